@@ -1,0 +1,69 @@
+// What the MTTKRP host code (mttkrp.hip) and the per-order kernel sources
+// (mttkrp_order.h, mttkrp_o<N>.hip) call of each other.
+#pragma once
+
+#include "internal.h"
+
+namespace tt {
+
+inline int grid_for(int64_t work, int block, int cap) {
+  int64_t g = (work + block - 1) / block;
+  if (g < 1) g = 1;
+  if (g > cap) g = cap;
+  return int(g);
+}
+
+// LDS capacities of the edge walk's node brackets (layout in mttkrp_order.h).
+constexpr int kUpperCap = 256;
+constexpr int kLeafCap = 1024;
+
+__host__ __device__ inline int32_t edge_leaf_cap(int32_t NB) {
+  return NB + 1 < kLeafCap ? NB + 1 : kLeafCap;
+}
+
+__host__ __device__ inline size_t edge_ep_bytes(int block, int lpr, int Rc) {
+  const size_t E = size_t(2) * (block / lpr);
+  return E * sizeof(int32_t) + E * size_t(Rc) * sizeof(float);
+}
+
+__host__ __device__ inline size_t edge_stage_ints(int order, int32_t NB) {
+  size_t n = size_t(2) * edge_leaf_cap(NB) + 1;  // level order-2
+  n += size_t(order - 2) * (2 * kUpperCap + 1);
+  return n;
+}
+
+__device__ __forceinline__ int32_t upper_index(const int64_t* __restrict__ off, int32_t n,
+                                               int64_t key) {
+  // largest t in [0, n) with off[t] <= key
+  int32_t lo = 0, hi = n - 1;
+  while (lo < hi) {
+    const int32_t mid = lo + ((hi - lo + 1) >> 1);
+    if (off[mid] <= key) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+
+// Defined per order N in mttkrp_o<N>.hip; the public launches of internal.h
+// pick the order.
+template <int N>
+int order_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A, int32_t a_rows,
+                 bool dense_root, const Variant& vr, void* ws, hipStream_t st);
+template <int N>
+int order_inner(const CsfDev& B, const LevelIndex& X, const FactorsDev& F, int level, int R,
+                float* A, int32_t a_rows, hipStream_t st);
+template <int N>
+int order_level(const CsfDev& B, const FactorsDev& F, int level, int R, float* A, int32_t a_rows,
+                hipStream_t st);
+template <int N>
+int order_batch(const BatchLaunch& L, hipStream_t st);
+template <int N>
+int order_batch_occupancy(int family, int block, int R, int32_t NB, int* per_cu);
+
+// Defined in mttkrp.hip: zero z_elems floats of Z and write the brackets of
+// nblk blocks of NB nonzeros; A = FP32(W) over n elements.
+int launch_edge_prep(const CsfDev& B, float* Z, int64_t z_elems, int32_t* brk, int32_t nblk,
+                     int32_t NB, hipStream_t st);
+int launch_narrow(const double* W, float* A, int64_t n, hipStream_t st);
+
+}  // namespace tt
