@@ -545,13 +545,7 @@ int auto_variant(const CsfStats& s, int order, int R) {
 }
 
 int lanes_per_row(int R) {
-  switch (R) {
-    case 16: return Lay<16>::LPR;
-    case 32: return Lay<32>::LPR;
-    case 64: return Lay<64>::LPR;
-    case 128: return Lay<128>::LPR;
-    default: return Lay<0>::LPR;
-  }
+  return with_rank_layout(R, [](auto r) { return Lay<r()>::LPR; });
 }
 
 int64_t nnz_per_block(const Variant& vr, int R) {
@@ -584,8 +578,8 @@ size_t mttkrp_workspace_bytes(const CsfDev& B, int R, const Variant& vr, int32_t
 int launch_mttkrp_inner(const CsfDev& B, const LevelIndex& X, const FactorsDev& F, int level,
                         int R, float* A, int32_t a_rows, hipStream_t st) {
   if (!X.built || X.level != level) return fail(TENTACO_EINVAL, "level %d index not built", level);
-  if (R <= 0 || R > Lay<0>::kMaxRank)
-    return fail(TENTACO_EUNSUPPORTED, "rank R=%d outside 1..%d", R, Lay<0>::kMaxRank);
+  if (R <= 0 || R > kMaxRankAny)
+    return fail(TENTACO_EUNSUPPORTED, "rank R=%d outside 1..%d", R, kMaxRankAny);
   switch (B.order) {
     case 3: return order_inner<3>(B, X, F, level, R, A, a_rows, st);
     case 4: return order_inner<4>(B, X, F, level, R, A, a_rows, st);
@@ -596,8 +590,8 @@ int launch_mttkrp_inner(const CsfDev& B, const LevelIndex& X, const FactorsDev& 
 
 int launch_mttkrp_level(const CsfDev& B, const FactorsDev& F, int level, int R, float* A,
                         int32_t a_rows, hipStream_t st) {
-  if (R <= 0 || R > Lay<0>::kMaxRank)
-    return fail(TENTACO_EUNSUPPORTED, "rank R=%d outside 1..%d", R, Lay<0>::kMaxRank);
+  if (R <= 0 || R > kMaxRankAny)
+    return fail(TENTACO_EUNSUPPORTED, "rank R=%d outside 1..%d", R, kMaxRankAny);
   switch (B.order) {
     case 2: return order_level<2>(B, F, level, R, A, a_rows, st);
     case 3: return order_level<3>(B, F, level, R, A, a_rows, st);
@@ -610,8 +604,8 @@ int launch_mttkrp_level(const CsfDev& B, const FactorsDev& F, int level, int R, 
 int launch_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A,
                   int32_t a_rows, bool dense_root, const Variant& vr, void* ws,
                   hipStream_t st) {
-  if (R <= 0 || R > Lay<0>::kMaxRank)
-    return fail(TENTACO_EUNSUPPORTED, "rank R=%d outside 1..%d", R, Lay<0>::kMaxRank);
+  if (R <= 0 || R > kMaxRankAny)
+    return fail(TENTACO_EUNSUPPORTED, "rank R=%d outside 1..%d", R, kMaxRankAny);
   if (vr.family < 0) return fail(TENTACO_EINVAL, "invalid variant");
   switch (B.order) {
     case 2: return order_mttkrp<2>(B, F, R, A, a_rows, dense_root, vr, ws, st);

@@ -62,7 +62,7 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
   const int32_t p0 = blk0 + gi * G;
   const int32_t p1 = min(p0 + G, blk1);
   const bool active = p0 < p1;
-  const int Rc = (R == 0) ? Rr : R;
+  const int Rc = (R <= 0) ? Rr : R;
 
   // ---- stage the node brackets in LDS
   int32_t lo[NL], hib[NL];
@@ -353,9 +353,11 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
     auto put = [&](int e, const V (&x)[NV]) {
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
-        const int k = RO::col(j, c);
+        const int k = RO::col(j, c, Rr);
         if constexpr (R == 0) {
           if (k < Rc) ev[size_t(e) * Rc + k] = x[j];
+        } else if constexpr (R < 0) {
+          store4(ev + size_t(e) * Rc + k, x[j]);
         } else {
           *reinterpret_cast<float4*>(ev + size_t(e) * Rc + k) = x[j];
         }
@@ -364,9 +366,11 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
     auto get = [&](int e, V (&x)[NV]) {
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
-        const int k = RO::col(j, c);
+        const int k = RO::col(j, c, Rr);
         if constexpr (R == 0) {
           x[j] = (k < Rc) ? ev[size_t(e) * Rc + k] : 0.f;
+        } else if constexpr (R < 0) {
+          x[j] = load4(ev + size_t(e) * Rc + k);
         } else {
           x[j] = *reinterpret_cast<const float4*>(ev + size_t(e) * Rc + k);
         }
@@ -631,34 +635,15 @@ __global__ __launch_bounds__(256) void inner_kernel(const int32_t* __restrict__ 
     if (gi == 0) RO::store(A, j, c, Rr, acc);
     return;
   }
-  const int Rc = (R == 0) ? Rr : R;
   if (gi == 0) {
-#pragma unroll
-    for (int q = 0; q < NV; ++q) {
-      const int k = RO::col(q, c);
-      if constexpr (R == 0) {
-        if (k < Rc) red[wv][k] = acc[q];
-      } else {
-        *reinterpret_cast<float4*>(&red[wv][k]) = acc[q];
-      }
-    }
+    RO::put(red[wv], c, acc);
   }
   __syncthreads();
   if (wv == 0 && gi == 0) {
     for (int w = 1; w < nwv; ++w) {
-#pragma unroll
-      for (int q = 0; q < NV; ++q) {
-        const int k = RO::col(q, c);
-        if constexpr (R == 0) {
-          if (k < Rc) acc[q] += red[w][k];
-        } else {
-          const float4 o = *reinterpret_cast<const float4*>(&red[w][k]);
-          acc[q].x += o.x;
-          acc[q].y += o.y;
-          acc[q].z += o.z;
-          acc[q].w += o.w;
-        }
-      }
+      V o[NV];
+      RO::get(red[w], c, o);
+      RO::add(acc, o);
     }
     RO::store(A, j, c, Rr, acc);
   }
@@ -848,34 +833,15 @@ __global__ __launch_bounds__(512) void slice_kernel(CsfDev B, FactorsDev F,
     if (gi == 0) RO::store(A, B.crd0[x], c, Rr, acc);
     return;
   }
-  const int Rc = (R == 0) ? Rr : R;
   if (gi == 0) {
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      const int k = RO::col(j, c);
-      if constexpr (R == 0) {
-        if (k < Rc) red[wv][k] = acc[j];
-      } else {
-        *reinterpret_cast<float4*>(&red[wv][k]) = acc[j];
-      }
-    }
+    RO::put(red[wv], c, acc);
   }
   __syncthreads();
   if (wv == 0 && gi == 0) {
     for (int w = 1; w < nwv; ++w) {
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        const int k = RO::col(j, c);
-        if constexpr (R == 0) {
-          if (k < Rc) acc[j] += red[w][k];
-        } else {
-          const float4 o = *reinterpret_cast<const float4*>(&red[w][k]);
-          acc[j].x += o.x;
-          acc[j].y += o.y;
-          acc[j].z += o.z;
-          acc[j].w += o.w;
-        }
-      }
+      V o[NV];
+      RO::get(red[w], c, o);
+      RO::add(acc, o);
     }
     RO::store(A, B.crd0[x], c, Rr, acc);
   }
@@ -908,20 +874,14 @@ __global__ __launch_bounds__(512) void slice_short_kernel(CsfDev B, FactorsDev F
     return;
   }
   if (gi == 0) {
-#pragma unroll
-    for (int j = 0; j < NV; ++j) *reinterpret_cast<float4*>(&red[wv][RO::col(j, c)]) = acc[j];
+    RO::put(red[wv], c, acc);
   }
   __syncthreads();
   if (wv == 0 && gi == 0) {
     for (int w = 1; w < nwv; ++w) {
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        const float4 o = *reinterpret_cast<const float4*>(&red[w][RO::col(j, c)]);
-        acc[j].x += o.x;
-        acc[j].y += o.y;
-        acc[j].z += o.z;
-        acc[j].w += o.w;
-      }
+      V o[NV];
+      RO::get(red[w], c, o);
+      RO::add(acc, o);
     }
     RO::store(A, B.crd0[x], c, Rr, acc);
   }
@@ -986,7 +946,7 @@ __global__ __launch_bounds__(64 * NW) void slice_pad_kernel(CsfDev B, FactorsDev
       const uint32_t od = real ? (kl0 & 0xFFFFu) * uint32_t(R * 4) : 0x80000000u;
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
-        const uint32_t cj = uint32_t(RO::col(j, c) * 4);
+        const uint32_t cj = uint32_t(RO::slot(j, c) * 4);
         cr[u][j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(crs, oc + cj, 0, 0));
         dr[u][j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(drs, od + cj, 0, 0));
       }
@@ -1017,21 +977,15 @@ __global__ __launch_bounds__(64 * NW) void slice_pad_kernel(CsfDev B, FactorsDev
     return;
   }
   if (gi == 0) {
-#pragma unroll
-    for (int j = 0; j < NV; ++j) *reinterpret_cast<float4*>(&red[wv][RO::col(j, c)]) = acc[j];
+    RO::put(red[wv], c, acc);
   }
   __syncthreads();
   if (wv == 0 && gi == 0) {
 #pragma unroll
     for (int w = 1; w < nwv; ++w) {
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        const float4 o = *reinterpret_cast<const float4*>(&red[w][RO::col(j, c)]);
-        acc[j].x += o.x;
-        acc[j].y += o.y;
-        acc[j].z += o.z;
-        acc[j].w += o.w;
-      }
+      V o[NV];
+      RO::get(red[w], c, o);
+      RO::add(acc, o);
     }
     RO::store(A, row, c, Rr, acc);
   }
@@ -1093,7 +1047,7 @@ __global__ __launch_bounds__(128) void slice_pair_kernel(const uint2* __restrict
       const uint32_t od = real ? (kl & 0xFFFFu) * uint32_t(R * 4) : 0x80000000u;
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
-        const uint32_t cj = uint32_t(RO::col(j, c) * 4);
+        const uint32_t cj = uint32_t(RO::slot(j, c) * 4);
         cr[u][j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(crs, oc + cj, 0, 0));
         dr[u][j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(drs, od + cj, 0, 0));
       }
@@ -1117,8 +1071,8 @@ __global__ __launch_bounds__(128) void slice_pair_kernel(const uint2* __restrict
   if (gi == 0) {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-      *reinterpret_cast<float4*>(&red[wv][0][RO::col(j, c)]) = aa[j];
-      *reinterpret_cast<float4*>(&red[wv][1][RO::col(j, c)]) = ab[j];
+      *reinterpret_cast<float4*>(&red[wv][0][RO::slot(j, c)]) = aa[j];
+      *reinterpret_cast<float4*>(&red[wv][1][RO::slot(j, c)]) = ab[j];
     }
   }
   __syncthreads();
@@ -1127,8 +1081,8 @@ __global__ __launch_bounds__(128) void slice_pair_kernel(const uint2* __restrict
     V t[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-      const float4 o0 = *reinterpret_cast<const float4*>(&red[0][wv][RO::col(j, c)]);
-      const float4 o1 = *reinterpret_cast<const float4*>(&red[1][wv][RO::col(j, c)]);
+      const float4 o0 = *reinterpret_cast<const float4*>(&red[0][wv][RO::slot(j, c)]);
+      const float4 o1 = *reinterpret_cast<const float4*>(&red[1][wv][RO::slot(j, c)]);
       t[j] = make_float4(o0.x + o1.x, o0.y + o1.y, o0.z + o1.z, o0.w + o1.w);
     }
     const int32_t row = wv == 0 ? inf.x : inf.y;
@@ -1221,7 +1175,7 @@ int launch_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A,
     }
     if (B.nodes[0] > 0) {
       ktimer_begin(st);
-      if constexpr (N == 3 && R != 0) {
+      if constexpr (N == 3 && R > 0) {
         // short fibres (nnz <= 1.25 x fibres) with the expansion built: the
         // kernel that skips the pos -> crd chain
         if (B.crd1_of_nnz && int64_t(B.nnz) * 4 <= int64_t(B.nodes[1]) * 5) {
@@ -1377,35 +1331,23 @@ int launch_level_order(const CsfDev& B, const FactorsDev& F, int level, int Rr, 
 template <int N>
 int order_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A, int32_t a_rows,
                  bool dense_root, const Variant& vr, void* ws, hipStream_t st) {
-  switch (R) {
-    case 16: return launch_typed<N, 16>(B, F, R, A, a_rows, dense_root, vr, ws, st);
-    case 32: return launch_typed<N, 32>(B, F, R, A, a_rows, dense_root, vr, ws, st);
-    case 64: return launch_typed<N, 64>(B, F, R, A, a_rows, dense_root, vr, ws, st);
-    case 128: return launch_typed<N, 128>(B, F, R, A, a_rows, dense_root, vr, ws, st);
-    default: return launch_typed<N, 0>(B, F, R, A, a_rows, dense_root, vr, ws, st);
-  }
+  return with_rank_layout(R, [&](auto r) {
+    return launch_typed<N, r()>(B, F, R, A, a_rows, dense_root, vr, ws, st);
+  });
 }
 
 template <int N>
 int order_inner(const CsfDev& B, const LevelIndex& X, const FactorsDev& F, int level, int R,
                 float* A, int32_t a_rows, hipStream_t st) {
-  switch (R) {
-    case 16: return launch_inner_order<N, 16>(B, X, F, level, R, A, a_rows, st);
-    case 32: return launch_inner_order<N, 32>(B, X, F, level, R, A, a_rows, st);
-    case 64: return launch_inner_order<N, 64>(B, X, F, level, R, A, a_rows, st);
-    default: return launch_inner_order<N, 0>(B, X, F, level, R, A, a_rows, st);
-  }
+  return with_rank_layout(
+      R, [&](auto r) { return launch_inner_order<N, r()>(B, X, F, level, R, A, a_rows, st); });
 }
 
 template <int N>
 int order_level(const CsfDev& B, const FactorsDev& F, int level, int R, float* A, int32_t a_rows,
                 hipStream_t st) {
-  switch (R) {
-    case 16: return launch_level_order<N, 16>(B, F, level, R, A, a_rows, st);
-    case 32: return launch_level_order<N, 32>(B, F, level, R, A, a_rows, st);
-    case 64: return launch_level_order<N, 64>(B, F, level, R, A, a_rows, st);
-    default: return launch_level_order<N, 0>(B, F, level, R, A, a_rows, st);
-  }
+  return with_rank_layout(
+      R, [&](auto r) { return launch_level_order<N, r()>(B, F, level, R, A, a_rows, st); });
 }
 
 template <int N>

@@ -160,34 +160,15 @@ __global__ __launch_bounds__(256) void tleaf_kernel(const int32_t* __restrict__ 
     if (gi == 0) RO::store(A, j, c, Rr, acc);
     return;
   }
-  const int Rc = (R == 0) ? Rr : R;
   if (gi == 0) {
-#pragma unroll
-    for (int q = 0; q < NV; ++q) {
-      const int k = RO::col(q, c);
-      if constexpr (R == 0) {
-        if (k < Rc) red[wv][k] = acc[q];
-      } else {
-        *reinterpret_cast<float4*>(&red[wv][k]) = acc[q];
-      }
-    }
+    RO::put(red[wv], c, acc);
   }
   __syncthreads();
   if (wv == 0 && gi == 0) {
     for (int w = 1; w < nwv; ++w) {
-#pragma unroll
-      for (int q = 0; q < NV; ++q) {
-        const int k = RO::col(q, c);
-        if constexpr (R == 0) {
-          if (k < Rc) acc[q] += red[w][k];
-        } else {
-          const float4 o = *reinterpret_cast<const float4*>(&red[w][k]);
-          acc[q].x += o.x;
-          acc[q].y += o.y;
-          acc[q].z += o.z;
-          acc[q].w += o.w;
-        }
-      }
+      V o[NV];
+      RO::get(red[w], c, o);
+      RO::add(acc, o);
     }
     RO::store(A, j, c, Rr, acc);
   }
@@ -317,15 +298,10 @@ int launch_mttkrp_leaf(const CsfDev& B, const LevelIndex& X, const FactorsDev& F
                        int32_t a_rows, hipStream_t st) {
   if (!X.built || X.level != B.order - 1 || !X.ent)
     return fail(TENTACO_EINVAL, "leaf index not built");
-  if (R <= 0 || R > Lay<0>::kMaxRank)
-    return fail(TENTACO_EUNSUPPORTED, "rank R=%d outside 1..%d", R, Lay<0>::kMaxRank);
-  switch (R) {
-    case 16: return launch_tleaf_rank<16>(B, X, F, R, A, a_rows, st);
-    case 32: return launch_tleaf_rank<32>(B, X, F, R, A, a_rows, st);
-    case 64: return launch_tleaf_rank<64>(B, X, F, R, A, a_rows, st);
-    case 128: return launch_tleaf_rank<128>(B, X, F, R, A, a_rows, st);
-    default: return launch_tleaf_rank<0>(B, X, F, R, A, a_rows, st);
-  }
+  if (R <= 0 || R > kMaxRankAny)
+    return fail(TENTACO_EUNSUPPORTED, "rank R=%d outside 1..%d", R, kMaxRankAny);
+  return with_rank_layout(
+      R, [&](auto r) { return launch_tleaf_rank<r()>(B, X, F, R, A, a_rows, st); });
 }
 
 }  // namespace tt
