@@ -552,14 +552,18 @@ int64_t nnz_per_block(const Variant& vr, int R) {
   return int64_t(vr.block / lanes_per_row(R)) * vr.group;
 }
 
+bool edge_tile_fits(int order, int R, const Variant& vr) {
+  constexpr int kUpperNodes = 256, kLeafNodes = 1024;
+  const int64_t leaf = std::min<int64_t>(nnz_per_block(vr, R) + 1, kLeafNodes);
+  const int64_t brackets = 4 * (2 * leaf + 1 + int64_t(order - 2) * (2 * kUpperNodes + 1));
+  const int64_t rows = 2 * (vr.block / lanes_per_row(R));
+  return brackets + (vr.family == kEdgeParallel ? rows * 4 * (R + 1) : 0) <= 65536;
+}
+
 bool variant_fits(int order, int R, int v) {
   const Variant vr = variant_of(v);
   if (vr.family < 0 || R <= 0) return false;
-  if (vr.family == kSliceRow) return true;
-  const int64_t NB = nnz_per_block(vr, R);
-  const size_t stage = edge_stage_ints(order, int32_t(NB)) * sizeof(int32_t);
-  if (vr.family == kEdgeSerial) return stage <= 65536;
-  return edge_ep_bytes(vr.block, lanes_per_row(R), R) + stage <= 65536;
+  return vr.family == kSliceRow || edge_tile_fits(order, R, vr);
 }
 
 size_t edge_brk_bytes(const CsfDev& B, int64_t NB) {

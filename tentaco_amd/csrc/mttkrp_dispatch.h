@@ -13,24 +13,11 @@ inline int grid_for(int64_t work, int block, int cap) {
   return int(g);
 }
 
-// LDS capacities of the edge walk's node brackets (layout in mttkrp_order.h).
-constexpr int kUpperCap = 256;
-constexpr int kLeafCap = 1024;
-
-__host__ __device__ inline int32_t edge_leaf_cap(int32_t NB) {
-  return NB + 1 < kLeafCap ? NB + 1 : kLeafCap;
-}
-
-__host__ __device__ inline size_t edge_ep_bytes(int block, int lpr, int Rc) {
-  const size_t E = size_t(2) * (block / lpr);
-  return E * sizeof(int32_t) + E * size_t(Rc) * sizeof(float);
-}
-
-__host__ __device__ inline size_t edge_stage_ints(int order, int32_t NB) {
-  size_t n = size_t(2) * edge_leaf_cap(NB) + 1;  // level order-2
-  n += size_t(order - 2) * (2 * kUpperCap + 1);
-  return n;
-}
+// Whether the variant table offers an edge tile at this order and rank: the
+// table's limit is 64 KB of node brackets and, for the edge-parallel family,
+// of two rows per row group (what a tile of that size once staged in LDS).
+// The walk itself needs less and takes every tile.
+bool edge_tile_fits(int order, int R, const Variant& vr);
 
 __device__ __forceinline__ int32_t upper_index(const int64_t* __restrict__ off, int32_t n,
                                                int64_t key) {

@@ -19,402 +19,410 @@ namespace {
 // (nonzeros [b*NB, (b+1)*NB)); shared by the per-tensor kernel and the
 // persistent batch kernel.
 //
-// LDS layout (dynamic, `smem`): the EP reduction area (edge_ep_bytes), then
-// for each walk level k = 0..N-2 the node bounds pos[k+1][lo..hi+1] and the
-// node coordinates crd[k][lo..hi] of the workgroup's bracket [lo, hi]. The
-// level above the nonzeros (k = N-2) gets room for min(NB+1, kLeafCap)
-// nodes (NB+1 is the most a CSF built from coordinates can have there); the
-// upper levels get kUpperCap. A level whose bracket does not fit is read
-// from global memory instead, so large brackets and runs of empty nodes cost
-// time, never correctness.
-// The edge-serial family (EP false) needs W (the edge-parallel family
-// ignores it): every row output goes to the FP64 buffer W instead of A.
-// Slices complete inside a group are stored; the
-// groups' first and last slices are combined across the wave's groups by a
-// segmented suffix scan over shuffles, and each slice's sum per wave is
-// added with one FP64 atomic. A giant slice then takes one atomic per wave,
-// without FP32 rounding at each add.
-// A device pointer the kernel knows to be global memory (loads through it
-// are global loads, never flat ones).
-__device__ __forceinline__ const __attribute__((address_space(1))) int32_t* as_global(
-    const int32_t* p) {
-  return reinterpret_cast<const __attribute__((address_space(1))) int32_t*>(
-      reinterpret_cast<uintptr_t>(p));
+// Every wave owns a contiguous run of NGW*G nonzeros (NGW row groups) and
+// walks it in chunks of up to 64, one nonzero per lane. A chunk's leaf pairs
+// and, per level, the next 64 node bounds and coordinates arrive in coalesced
+// loads one chunk ahead. A lane's node at a level is the chunk's first node
+// plus the number of later nodes that start at or before its child: a
+// histogram of the starts over the chunk's children and a lane scan, so no
+// lane searches or branches on its own. The chunk then splits into pieces of
+// one slice and at most PF fibres (a whole chunk where slices are long). For
+// a piece, the product of the upper levels' rows is formed once per fibre and
+// kept in LDS (P); the row groups take the piece's nonzeros in turn, each
+// step one leaf row by a global load and one P row from LDS:
+//   acc += (val * P(fibre, :)) (.) M_{N-1}(l, :).
+// Slice changes are uniform over the wave: the row groups' accumulators are
+// summed over the wave and the row is stored.
+//
+// The serial walk it replaces gave every row group a run of its own and
+// closed fibres per group; some group of a wave closed one on most steps, and
+// the closing's instructions bound it where the factors fit L2, and drained
+// the row gathers in flight where they do not. Per call, before and after:
+// 2M nonzeros, 3-mode, rank 32 (10007 x 20011 x 5003) 61 and 45 us; 100M,
+// 3-mode, rank 32 (500k^3) 2281 and 2099 us (of 1960 us at the random-row rate
+// of a 64 MB factor); 60M, 4-mode, rank 64 (200k^4) 2845 and 2415 us; 5M at
+// rank 50 229 and 165 us. What is left where the factors fit L2 is the
+// latency of a chunk's dependent steps and about 4 vector instructions a
+// nonzero.
+//
+// LDS per wave (edge_wave_lds bytes): a record per nonzero of the chunk
+// (leaf row, value, fibre), the histogram, P, and the wave's first slice's
+// row; the block's combine reuses P and the histogram.
+constexpr int kRecBytes = 64 * 16;
+constexpr int kHistBytes = 64 * 4;
+constexpr int kFibBytes = 4096;
+
+template <int R>
+constexpr size_t edge_wave_lds() {
+  return kRecBytes + kHistBytes + kFibBytes + Lay<R>::kMaxRank * sizeof(float);
+}
+
+// The pointer as one to global memory. In the batch kernel the pointers come
+// from the task table in memory; loads through them would be flat loads,
+// whose waits also drain the LDS reads in flight.
+template <class T>
+__device__ __forceinline__ T* global_ptr(T* p) {
+  typedef __attribute__((address_space(1))) T* G;
+  return (T*)reinterpret_cast<G>(reinterpret_cast<uintptr_t>(p));
+}
+
+// Orders the wave's LDS accesses: what its lanes wrote before is read after.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Inclusive sum over the lanes up to this one (DPP row shifts, then the rows'
+// last lanes broadcast to the next rows).
+__device__ __forceinline__ int32_t wave_scan_add(int32_t x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+  return x;
+}
+
+// Largest x in [lo, hi] with a[x] <= key (requires a[lo] <= key), 64 probes a
+// step, uniform over the wave.
+__device__ __forceinline__ int32_t wave_search_le(const int32_t* __restrict__ a, int32_t lo,
+                                                  int32_t hi, int32_t key, int lane) {
+  while (lo < hi) {
+    const uint32_t n = uint32_t(hi - lo);
+    const uint32_t step = (n + 63u) >> 6;
+    const uint32_t off = uint32_t(lane + 1) * step;
+    const bool le = off <= n && a[lo + int32_t(off <= n ? off : n)] <= key;
+    const uint32_t cnt = uint32_t(__popcll(__ballot(le)));
+    const uint32_t next = cnt * step;
+    hi = lo + int32_t(min(n, next + step - 1u));
+    lo += int32_t(next);
+  }
+  return lo;
 }
 
 template <int N, int R, bool EP>
-__device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
-                                           float* __restrict__ A, int Rr,
-                                           const int32_t* __restrict__ brk, int32_t b,
-                                           int32_t G, int32_t NB, unsigned char* smem,
-                                           double* __restrict__ W) {
+__device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F, float* out_a,
+                                           int Rr, const int32_t* brk_p, int32_t b, int32_t G,
+                                           int32_t NB, unsigned char* smem, double* out_w) {
   using RO = Row<R>;
   using V = typename RO::V;
   constexpr int NV = RO::NV;
   constexpr int LPR = RO::LPR;
-  constexpr int NL = N - 1;  // levels 0..N-2 carry walk state
+  constexpr int KR = Lay<R>::kMaxRank;
+  constexpr int NGW = 64 / LPR;             // row groups of a wave
+  constexpr int NL = N - 1;                 // levels 0..N-2 hold nodes
+  constexpr int FL = N - 2;                 // the nonzeros' parents (fibres)
+  constexpr int PF0 = kFibBytes / (KR * 4); // fibres whose product rows fit P
+  constexpr int PF = PF0 < 64 ? PF0 : 64;
+  // leaf rows in flight per row group, at most 32 VGPRs of them
+  constexpr int SB = NV >= 4 ? 2 : NV == 2 ? 4 : LPR < 8 ? LPR : 8;
+  float* __restrict__ A = global_ptr(out_a);
+  double* __restrict__ W = global_ptr(out_w);
+  const int32_t* __restrict__ brk = global_ptr(brk_p);
 
-  const int gi = threadIdx.x / LPR;
-  const int c = threadIdx.x % LPR;
-  const int32_t nnz = B.nnz;
+  const int lane = int(threadIdx.x) & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int nwv = int(blockDim.x) >> 6;
+  const int gi = lane / LPR;
+  const int c = lane % LPR;
+  auto wave_mem = [&](int w) { return smem + size_t(w) * edge_wave_lds<R>(); };
+  int4* rec = reinterpret_cast<int4*>(wave_mem(wv));
+  int32_t* hist = reinterpret_cast<int32_t*>(wave_mem(wv) + kRecBytes);
+  float* P = reinterpret_cast<float*>(wave_mem(wv) + kRecBytes + kHistBytes);
+  float* head_row = P + kFibBytes / 4;
+
+  // the wave's run [w0, w1)
   const int32_t blk0 = b * NB;
-  const int32_t blk1 = min(blk0 + NB, nnz);
-  const int32_t p0 = blk0 + gi * G;
-  const int32_t p1 = min(p0 + G, blk1);
-  const bool active = p0 < p1;
-  const int Rc = (R <= 0) ? Rr : R;
+  const int32_t len = min(NB, B.nnz - blk0);
+  const int32_t off = wv * (NGW * G);
+  const bool active = off < len;
+  const int32_t w0 = blk0 + off;
+  const int32_t w1 = active ? w0 + min(NGW * G, len - off) : w0;
 
-  // ---- stage the node brackets in LDS
-  int32_t lo[NL], hib[NL];
-  bool staged[NL];
-  int32_t* spos[NL];
-  int32_t* scrd[NL];
-  {
-    int32_t* base = reinterpret_cast<int32_t*>(
-        smem + (EP ? edge_ep_bytes(blockDim.x, LPR, Rc) : size_t(0)));
+  V acc[NV];
+  RO::zero(acc);
+  int32_t head = INT_MAX, open = INT_MAX;
+  bool head_closed = false;
+
+  if (active) {
+    const int32_t* __restrict__ lcrd = global_ptr(B.crd[N - 1]);
+    const float* __restrict__ vals = global_ptr(B.vals);
+    const float* __restrict__ Mleaf = global_ptr(F.M[N - 1]);
+    // per level: its nodes' child ranges, their coordinates and factor
+    const int32_t* __restrict__ pos[NL];
+    const int32_t* __restrict__ crd[NL];
+    const float* __restrict__ M[NL];
 #pragma unroll
-    for (int k = NL - 1; k >= 0; --k) {
-      const int32_t cap = (k == NL - 1) ? edge_leaf_cap(NB) : kUpperCap;
-      lo[k] = brk[b * NL + k];
-      hib[k] = brk[(b + 1) * NL + k];
-      staged[k] = hib[k] - lo[k] + 1 <= cap;
-      spos[k] = base;
-      scrd[k] = base + cap + 1;
-      base += 2 * cap + 1;
-      if (staged[k]) {
-        const int32_t* pk = B.pos[k + 1];
-        const int32_t* ck = (k == 0) ? B.crd0 : B.crd[k];
-        const int32_t n = hib[k] - lo[k] + 1;
-        for (int32_t j = threadIdx.x; j <= n; j += blockDim.x) {
-          spos[k][j] = pk[lo[k] + j];
-          if (j < n) scrd[k][j] = ck[lo[k] + j];
+    for (int k = 0; k < NL; ++k) {
+      pos[k] = global_ptr(B.pos[k + 1]);
+      crd[k] = global_ptr(k == 0 ? B.crd0 : B.crd[k]);
+      M[k] = global_ptr(F.M[k]);
+    }
+    // cur[k]: the node at level k that holds the chunk's first nonzero
+    int32_t cur[NL];
+    {
+      int32_t key = w0;
+#pragma unroll
+      for (int k = FL; k >= 0; --k) {
+        const int32_t lo = brk[b * NL + k];
+        const int32_t hi = wv == 0 ? lo : brk[(b + 1) * NL + k];
+        cur[k] = wave_search_le(pos[k], lo, hi, key, lane);
+        key = cur[k];
+      }
+    }
+    head = open = cur[0];
+
+    // The windows of a chunk: wp[k] lane j = where node cur[k]+1+j starts
+    // among the level's children (the level's total past its last node),
+    // wc[k] lane j = coordinate of node cur[k]+j.
+    int32_t wp[NL], wc[NL];
+    auto window = [&](int k, int32_t x, int32_t& p, int32_t& cc) {
+      p = pos[k][min(x + 1 + lane, B.nodes[k])];
+      cc = crd[k][min(x + lane, B.nodes[k] - 1)];
+    };
+    auto pairs = [&](int32_t q, int32_t& l, float& v) {
+      const int32_t t = min(q + lane, w1 - 1);
+      l = lcrd[t];
+      v = vals[t];
+    };
+    // lane x: how many of the starts p (ascending over the lanes) are <= base + x
+    auto rank = [&](int32_t p, int32_t base) -> int32_t {
+      const uint32_t s = uint32_t(p - base);
+      hist[lane] = 0;
+      wave_lds_sync();
+      if (s < 64u) atomicAdd(&hist[s], 1);
+      wave_lds_sync();
+      const int32_t n = hist[lane];
+      wave_lds_sync();
+      return wave_scan_add(n);
+    };
+    auto lane_of = [&](int32_t x, int32_t src) { return __builtin_amdgcn_readlane(x, src); };
+
+    int32_t open_row = 0;
+    auto close_slice = [&]() {
+      RO::wave_sum(acc);
+      if (open == head && !head_closed) {
+        head_closed = true;
+        if (gi == 0) RO::put(head_row, c, acc);
+      } else if (gi == 0) {
+        if constexpr (EP) RO::store(A, open_row, c, Rr, acc);
+        else RO::store_f64(W, open_row, c, Rr, acc);
+      }
+      RO::zero(acc);
+    };
+
+    int32_t l, lnext = 0;
+    float v, vnext = 0.f;
+    pairs(w0, l, v);
+#pragma unroll
+    for (int k = 0; k < NL; ++k) window(k, cur[k], wp[k], wc[k]);
+
+    for (int32_t q = w0; q < w1;) {
+      // move past nodes that end at or before the chunk's first child (empty
+      // nodes, or a window the last chunk used up)
+#pragma unroll
+      for (int k = FL; k >= 0; --k) {
+        const int32_t key = k == FL ? q : cur[k + 1];
+        const int past = __popcll(__ballot(wp[k] <= key));
+        if (past) {
+          cur[k] += past;
+          if (past == 64)
+            cur[k] = wave_search_le(pos[k], cur[k], B.nodes[k] - 1, key, lane);
+          window(k, cur[k], wp[k], wc[k]);
         }
       }
+      // the chunk ends where a level's window does
+      int32_t n = 64;
+#pragma unroll
+      for (int k = 0; k < NL; ++k) {
+        const int32_t key = k == FL ? q : cur[k + 1];
+        n = min(64, lane_of(wp[k], n - 1) - key);
+      }
+      n = min(n, w1 - q);
+      // local node of every child, bottom up; then the fibres' ancestors
+      int32_t loc[NL];  // loc[k] lane x: node of child x of the chunk
+      int32_t cnt[NL];  // nodes of the chunk
+#pragma unroll
+      for (int k = FL; k >= 0; --k) {
+        const int32_t key = k == FL ? q : cur[k + 1];
+        const int32_t m = k == FL ? n : cnt[k + 1];
+        loc[k] = 0;
+        if (lane_of(wp[k], 0) < key + m) loc[k] = rank(wp[k], key);
+        cnt[k] = lane_of(loc[k], m - 1) + 1;
+      }
+      int32_t fc[NL];      // fc[k] lane f: coordinate at level k above fibre f
+      int32_t root = loc[0];  // lane f: root node of fibre f (of nonzero f for N = 2)
+      {
+        int32_t an = lane;
+        fc[FL] = wc[FL];
+#pragma unroll
+        for (int k = FL - 1; k >= 0; --k) {
+          an = k == FL - 1 ? loc[k] : __shfl(loc[k], an);
+          fc[k] = __shfl(wc[k], an);
+        }
+        if constexpr (N > 2) root = an;
+      }
+      rec[lane] = make_int4(l, __float_as_int(v), loc[FL], 0);
+      wave_lds_sync();
+      // the next chunk's loads
+      const int32_t qn = q + n;
+      int32_t curn[NL], wpn[NL], wcn[NL];
+      if (qn < w1) {
+        pairs(qn, lnext, vnext);
+#pragma unroll
+        for (int k = FL; k >= 0; --k) {
+          const int32_t key = k == FL ? qn : curn[k + 1];
+          curn[k] = cur[k] + __popcll(__ballot(wp[k] <= key));
+          window(k, curn[k], wpn[k], wcn[k]);
+        }
+      }
+      // pieces: nonzeros [a, e) of one slice in fibres [fa, fe)
+      const int32_t nf = N > 2 ? cnt[FL] : n;
+      for (int32_t a = 0, fa = 0; a < n;) {
+        const int32_t r = lane_of(root, fa);
+        const int32_t fe =
+            fa + __popcll(__ballot(lane >= fa && lane < min(nf, N > 2 ? fa + PF : 64) && root == r));
+        const int32_t e = N == 2 ? fe : (fe >= nf ? n : lane_of(wp[FL], fe - 1) - q);
+        if (cur[0] + r != open) {
+          close_slice();
+          open = cur[0] + r;
+        }
+        open_row = lane_of(wc[0], r);
+        bool staged = N == 2;
+        auto stage = [&]() {
+          constexpr int U = NV >= 4 ? 1 : 2;
+          for (int32_t f0 = fa; f0 < fe; f0 += U * NGW) {
+            V p[U][NV];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              const int32_t f = min(f0 + u * NGW + gi, fe - 1);
+              RO::load(p[u], M[FL], __shfl(fc[FL], f), c, Rr);
+#pragma unroll
+              for (int k = FL - 1; k >= 1; --k) {
+                V m[NV];
+                RO::load(m, M[k], __shfl(fc[k], f), c, Rr);
+                RO::hmul(p[u], m);
+              }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              const int32_t f = f0 + u * NGW + gi;
+              if (f < fe) RO::put(P + (f - fa) * KR, c, p[u]);
+            }
+          }
+          wave_lds_sync();
+        };
+        auto steps = [&](auto S, int32_t t0) {
+          V d[S()][NV];
+          float w[S()];
+          int32_t slot[S()];
+#pragma unroll
+          for (int u = 0; u < S(); ++u) {
+            const int32_t t = t0 + u * NGW + gi;
+            const int4 x = rec[min(t, e - 1)];
+            w[u] = t < e ? __int_as_float(x.y) : 0.f;
+            slot[u] = x.z - fa;
+            RO::load(d[u], Mleaf, x.x, c, Rr);
+          }
+          if constexpr (N > 2) {
+            if (!staged) stage();
+            staged = true;
+          }
+#pragma unroll
+          for (int u = 0; u < S(); ++u) {
+            if constexpr (N > 2) {
+              V p[NV], s[NV];
+              RO::get(P + slot[u] * KR, c, p);
+              RO::zero(s);
+              RO::axpy(s, w[u], p);
+              RO::hfma(acc, s, d[u]);
+            } else {
+              RO::axpy(acc, w[u], d[u]);
+            }
+          }
+        };
+        for (int32_t t0 = a; t0 < e;) {
+          if (SB == 8 && e - t0 > 4 * NGW) {
+            steps(std::integral_constant<int, SB>(), t0);
+            t0 += SB * NGW;
+          } else if (SB >= 4 && e - t0 > 2 * NGW) {
+            steps(std::integral_constant<int, SB < 4 ? SB : 4>(), t0);
+            t0 += 4 * NGW;
+          } else {
+            steps(std::integral_constant<int, 2>(), t0);
+            t0 += 2 * NGW;
+          }
+        }
+        wave_lds_sync();
+        a = e;
+        fa = fe;
+      }
+      q = qn;
+      l = lnext;
+      v = vnext;
+#pragma unroll
+      for (int k = 0; k < NL; ++k) {
+        cur[k] = curn[k];
+        wp[k] = wpn[k];
+        wc[k] = wcn[k];
+      }
+    }
+    RO::wave_sum(acc);
+  }
+
+  // The workgroup's slices: two entries per wave (its first slice, complete
+  // or 0 where it is still open; the slice open at the run's end), keys in
+  // ascending order. Every column sums runs of equal keys in FP64; only the
+  // workgroup's first and last slice can be shared with another workgroup.
+  if (gi == 0) {
+    V h[NV];
+    RO::zero(h);
+    if (head_closed) RO::get(head_row, c, h);
+    RO::put(P, c, h);
+    RO::put(P + KR, c, acc);
+    if (c == 0) {
+      hist[0] = head;
+      hist[1] = open;
     }
   }
   __syncthreads();
-  // An LDS read when the level's brackets are staged, a global read
-  // otherwise, as two loads of their own: one load through a pointer that
-  // may be either would be a flat load, whose wait also drains every global
-  // load in flight (the walk's row gathers). The global read is waited for
-  // on its own path (the empty asm uses its value), so a use after the two
-  // paths join waits only for the LDS read, not for the rows in flight.
-  auto POS = [&](int k, int32_t x) -> int32_t {
-    if (staged[k]) return spos[k][x - lo[k]];
-    const int32_t v = as_global(B.pos[k + 1])[x];
-    asm volatile("" ::"v"(v));
-    return v;
+  auto key_of = [&](int en) {
+    return reinterpret_cast<const int32_t*>(wave_mem(en >> 1) + kRecBytes)[en & 1];
   };
-  auto CRD = [&](int k, int32_t x) -> int32_t {
-    if (staged[k]) return scrd[k][x - lo[k]];
-    const int32_t v = as_global((k == 0) ? B.crd0 : B.crd[k])[x];
-    asm volatile("" ::"v"(v));
-    return v;
+  auto row_of = [&](int en) {
+    return reinterpret_cast<const float*>(wave_mem(en >> 1) + kRecBytes + kHistBytes) +
+           (en & 1) * KR;
   };
-  auto SEARCH = [&](int k, int32_t a, int32_t z, int32_t key) {
-    // largest x in [a, z] with POS(k, x) <= key (requires POS(k, a) <= key)
-    while (a < z) {
-      const int32_t mid = a + ((z - a + 1) >> 1);
-      if (POS(k, mid) <= key) a = mid;
-      else z = mid - 1;
-    }
-    return a;
-  };
-
-  int32_t cur[NL], cend[NL];
-  V acc[NL][NV];
-  V rowc[NL][NV];
-#pragma unroll
-  for (int k = 0; k < NL; ++k) {
-    RO::zero(acc[k]);
-    RO::zero(rowc[k]);
-    cur[k] = 0;
-    cend[k] = 0;
-  }
-  int32_t head = INT_MAX;
-  int32_t head_row = 0;
-  bool head_closed = false;
-  V head_acc[NV];
-  RO::zero(head_acc);
-
-  if (active) {
-    int32_t key = p0;
-#pragma unroll
-    for (int k = NL - 1; k >= 0; --k) {
-      cur[k] = SEARCH(k, lo[k], hib[k], key);
-      key = cur[k];
-    }
-#pragma unroll
-    for (int k = 0; k < NL; ++k) {
-      cend[k] = POS(k, cur[k] + 1);
-      if (k >= 1) RO::load(rowc[k], F.M[k], CRD(k, cur[k]), c, Rr);
-    }
-    head = cur[0];
-    head_row = CRD(0, cur[0]);
-
-    const int32_t* __restrict__ lcrd = B.crd[N - 1];
-    const float* __restrict__ vals = B.vals;
-    const float* __restrict__ Mleaf = F.M[N - 1];
-    // Leaf (coordinate, value) pairs arrive U at a time: lane c < U of a row
-    // group loads pair t0 + c (one coalesced load per group and batch) and
-    // the group's lanes exchange them with shuffles. Pairs are fetched two
-    // batches ahead and leaf rows one batch ahead of their use.
-    constexpr int U = LPR < 4 ? LPR : 4;
-    const int gbase = (threadIdx.x & 63) - c;  // lane of this group's lane 0
-    // (loads of an in-range position for every lane, masked afterwards: a
-    // load behind a branch makes the compiler wait for it at the join)
-    auto load_pairs = [&](int32_t t0, int32_t& lq, float& vq) {
-      const int32_t t = t0 + c;
-      const bool ok = c < U && t < p1;
-      const int32_t tc = min(t, p1 - 1);
-      const int32_t l = lcrd[tc];
-      const float w = vals[tc];
-      lq = ok ? l : 0;
-      vq = ok ? w : 0.f;
-    };
-    auto issue = [&](int32_t lq, float vq, V (&d)[U][NV], float (&v)[U]) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int32_t l = __shfl(lq, gbase + u);
-        v[u] = __shfl(vq, gbase + u);
-        RO::load(d[u], Mleaf, l, c, Rr);
-      }
-    };
-    auto consume = [&](int32_t t0, const V (&d)[U][NV], const float (&v)[U]) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int32_t t = t0 + u;
-        if (t >= p1) break;
-        if (t >= cend[NL - 1]) {
-          // close the fiber at level N-2 and every ancestor that ends here
-          bool closing = true;
-          int32_t ckey = t;
-#pragma unroll
-          for (int k = NL - 1; k >= 0; --k) {
-            if (closing) {
-              const int32_t old = cur[k];
-              if (k >= 1) {
-                RO::hfma(acc[k - 1], acc[k], rowc[k]);
-              } else {
-                const int64_t row = CRD(0, old);
-                if (old == head && !head_closed) {
-                  head_closed = true;
-#pragma unroll
-                  for (int j = 0; j < NV; ++j) head_acc[j] = acc[0][j];
-                } else {
-                  if constexpr (EP) RO::store(A, row, c, Rr, acc[0]);
-                  else RO::store_f64(W, row, c, Rr, acc[0]);
-                }
-              }
-              RO::zero(acc[k]);
-              int32_t x = old + 1;
-              int32_t e = POS(k, x + 1);
-              if (e <= ckey) {
-                x = SEARCH(k, x + 1, hib[k], ckey);
-                e = POS(k, x + 1);
-              }
-              cur[k] = x;
-              cend[k] = e;
-              if (k >= 1) {
-                RO::load(rowc[k], F.M[k], CRD(k, x), c, Rr);
-                closing = x >= cend[k - 1];
-                ckey = x;
-              }
-            }
-          }
-        }
-        RO::axpy(acc[NL - 1], v[u], d[u]);
-      }
-    };
-    V dA[U][NV], dB[U][NV];
-    float vA[U], vB[U];
-    int32_t lA, lB;
-    float wA, wB;
-    load_pairs(p0, lA, wA);
-    load_pairs(p0 + U, lB, wB);
-    issue(lA, wA, dA, vA);
-    for (int32_t t0 = p0; t0 < p1; t0 += 2 * U) {
-      // invariant: rows of batch t0 in dA; pairs of batch t0+U in (lB, wB)
-      if (t0 + U < p1) {
-        load_pairs(t0 + 2 * U, lA, wA);
-        issue(lB, wB, dB, vB);
-      }
-      consume(t0, dA, vA);
-      if (t0 + U >= p1) break;
-      if (t0 + 2 * U < p1) {
-        load_pairs(t0 + 3 * U, lB, wB);
-        issue(lA, wA, dA, vA);
-      }
-      consume(t0 + U, dB, vB);
-    }
-    // fold the open nodes into the open slice
-#pragma unroll
-    for (int k = NL - 1; k >= 1; --k) RO::hfma(acc[k - 1], acc[k], rowc[k]);
-  }
-
-  if constexpr (!EP) {
-    // Entries e = 2 * gw + q of the wave's NGW groups: q = 0 is the group's
-    // first slice (its partial if it closed inside the run, else 0), q = 1
-    // the slice open at the run's end. Keys do not decrease with e; idle
-    // groups (trailing) hold INT_MAX. Suffix scan: at stride s, entry e adds
-    // entry e + s when both have the same key, so each key's first entry ends
-    // with the key's sum over the wave. Stride 1 pairs (gw, 0) with (gw, 1)
-    // and (gw, 1) with (gw + 1, 0); an even stride pairs (gw, q) with
-    // (gw + s / 2, q). Every lane runs every shuffle.
-    constexpr int NGW = 64 / LPR;
-    const int lane = int(threadIdx.x) & 63;
-    const int gw = lane / LPR;
-    const int32_t k0 = active ? head : INT_MAX;
-    const int32_t k1 = active ? cur[0] : INT_MAX;
-    V v0[NV], v1[NV];
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      v0[j] = head_acc[j];
-      v1[j] = acc[0][j];
-    }
-    auto shfl_v = [&](const V (&x)[NV], int src, V (&out)[NV]) {
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        if constexpr (R == 0) {
-          out[j] = __shfl(x[j], src);
-        } else {
-          out[j].x = __shfl(x[j].x, src);
-          out[j].y = __shfl(x[j].y, src);
-          out[j].z = __shfl(x[j].z, src);
-          out[j].w = __shfl(x[j].w, src);
-        }
-      }
-    };
-#pragma unroll
-    for (int st = 1; st < 2 * NGW; st <<= 1) {
-      const int dg = st == 1 ? 1 : st / 2;  // groups ahead of the source
-      const int src = (lane + dg * LPR) & 63;
-      const bool in_wave = gw + dg < NGW;
-      V a0[NV], a1[NV], b0[NV], b1[NV];
-      shfl_v(v0, src, b0);
-      shfl_v(v1, src, b1);
-      const int32_t n0 = __shfl(k0, src);
-      const int32_t n1 = __shfl(k1, src);
-      int32_t t0, t1;
-      bool ok0, ok1;
-      if (st == 1) {
-        // (gw, 0) + (gw, 1) in this lane; (gw, 1) + (gw + 1, 0)
-#pragma unroll
-        for (int j = 0; j < NV; ++j) {
-          a0[j] = v1[j];
-          a1[j] = b0[j];
-        }
-        t0 = k1;
-        t1 = n0;
-        ok0 = true;
-        ok1 = in_wave;
+  const int nent = 2 * int(min(int64_t(nwv), (int64_t(len) + NGW * G - 1) / (NGW * G)));
+  const int32_t first = key_of(0), last = key_of(nent - 1);
+  const int cols = R > 0 ? R : Rr;
+  for (int col = int(threadIdx.x); col < cols; col += int(blockDim.x)) {
+    const int at = RO::slot_of(col, Rr);
+    double s = 0.0;
+    int32_t key = first;
+    auto out = [&]() {
+      const int64_t o = int64_t(global_ptr(B.crd0)[key]) * cols + col;
+      const bool shared = key == first || key == last;
+      if constexpr (EP) {
+        if (shared) unsafeAtomicAdd(A + o, float(s));
+        else A[o] = float(s);
       } else {
-#pragma unroll
-        for (int j = 0; j < NV; ++j) {
-          a0[j] = b0[j];
-          a1[j] = b1[j];
-        }
-        t0 = n0;
-        t1 = n1;
-        ok0 = in_wave;
-        ok1 = in_wave;
-      }
-      if (ok0 && k0 != INT_MAX && t0 == k0) RO::add(v0, a0);
-      if (ok1 && k1 != INT_MAX && t1 == k1) RO::add(v1, a1);
-    }
-    // a key's first entry in the wave adds the sum
-    const int32_t kprev = __shfl(k1, (lane - LPR) & 63);  // (gw - 1, 1)
-    if (k0 != INT_MAX && (gw == 0 || kprev != k0))
-      RO::atomic_add_f64(W, CRD(0, k0), c, Rr, v0);
-    if (k1 != INT_MAX && k1 != k0) RO::atomic_add_f64(W, CRD(0, k1), c, Rr, v1);
-  }
-
-  if constexpr (EP) {
-    // Segmented suffix scan over the 2 entries per row group (first slice,
-    // last slice) of the workgroup; keys are nondecreasing, idle groups use
-    // INT_MAX. Entry 2g = (head slice, its closed partial or 0), entry
-    // 2g+1 = (open slice at run end, its partial).
-    const int NGB = blockDim.x / LPR;
-    const int E = 2 * NGB;
-    int32_t* keys = reinterpret_cast<int32_t*>(smem);
-    float* ev = reinterpret_cast<float*>(smem + size_t(E) * sizeof(int32_t));
-    V val[2][NV];
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      val[0][j] = head_acc[j];
-      val[1][j] = acc[0][j];
-    }
-    const int32_t key0 = active ? head : INT_MAX;
-    const int32_t key1 = active ? cur[0] : INT_MAX;
-    if (c == 0) {
-      keys[2 * gi] = key0;
-      keys[2 * gi + 1] = key1;
-    }
-    auto put = [&](int e, const V (&x)[NV]) {
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        const int k = RO::col(j, c, Rr);
-        if constexpr (R == 0) {
-          if (k < Rc) ev[size_t(e) * Rc + k] = x[j];
-        } else if constexpr (R < 0) {
-          store4(ev + size_t(e) * Rc + k, x[j]);
-        } else {
-          *reinterpret_cast<float4*>(ev + size_t(e) * Rc + k) = x[j];
-        }
+        if (shared) unsafeAtomicAdd(W + o, s);
+        else W[o] = s;
       }
     };
-    auto get = [&](int e, V (&x)[NV]) {
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        const int k = RO::col(j, c, Rr);
-        if constexpr (R == 0) {
-          x[j] = (k < Rc) ? ev[size_t(e) * Rc + k] : 0.f;
-        } else if constexpr (R < 0) {
-          x[j] = load4(ev + size_t(e) * Rc + k);
-        } else {
-          x[j] = *reinterpret_cast<const float4*>(ev + size_t(e) * Rc + k);
-        }
+    for (int en = 0; en < nent; ++en) {
+      const int32_t k = key_of(en);
+      if (k != key) {
+        out();
+        s = 0.0;
+        key = k;
       }
-    };
-    put(2 * gi, val[0]);
-    put(2 * gi + 1, val[1]);
-    __syncthreads();
-    for (int s = 1; s < E; s <<= 1) {
-      V add[2][NV];
-      bool take[2];
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int e = 2 * gi + q;
-        take[q] = (e + s < E) && keys[e] != INT_MAX && keys[e + s] == keys[e];
-        if (take[q]) get(e + s, add[q]);
-      }
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        if (take[q]) {
-          RO::add(val[q], add[q]);
-          put(2 * gi + q, val[q]);
-        }
-      }
-      __syncthreads();
+      s += double(row_of(en)[at]);
     }
-    // segment heads write their totals; only the workgroup's first and last
-    // slice can be shared with another workgroup
-    const int32_t g_last = (blk1 - 1 - blk0) / G;
-    const int32_t first_key = keys[0];
-    const int32_t last_key = keys[2 * g_last + 1];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int e = 2 * gi + q;
-      const int32_t k = keys[e];
-      if (k == INT_MAX) continue;
-      if (e > 0 && keys[e - 1] == k) continue;
-      const int64_t row = CRD(0, k);
-      if (k == first_key || k == last_key) RO::atomic_add(A, row, c, Rr, val[q]);
-      else RO::store(A, row, c, Rr, val[q]);
-    }
+    out();
   }
-  (void)head_row;
 }
 
 template <int N, int R, bool EP>
@@ -665,7 +673,7 @@ __device__ __forceinline__ void slice3_accumulate(const CsfDev& B, const Factors
   constexpr int NV = RO::NV;
   constexpr int NG = 64 / RO::LPR;
   constexpr int NT = 64 / NG;                 // fibers per row group per chunk
-  constexpr int TB = NT < 8 ? NT : 8;         // fibers whose rows are in flight per batch
+  constexpr int TB = NV >= 4 ? 2 : NT < 8 ? NT : 8;  // fibers whose rows are in flight per batch
   const int32_t* __restrict__ p2 = B.pos[2];
   const int32_t* __restrict__ c1 = B.crd[1];
   const int32_t* __restrict__ c2 = B.crd[2];
@@ -1139,10 +1147,8 @@ template <int N, int R>
 int launch_batch_order(const BatchLaunch& L, hipStream_t st) {
   const int32_t i_lo = L.grp_item[N], i_hi = L.grp_item[N + 1];
   if (i_hi <= i_lo) return TENTACO_OK;
-  const int lpr = Row<R>::LPR;
   const int blk = L.blk[N];
-  const size_t lds = edge_stage_ints(N, L.nb[N]) * sizeof(int32_t) + edge_ep_bytes(blk, lpr, L.R);
-  if (lds > 65536) return fail(TENTACO_EUNSUPPORTED, "batch LDS %zu B", lds);
+  const size_t lds = size_t(blk / 64) * edge_wave_lds<R>();
   const int grid = std::max(1, std::min<int>(L.grp_grid[N], i_hi - i_lo));
   batch_kernel<N, R, true><<<grid, blk, lds, st>>>(
       L.tasks, L.grp_task[N], L.grp_task[N + 1], L.item_off, i_lo, i_hi, L.counter + N, L.R,
@@ -1153,10 +1159,9 @@ int launch_batch_order(const BatchLaunch& L, hipStream_t st) {
 
 template <int N, int R>
 int batch_occupancy_order(int family, int block, int Rr, int32_t NB, int* per_cu) {
-  const int lpr = Row<R>::LPR;
   if (family != kEdgeParallel)
     return fail(TENTACO_EUNSUPPORTED, "the batch runs the edge-parallel walk only");
-  const size_t lds = edge_stage_ints(N, NB) * sizeof(int32_t) + edge_ep_bytes(block, lpr, Rr);
+  const size_t lds = size_t(block / 64) * edge_wave_lds<R>();
   const hipError_t e =
       hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, batch_kernel<N, R, true>, block, lds);
   if (e != hipSuccess) return fail(TENTACO_EHIP, "occupancy query: %s", hipGetErrorString(e));
@@ -1230,30 +1235,23 @@ int launch_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A,
     if (rc) return rc;
   }
   if (nblk == 0) return TENTACO_OK;
-  const int lpr = Row<R>::LPR;
-  const size_t stage = edge_stage_ints(N, int32_t(NB)) * sizeof(int32_t);
+  // the variant table's tile limit (tentaco_variant_fits)
+  if (!edge_tile_fits(N, Rr, vr)) {
+    return fail(TENTACO_EUNSUPPORTED, "edge tile of block %d and group %d at rank %d is over the "
+                "tile limit of order %d", vr.block, vr.group, Rr, N);
+  }
+  const size_t lds = size_t(vr.block / 64) * edge_wave_lds<R>();
+  ktimer_begin(st);
   if (vr.family == kEdgeSerial) {
-    if (stage > 65536)
-      return fail(TENTACO_EUNSUPPORTED, "edge-serial tile of %lld nonzeros needs %zu B of LDS",
-                  (long long)NB, stage);
-    ktimer_begin(st);
-    edge_kernel<N, R, false><<<int(nblk), vr.block, stage, st>>>(
-        B, F, A, Rr, brk, vr.group, int32_t(NB), W);
-    TT_HIP_CHECK(hipGetLastError());
-    ktimer_end(st, "edge_kernel");
-    return launch_narrow(W, A, a_elems, st);
+    edge_kernel<N, R, false><<<int(nblk), vr.block, lds, st>>>(B, F, A, Rr, brk, vr.group,
+                                                               int32_t(NB), W);
   } else {
-    const size_t lds = edge_ep_bytes(vr.block, lpr, Rr) + stage;
-    if (lds > 65536)
-      return fail(TENTACO_EUNSUPPORTED, "edge-parallel block %d at rank %d needs %zu B of LDS",
-                  vr.block, Rr, lds);
-    ktimer_begin(st);
-    edge_kernel<N, R, true><<<int(nblk), vr.block, lds, st>>>(
-        B, F, A, Rr, brk, vr.group, int32_t(NB), nullptr);
+    edge_kernel<N, R, true><<<int(nblk), vr.block, lds, st>>>(B, F, A, Rr, brk, vr.group,
+                                                              int32_t(NB), nullptr);
   }
   TT_HIP_CHECK(hipGetLastError());
   ktimer_end(st, "edge_kernel");
-  return TENTACO_OK;
+  return W ? launch_narrow(W, A, a_elems, st) : TENTACO_OK;
 }
 
 template <int N, int L, int R>

@@ -15,9 +15,9 @@
 //           lane owns. No load is predicated and none leaves the row, at
 //           4-byte alignment;
 //   R == 0  ranks 1..3: one column per lane of 4.
-// Ranks 4..256 used to share one scalar layout of 16 columns-predicated loads
-// per lane and row: the 5M-nonzero 3-mode tensor at rank 50 takes 0.59 ms
-// with it and 0.20 ms with the float4 layout.
+// Ranks 4..256 used to share one scalar layout of 16 column-predicated loads
+// per lane and row: a 5M-nonzero 3-mode MTTKRP at rank 50 took 598 us with it
+// and 229 us with the float4 layout (the walk of that time).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -94,6 +94,12 @@ struct Row {
   __device__ __forceinline__ static int col(int j, int c, int Rr) {
     if constexpr (R < 0) return min(slot(j, c), Rr - 4);
     else return slot(j, c);
+  }
+
+  // Where column k is in such a row.
+  __device__ __forceinline__ static int slot_of(int k, int Rr) {
+    if constexpr (R < 0) return (k & ~3) + (k - min(k & ~3, Rr - 4));
+    else return k;
   }
 
   // base[slot] = a, a += base[slot]: a row of kMaxRank floats, 16-byte
