@@ -221,7 +221,11 @@ int tentaco_csf_info(const tentaco_csf* h, int* order, int64_t* nnz,
                      int32_t* nodes);
 /* Reserve the per-handle workspace a variant needs, so that later calls on
  * this handle with at most dims[0] output rows allocate nothing (required
- * before graph capture). Edge variants need the partition brackets; the
+ * before graph capture). Edge variants need the partition brackets, and for
+ * the variant named here (AUTO: the one it resolves to) the call builds the
+ * table of the waves' start nodes, which later calls read instead of writing
+ * brackets (4(order-1) B per 16 to 1024 nonzeros; without a reserve call, the
+ * first call of a run length builds it and synchronizes its stream); the
  * edge-serial family also accumulates its rows in FP64 (output rows x R
  * doubles), which keeps atomics on giant slices accurate. For 3-mode
  * handles it also builds the slice-row structures: the expansion (4 B per

@@ -23,7 +23,7 @@ struct tentaco_batch {
   int64_t* d_item_off = nullptr;
   uint32_t* d_rowbits = nullptr;  // per task, one bit per output row
   int32_t* d_counter = nullptr;
-  int32_t* d_brk = nullptr;
+  int32_t* d_starts = nullptr;
   size_t brk_bytes = 0;
   tt::BatchLaunch L;
   std::vector<int64_t> h_fill, h_bnd;  // host prefix tables (ntasks + 1)
@@ -62,10 +62,10 @@ void free_tables(tentaco_batch* b) {
   (void)hipFree(b->d_tasks);
   (void)hipFree(b->d_bnd_off);
   (void)hipFree(b->d_item_off);
-  (void)hipFree(b->d_brk);
+  (void)hipFree(b->d_starts);
   b->d_tasks = nullptr;
   b->d_bnd_off = b->d_item_off = nullptr;
-  b->d_brk = nullptr;
+  b->d_starts = nullptr;
   b->brk_bytes = 0;
 }
 
@@ -93,7 +93,7 @@ int configure_tables(tentaco_batch* b) {
   BatchLaunch& L = b->L;
   const int lpr = lanes_per_row(b->R);
   for (int N = 0; N <= kMaxOrder; ++N) L.nb[N] = int32_t((L.blk[N] / lpr) * L.grp[N]);
-  std::vector<int64_t> bnd(b->ntasks + 1, 0), item(b->ntasks + 1, 0), brk_off(b->ntasks + 1, 0);
+  std::vector<int64_t> bnd(b->ntasks + 1, 0), item(b->ntasks + 1, 0), start_off(b->ntasks + 1, 0);
   for (int t = 0; t < b->ntasks; ++t) {
     const tentaco_csf* h = b->tasks[t];
     const int64_t nnz = h->nodes[h->order - 1];
@@ -101,7 +101,7 @@ int configure_tables(tentaco_batch* b) {
     const int64_t nblk = (nnz + NB - 1) / NB;
     item[t + 1] = item[t] + nblk;
     bnd[t + 1] = bnd[t] + nblk + 1;
-    brk_off[t + 1] = brk_off[t] + (nblk + 1) * (h->order - 1);
+    start_off[t + 1] = start_off[t] + (nblk + 1) * (L.blk[h->order] / 64) * (h->order - 1);
   }
   if (item[b->ntasks] >= (int64_t(1) << 31))
     return fail(TENTACO_EUNSUPPORTED, "batch has too many work items");
@@ -109,9 +109,9 @@ int configure_tables(tentaco_batch* b) {
   int rc = dev_alloc(&b->d_tasks, size_t(b->ntasks));
   if (!rc) rc = dev_alloc(&b->d_bnd_off, size_t(b->ntasks));
   if (!rc) rc = dev_alloc(&b->d_item_off, size_t(b->ntasks) + 1);  // + the total
-  if (!rc) rc = dev_alloc(&b->d_brk, size_t(brk_off[b->ntasks]));
+  if (!rc) rc = dev_alloc(&b->d_starts, size_t(start_off[b->ntasks]));
   if (rc) return rc;
-  for (int t = 0; t < b->ntasks; ++t) b->host_tasks[t].brk = b->d_brk + brk_off[t];
+  for (int t = 0; t < b->ntasks; ++t) b->host_tasks[t].starts = b->d_starts + start_off[t];
   TT_HIP_CHECK(hipMemcpy(b->d_tasks, b->host_tasks.data(), sizeof(BatchTaskDev) * b->ntasks,
                          hipMemcpyHostToDevice));
   TT_HIP_CHECK(hipMemcpy(b->d_bnd_off, bnd.data(), sizeof(int64_t) * b->ntasks,

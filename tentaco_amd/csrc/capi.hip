@@ -61,6 +61,7 @@ void free_handle(tentaco_csf* h) {
   (void)hipFree(h->d_vals);
   (void)hipFree(h->ws);
   for (void* w : h->ws_retired) (void)hipFree(w);
+  for (int i = 0; i < h->starts.n; ++i) (void)hipFree(h->starts.p[i]);
   for (int m = 0; m < kMaxOrder; ++m) (void)hipFree(h->stage_f[m]);
   (void)hipFree(h->stage_a);
   (void)hipFree(h->d_crd1_of_nnz);
@@ -205,6 +206,38 @@ int reserve_ws(tentaco_csf* h, size_t bytes, hipStream_t st) {
   return TENTACO_OK;
 }
 
+// The handle's wave starts for variant vr at rank R (edge families), or null.
+// With `build`, a missing table is built on st and waited for, so that it is
+// complete for every stream; not under capture. A failed build leaves the
+// calls on the brackets they write themselves.
+const int32_t* walk_starts(tentaco_csf* h, const Variant& vr, int R, bool build, hipStream_t st) {
+  const CsfDev B = h->view();
+  if (vr.family == kSliceRow || vr.family < 0 || B.nnz <= 0) return nullptr;
+  const int64_t wn = nnz_per_wave(vr, R);
+  WalkStarts& s = h->starts;
+  std::lock_guard<std::mutex> lk(s.mu);
+  for (int i = 0; i < s.n; ++i)
+    if (s.wn[i] == wn) return s.p[i];
+  if (!build || s.n >= WalkStarts::kTables) return nullptr;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone)
+    return nullptr;
+  int32_t* p = nullptr;
+  if (hipMalloc(reinterpret_cast<void**>(&p), edge_brk_bytes(B, wn)) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  const int rc = launch_walk_starts(B, wn, p, st);
+  if (hipStreamSynchronize(st) != hipSuccess || rc) {
+    (void)hipFree(p);
+    clear_error();
+    return nullptr;
+  }
+  s.wn[s.n] = wn;
+  s.p[s.n++] = p;
+  return p;
+}
+
 int resolve_variant(const tentaco_csf* h, int R, int variant) {
   if (variant == TENTACO_VARIANT_DEFAULT) return default_variant();
   if (variant == TENTACO_VARIANT_AUTO) {
@@ -302,6 +335,7 @@ int host_mttkrp(int order, taco_tensor_t* A, taco_tensor_t* B,
   if (vr.family < 0) return fail(TENTACO_EINVAL, "variant %d out of range", variant);
   rc = reserve_ws(h, mttkrp_workspace_bytes(h->view(), R, vr, a_rows), nullptr);
   if (rc) return rc;
+  h->reserved = true;  // a handle for one call: its start table would be used once
   if (vr.family == kSliceRow) {
     rc = ensure_expand3(h, nullptr);  // per-handle structure, outside the timed region
     if (rc) return rc;
@@ -671,7 +705,12 @@ int tentaco_csf_reserve_rows(tentaco_csf* h, int R, int variant, int32_t a_rows)
   if (!rc) rc = (hipDeviceSynchronize() == hipSuccess) ? TENTACO_OK
                                                        : fail(TENTACO_EHIP, "synchronize failed");
   if (rc) return rc;
-  return reserve_ws(h, need, nullptr);
+  rc = reserve_ws(h, need, nullptr);
+  if (rc) return rc;
+  // the wave starts of the variant that calls with this argument run
+  (void)walk_starts(h, variant_of(resolve_variant(h, R, variant)), R, true, nullptr);
+  h->reserved = true;
+  return TENTACO_OK;
 }
 
 int tentaco_csf_reserve(tentaco_csf* h, int R, int variant) {
@@ -766,8 +805,10 @@ int tentaco_mttkrp_dev(tentaco_csf* h, int R, const float* const* factors_dev, f
   const CsfDev B = h->view();
   rc = reserve_ws(h, mttkrp_workspace_bytes(B, R, vr, a_rows), static_cast<hipStream_t>(stream));
   if (rc) return rc;
+  const int32_t* starts =
+      walk_starts(h, vr, R, !h->reserved, static_cast<hipStream_t>(stream));
   const bool dense = h->dense_root && a_rows == h->nodes[0];
-  return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws,
+  return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws, starts,
                        static_cast<hipStream_t>(stream));
 }
 
@@ -804,7 +845,8 @@ int tentaco_mttkrp_dev_noalloc(tentaco_csf* h, int R, const float* const* factor
   // slice-row: the 3-mode expansion and padded layout are used when a
   // reserve call built them, never built here
   const bool dense = h->dense_root && a_rows == h->nodes[0];
-  return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, ws, static_cast<hipStream_t>(stream));
+  return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, ws, nullptr,
+                       static_cast<hipStream_t>(stream));
 }
 
 // The sweep over the variants with use[v] set (all when use is NULL);
@@ -821,6 +863,9 @@ static int sweep_impl(tentaco_csf* h, int R, const float* const* factors_dev, fl
       need = std::max(need, mttkrp_workspace_bytes(h->view(), R, variant_of(v), a_rows));
     int rc = reserve_ws(h, need, st);
     if (rc) return rc;
+    for (int v = 0; v < kNumVariants; ++v)
+      if ((!use || use[v]) && variant_fits(h->order, R, v))
+        (void)walk_starts(h, variant_of(v), R, true, st);
   }
   hipEvent_t e0, e1;
   TT_HIP_CHECK(hipEventCreate(&e0));

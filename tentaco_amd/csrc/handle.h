@@ -1,10 +1,28 @@
 // Device-resident CSF handle (the opaque tentaco_csf of the C ABI).
 #pragma once
 
+#include <mutex>
 #include <vector>
 
 #include "internal.h"
 #include "tuning.h"
+
+namespace tt {
+// The edge walk's wave starts of a handle, one table per run length (a power
+// of two from 16 to 1024 nonzeros): they depend on the CSF alone. A table is
+// complete when it is entered and stays until the handle is freed, so calls
+// on any stream or thread, and captured graphs, may read it. Writing the
+// brackets on every call took 11-16 us of serial searches and left each wave
+// a search of its own (1.5M nonzeros, 5-mode, rank 16: 67 us a call, 47 us
+// with the table).
+struct WalkStarts {
+  static constexpr int kTables = 8;
+  std::mutex mu;
+  int n = 0;
+  int64_t wn[kTables] = {};
+  int32_t* p[kTables] = {};
+};
+}  // namespace tt
 
 struct tentaco_csf {
   int order = 0;
@@ -21,6 +39,10 @@ struct tentaco_csf {
   // workspaces replaced by a larger one; a graph captured earlier may still
   // use them, so they are freed with the handle, never before
   std::vector<void*> ws_retired;
+  tt::WalkStarts starts;
+  // workspace reserved by the caller (or for one host call): later calls
+  // allocate nothing, so they write brackets where no start table exists
+  bool reserved = false;
   tt::TuneTable tune;  // per-rank best variant found by the autotuner
   tt::CsfStats stats;
   // device buffers of the stream-ordered host-pointer path (factors of

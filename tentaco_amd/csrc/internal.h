@@ -87,9 +87,16 @@ size_t ttv_workspace_bytes(const CsfDev& B);
 // Enqueue one MTTKRP on `stream`. A (a_rows x R) is fully overwritten;
 // `dense_root` says crd0 == 0..n0-1 with n0 == a_rows (no zero fill needed
 // for the slice-row family). ws must hold mttkrp_workspace_bytes bytes.
+// starts: the walk's wave starts for nnz_per_wave(vr, R) (edge families; see
+// launch_walk_starts), or null: the call then writes the brackets into ws.
 int launch_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A,
                   int32_t a_rows, bool dense_root, const Variant& vr,
-                  void* ws, hipStream_t stream);
+                  void* ws, const int32_t* starts, hipStream_t stream);
+// Nonzeros one wave of an edge-family variant walks at rank R.
+int64_t nnz_per_wave(const Variant& vr, int R);
+// Write the node at every level 0..N-2 that holds the first nonzero of each
+// run of wn nonzeros (edge_brk_bytes(B, wn) bytes) on `stream`.
+int launch_walk_starts(const CsfDev& B, int64_t wn, int32_t* starts, hipStream_t stream);
 // Fill the 3-mode expansion arrays of CsfDev (crd1_of_nnz: nnz entries,
 // nnz_of_root: n0 + 1 entries) from the CSF's own pos/crd on `stream`.
 int launch_expand3(const CsfDev& B, int32_t* crd1_of_nnz, int32_t* nnz_of_root,
@@ -218,12 +225,12 @@ int launch_ttv_units(const CsfDev& B, const TtvPlan& plan, const float* c, float
                      hipStream_t stream);
 
 // One task of a batched persistent launch (a CSF with its factors, output
-// and bracket workspace).
+// and the walk's wave starts).
 struct BatchTaskDev {
   CsfDev B;
   FactorsDev F;
   float* A = nullptr;
-  int32_t* brk = nullptr;
+  int32_t* starts = nullptr;  // per item and wave, the nodes of its first nonzero
   // output rows, and one bit per row, set where a root node with at least
   // one nonzero writes the row
   int32_t rows = 0;
@@ -282,10 +289,10 @@ struct BatchLaunch {
   hipEvent_t cev[kMaxOrder + 1] = {};
 };
 
-// One launch of the batch. The brackets must have been written by
+// One launch of the batch. The waves' starts must have been written by
 // launch_batch_brackets for the current tiles.
 int launch_batch(const BatchLaunch& L, hipStream_t stream);
-// Write every task's partition brackets for the current tiles (they depend
+// Write every task's wave starts for the current tiles (they depend
 // on the CSFs and the tiles only).
 int launch_batch_brackets(const BatchLaunch& L, hipStream_t stream);
 // Zero every output row that no launch stores (and the boundary rows): the

@@ -179,20 +179,22 @@ __device__ __forceinline__ void zero_row(float* A, int64_t row, int R) {
 // stores, write the brackets, zero the rows of the slices at item boundaries.
 constexpr int kPrepFill = 1, kPrepBrackets = 2, kPrepBoundary = 4;
 
-// Nonzeros per work item of each order group (kernel argument, by value).
+// Nonzeros per work item and waves per workgroup of each order group (kernel
+// argument, by value).
 struct BatchNB {
   int32_t nb[kMaxOrder + 1];
+  int32_t nw[kMaxOrder + 1];
 };
 
 // Prep of the order group holding sorted tasks [t_lo, t_hi): reset that
 // order's work counter; with kPrepFill zero the outputs (quads [q_lo,
 // q_hi)), skipping a row whose bit is set in the task's rowbits, because a
-// root node with nonzeros stores it; with kPrepBrackets write the brackets
-// (entries [b_lo, b_hi)); with kPrepBoundary zero the row of each slice
+// root node with nonzeros stores it; with kPrepBrackets write where the waves
+// of each item start (entries [b_lo, b_hi)); with kPrepBoundary zero the row of each slice
 // holding position b*NB or b*NB - 1 of a boundary b: those are the
 // edge-parallel walk's only atomically updated rows (the slices holding an
 // item's first and last nonzero). Without kPrepBrackets the boundary rows
-// come from the brackets written before.
+// come from the starts written before.
 __global__ __launch_bounds__(256) void batch_prep_kernel(const BatchTaskDev* __restrict__ tasks,
                                                          int32_t t_lo, int32_t t_hi,
                                                          const int64_t* __restrict__ fill_off,
@@ -270,15 +272,19 @@ __global__ __launch_bounds__(256) void batch_prep_kernel(const BatchTaskDev* __r
     int64_t p = bi * int64_t(NB);
     if (p > T.B.nnz - 1) p = T.B.nnz - 1;
     int32_t key = int32_t(p);
+    const int32_t nw = nbs.nw[N];
     if (mode & kPrepBrackets) {
-      for (int m = N - 2; m >= 0; --m) {
-        const int32_t x = search_le(T.B.pos[m + 1], 0, T.B.nodes[m] - 1, key);
-        T.brk[bi * (N - 1) + m] = x;
-        key = x;
+      // the starts of the item's waves
+      for (int w = 0; w < nw; ++w) {
+        key = int32_t(min(bi * int64_t(NB) + w * (NB / nw), int64_t(T.B.nnz) - 1));
+        for (int m = N - 2; m >= 0; --m) {
+          const int32_t x = search_le(T.B.pos[m + 1], 0, T.B.nodes[m] - 1, key);
+          T.starts[(bi * nw + w) * (N - 1) + m] = x;
+          key = x;
+        }
       }
-    } else {
-      key = T.brk[bi * (N - 1)];  // the root node holding position p
     }
+    key = T.starts[bi * nw * (N - 1)];  // the root node holding position p
     if (mode & kPrepBoundary) {
       zero_row(T.A, T.B.crd0[key], R);
       // position p - 1 (the previous item's last nonzero) lies in another
@@ -323,7 +329,10 @@ int launch_batch_prep_range(const BatchLaunch& L, int n_lo, int n_hi, hipStream_
   const int64_t work = std::max<int64_t>(fill_quads, b1 - b0);
   const int qshift = L.R == 16 ? 2 : L.R == 32 ? 3 : 4;  // log2(R / 4), R in {16, 32, 64}
   BatchNB nbs{};
-  for (int N = 0; N <= kMaxOrder; ++N) nbs.nb[N] = L.nb[N];
+  for (int N = 0; N <= kMaxOrder; ++N) {
+    nbs.nb[N] = L.nb[N];
+    nbs.nw[N] = std::max(1, L.blk[N] / 64);
+  }
   batch_prep_kernel<<<grid_for(work, 256, 16384), 256, 0, st>>>(
       L.tasks, t_lo, t_hi, L.fill_off, f0 >> 2, f1 >> 2, L.bnd_off, b0, b1, L.counter, n_lo, n_hi,
       nbs, L.R, qshift, mode);
@@ -566,6 +575,16 @@ bool variant_fits(int order, int R, int v) {
   return vr.family == kSliceRow || edge_tile_fits(order, R, vr);
 }
 
+int64_t nnz_per_wave(const Variant& vr, int R) {
+  return int64_t(64 / lanes_per_row(R)) * vr.group;
+}
+
+int launch_walk_starts(const CsfDev& B, int64_t wn, int32_t* starts, hipStream_t st) {
+  // the brackets of runs of wn nonzeros (one entry past the last run too)
+  const int64_t runs = (int64_t(B.nnz) + wn - 1) / wn;
+  return launch_edge_prep(B, nullptr, 0, starts, int32_t(runs), int32_t(wn), st);
+}
+
 size_t edge_brk_bytes(const CsfDev& B, int64_t NB) {
   const int64_t nblk = (int64_t(B.nnz) + NB - 1) / NB;
   const size_t bytes = size_t(nblk + 1) * size_t(B.order - 1) * sizeof(int32_t);
@@ -607,15 +626,15 @@ int launch_mttkrp_level(const CsfDev& B, const FactorsDev& F, int level, int R, 
 
 int launch_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A,
                   int32_t a_rows, bool dense_root, const Variant& vr, void* ws,
-                  hipStream_t st) {
+                  const int32_t* starts, hipStream_t st) {
   if (R <= 0 || R > kMaxRankAny)
     return fail(TENTACO_EUNSUPPORTED, "rank R=%d outside 1..%d", R, kMaxRankAny);
   if (vr.family < 0) return fail(TENTACO_EINVAL, "invalid variant");
   switch (B.order) {
-    case 2: return order_mttkrp<2>(B, F, R, A, a_rows, dense_root, vr, ws, st);
-    case 3: return order_mttkrp<3>(B, F, R, A, a_rows, dense_root, vr, ws, st);
-    case 4: return order_mttkrp<4>(B, F, R, A, a_rows, dense_root, vr, ws, st);
-    case 5: return order_mttkrp<5>(B, F, R, A, a_rows, dense_root, vr, ws, st);
+    case 2: return order_mttkrp<2>(B, F, R, A, a_rows, dense_root, vr, ws, starts, st);
+    case 3: return order_mttkrp<3>(B, F, R, A, a_rows, dense_root, vr, ws, starts, st);
+    case 4: return order_mttkrp<4>(B, F, R, A, a_rows, dense_root, vr, ws, starts, st);
+    case 5: return order_mttkrp<5>(B, F, R, A, a_rows, dense_root, vr, ws, starts, st);
     default: return fail(TENTACO_EUNSUPPORTED, "order %d outside 2..5", B.order);
   }
 }

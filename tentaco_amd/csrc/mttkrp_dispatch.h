@@ -35,7 +35,8 @@ __device__ __forceinline__ int32_t upper_index(const int64_t* __restrict__ off, 
 // pick the order.
 template <int N>
 int order_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A, int32_t a_rows,
-                 bool dense_root, const Variant& vr, void* ws, hipStream_t st);
+                 bool dense_root, const Variant& vr, void* ws, const int32_t* starts,
+                 hipStream_t st);
 template <int N>
 int order_inner(const CsfDev& B, const LevelIndex& X, const FactorsDev& F, int level, int R,
                 float* A, int32_t a_rows, hipStream_t st);

@@ -101,10 +101,16 @@ __device__ __forceinline__ int32_t wave_search_le(const int32_t* __restrict__ a,
   return lo;
 }
 
+// Where a wave's run starts comes from `starts` (the node of its first
+// nonzero at every level, N-1 per wave, waves in order), a table that depends
+// on the CSF and the run length only and that a handle or a batch keeps; or,
+// with starts null, from the block's brackets brk (the same per block) by a
+// search of its own.
 template <int N, int R, bool EP>
 __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F, float* out_a,
-                                           int Rr, const int32_t* brk_p, int32_t b, int32_t G,
-                                           int32_t NB, unsigned char* smem, double* out_w) {
+                                           int Rr, const int32_t* brk_p, const int32_t* starts_p,
+                                           int32_t b, int32_t G, int32_t NB, unsigned char* smem,
+                                           double* out_w) {
   using RO = Row<R>;
   using V = typename RO::V;
   constexpr int NV = RO::NV;
@@ -120,6 +126,7 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
   float* __restrict__ A = global_ptr(out_a);
   double* __restrict__ W = global_ptr(out_w);
   const int32_t* __restrict__ brk = global_ptr(brk_p);
+  const int32_t* __restrict__ starts = global_ptr(starts_p);
 
   const int lane = int(threadIdx.x) & 63;
   const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
@@ -161,7 +168,11 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
     }
     // cur[k]: the node at level k that holds the chunk's first nonzero
     int32_t cur[NL];
-    {
+    if (starts) {
+      const int32_t* st = starts + (int64_t(b) * nwv + wv) * NL;
+#pragma unroll
+      for (int k = 0; k < NL; ++k) cur[k] = __builtin_amdgcn_readfirstlane(st[k]);
+    } else {
       int32_t key = w0;
 #pragma unroll
       for (int k = FL; k >= 0; --k) {
@@ -429,10 +440,11 @@ template <int N, int R, bool EP>
 __global__ __launch_bounds__(512) void edge_kernel(CsfDev B, FactorsDev F,
                                                    float* __restrict__ A, int Rr,
                                                    const int32_t* __restrict__ brk,
+                                                   const int32_t* __restrict__ starts,
                                                    int32_t G, int32_t NB,
                                                    double* __restrict__ W) {
   extern __shared__ __align__(16) unsigned char smem[];
-  edge_block<N, R, EP>(B, F, A, Rr, brk, blockIdx.x, G, NB, smem, W);
+  edge_block<N, R, EP>(B, F, A, Rr, brk, starts, blockIdx.x, G, NB, smem, W);
 }
 
 
@@ -1101,45 +1113,54 @@ __global__ __launch_bounds__(128) void slice_pair_kernel(const uint2* __restrict
 
 // Persistent workgroups over the items of one order's tasks (the device
 // task table is sorted by order: tasks [t_lo, t_hi) hold items [i_lo, i_hi)),
-// so each order runs with its own register and LDS footprint. schedule 0
-// pulls items from the order's device counter (reset by the prep launch) in
-// arrival order; schedule 1 is a static cyclic assignment (item = i_lo +
-// block + k * grid). Either way a workgroup's items increase, so its task
-// cursor only moves forward.
+// so each order runs with its own register and LDS footprint. Items go out
+// in chunks of `chunk` consecutive ones: a workgroup's first chunk is its own
+// index; later ones come from the order's device counter (schedule 0, reset
+// by the prep launch; not touched when the first chunks cover every item) or
+// by a static cyclic assignment (schedule 1). Either way a workgroup's items
+// increase, so its task cursor only moves forward.
 template <int N, int R, bool EP>
 __global__ __launch_bounds__(512) void batch_kernel(const BatchTaskDev* __restrict__ tasks,
                                                     int32_t t_lo, int32_t t_hi,
                                                     const int64_t* __restrict__ item_off,
                                                     int32_t i_lo, int32_t i_hi,
                                                     int32_t* __restrict__ counter, int Rr,
-                                                    int32_t G, int32_t NB, int dynamic) {
+                                                    int32_t G, int32_t NB, int32_t chunk,
+                                                    int dynamic) {
   // the batch has no FP64 row buffer, which the edge-serial walk needs
   static_assert(EP, "the batch runs the edge-parallel walk only");
   extern __shared__ __align__(16) unsigned char smem[];
-  __shared__ int32_t s_item;
+  __shared__ int32_t s_chunk;
+  const int32_t nchunks = (i_hi - i_lo + chunk - 1) / chunk;
+  const int32_t grid = int32_t(gridDim.x);
   int32_t t = -1;
   int64_t t_end = 0;
-  int32_t item = i_lo + int32_t(blockIdx.x);
-  for (;;) {
-    __syncthreads();  // the previous item's LDS reads are done
+  for (int32_t ch = int32_t(blockIdx.x); ch < nchunks;) {
+    const int32_t first = i_lo + ch * chunk;
+    const int32_t last = min(i_hi - first, chunk) + first;
+    for (int32_t item = first; item < last; ++item) {
+      __syncthreads();  // the previous item's LDS reads are done
+      if (t < 0) {
+        t = t_lo + upper_index(item_off + t_lo, t_hi - t_lo, item);
+        t_end = item_off[t + 1];
+      }
+      while (item >= t_end) {
+        ++t;
+        t_end = item_off[t + 1];
+      }
+      const BatchTaskDev& T = tasks[t];
+      const int32_t b = item - int32_t(item_off[t]);
+      edge_block<N, R, EP>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, G, NB, smem, nullptr);
+    }
     if (dynamic) {
-      if (threadIdx.x == 0) s_item = i_lo + atomicAdd(counter, 1);
+      if (nchunks <= grid) break;
+      __syncthreads();  // every thread has read the previous s_chunk
+      if (threadIdx.x == 0) s_chunk = grid + atomicAdd(counter, 1);
       __syncthreads();
-      item = __builtin_amdgcn_readfirstlane(s_item);
+      ch = __builtin_amdgcn_readfirstlane(s_chunk);
+    } else {
+      ch += grid;
     }
-    if (item >= i_hi) break;
-    if (t < 0) {
-      t = t_lo + upper_index(item_off + t_lo, t_hi - t_lo, item);
-      t_end = item_off[t + 1];
-    }
-    while (item >= t_end) {
-      ++t;
-      t_end = item_off[t + 1];
-    }
-    const BatchTaskDev& T = tasks[t];
-    const int32_t b = item - int32_t(item_off[t]);
-    edge_block<N, R, EP>(T.B, T.F, T.A, Rr, T.brk, b, G, NB, smem, nullptr);
-    if (!dynamic) item += int32_t(gridDim.x);
   }
 }
 
@@ -1150,9 +1171,14 @@ int launch_batch_order(const BatchLaunch& L, hipStream_t st) {
   const int blk = L.blk[N];
   const size_t lds = size_t(blk / 64) * edge_wave_lds<R>();
   const int grid = std::max(1, std::min<int>(L.grp_grid[N], i_hi - i_lo));
+  // An add to the one counter takes 10-12 ns whatever the workgroups do, so
+  // items taken one at a time cost that each (8 tensors, 38k items of 512
+  // nonzeros: 815 us a replay, 676 us in chunks and with the starts kept). About eight chunks per
+  // workgroup keep the ends even.
+  const int32_t chunk = L.sch[N] == 0 ? std::max(1, (i_hi - i_lo) / (8 * grid)) : 1;
   batch_kernel<N, R, true><<<grid, blk, lds, st>>>(
       L.tasks, L.grp_task[N], L.grp_task[N + 1], L.item_off, i_lo, i_hi, L.counter + N, L.R,
-      L.grp[N], L.nb[N], L.sch[N] == 0);
+      L.grp[N], L.nb[N], chunk, L.sch[N] == 0);
   TT_HIP_CHECK(hipGetLastError());
   return TENTACO_OK;
 }
@@ -1171,7 +1197,7 @@ int batch_occupancy_order(int family, int block, int Rr, int32_t NB, int* per_cu
 template <int N, int R>
 int launch_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A,
                  int32_t a_rows, bool dense_root, const Variant& vr, void* ws,
-                 hipStream_t st) {
+                 const int32_t* starts, hipStream_t st) {
   const int64_t a_elems = int64_t(a_rows) * Rr;
   if (vr.family == kSliceRow) {
     if (!dense_root) {
@@ -1231,7 +1257,8 @@ int launch_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A,
   {
     float* Z = W ? reinterpret_cast<float*>(W) : A;
     const int64_t z_elems = W ? 2 * a_elems : a_elems;
-    const int rc = launch_edge_prep(B, Z, z_elems, brk, int32_t(nblk), int32_t(NB), st);
+    const int rc = starts ? launch_fill(Z, z_elems, 0.f, st)
+                          : launch_edge_prep(B, Z, z_elems, brk, int32_t(nblk), int32_t(NB), st);
     if (rc) return rc;
   }
   if (nblk == 0) return TENTACO_OK;
@@ -1243,11 +1270,11 @@ int launch_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A,
   const size_t lds = size_t(vr.block / 64) * edge_wave_lds<R>();
   ktimer_begin(st);
   if (vr.family == kEdgeSerial) {
-    edge_kernel<N, R, false><<<int(nblk), vr.block, lds, st>>>(B, F, A, Rr, brk, vr.group,
-                                                               int32_t(NB), W);
+    edge_kernel<N, R, false><<<int(nblk), vr.block, lds, st>>>(B, F, A, Rr, brk, starts,
+                                                               vr.group, int32_t(NB), W);
   } else {
-    edge_kernel<N, R, true><<<int(nblk), vr.block, lds, st>>>(B, F, A, Rr, brk, vr.group,
-                                                              int32_t(NB), nullptr);
+    edge_kernel<N, R, true><<<int(nblk), vr.block, lds, st>>>(B, F, A, Rr, brk, starts,
+                                                              vr.group, int32_t(NB), nullptr);
   }
   TT_HIP_CHECK(hipGetLastError());
   ktimer_end(st, "edge_kernel");
@@ -1328,9 +1355,10 @@ int launch_level_order(const CsfDev& B, const FactorsDev& F, int level, int Rr, 
 // ---- one tensor order's entry points (mttkrp_dispatch.h) --------------------
 template <int N>
 int order_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A, int32_t a_rows,
-                 bool dense_root, const Variant& vr, void* ws, hipStream_t st) {
+                 bool dense_root, const Variant& vr, void* ws, const int32_t* starts,
+                 hipStream_t st) {
   return with_rank_layout(R, [&](auto r) {
-    return launch_typed<N, r()>(B, F, R, A, a_rows, dense_root, vr, ws, st);
+    return launch_typed<N, r()>(B, F, R, A, a_rows, dense_root, vr, ws, starts, st);
   });
 }
 
@@ -1371,7 +1399,7 @@ int order_batch_occupancy(int family, int block, int R, int32_t NB, int* per_cu)
 // Instantiates order N's entry points (one source per order).
 #define TT_INSTANTIATE_ORDER(N)                                                                 \
   template int tt::order_mttkrp<N>(const CsfDev&, const FactorsDev&, int, float*, int32_t, bool, \
-                                   const Variant&, void*, hipStream_t);                         \
+                                   const Variant&, void*, const int32_t*, hipStream_t);         \
   template int tt::order_inner<N>(const CsfDev&, const LevelIndex&, const FactorsDev&, int, int, \
                                   float*, int32_t, hipStream_t);                                \
   template int tt::order_level<N>(const CsfDev&, const FactorsDev&, int, int, float*, int32_t,  \
