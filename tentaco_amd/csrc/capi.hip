@@ -248,6 +248,14 @@ int resolve_variant(const tentaco_csf* h, int R, int variant) {
   return variant;
 }
 
+// What a call with `variant` that resolved to v runs: AUTO's structural choice
+// is resized to the tensor, anything else is the variant's own tile.
+Variant tile_of(const tentaco_csf* h, int R, int variant, int v) {
+  if (variant == TENTACO_VARIANT_AUTO && h->tune.lookup(R) < 0)
+    return auto_tile(h->stats, h->order, R);
+  return variant_of(v);
+}
+
 // Load the MTTKRP and TTV code objects on the current device once, before
 // the first timed region (the first launch from a code object loads it,
 // which would otherwise land inside get_gpu_timer_result's region).
@@ -331,7 +339,7 @@ int host_mttkrp(int order, taco_tensor_t* A, taco_tensor_t* B,
   if (hipMalloc(&abuf.p, std::max<size_t>(abytes, 4)) != hipSuccess)
     return fail(TENTACO_ENOMEM, "hipMalloc of A (%zu bytes) failed", abytes);
   const int v = resolve_variant(h, R, variant);
-  const Variant vr = variant_of(v);
+  const Variant vr = tile_of(h, R, variant, v);
   if (vr.family < 0) return fail(TENTACO_EINVAL, "variant %d out of range", variant);
   rc = reserve_ws(h, mttkrp_workspace_bytes(h->view(), R, vr, a_rows), nullptr);
   if (rc) return rc;
@@ -348,7 +356,7 @@ int host_mttkrp(int order, taco_tensor_t* A, taco_tensor_t* B,
     rc = ensure_events();
     if (rc) return rc;
     TT_HIP_CHECK(hipEventRecord(g_ev0, nullptr));
-    rc = tentaco_mttkrp_dev(h, R, fdev, static_cast<float*>(abuf.p), a_rows, v, nullptr);
+    rc = tentaco_mttkrp_dev(h, R, fdev, static_cast<float*>(abuf.p), a_rows, variant, nullptr);
     if (rc) return rc;
     TT_HIP_CHECK(hipEventRecord(g_ev1, nullptr));
     TT_HIP_CHECK(hipEventSynchronize(g_ev1));
@@ -708,7 +716,7 @@ int tentaco_csf_reserve_rows(tentaco_csf* h, int R, int variant, int32_t a_rows)
   rc = reserve_ws(h, need, nullptr);
   if (rc) return rc;
   // the wave starts of the variant that calls with this argument run
-  (void)walk_starts(h, variant_of(resolve_variant(h, R, variant)), R, true, nullptr);
+  (void)walk_starts(h, tile_of(h, R, variant, resolve_variant(h, R, variant)), R, true, nullptr);
   h->reserved = true;
   return TENTACO_OK;
 }
@@ -796,7 +804,7 @@ int tentaco_mttkrp_dev(tentaco_csf* h, int R, const float* const* factors_dev, f
   } else {
     v = resolve_variant(h, R, variant);
   }
-  const Variant vr = variant_of(v);
+  const Variant vr = tile_of(h, R, variant, v);
   if (vr.family < 0) return fail(TENTACO_EINVAL, "variant %d out of range", variant);
   if (vr.family == kSliceRow) {
     rc = ensure_expand3(h, static_cast<hipStream_t>(stream));
@@ -828,7 +836,7 @@ int tentaco_mttkrp_dev_noalloc(tentaco_csf* h, int R, const float* const* factor
   // AUTO: the recorded choice or the structural heuristic (the selector and
   // the sweep allocate and synchronise)
   const int v = resolve_variant(h, R, variant);
-  const Variant vr = variant_of(v);
+  const Variant vr = tile_of(h, R, variant, v);
   if (vr.family < 0) return fail(TENTACO_EINVAL, "variant %d out of range", variant);
   const CsfDev B = h->view();
   const size_t need = mttkrp_workspace_bytes(B, R, vr, a_rows);

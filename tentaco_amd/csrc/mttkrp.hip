@@ -553,6 +553,26 @@ int auto_variant(const CsfStats& s, int order, int R) {
   return 2 * per_family + 1;  // sr_b256 (always fits)
 }
 
+Variant auto_tile(const CsfStats& s, int order, int R) {
+  const Variant vr = variant_of(auto_variant(s, order, R));
+  if (vr.family != kEdgeParallel) return vr;
+  // A wave's run of nonzeros is a serial chain, so up to about 3000 runs in
+  // all (12 waves per CU) shorter runs are faster; beyond that more runs only
+  // add each one's start and end. Runs hold 32 to 512 nonzeros, in 512-thread
+  // workgroups below 300k nonzeros (fewer workgroups to combine) and 256 from
+  // there. From 30M nonzeros on 512 threads and runs of 256 are 2-4% faster
+  // again (100M, 3-mode, rank 32: 2023 us against 2101). Over 60 tensors drawn
+  // from 10k to 12.6M nonzeros, orders 3-5, ranks 7-128, this is 1.08x the
+  // sweep's best edge-parallel tile (geometric mean); the variants' own sizes
+  // (256 x 16 and 512 x 64) are 1.33x.
+  const int groups = 64 / lanes_per_row(R);
+  const bool large = s.nnz >= 30000000;
+  const int64_t want = std::max<int64_t>(32, std::min<int64_t>(large ? 256 : 512, s.nnz / 3000));
+  Variant t{kEdgeParallel, s.nnz < 300000 || large ? 512 : 256, 4};
+  while (t.group < 64 && int64_t(groups) * t.group * 3 / 2 <= want) t.group *= 2;
+  return edge_tile_fits(order, R, t) ? t : vr;
+}
+
 int lanes_per_row(int R) {
   return with_rank_layout(R, [](auto r) { return Lay<r()>::LPR; });
 }

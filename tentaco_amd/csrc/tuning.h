@@ -53,4 +53,8 @@ struct CsfStats {
 // root slices are many and even, edge-parallel otherwise.
 int auto_variant(const CsfStats& s, int order, int R);
 
+// The tile that choice runs: an edge-parallel variant resized to the
+// tensor, any other unchanged.
+Variant auto_tile(const CsfStats& s, int order, int R);
+
 }  // namespace tt
