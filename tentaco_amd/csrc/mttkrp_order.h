@@ -57,21 +57,6 @@ constexpr size_t edge_wave_lds() {
   return kRecBytes + kHistBytes + kFibBytes + Lay<R>::kMaxRank * sizeof(float);
 }
 
-// The pointer as one to global memory. In the batch kernel the pointers come
-// from the task table in memory; loads through them would be flat loads,
-// whose waits also drain the LDS reads in flight.
-template <class T>
-__device__ __forceinline__ T* global_ptr(T* p) {
-  typedef __attribute__((address_space(1))) T* G;
-  return (T*)reinterpret_cast<G>(reinterpret_cast<uintptr_t>(p));
-}
-
-// Orders the wave's LDS accesses: what its lanes wrote before is read after.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 // Inclusive sum over the lanes up to this one (DPP row shifts, then the rows'
 // last lanes broadcast to the next rows).
 __device__ __forceinline__ int32_t wave_scan_add(int32_t x) {
@@ -121,6 +106,9 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
   constexpr int FL = N - 2;                 // the nonzeros' parents (fibres)
   constexpr int PF0 = kFibBytes / (KR * 4); // fibres whose product rows fit P
   constexpr int PF = PF0 < 64 ? PF0 : 64;
+  // slices of a chunk from which their nonzeros' products are summed from LDS,
+  // PF at a time: about twice as many as the chunk has such rounds
+  constexpr int kManySlices = 128 / PF < 3 ? 3 : 128 / PF;
   // leaf rows in flight per row group, at most 32 VGPRs of them
   constexpr int SB = NV >= 4 ? 2 : NV == 2 ? 4 : LPR < 8 ? LPR : 8;
   float* __restrict__ A = global_ptr(out_a);
@@ -288,9 +276,95 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
           window(k, curn[k], wpn[k], wcn[k]);
         }
       }
-      // pieces: nonzeros [a, e) of one slice in fibres [fa, fe)
+      // slices of the chunk: the mask of their first nonzeros
+      const int32_t rq = N > 2 ? __shfl(root, loc[FL]) : root;  // lane q: nonzero q's root
+      const int32_t rbefore = __shfl_up(rq, 1);
+      const bool first_of = lane < n && (lane == 0 || rq != rbefore);
+      const uint64_t starts_of = __ballot(first_of);
+      const int32_t ns = __popcll(starts_of);
+      const bool many = ns >= kManySlices;
+      if (many) {
+        // Many slices: the products of PB nonzeros at a time go to LDS, all
+        // their rows in flight at once, and the row groups then sum a slice
+        // each. Taken as pieces, every slice would wait for its own rows.
+        const int32_t ord = __popcll(starts_of & ((2ull << lane) - 1ull)) - 1;
+        if (first_of) hist[ord] = lane;  // first nonzero of slice `ord`
+        wave_lds_sync();
+        constexpr int PB = PF;
+        constexpr int U = PB / NGW;
+        for (int32_t s0 = 0; s0 < n; s0 += PB) {
+          const int32_t m = min(PB, n - s0);
+          V d[U][NV];
+          float w[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int4 x = rec[s0 + min(u * NGW + gi, m - 1)];
+            w[u] = __int_as_float(x.y);
+            RO::load(d[u], Mleaf, x.x, c, Rr);
+            if constexpr (N > 2) {
+#pragma unroll
+              for (int k = FL; k >= 1; --k) {
+                V p[NV];
+                RO::load(p, M[k], __shfl(fc[k], x.z), c, Rr);
+                RO::hmul(d[u], p);
+              }
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            V p[NV];
+            RO::zero(p);
+            RO::axpy(p, w[u], d[u]);
+            if (u * NGW + gi < m) RO::put(P + (u * NGW + gi) * KR, c, p);
+          }
+          wave_lds_sync();
+          const int32_t o0 = lane_of(ord, s0), o1 = lane_of(ord, s0 + m - 1);
+          const int32_t r0 = lane_of(rq, s0);
+          if (cur[0] + r0 != open) {
+            close_slice();
+            open = cur[0] + r0;
+            open_row = lane_of(wc[0], r0);
+          }
+          // slice o0 continues the open one, o1 stays open
+          V last[NV];
+          RO::zero(last);
+          for (int32_t ob = o0; ob <= o1; ob += NGW) {
+            const int32_t o = min(ob + gi, o1);
+            const int32_t a = max(hist[o], s0);
+            const int32_t e = o + 1 < ns ? min(hist[min(o + 1, 63)], s0 + m) : s0 + m;
+            const int32_t row = __shfl(wc[0], __shfl(rq, a));
+            V sum[NV];
+            RO::zero(sum);
+            if (ob + gi <= o1)
+              for (int32_t i = a; i < e; ++i) {
+                V p[NV];
+                RO::get(P + (i - s0) * KR, c, p);
+                RO::add(sum, p);
+              }
+            if (o == o0) {
+              RO::add(acc, sum);
+            } else if (o == o1) {
+              RO::add(last, sum);
+            } else if constexpr (EP) {
+              RO::store(A, row, c, Rr, sum);
+            } else {
+              RO::store_f64(W, row, c, Rr, sum);
+            }
+          }
+          if (o1 > o0) {
+            close_slice();
+#pragma unroll
+            for (int j = 0; j < NV; ++j) acc[j] = last[j];
+            const int32_t r1 = lane_of(rq, s0 + m - 1);
+            open = cur[0] + r1;
+            open_row = lane_of(wc[0], r1);
+          }
+          wave_lds_sync();
+        }
+      }
+      // few: pieces, nonzeros [a, e) of one slice in fibres [fa, fe)
       const int32_t nf = N > 2 ? cnt[FL] : n;
-      for (int32_t a = 0, fa = 0; a < n;) {
+      for (int32_t a = many ? n : 0, fa = 0; a < n;) {
         const int32_t r = lane_of(root, fa);
         const int32_t fe =
             fa + __popcll(__ballot(lane >= fa && lane < min(nf, N > 2 ? fa + PF : 64) && root == r));
@@ -326,30 +400,26 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
         };
         auto steps = [&](auto S, int32_t t0) {
           V d[S()][NV];
-          float w[S()];
-          int32_t slot[S()];
+          auto record = [&](int u) { return rec[min(t0 + u * NGW + gi, e - 1)]; };
 #pragma unroll
-          for (int u = 0; u < S(); ++u) {
-            const int32_t t = t0 + u * NGW + gi;
-            const int4 x = rec[min(t, e - 1)];
-            w[u] = t < e ? __int_as_float(x.y) : 0.f;
-            slot[u] = x.z - fa;
-            RO::load(d[u], Mleaf, x.x, c, Rr);
-          }
+          for (int u = 0; u < S(); ++u) RO::load(d[u], Mleaf, record(u).x, c, Rr);
           if constexpr (N > 2) {
             if (!staged) stage();
             staged = true;
           }
+          // (the records are read again rather than held: 16 registers less)
 #pragma unroll
           for (int u = 0; u < S(); ++u) {
+            const int4 x = record(u);
+            const float w = t0 + u * NGW + gi < e ? __int_as_float(x.y) : 0.f;
             if constexpr (N > 2) {
               V p[NV], s[NV];
-              RO::get(P + slot[u] * KR, c, p);
+              RO::get(P + (x.z - fa) * KR, c, p);
               RO::zero(s);
-              RO::axpy(s, w[u], p);
+              RO::axpy(s, w, p);
               RO::hfma(acc, s, d[u]);
             } else {
-              RO::axpy(acc, w[u], d[u]);
+              RO::axpy(acc, w, d[u]);
             }
           }
         };
@@ -436,8 +506,15 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
   }
 }
 
+// Waves per SIMD asked of the compiler (its register budget is 512 over this):
+// left alone it takes 114 registers at order 3 and 140 at order 5.
+template <int N, int R>
+constexpr int edge_waves() {
+  return Row<R>::NV >= 4 ? 2 : Row<R>::NV == 2 ? 4 : N <= 3 ? 5 : 4;
+}
+
 template <int N, int R, bool EP>
-__global__ __launch_bounds__(512) void edge_kernel(CsfDev B, FactorsDev F,
+__global__ __launch_bounds__(512, (edge_waves<N, R>())) void edge_kernel(CsfDev B, FactorsDev F,
                                                    float* __restrict__ A, int Rr,
                                                    const int32_t* __restrict__ brk,
                                                    const int32_t* __restrict__ starts,
@@ -1120,7 +1197,7 @@ __global__ __launch_bounds__(128) void slice_pair_kernel(const uint2* __restrict
 // by a static cyclic assignment (schedule 1). Either way a workgroup's items
 // increase, so its task cursor only moves forward.
 template <int N, int R, bool EP>
-__global__ __launch_bounds__(512) void batch_kernel(const BatchTaskDev* __restrict__ tasks,
+__global__ __launch_bounds__(512, (edge_waves<N, R>())) void batch_kernel(const BatchTaskDev* __restrict__ tasks,
                                                     int32_t t_lo, int32_t t_hi,
                                                     const int64_t* __restrict__ item_off,
                                                     int32_t i_lo, int32_t i_hi,

@@ -27,6 +27,21 @@
 
 namespace tt {
 
+// The pointer as one to global memory. Loads through a pointer that was itself
+// read from memory (the task and job tables) are flat loads otherwise, whose
+// waits also drain the LDS reads in flight.
+template <class T>
+__device__ __forceinline__ T* global_ptr(T* p) {
+  typedef __attribute__((address_space(1))) T* G;
+  return (T*)reinterpret_cast<G>(reinterpret_cast<uintptr_t>(p));
+}
+
+// Orders the wave's LDS accesses: what its lanes wrote before is read after.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 constexpr int kMaxRankAny = 256;
 
 template <int R>
