@@ -24,6 +24,7 @@ struct tentaco_batch {
   uint32_t* d_rowbits = nullptr;  // per task, one bit per output row
   int32_t* d_counter = nullptr;
   int32_t* d_starts = nullptr;
+  float4** d_bnd_rows = nullptr;  // the rows zeroed before every run
   size_t brk_bytes = 0;
   tt::BatchLaunch L;
   std::vector<int64_t> h_fill, h_bnd;  // host prefix tables (ntasks + 1)
@@ -63,9 +64,11 @@ void free_tables(tentaco_batch* b) {
   (void)hipFree(b->d_bnd_off);
   (void)hipFree(b->d_item_off);
   (void)hipFree(b->d_starts);
+  (void)hipFree(b->d_bnd_rows);
   b->d_tasks = nullptr;
   b->d_bnd_off = b->d_item_off = nullptr;
   b->d_starts = nullptr;
+  b->d_bnd_rows = nullptr;
   b->brk_bytes = 0;
 }
 
@@ -110,6 +113,7 @@ int configure_tables(tentaco_batch* b) {
   if (!rc) rc = dev_alloc(&b->d_bnd_off, size_t(b->ntasks));
   if (!rc) rc = dev_alloc(&b->d_item_off, size_t(b->ntasks) + 1);  // + the total
   if (!rc) rc = dev_alloc(&b->d_starts, size_t(start_off[b->ntasks]));
+  if (!rc) rc = dev_alloc(&b->d_bnd_rows, size_t(bnd[b->ntasks]) * 2);
   if (rc) return rc;
   for (int t = 0; t < b->ntasks; ++t) b->host_tasks[t].starts = b->d_starts + start_off[t];
   TT_HIP_CHECK(hipMemcpy(b->d_tasks, b->host_tasks.data(), sizeof(BatchTaskDev) * b->ntasks,
@@ -125,6 +129,7 @@ int configure_tables(tentaco_batch* b) {
   L.ntasks = b->ntasks;
   L.bnd_off = b->d_bnd_off;
   L.total_bnd = bnd[b->ntasks];
+  L.bnd_rows = b->d_bnd_rows;
   L.item_off = b->d_item_off;
   L.total_items = int32_t(item[b->ntasks]);
   L.counter = b->d_counter;
@@ -278,8 +283,12 @@ int tentaco_batch_set_operands(tentaco_batch* b, const float* const* factors_dev
   b->h_fill = fill;
   b->L.h_fill_off = b->h_fill.data();
   b->have_operands = true;
-  if (b->L.blk[kMaxOrder] == 0)  // never configured: edge-parallel, 256 threads, group 16
-    for (int N = 0; N <= kMaxOrder; ++N) set_tile(b, N, kEdgeParallel, 256, 16);
+  if (b->L.blk[kMaxOrder] == 0) {  // never configured
+    int64_t nnz = 0;
+    for (const tentaco_csf* h : b->tasks) nnz += h->nodes[h->order - 1];
+    const int group = batch_group(nnz, b->R);
+    for (int N = 0; N <= kMaxOrder; ++N) set_tile(b, N, kEdgeParallel, 256, group);
+  }
   rc = configure_tables(b);
   if (rc) return rc;
   return zero_retained_outputs(b);

@@ -74,6 +74,9 @@ int default_variant();
 // Lanes that share one factor row for rank R (float4 per lane); 16 for the
 // generic (non-specialised) rank path.
 int lanes_per_row(int R);
+// Nonzeros per lane group of a batch tile of 256 threads that nobody chose,
+// for tasks of nnz nonzeros in all.
+int batch_group(int64_t nnz, int R);
 // Nonzeros one workgroup covers for an edge-family variant at rank R.
 int64_t nnz_per_block(const Variant& vr, int R);
 // Workspace bytes an MTTKRP call with a_rows output rows needs (0 for the
@@ -244,6 +247,7 @@ struct BatchLaunch {
   int64_t total_fill = 0;
   const int64_t* bnd_off = nullptr;     // device, prefix of (items+1) per task
   int64_t total_bnd = 0;
+  float4** bnd_rows = nullptr;          // device, two output rows (or null) per boundary
   const int64_t* item_off = nullptr;    // device, prefix of items per task (ntasks + 1)
   int32_t total_items = 0;
   int32_t* counter = nullptr;           // device work counter

@@ -170,11 +170,6 @@ __device__ __forceinline__ int32_t root_of_position(const CsfDev& B, int32_t p) 
   return key;
 }
 
-__device__ __forceinline__ void zero_row(float* A, int64_t row, int R) {
-  float4* A4 = reinterpret_cast<float4*>(A + row * R);
-  for (int q = 0; q < (R >> 2); ++q) A4[q] = make_float4(0.f, 0.f, 0.f, 0.f);
-}
-
 // What a batch prep launch does (bits): zero the output rows no root node
 // stores, write the brackets, zero the rows of the slices at item boundaries.
 constexpr int kPrepFill = 1, kPrepBrackets = 2, kPrepBoundary = 4;
@@ -190,11 +185,14 @@ struct BatchNB {
 // order's work counter; with kPrepFill zero the outputs (quads [q_lo,
 // q_hi)), skipping a row whose bit is set in the task's rowbits, because a
 // root node with nonzeros stores it; with kPrepBrackets write where the waves
-// of each item start (entries [b_lo, b_hi)); with kPrepBoundary zero the row of each slice
-// holding position b*NB or b*NB - 1 of a boundary b: those are the
+// of each item start (entries [b_lo, b_hi)) and, per boundary b, the output
+// rows of the slices holding positions b*NB and b*NB - 1: those are the
 // edge-parallel walk's only atomically updated rows (the slices holding an
-// item's first and last nonzero). Without kPrepBrackets the boundary rows
-// come from the starts written before.
+// item's first and last nonzero); with kPrepBoundary zero the listed rows.
+// The list (two row addresses per boundary, null where an earlier boundary
+// lists the row) depends on the CSFs, outputs and tiles only; finding the
+// rows on every run took 17 us a launch in a CP-ALS sweep over three tensors,
+// reading the list 4 us.
 __global__ __launch_bounds__(256) void batch_prep_kernel(const BatchTaskDev* __restrict__ tasks,
                                                          int32_t t_lo, int32_t t_hi,
                                                          const int64_t* __restrict__ fill_off,
@@ -203,7 +201,8 @@ __global__ __launch_bounds__(256) void batch_prep_kernel(const BatchTaskDev* __r
                                                          int64_t b_lo, int64_t b_hi,
                                                          int32_t* __restrict__ counter,
                                                          int n_lo, int n_hi, BatchNB nbs, int R,
-                                                         int qshift, int mode) {
+                                                         int qshift, int mode,
+                                                         float4** __restrict__ bnd_rows) {
   const int64_t tid = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const int64_t nthr = int64_t(gridDim.x) * blockDim.x;
   // the work counters of order groups [n_lo, n_hi)
@@ -262,42 +261,45 @@ __global__ __launch_bounds__(256) void batch_prep_kernel(const BatchTaskDev* __r
         if (dst[u] && !((w[u] >> sh[u]) & 1u)) *dst[u] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
   }
+  if (mode & kPrepBoundary) {
+    const int64_t n = (b_hi - b_lo) << (qshift + 1);
+    for (int64_t i = tid; i < n; i += nthr) {
+      float4* row = bnd_rows[2 * b_lo + (i >> qshift)];
+      if (row) row[i & ((1 << qshift) - 1)] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  }
+  if (!(mode & kPrepBrackets)) return;
   for (int64_t i = b_lo + tid; i < b_hi; i += nthr) {
     const int32_t t = t_lo + upper_index(bnd_off + t_lo, nt, i);
     const BatchTaskDev& T = tasks[t];
+    bnd_rows[2 * i] = bnd_rows[2 * i + 1] = nullptr;
     if (T.B.nnz <= 0) continue;
     const int64_t bi = i - bnd_off[t];
     const int N = T.B.order;
     const int32_t NB = nbs.nb[N];
-    int64_t p = bi * int64_t(NB);
-    if (p > T.B.nnz - 1) p = T.B.nnz - 1;
-    int32_t key = int32_t(p);
     const int32_t nw = nbs.nw[N];
-    if (mode & kPrepBrackets) {
-      // the starts of the item's waves
-      for (int w = 0; w < nw; ++w) {
-        key = int32_t(min(bi * int64_t(NB) + w * (NB / nw), int64_t(T.B.nnz) - 1));
-        for (int m = N - 2; m >= 0; --m) {
-          const int32_t x = search_le(T.B.pos[m + 1], 0, T.B.nodes[m] - 1, key);
-          T.starts[(bi * nw + w) * (N - 1) + m] = x;
-          key = x;
-        }
+    // the starts of the item's waves
+    for (int w = 0; w < nw; ++w) {
+      int32_t key = int32_t(min(bi * int64_t(NB) + w * (NB / nw), int64_t(T.B.nnz) - 1));
+      for (int m = N - 2; m >= 0; --m) {
+        const int32_t x = search_le(T.B.pos[m + 1], 0, T.B.nodes[m] - 1, key);
+        T.starts[(bi * nw + w) * (N - 1) + m] = x;
+        key = x;
       }
     }
-    key = T.starts[bi * nw * (N - 1)];  // the root node holding position p
-    if (mode & kPrepBoundary) {
-      zero_row(T.A, T.B.crd0[key], R);
-      // position p - 1 (the previous item's last nonzero) lies in another
-      // slice only when slice `key` starts exactly at p; its first nonzero
-      // is found by descending the pos arrays
-      if (bi > 0 && p > 0 && p == bi * int64_t(NB)) {
-        int32_t first = key;
-        for (int m = 1; m < N; ++m) first = T.B.pos[m][first];
-        if (first == p) {
-          const int32_t x1 = root_of_position(T.B, int32_t(p - 1));
-          if (x1 != key) zero_row(T.A, T.B.crd0[x1], R);
-        }
-      }
+    // the boundary's rows: the slice of position p, and that of p - 1 (the
+    // previous item's last nonzero), another one only when p is a slice's
+    // first position
+    const int64_t p = min(bi * int64_t(NB), int64_t(T.B.nnz) - 1);
+    const int32_t here = T.starts[bi * nw * (N - 1)];
+    const int32_t prev = bi > 0 ? root_of_position(T.B, int32_t((bi - 1) * NB)) : -1;
+    auto row_of = [&](int32_t x) {
+      return reinterpret_cast<float4*>(T.A + int64_t(T.B.crd0[x]) * R);
+    };
+    if (here != prev) bnd_rows[2 * i] = row_of(here);
+    if (bi > 0 && p == bi * int64_t(NB)) {
+      const int32_t before = root_of_position(T.B, int32_t(p - 1));
+      if (before != here && before != prev) bnd_rows[2 * i + 1] = row_of(before);
     }
   }
 }
@@ -326,8 +328,9 @@ int launch_batch_prep_range(const BatchLaunch& L, int n_lo, int n_hi, hipStream_
   const int64_t f0 = L.h_fill_off[t_lo], f1 = L.h_fill_off[t_hi];
   const int64_t b0 = L.h_bnd_off[t_lo], b1 = L.h_bnd_off[t_hi];
   const int64_t fill_quads = (mode & kPrepFill) ? (f1 - f0) >> 2 : 0;
-  const int64_t work = std::max<int64_t>(fill_quads, b1 - b0);
   const int qshift = L.R == 16 ? 2 : L.R == 32 ? 3 : 4;  // log2(R / 4), R in {16, 32, 64}
+  const int64_t work = std::max<int64_t>(
+      fill_quads, (mode & kPrepBoundary) ? (b1 - b0) << (qshift + 1) : b1 - b0);
   BatchNB nbs{};
   for (int N = 0; N <= kMaxOrder; ++N) {
     nbs.nb[N] = L.nb[N];
@@ -335,7 +338,7 @@ int launch_batch_prep_range(const BatchLaunch& L, int n_lo, int n_hi, hipStream_
   }
   batch_prep_kernel<<<grid_for(work, 256, 16384), 256, 0, st>>>(
       L.tasks, t_lo, t_hi, L.fill_off, f0 >> 2, f1 >> 2, L.bnd_off, b0, b1, L.counter, n_lo, n_hi,
-      nbs, L.R, qshift, mode);
+      nbs, L.R, qshift, mode, L.bnd_rows);
   TT_HIP_CHECK(hipGetLastError());
   return TENTACO_OK;
 }
@@ -571,6 +574,14 @@ Variant auto_tile(const CsfStats& s, int order, int R) {
   Variant t{kEdgeParallel, s.nnz < 300000 || large ? 512 : 256, 4};
   while (t.group < 64 && int64_t(groups) * t.group * 3 / 2 <= want) t.group *= 2;
   return edge_tile_fits(order, R, t) ? t : vr;
+}
+
+int batch_group(int64_t nnz, int R) {
+  // runs of 512 nonzeros a wave from 4M nonzeros in all, 256 below: at 256
+  // threads, 19.6M nonzeros, rank 32: group 64 547 us a replay, 16 669; 1.26M:
+  // 32 88, 64 103, 16 91; 19.6M, rank 16: 32 445, 64 542, 16 488
+  const int groups = 64 / lanes_per_row(R);
+  return std::min(64, (nnz >= 4000000 ? 512 : 256) / groups);
 }
 
 int lanes_per_row(int R) {
