@@ -30,6 +30,7 @@
 
 #include "handle.h"
 #include "internal.h"
+#include "rowops.h"
 
 namespace tt {
 namespace {
@@ -37,7 +38,10 @@ namespace {
 constexpr int kMaxR = 64;
 constexpr int kApplyRows = 64;    // rows per block of the apply / scale kernels
 constexpr int kStatRows = 2048;   // rows per block of the reduction kernels
-constexpr int kUpdRows = 4096;    // rows per block of the fused update kernel
+// Blocks of a mode step's fused update: the rows per block are chosen so that
+// about this many cover the chip without many partials to sum.
+constexpr int kUpdBlocks = 256;
+constexpr int kUpdUnit = 128;     // rows per block: a multiple of this
 
 struct CpdJob {
   const float* M = nullptr;  // MTTKRP result, rows x R
@@ -51,8 +55,16 @@ struct CpdJob {
   int32_t rows = 0;
   int32_t ablk0 = 0, nablk = 0;  // apply blocks (kApplyRows rows each)
   int32_t sblk0 = 0, nsblk = 0;  // reduction blocks (kStatRows rows each)
-  int32_t ublk0 = 0, nublk = 0;  // update blocks (kUpdRows rows each)
+  int32_t ublk0 = 0, nublk = 0;  // update blocks (urows rows each)
+  int32_t urows = 0;
 };
+
+// Sum over the wave, in a fixed order; every lane gets it.
+__device__ __forceinline__ double wave_sum_f64(double x) {
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) x += __shfl_xor(x, o);
+  return x;
+}
 
 __device__ __forceinline__ int find_job(const int32_t* __restrict__ off, int n, int32_t blk) {
   int lo = 0, hi = n - 1;  // largest j with off[j] <= blk
@@ -64,60 +76,60 @@ __device__ __forceinline__ int find_job(const int32_t* __restrict__ off, int n, 
   return lo;
 }
 
-// V = Hadamard product of the job's Grams; Vinv = V^-1 through Cholesky in
-// FP64. A non-positive pivot (a rank-deficient V) is lifted to 1e-12 times
-// the largest diagonal, which keeps the solve finite.
-__global__ __launch_bounds__(256) void hadamard_inverse_kernel(const CpdJob* __restrict__ jobs,
-                                                               int R) {
-  __shared__ double L[kMaxR][kMaxR + 1];
-  __shared__ float W[kMaxR][kMaxR + 1];  // L^-1 (lower triangle)
-  __shared__ double dmax;
+// V = Hadamard product of the job's Grams; Vinv = V^-1 by Gauss-Jordan
+// elimination in FP64 (V is symmetric positive semidefinite, so the diagonal
+// is the pivot). A pivot at or below 1e-12 times the largest diagonal (a
+// rank-deficient V) is lifted to that value, which keeps the solve finite; the
+// pivots are those of a Cholesky factorisation.
+//
+// A chain of R dependent steps bounds it, so a step is one barrier: every
+// thread keeps EPT entries of a row in registers, the owners of the step's
+// row and column publish them in one of two LDS buffers in turn, and every
+// thread eliminates its own entries. One workgroup per job, R*R / EPT threads.
+// (A Cholesky factorisation with a thread per pivot and a forward substitution
+// per column took 69 us at R = 32, this 18 us.)
+template <int R>
+__global__ __launch_bounds__(R * R / (R == 16 ? 1 : 4)) void hadamard_inverse_kernel(
+    const CpdJob* __restrict__ jobs) {
+  constexpr int EPT = R == 16 ? 1 : 4;
+  __shared__ double rowk[2][R], colk[2][R];
+  __shared__ double diag[R];
   const CpdJob& J = jobs[blockIdx.x];
-  for (int e = threadIdx.x; e < R * R; e += blockDim.x) {
-    const int i = e / R, j = e % R;
-    double v = 1.0;
-    for (int g = 0; g < J.nG; ++g) v *= double(J.Gk[g][e]);
-    L[i][j] = v;
+  const int i = int(threadIdx.x) / (R / EPT), j0 = int(threadIdx.x) % (R / EPT) * EPT;
+  double v[EPT];
+#pragma unroll
+  for (int u = 0; u < EPT; ++u) {
+    v[u] = 1.0;
+    for (int g = 0; g < J.nG; ++g) v[u] *= double(J.Gk[g][i * R + j0 + u]);
+    if (i == j0 + u) diag[i] = v[u];
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double m = 0.0;
-    for (int i = 0; i < R; ++i) m = fmax(m, L[i][i]);
-    dmax = m > 0.0 ? m : 1.0;
-  }
-  __syncthreads();
+  double dmax = 0.0;
+  for (int q = 0; q < R; ++q) dmax = fmax(dmax, diag[q]);
+  const double least = 1e-12 * (dmax > 0.0 ? dmax : 1.0);
   for (int k = 0; k < R; ++k) {
-    if (threadIdx.x == 0) {
-      double d = L[k][k];
-      for (int j = 0; j < k; ++j) d -= L[k][j] * L[k][j];
-      L[k][k] = sqrt(d > 1e-12 * dmax ? d : 1e-12 * dmax);
+    double* rk = rowk[k & 1];
+    double* ck = colk[k & 1];
+    if (i == k) {
+#pragma unroll
+      for (int u = 0; u < EPT; ++u) rk[j0 + u] = v[u];
     }
-    __syncthreads();
-    for (int i = k + 1 + threadIdx.x; i < R; i += blockDim.x) {
-      double s = L[i][k];
-      for (int j = 0; j < k; ++j) s -= L[i][j] * L[k][j];
-      L[i][k] = s / L[k][k];
-    }
-    __syncthreads();
-  }
-  // column c of L^-1 by forward substitution (one thread per column)
-  for (int c = threadIdx.x; c < R; c += blockDim.x) {
-    for (int i = 0; i < R; ++i) W[i][c] = 0.f;
-    W[c][c] = float(1.0 / L[c][c]);
-    for (int i = c + 1; i < R; ++i) {
-      double s = 0.0;
-      for (int j = c; j < i; ++j) s += L[i][j] * double(W[j][c]);
-      W[i][c] = float(-s / L[i][i]);
+#pragma unroll
+    for (int u = 0; u < EPT; ++u)
+      if (j0 + u == k) ck[i] = v[u];
+    __syncthreads();  // (the other buffer's readers are past the last barrier)
+    const double d = rk[k];
+    const double p = 1.0 / (d > least ? d : least);
+    const double f = ck[i] * p;
+#pragma unroll
+    for (int u = 0; u < EPT; ++u) {
+      const int j = j0 + u;
+      if (i == k) v[u] = j == k ? p : v[u] * p;
+      else v[u] = j == k ? -f : v[u] - f * rk[j];
     }
   }
-  __syncthreads();
-  // V^-1 = L^-T L^-1
-  for (int e = threadIdx.x; e < R * R; e += blockDim.x) {
-    const int i = e / R, j = e % R;
-    double s = 0.0;
-    for (int k = max(i, j); k < R; ++k) s += double(W[k][i]) * double(W[k][j]);
-    J.Vinv[e] = float(s);
-  }
+#pragma unroll
+  for (int u = 0; u < EPT; ++u) J.Vinv[i * R + j0 + u] = float(v[u]);
 }
 
 // Gram partials: part[block][i*R + j] = sum over the block's rows of
@@ -176,7 +188,7 @@ __global__ __launch_bounds__(256) void gram_reduce_kernel(const CpdJob* __restri
   }
 }
 
-// Pass 1 of a mode step, kUpdRows rows of one job per block, in tiles of
+// Pass 1 of a mode step, urows rows of one job per block, in tiles of
 // TR = 1024 / R rows (one float4 of M per thread per tile):
 //   A = M V^-1, written unnormalised;
 //   per-block FP64 partials of A^T A (FP32 within a tile), of the column
@@ -196,11 +208,11 @@ __global__ __launch_bounds__(256) void update_kernel(const CpdJob* __restrict__ 
   __shared__ __align__(16) float Vs[R][R];
   __shared__ float Ms[TR][R + 1];
   __shared__ float As[TR][R + 1];
-  __shared__ double red[256];
+  __shared__ double red[4];
   const int j = find_job(ublk0, njobs, blockIdx.x);
   const CpdJob& J = jobs[j];
-  const int32_t r0 = (int32_t(blockIdx.x) - J.ublk0) * kUpdRows;
-  const int32_t r1 = min(r0 + kUpdRows, J.rows);
+  const int32_t r0 = (int32_t(blockIdx.x) - J.ublk0) * J.urows;
+  const int32_t r1 = min(r0 + J.urows, J.rows);
   for (int e = threadIdx.x; e < R * R; e += 256) Vs[e / R][e % R] = J.Vinv[e];
   const int rr = int(threadIdx.x) / Q, q = int(threadIdx.x) % Q;
   double g[EPT];
@@ -263,30 +275,27 @@ __global__ __launch_bounds__(256) void update_kernel(const CpdJob* __restrict__ 
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < 4; ++u) As[rr][4 * q + u] = cmax[u];
-  red[threadIdx.x] = inner;
+  inner = wave_sum_f64(inner);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = inner;
   __syncthreads();
   if (threadIdx.x < R) {
     float mx = 0.f;
     for (int r = 0; r < TR; ++r) mx = fmaxf(mx, As[r][threadIdx.x]);
     pm[int64_t(blockIdx.x) * R + threadIdx.x] = double(mx);
   }
-  if (threadIdx.x == 0) {
-    double sacc = 0.0;
-    for (int t = 0; t < 256; ++t) sacc += red[t];
-    pi[blockIdx.x] = sacc;
-  }
+  if (threadIdx.x == 0) pi[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
 }
 
 // update_kernel for R = 32 on the matrix cores. Each wave takes 32-row tiles
-// (tile w + 4k of the block); per tile:
+// (tile w + 4k of the block) on its own, the next tile's M loaded while this
+// one is computed; per tile:
 //   A = M V^-1 as 16 v_mfma_f32_32x32x2f32 steps (operands from LDS: M tile
 //   and V^-1), then A^T A as 16 more on the A tile staged in LDS; the Gram
 //   accumulators are added into FP64 registers after every tile.
 // Accumulator layout of the 32x32 result: lane l holds column l % 32 and,
 // in register r, row (r % 4) + 4 * (l / 32) + 8 * (r / 4). Operand layout:
 // lane l supplies A[l % 32][k = l / 32] and B[k = l / 32][l % 32] for the
-// step's two k values. The loop is uniform over the block (idle tiles are
-// zero rows), so its barriers are reached by every wave.
+// step's two k values.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 __global__ __launch_bounds__(256) void update32_mfma_kernel(const CpdJob* __restrict__ jobs,
@@ -300,38 +309,48 @@ __global__ __launch_bounds__(256) void update32_mfma_kernel(const CpdJob* __rest
   __shared__ float Ts[W][32][R + 1];  // per wave: the M tile, then the A tile
   __shared__ double Gs[R][R];         // cross-wave Gram reduction
   __shared__ float Cm[W][64];
-  __shared__ double Is[W][64];
+  __shared__ double Is[W];
   const int j = find_job(ublk0, njobs, blockIdx.x);
   const CpdJob& J = jobs[j];
-  const int32_t r0 = (int32_t(blockIdx.x) - J.ublk0) * kUpdRows;
-  const int32_t r1 = min(r0 + kUpdRows, J.rows);
+  const int32_t r0 = (int32_t(blockIdx.x) - J.ublk0) * J.urows;
+  const int32_t r1 = min(r0 + J.urows, J.rows);
   const int lane = int(threadIdx.x) & 63;
   const int w = int(threadIdx.x) >> 6;
   const int col = lane & 31, half = lane >> 5;
-  for (int e = threadIdx.x; e < R * R; e += 256) Vs[e / R][e % R] = J.Vinv[e];
+  const float* __restrict__ M = global_ptr(J.M);
+  float* __restrict__ A = global_ptr(J.A);
+  const float* __restrict__ Vinv = global_ptr(J.Vinv);
+  for (int e = threadIdx.x; e < R * R; e += 256) Vs[e / R][e % R] = Vinv[e];
   double gd[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) gd[r] = 0.0;
   float cmax = 0.f;
   double inner = 0.0;
-  const int32_t ntiles = (r1 - r0 + 31) / 32;
-  const int32_t rounds = (ntiles + W - 1) / W;
-  for (int32_t k = 0; k < rounds; ++k) {
-    const int32_t t0 = r0 + (k * W + w) * 32;  // this wave's tile
-    __syncthreads();  // previous readers of Ts are done (and Vs is loaded)
-    // M tile -> LDS: 32 rows x 32 floats, float4 per lane, 4 passes
+  // M tile: 32 rows x 32 floats, float4 per lane, 4 passes
+  float4 mt[4];
+  auto load_tile = [&](int32_t t0) {
 #pragma unroll
     for (int pss = 0; pss < 4; ++pss) {
       const int e = pss * 64 + lane;  // float4 index in the tile
-      const int rr = e >> 3, q = e & 7;
-      float4 m4 = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (t0 + rr < r1) m4 = *reinterpret_cast<const float4*>(J.M + int64_t(t0 + rr) * R + 4 * q);
-      Ts[w][rr][4 * q] = m4.x;
-      Ts[w][rr][4 * q + 1] = m4.y;
-      Ts[w][rr][4 * q + 2] = m4.z;
-      Ts[w][rr][4 * q + 3] = m4.w;
+      const int32_t row = t0 + (e >> 3);
+      mt[pss] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (row < r1) mt[pss] = *reinterpret_cast<const float4*>(M + int64_t(row) * R + 4 * (e & 7));
     }
-    __syncthreads();
+  };
+  load_tile(r0 + w * 32);
+  __syncthreads();  // Vs is loaded
+  for (int32_t t0 = r0 + w * 32; t0 < r1; t0 += W * 32) {
+#pragma unroll
+    for (int pss = 0; pss < 4; ++pss) {
+      const int e = pss * 64 + lane;
+      float* row = &Ts[w][e >> 3][4 * (e & 7)];
+      row[0] = mt[pss].x;
+      row[1] = mt[pss].y;
+      row[2] = mt[pss].z;
+      row[3] = mt[pss].w;
+    }
+    wave_lds_sync();
+    if (t0 + W * 32 < r1) load_tile(t0 + W * 32);
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
@@ -346,18 +365,18 @@ __global__ __launch_bounds__(256) void update32_mfma_kernel(const CpdJob* __rest
     for (int r = 0; r < 16; ++r) {
       const int i = (r & 3) + 4 * half + 8 * (r >> 2);
       if (t0 + i < r1) {
-        J.A[int64_t(t0 + i) * R + col] = acc[r];
+        A[int64_t(t0 + i) * R + col] = acc[r];
         cmax = fmaxf(cmax, fabsf(acc[r]));
         inner += double(Ts[w][i][col]) * double(acc[r]);
       }
     }
-    __syncthreads();  // every lane has read its M values
+    wave_lds_sync();  // every lane has read its M values
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int i = (r & 3) + 4 * half + 8 * (r >> 2);
       Ts[w][i][col] = (t0 + i < r1) ? acc[r] : 0.f;
     }
-    __syncthreads();
+    wave_lds_sync();
     f32x16 g;
 #pragma unroll
     for (int r = 0; r < 16; ++r) g[r] = 0.f;
@@ -368,6 +387,7 @@ __global__ __launch_bounds__(256) void update32_mfma_kernel(const CpdJob* __rest
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) gd[r] += double(g[r]);
+    wave_lds_sync();  // the tile's readers are done
   }
   // the block's partials, waves summed in order
   for (int ww = 0; ww < W; ++ww) {
@@ -381,7 +401,8 @@ __global__ __launch_bounds__(256) void update32_mfma_kernel(const CpdJob* __rest
     }
   }
   Cm[w][lane] = cmax;
-  Is[w][lane] = inner;
+  inner = wave_sum_f64(inner);
+  if (lane == 0) Is[w] = inner;
   __syncthreads();
   for (int e = threadIdx.x; e < R * R; e += 256) pg[int64_t(blockIdx.x) * R * R + e] = Gs[e / R][e % R];
   if (threadIdx.x < R) {
@@ -389,58 +410,71 @@ __global__ __launch_bounds__(256) void update32_mfma_kernel(const CpdJob* __rest
     for (int ww = 0; ww < W; ++ww) mx = fmaxf(mx, fmaxf(Cm[ww][threadIdx.x], Cm[ww][threadIdx.x + 32]));
     pm[int64_t(blockIdx.x) * R + threadIdx.x] = double(mx);
   }
-  if (threadIdx.x == 0) {
-    double sacc = 0.0;
-    for (int ww = 0; ww < W; ++ww)
-      for (int l = 0; l < 64; ++l) sacc += Is[ww][l];
-    pi[blockIdx.x] = sacc;
-  }
+  if (threadIdx.x == 0) pi[blockIdx.x] = ((Is[0] + Is[1]) + Is[2]) + Is[3];
 }
 
-// Per job and chunk of 256 Gram entries (grid = jobs x ceil(R*R / 256)):
-// lambda (2-norms from the Gram diagonal on the first sweep, else
+// Per job and chunk of 256 Gram entries (grid = jobs x ceil(R*R / 256), 1024
+// threads): lambda (2-norms from the Gram diagonal on the first sweep, else
 // max(1, max |a|)), the Gram of the normalised factor G = (A^T A) ./
-// (lambda lambda^T), and the fit's inner product; partials in block order.
-// Every block of a job computes the same lambda; the chunk-0 block stores it.
-__global__ __launch_bounds__(256) void finish_kernel(const CpdJob* __restrict__ jobs, int R,
-                                                     int use_max,
-                                                     const double* __restrict__ pg,
-                                                     const double* __restrict__ pm,
-                                                     const double* __restrict__ pi) {
+// (lambda lambda^T), and the fit's inner product. The partials of an entry
+// are summed in four contiguous segments by four threads, each in block order,
+// and the segments in order, so the results do not depend on scheduling. Every
+// block of a job computes the same lambda; the chunk-0 block stores it.
+__global__ __launch_bounds__(1024) void finish_kernel(const CpdJob* __restrict__ jobs, int R,
+                                                      int use_max,
+                                                      const double* __restrict__ pg,
+                                                      const double* __restrict__ pm,
+                                                      const double* __restrict__ pi) {
+  __shared__ double part[4][256];
   __shared__ double lam[kMaxR];
   const int chunks = (R * R + 255) / 256;
   const int chunk = int(blockIdx.x) % chunks;
   const CpdJob& J = jobs[blockIdx.x / chunks];
-  // sums in block order; eight partials are loaded ahead of their adds
-  auto ordered_sum = [&](const double* base, int64_t stride) {
+  const int t = int(threadIdx.x) & 255, seg = int(threadIdx.x) >> 8;
+  const int per = (J.nublk + 3) / 4;
+  const int b0 = min(seg * per, J.nublk), b1 = min(b0 + per, J.nublk);
+  // this segment's partials, sixteen loaded ahead of their adds
+  auto segment = [&](const double* base, int64_t stride, auto&& add) {
     double s = 0.0;
-    int b = 0;
-    for (; b + 8 <= J.nublk; b += 8) {
-      double v[8];
+    int b = b0;
+    for (; b + 16 <= b1; b += 16) {
+      double v[16];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = base[int64_t(J.ublk0 + b + u) * stride];
+      for (int u = 0; u < 16; ++u) v[u] = base[int64_t(J.ublk0 + b + u) * stride];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) s += v[u];
+      for (int u = 0; u < 16; ++u) s = add(s, v[u]);
     }
-    for (; b < J.nublk; ++b) s += base[int64_t(J.ublk0 + b) * stride];
+    for (; b < b1; ++b) s = add(s, base[int64_t(J.ublk0 + b) * stride]);
     return s;
   };
-  for (int c = threadIdx.x; c < R; c += blockDim.x) {
-    const double sq = ordered_sum(pg + c * R + c, int64_t(R) * R);
-    double mx = 0.0;
-    for (int b = 0; b < J.nublk; ++b) mx = fmax(mx, pm[int64_t(J.ublk0 + b) * R + c]);
-    double l = use_max ? fmax(mx, 1.0) : sqrt(sq);
+  auto plus = [](double x, double y) { return x + y; };
+  auto larger = [](double x, double y) { return fmax(x, y); };
+  // lambda
+  if (t < R) part[seg][t] = use_max ? segment(pm + t, R, larger)
+                                    : segment(pg + t * R + t, int64_t(R) * R, plus);
+  __syncthreads();
+  if (int(threadIdx.x) < R) {
+    double l;
+    if (use_max) l = fmax(fmax(fmax(part[0][t], part[1][t]), fmax(part[2][t], part[3][t])), 1.0);
+    else l = sqrt(((part[0][t] + part[1][t]) + part[2][t]) + part[3][t]);
     if (!(l > 0.0)) l = 1.0;
-    lam[c] = double(float(l));
-    if (chunk == 0) J.lam[c] = float(l);
+    lam[t] = double(float(l));
+    if (chunk == 0) J.lam[t] = float(l);
   }
   __syncthreads();
-  const int e = chunk * 256 + int(threadIdx.x);
-  if (e < R * R) {
-    const double s = ordered_sum(pg + e, int64_t(R) * R);
+  const int e = chunk * 256 + t;
+  if (e < R * R) part[seg][t] = segment(pg + e, int64_t(R) * R, plus);
+  __syncthreads();
+  if (seg == 0 && e < R * R) {
+    const double s = ((part[0][t] + part[1][t]) + part[2][t]) + part[3][t];
     J.G[e] = float(s / (lam[e / R] * lam[e % R]));
   }
-  if (chunk == 0 && threadIdx.x == 0 && J.inner) *J.inner = ordered_sum(pi, 1);
+  if (chunk == 0 && J.inner) {
+    __syncthreads();
+    if (t == 0) part[seg][0] = segment(pi, 1, plus);
+    __syncthreads();
+    if (threadIdx.x == 0) *J.inner = ((part[0][0] + part[1][0]) + part[2][0]) + part[3][0];
+  }
 }
 
 // A /= lambda over every job's rows, float4 at a time (kApplyRows rows per
@@ -511,6 +545,10 @@ struct tentaco_cpd {
   // partials of the fused update (Gram, column max, inner product)
   double *upg = nullptr, *upm = nullptr, *upi = nullptr;
   hipStream_t own = nullptr;
+  // V^-1 needs only the other modes' Grams: it runs beside the batched MTTKRP
+  // on this stream (default priority), forked from and joined to the sweep's
+  hipStream_t side = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr;
 
   ~tentaco_cpd() {
     for (auto& s : step) {
@@ -534,6 +572,9 @@ struct tentaco_cpd {
     (void)hipFree(upi);
     (void)hipFree(d_inner);
     if (own) (void)hipStreamDestroy(own);
+    if (side) (void)hipStreamDestroy(side);
+    if (fork) (void)hipEventDestroy(fork);
+    if (join) (void)hipEventDestroy(join);
   }
 };
 
@@ -551,6 +592,10 @@ int build_jobs(tentaco_cpd* c, int m, const std::vector<int>& tensors, std::vect
   if (ublk0) ublk0->clear();
   nablk = nsblk = 0;
   int32_t nu = 0;
+  int64_t total = 0;
+  for (int t : tensors) total += c->dims[size_t(t)][size_t(m)];
+  const int64_t per = (total + kUpdBlocks - 1) / kUpdBlocks;
+  const int32_t urows = int32_t((per + kUpdUnit - 1) / kUpdUnit * kUpdUnit);
   for (int t : tensors) {
     CpdJob J;
     J.M = c->M[size_t(t)][size_t(m)];
@@ -566,7 +611,8 @@ int build_jobs(tentaco_cpd* c, int m, const std::vector<int>& tensors, std::vect
     J.sblk0 = nsblk;
     J.nsblk = (J.rows + kStatRows - 1) / kStatRows;
     J.ublk0 = nu;
-    J.nublk = (J.rows + kUpdRows - 1) / kUpdRows;
+    J.urows = urows;
+    J.nublk = (J.rows + urows - 1) / urows;
     // the fit needs <X, model> from each tensor's last mode update
     if (c->d_inner && m == c->order[size_t(t)] - 1) J.inner = c->d_inner + t;
     ablk0.push_back(J.ablk0);
@@ -756,7 +802,6 @@ int tentaco_cpd_create(tentaco_csf* const* handles, const int* level_modes, int 
     }
     int rc = tentaco_batch_create(tasks.data(), int(tasks.size()), R, &S.batch);
     if (!rc) rc = tentaco_batch_set_operands(S.batch, facs.data(), outs.data(), rows.data());
-    if (!rc) rc = tentaco_batch_configure(S.batch, 1, 128, 64);
     if (!rc) rc = tentaco_batch_set_output_mode(S.batch, TENTACO_BATCH_OUTPUTS_RETAINED);
     if (rc) return bail(rc);
     std::vector<int32_t> ab, sb, ub;
@@ -817,6 +862,11 @@ int tentaco_cpd_iterate(tentaco_cpd* c, int sweeps, int use_graphs, void* stream
     if (!c->own) TT_HIP_CHECK(hipStreamCreate(&c->own));
     st = c->own;
   }
+  if (!c->side) {
+    TT_HIP_CHECK(hipEventCreateWithFlags(&c->fork, hipEventDisableTiming));
+    TT_HIP_CHECK(hipEventCreateWithFlags(&c->join, hipEventDisableTiming));
+    TT_HIP_CHECK(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
+  }
   const int R = c->R;
   std::vector<double> inner(size_t(c->nt), 0.0);
   for (int it = 0; it < sweeps; ++it) {
@@ -826,19 +876,23 @@ int tentaco_cpd_iterate(tentaco_cpd* c, int sweeps, int use_graphs, void* stream
       if (S.tensors.empty()) continue;
       const int nj = int(S.jobs.size());
       int rc;
-      if (use_graphs) {
-        if (!S.captured) {
-          rc = tentaco_batch_capture(S.batch, st);
-          if (rc) return rc;
-          S.captured = true;
-        }
-        rc = tentaco_batch_launch(S.batch, st);
-      } else {
-        rc = tentaco_batch_run(S.batch, st);
+      if (use_graphs && !S.captured) {
+        rc = tentaco_batch_capture(S.batch, st);
+        if (rc) return rc;
+        S.captured = true;
       }
-      if (rc) return rc;
-      hadamard_inverse_kernel<<<nj, 256, 0, st>>>(S.d_jobs, R);
+      TT_HIP_CHECK(hipEventRecord(c->fork, st));
+      TT_HIP_CHECK(hipStreamWaitEvent(c->side, c->fork, 0));
+      switch (R) {
+        case 16: hadamard_inverse_kernel<16><<<nj, 256, 0, c->side>>>(S.d_jobs); break;
+        case 32: hadamard_inverse_kernel<32><<<nj, 256, 0, c->side>>>(S.d_jobs); break;
+        default: hadamard_inverse_kernel<64><<<nj, 1024, 0, c->side>>>(S.d_jobs); break;
+      }
       TT_HIP_CHECK(hipGetLastError());
+      TT_HIP_CHECK(hipEventRecord(c->join, c->side));
+      rc = use_graphs ? tentaco_batch_launch(S.batch, st) : tentaco_batch_run(S.batch, st);
+      if (rc) return rc;
+      TT_HIP_CHECK(hipStreamWaitEvent(st, c->join, 0));
       switch (R) {
         case 16:
           update_kernel<16><<<S.nublk, 256, 0, st>>>(S.d_jobs, S.d_ublk0, nj, c->upg, c->upm, c->upi);
@@ -852,7 +906,7 @@ int tentaco_cpd_iterate(tentaco_cpd* c, int sweeps, int use_graphs, void* stream
           break;
       }
       TT_HIP_CHECK(hipGetLastError());
-      finish_kernel<<<nj * ((R * R + 255) / 256), 256, 0, st>>>(S.d_jobs, R, use_max, c->upg,
+      finish_kernel<<<nj * ((R * R + 255) / 256), 1024, 0, st>>>(S.d_jobs, R, use_max, c->upg,
                                                                  c->upm, c->upi);
       TT_HIP_CHECK(hipGetLastError());
       scale4_kernel<<<S.nablk, 256, 0, st>>>(S.d_jobs, S.d_ablk0, nj, R);
@@ -920,6 +974,7 @@ int tentaco_cpd_set_factor(tentaco_cpd* c, int t, int m, const float* factor) {
 }
 
 int tentaco_cpd_free(tentaco_cpd* c) {
+  if (c && c->side) (void)hipStreamSynchronize(c->side);
   delete c;
   return TENTACO_OK;
 }
