@@ -374,16 +374,16 @@ def run_level_modes(tt, metrics, B, K):
         def lstep():
             H.mttkrp_level(L, fl, A, R)
 
-        # the level's transposed index, built once from B alone: leaf, one
-        # (level N-2 node, value) pair per nonzero plus the ancestors of the
-        # level N-2 nodes; inner, the level-L nodes with their ancestors
+        # the level's transposed index of this 3-mode tensor, built once from
+        # B alone: leaf, the nonzeros' coordinates and values; inner, the
+        # level-1 nodes' ranges and coordinates
         leaf = L == B.order - 1
         tt.synchronize()
         t0 = time.perf_counter()
         H.reserve_level(L)
         index = {"build_ms": round((time.perf_counter() - t0) * 1e3, 3),
-                 "device_bytes": (8 * B.nnz + 4 * (B.order - 1) * B.nodes(B.order - 2) if leaf
-                                  else 4 * (L + 1) * B.nodes(L)) + 4 * (B.dims[L] + 1)}
+                 "device_bytes": 4 * B.order * (B.nnz if leaf else B.nodes(B.order - 2))
+                 + 4 * (B.dims[L] + 1)}
         lstep()
         lms = time_steps(lstep, K)[0] / K
         got = A.numpy()
@@ -412,7 +412,7 @@ def run_level_modes(tt, metrics, B, K):
             "rooted_csf_device_bytes": int(sum(np.asarray(Bm.pos[m]).nbytes + np.asarray(Bm.crd[m]).nbytes
                                                for m in range(Bm.order)) + Bm.nnz * 4),
             "rel_l2_one_csf_vs_rooted_csf": rel_l2(got, Am.numpy()),
-            "one_csf_kernel": ("tleaf_kernel" if leaf else "inner_kernel") +
+            "one_csf_kernel": ("tleaf_kernel" if leaf else "inner_leaf_kernel") +
                               " (transposed level index, no atomics)",
             "level_index": index,
         }

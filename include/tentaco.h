@@ -419,8 +419,9 @@ int tentaco_mttkrp_dev_repeat(tentaco_csf* h, int R, const float* const* factors
  * the level's largest coordinate. Each level runs through a per-handle
  * transposed index of its nodes sorted by coordinate, built on the level's
  * first call outside stream capture or by tentaco_csf_reserve_level: 4 B
- * per coordinate plus, for the leaf level, 8 B per nonzero and 4(order-1)
- * B per level order-2 node, or, for an inner level L, 4(L+1) B per level-L
+ * per coordinate plus, for the leaf level, 4 order B per nonzero up to order 3
+ * and from there 8 B per nonzero and 4(order-1) B per level order-2 node, or,
+ * for an inner level, 4 order B per level order-2
  * node. Every row is then written once, without atomics, bitwise
  * reproducible. A call captured before its level's index exists zero-fills
  * A and accumulates with FP32 atomics instead.

@@ -125,18 +125,20 @@ int launch_mttkrp_level(const CsfDev& B, const FactorsDev& F, int level, int R, 
 // Per-handle transposed index of one level L >= 1 of a CSF, for the
 // MTTKRP of that level's mode on a CSF rooted elsewhere (one allocation):
 // tpos has dim + 1 entry offsets (entries sorted by level-L coordinate,
-// ties in CSF order). The leaf level (L = N-1) keeps per entry its level N-2
-// node and value bits (ent) and per level N-2 node the coordinates at
-// levels 0..N-2 (anc, N-1 per node). An inner level keeps per entry its
-// level-L node (node) and per level-L node the coordinates at levels
-// 0..L-1 (anc, L per node).
+// ties in CSF order). The leaf level (L = N-1) keeps per entry (ent) its
+// coordinates at levels 0..N-2 and value up to order 3, else its level N-2
+// node and value bits, and per level N-2 node the coordinates at levels
+// 0..N-2 (anc, N-1 per node). An inner level's entries are the level N-2
+// nodes by their ancestor's coordinate, each with its range of nonzeros
+// (node: the starts, then the ends) and its coordinates at the other levels
+// 0..N-2 (anc, level by level).
 struct LevelIndex {
   bool built = false;
   int level = 0;
   int32_t dim = 0;
   void* mem = nullptr;
   int32_t* tpos = nullptr;
-  uint2* ent = nullptr;
+  void* ent = nullptr;
   int32_t* node = nullptr;
   int32_t* anc = nullptr;
 };

@@ -629,19 +629,6 @@ size_t mttkrp_workspace_bytes(const CsfDev& B, int R, const Variant& vr, int32_t
   return brk + size_t(std::max<int32_t>(a_rows, 0)) * size_t(R) * sizeof(double);
 }
 
-int launch_mttkrp_inner(const CsfDev& B, const LevelIndex& X, const FactorsDev& F, int level,
-                        int R, float* A, int32_t a_rows, hipStream_t st) {
-  if (!X.built || X.level != level) return fail(TENTACO_EINVAL, "level %d index not built", level);
-  if (R <= 0 || R > kMaxRankAny)
-    return fail(TENTACO_EUNSUPPORTED, "rank R=%d outside 1..%d", R, kMaxRankAny);
-  switch (B.order) {
-    case 3: return order_inner<3>(B, X, F, level, R, A, a_rows, st);
-    case 4: return order_inner<4>(B, X, F, level, R, A, a_rows, st);
-    case 5: return order_inner<5>(B, X, F, level, R, A, a_rows, st);
-    default: return fail(TENTACO_EINVAL, "order %d has no inner level", B.order);
-  }
-}
-
 int launch_mttkrp_level(const CsfDev& B, const FactorsDev& F, int level, int R, float* A,
                         int32_t a_rows, hipStream_t st) {
   if (R <= 0 || R > kMaxRankAny)

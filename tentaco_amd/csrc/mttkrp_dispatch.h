@@ -38,9 +38,6 @@ int order_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A, int32_t 
                  bool dense_root, const Variant& vr, void* ws, const int32_t* starts,
                  hipStream_t st);
 template <int N>
-int order_inner(const CsfDev& B, const LevelIndex& X, const FactorsDev& F, int level, int R,
-                float* A, int32_t a_rows, hipStream_t st);
-template <int N>
 int order_level(const CsfDev& B, const FactorsDev& F, int level, int R, float* A, int32_t a_rows,
                 hipStream_t st);
 template <int N>

@@ -57,18 +57,6 @@ constexpr size_t edge_wave_lds() {
   return kRecBytes + kHistBytes + kFibBytes + Lay<R>::kMaxRank * sizeof(float);
 }
 
-// Inclusive sum over the lanes up to this one (DPP row shifts, then the rows'
-// last lanes broadcast to the next rows).
-__device__ __forceinline__ int32_t wave_scan_add(int32_t x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
-  return x;
-}
-
 // Largest x in [lo, hi] with a[x] <= key (requires a[lo] <= key), 64 probes a
 // step, uniform over the wave.
 __device__ __forceinline__ int32_t wave_search_le(const int32_t* __restrict__ a, int32_t lo,
@@ -678,71 +666,6 @@ __global__ __launch_bounds__(256) void level_kernel(CsfDev B, FactorsDev F, floa
       }
       RO::atomic_add(A, B.crd[L][y], c, Rr, out);
     }
-  }
-}
-
-// MTTKRP for the mode held at inner level L (1 <= L <= N-2) through the
-// per-handle transposed index of that level: the level-L nodes sorted by
-// coordinate (node[t], rows tpos[j]..tpos[j+1]) and, per node, the
-// coordinates of its ancestors at levels 0..L-1 (anc[y * L + m]). One
-// workgroup of 1-4 waves computes output row j: its row groups take the
-// row's nodes in turn, each adding (product of the node's ancestor rows) x
-// (sum of the node's children's subtrees), and the row is reduced over the
-// wave and the workgroup and stored once: no atomics, no zero fill,
-// bitwise reproducible.
-template <int N, int L, int R>
-__global__ __launch_bounds__(256) void inner_kernel(const int32_t* __restrict__ tpos, int32_t tdim,
-                                                    const int32_t* __restrict__ node,
-                                                    const int32_t* __restrict__ anc, CsfDev B,
-                                                    FactorsDev F, float* __restrict__ A, int Rr) {
-  using RO = Row<R>;
-  using V = typename RO::V;
-  constexpr int NV = RO::NV;
-  constexpr int LPR = RO::LPR;
-  constexpr int NG = 64 / LPR;
-  __shared__ __align__(16) float red[4][Lay<R>::kMaxRank];
-  const int32_t j = blockIdx.x;
-  const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
-  const int nwv = blockDim.x >> 6;
-  const int gi = lane / LPR;
-  const int c = lane % LPR;
-  V acc[NV];
-  RO::zero(acc);
-  if (j < tdim) {
-    const int32_t t1 = tpos[j + 1];
-    for (int32_t t = tpos[j] + wv * NG + gi; t < t1; t += NG * nwv) {
-      const int32_t y = node[t];
-      const int32_t* a = anc + int64_t(y) * L;
-      V above[NV];
-      RO::load(above, F.M[0], a[0], c, Rr);
-#pragma unroll
-      for (int m = 1; m < L; ++m) {
-        V r[NV];
-        RO::load(r, F.M[m], a[m], c, Rr);
-        RO::hmul(above, r);
-      }
-      V below[NV];
-      children_sum<N, L, R>(B, F, y, c, Rr, below);
-      RO::hfma(acc, above, below);
-    }
-  }
-  RO::wave_sum(acc);
-  if (nwv == 1) {
-    if (gi == 0) RO::store(A, j, c, Rr, acc);
-    return;
-  }
-  if (gi == 0) {
-    RO::put(red[wv], c, acc);
-  }
-  __syncthreads();
-  if (wv == 0 && gi == 0) {
-    for (int w = 1; w < nwv; ++w) {
-      V o[NV];
-      RO::get(red[w], c, o);
-      RO::add(acc, o);
-    }
-    RO::store(A, j, c, Rr, acc);
   }
 }
 
@@ -1359,37 +1282,6 @@ int launch_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A,
 }
 
 template <int N, int L, int R>
-int launch_inner_typed(const CsfDev& B, const LevelIndex& X, const FactorsDev& F, int Rr, float* A,
-                       int32_t a_rows, hipStream_t st) {
-  if (a_rows <= 0) return TENTACO_OK;
-  // 1-4 waves per row, from the mean level-L nodes per row
-  const int64_t mean = (int64_t(B.nodes[L]) + X.dim - 1) / std::max<int32_t>(X.dim, 1);
-  const int per_wave = 64 / Row<R>::LPR;
-  const int nwv = int(std::max<int64_t>(1, std::min<int64_t>(4, (mean + 4 * per_wave - 1) /
-                                                                   (4 * per_wave))));
-  ktimer_begin(st);
-  inner_kernel<N, L, R><<<a_rows, 64 * nwv, 0, st>>>(X.tpos, X.dim, X.node, X.anc, B, F, A, Rr);
-  TT_HIP_CHECK(hipGetLastError());
-  ktimer_end(st, "inner_kernel");
-  return TENTACO_OK;
-}
-
-template <int N, int R>
-int launch_inner_order(const CsfDev& B, const LevelIndex& X, const FactorsDev& F, int level,
-                       int Rr, float* A, int32_t a_rows, hipStream_t st) {
-  if constexpr (N >= 3) {
-    if (level == 1) return launch_inner_typed<N, 1, R>(B, X, F, Rr, A, a_rows, st);
-  }
-  if constexpr (N >= 4) {
-    if (level == 2) return launch_inner_typed<N, 2, R>(B, X, F, Rr, A, a_rows, st);
-  }
-  if constexpr (N >= 5) {
-    if (level == 3) return launch_inner_typed<N, 3, R>(B, X, F, Rr, A, a_rows, st);
-  }
-  return fail(TENTACO_EINVAL, "level %d is not an inner level of an order-%d tensor", level, N);
-}
-
-template <int N, int L, int R>
 int launch_level_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A, int32_t a_rows,
                        hipStream_t st) {
   const int64_t a_elems = int64_t(a_rows) * Rr;
@@ -1440,13 +1332,6 @@ int order_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A, int32_t 
 }
 
 template <int N>
-int order_inner(const CsfDev& B, const LevelIndex& X, const FactorsDev& F, int level, int R,
-                float* A, int32_t a_rows, hipStream_t st) {
-  return with_rank_layout(
-      R, [&](auto r) { return launch_inner_order<N, r()>(B, X, F, level, R, A, a_rows, st); });
-}
-
-template <int N>
 int order_level(const CsfDev& B, const FactorsDev& F, int level, int R, float* A, int32_t a_rows,
                 hipStream_t st) {
   return with_rank_layout(
@@ -1477,8 +1362,6 @@ int order_batch_occupancy(int family, int block, int R, int32_t NB, int* per_cu)
 #define TT_INSTANTIATE_ORDER(N)                                                                 \
   template int tt::order_mttkrp<N>(const CsfDev&, const FactorsDev&, int, float*, int32_t, bool, \
                                    const Variant&, void*, const int32_t*, hipStream_t);         \
-  template int tt::order_inner<N>(const CsfDev&, const LevelIndex&, const FactorsDev&, int, int, \
-                                  float*, int32_t, hipStream_t);                                \
   template int tt::order_level<N>(const CsfDev&, const FactorsDev&, int, int, float*, int32_t,  \
                                   hipStream_t);                                                 \
   template int tt::order_batch<N>(const BatchLaunch&, hipStream_t);                             \
