@@ -73,6 +73,16 @@ void free_handle(tentaco_csf* h) {
   delete h;
 }
 
+// Whether the paired slice layout is built for this handle: 3-mode short
+// fibres, packable coordinates, slices that pair within the slots, at most
+// twice the nonzeros in slots.
+bool pairs_apply(const tentaco_csf* h) {
+  if (h->order != 3) return false;
+  const int64_t nnz = h->nodes[2], np = int64_t(h->host_pairs.size() / 2);
+  return nnz * 4 <= int64_t(h->nodes[1]) * 5 && h->max_crd[1] < 65535 && h->max_crd[2] < 65535 &&
+         h->stats.max_slice_nnz <= kPairSlots && np > 0 && np * kPairSlots <= 2 * nnz;
+}
+
 // The 3-mode expansion (level-1 coordinate per nonzero, first nonzero per
 // root node) that the slice-row kernel's short-fibre path reads; built once,
 // on `st`.
@@ -129,8 +139,7 @@ int ensure_expand3(tentaco_csf* h, hipStream_t st) {
   // that fits), and at most twice the nonzeros in slots; optional
   static_assert(kPairCap == kPairSlots, "pairing capacity");
   const int32_t np = int32_t(h->host_pairs.size() / 2);
-  if (short_fibres && h->max_crd[1] < 65535 && h->max_crd[2] < 65535 &&
-      h->stats.max_slice_nnz <= kPairSlots && np > 0 && int64_t(np) * kPairSlots <= 2 * nnz) {
+  if (pairs_apply(h)) {
     // one allocation: slots, per-pair info, the pairs (kept with it)
     const size_t b_slots = size_t(np) * kPairSlots * sizeof(uint2);
     const size_t b_info = (size_t(np) * sizeof(int4) + 255) & ~size_t(255);
@@ -252,7 +261,7 @@ int resolve_variant(const tentaco_csf* h, int R, int variant) {
 // is resized to the tensor, anything else is the variant's own tile.
 Variant tile_of(const tentaco_csf* h, int R, int variant, int v) {
   if (variant == TENTACO_VARIANT_AUTO && h->tune.lookup(R) < 0)
-    return auto_tile(h->stats, h->order, R);
+    return auto_tile(h->stats, h->order, R, pairs_apply(h));
   return variant_of(v);
 }
 

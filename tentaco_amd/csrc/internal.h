@@ -58,7 +58,8 @@ enum Family { kEdgeSerial = 0, kEdgeParallel = 1, kSliceRow = 2 };
 struct Variant {
   int family;
   int block;  // threads per workgroup
-  int group;  // nonzeros per lane group (edge families); 0 for slice-row
+  int group;  // nonzeros per lane group (edge families); slice-row: 0, or the
+              // nonzeros a wave's slices start among (slice_group_kernel)
 };
 
 constexpr int kNumGridBlocks = 3;

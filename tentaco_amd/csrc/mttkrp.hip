@@ -556,8 +556,20 @@ int auto_variant(const CsfStats& s, int order, int R) {
   return 2 * per_family + 1;  // sr_b256 (always fits)
 }
 
-Variant auto_tile(const CsfStats& s, int order, int R) {
+Variant auto_tile(const CsfStats& s, int order, int R, bool paired) {
   const Variant vr = variant_of(auto_variant(s, order, R));
+  if (vr.family == kSliceRow) {
+    // 3-mode short fibres (the kernels over the expansion): the paired layout
+    // where it exists; else whole slices by the wave below 12 nonzeros a
+    // slice, one wave a slice up to 48 and two from there. Against the
+    // variant's 256 threads, us at rank 32 / 50: mean 8 nonzeros 49 -> 13 /
+    // 80 -> 21, mean 30 27 -> 15 / 46 -> 26, mean 60 15 -> 12 / 28 -> 21
+    if (order != 3 || s.nnz <= 0 || s.child_mean[2] > 1.25) return vr;
+    if (paired && (R == 16 || R == 32 || R == 64)) return vr;
+    const double mean = double(s.nnz) / std::max(s.nonempty_slices, 1);
+    if (mean < 12.0) return Variant{kSliceRow, vr.block, s.nnz < 500000 ? 64 : 128};
+    return Variant{kSliceRow, mean <= 48.0 ? 64 : 128, 0};
+  }
   if (vr.family != kEdgeParallel) return vr;
   // A wave's run of nonzeros is a serial chain, so up to about 3000 runs in
   // all (12 waves per CU) shorter runs are faster; beyond that more runs only

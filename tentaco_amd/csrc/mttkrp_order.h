@@ -907,6 +907,131 @@ __global__ __launch_bounds__(512) void slice_short_kernel(CsfDev B, FactorsDev F
   }
 }
 
+// Slice-row kernel for 3-mode tensors of short fibres and short slices, over
+// the expansion: a wave takes the consecutive slices that start among its WN
+// nonzeros (whole, the empty ones too), PB nonzeros at a time. Their products
+// val * C(k,:) (.) D(l,:) go to LDS with all rows in flight, and the row
+// groups then sum a slice each and store its row; a slice that runs past the
+// batch is carried to the next. No atomics, no zero fill on a dense root,
+// deterministic. A workgroup per slice (slice_short_kernel) leaves most of its
+// lanes idle below some 12 nonzeros a slice: 40000 slices of 7.5, rank 32:
+// 50 us a call with 256 threads a slice, 32 with 128, 13 here.
+template <int R>
+constexpr int group_batch() {
+  constexpr int p = 4096 / (Lay<R>::kMaxRank * 4);
+  return p > 64 ? 64 : Lay<R>::kMaxRank == 128 ? 16 : Lay<R>::kMaxRank == 256 ? 8 : p;
+}
+
+template <int R>
+__global__ __launch_bounds__(256) void slice_group_kernel(CsfDev B, FactorsDev F,
+                                                          float* __restrict__ A, int Rr,
+                                                          int32_t WN) {
+  using RO = Row<R>;
+  using V = typename RO::V;
+  constexpr int NV = RO::NV;
+  constexpr int LPR = RO::LPR;
+  constexpr int KR = Lay<R>::kMaxRank;
+  constexpr int NGW = 64 / LPR;
+  constexpr int PB = group_batch<R>();
+  constexpr int U = PB / NGW;
+  static_assert(U >= 1 && PB % NGW == 0, "whole steps");
+  __shared__ __align__(16) float lds[4][PB * KR];
+  const int lane = int(threadIdx.x) & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int gi = lane / LPR;
+  const int c = lane % LPR;
+  float* P = lds[wv];
+  const int32_t* __restrict__ nzr = B.nnz_of_root;
+  const int32_t* __restrict__ kq = B.crd1_of_nnz;
+  const int32_t* __restrict__ lq = B.crd[2];
+  const float* __restrict__ vq = B.vals;
+  const int32_t n0 = B.nodes[0];
+  const int32_t nnz = B.nnz;
+  const int64_t w = int64_t(blockIdx.x) * 4 + wv;
+  if (w * WN >= nnz) return;
+  // slices [x0, x1): those whose first nonzero is in [w*WN, (w+1)*WN); the
+  // first wave takes the leading empty ones, the last the trailing ones
+  const int64_t hi = (w + 1) * WN;
+  const int32_t x0 = w == 0 ? 0 : wave_search_le(nzr, 0, n0 - 1, int32_t(w * WN) - 1, lane) + 1;
+  const int32_t x1 =
+      hi >= nnz ? n0 : wave_search_le(nzr, max(x0 - 1, 0), n0 - 1, int32_t(hi) - 1, lane) + 1;
+  V carry[NV];
+  RO::zero(carry);
+  bool carried = false;
+  for (int32_t xb = x0; xb < x1; xb += 64) {
+    // a window of slices, one per lane
+    const int32_t nx = min(64, x1 - xb);
+    const int32_t x = min(xb + lane, x1 - 1);
+    const int32_t st = nzr[x];
+    const int32_t en = nzr[x + 1];
+    const int32_t row = B.crd0[x];
+    for (int32_t rb = 0; rb < nx; rb += NGW) {
+      const int32_t r = min(rb + gi, nx - 1);
+      const int32_t len = __shfl(en - st, r);
+      const int32_t rr = __shfl(row, r);
+      if (rb + gi < nx && len == 0) {
+        V z[NV];
+        RO::zero(z);
+        RO::store(A, rr, c, Rr, z);
+      }
+    }
+    const int32_t q0 = __builtin_amdgcn_readlane(st, 0);
+    const int32_t q1 = __builtin_amdgcn_readlane(en, nx - 1);
+    for (int32_t s0 = q0; s0 < q1; s0 += PB) {
+      const int32_t m = min(PB, q1 - s0);
+      V cr[U][NV], dr[U][NV];
+      float vt[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int32_t q = s0 + min(u * NGW + gi, m - 1);
+        vt[u] = vq[q];
+        RO::load(cr[u], F.M[1], kq[q], c, Rr);
+        RO::load(dr[u], F.M[2], lq[q], c, Rr);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        V p[NV];
+        RO::zero(p);
+        RO::axpy(p, vt[u], dr[u]);
+        RO::hmul(p, cr[u]);
+        if (u * NGW + gi < m) RO::put(P + (u * NGW + gi) * KR, c, p);
+      }
+      wave_lds_sync();
+      const int32_t s1 = s0 + m;
+      // slices that reach into the batch
+      const int32_t r0 = __popcll(__ballot(lane < nx && en <= s0));
+      const int32_t r1 = __popcll(__ballot(lane < nx && st < s1)) - 1;
+      V last[NV];
+      RO::zero(last);
+      for (int32_t rb = r0; rb <= r1; rb += NGW) {
+        const int32_t r = min(rb + gi, r1);
+        const int32_t a = max(__shfl(st, r), s0);
+        const int32_t b = __shfl(en, r);
+        const int32_t rr = __shfl(row, r);
+        if (rb + gi > r1) continue;
+        V sum[NV];
+        RO::zero(sum);
+        for (int32_t i = a; i < min(b, s1); ++i) {
+          V p[NV];
+          RO::get(P + (i - s0) * KR, c, p);
+          RO::add(sum, p);
+        }
+        if (r == r0 && carried) RO::add(sum, carry);
+        if (b > s1) RO::add(last, sum);
+        else if (a < b) RO::store(A, rr, c, Rr, sum);
+      }
+      carried = __builtin_amdgcn_readlane(en, r1) > s1;
+      if (carried) {
+        // to every row group: the next batch's first one adds it
+        RO::wave_sum(last);
+#pragma unroll
+        for (int j = 0; j < NV; ++j) carry[j] = last[j];
+      }
+      wave_lds_sync();
+    }
+  }
+}
+
 // Slice-row kernel over the padded layout: one workgroup of pad_width
 // threads per root node, each thread holding one slot, so the slice's
 // nonzeros are read at addresses fixed at launch (no offset load first).
@@ -1206,10 +1331,21 @@ int launch_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A,
     }
     if (B.nodes[0] > 0) {
       ktimer_begin(st);
-      if constexpr (N == 3 && R > 0) {
-        // short fibres (nnz <= 1.25 x fibres) with the expansion built: the
-        // kernel that skips the pos -> crd chain
-        if (B.crd1_of_nnz && int64_t(B.nnz) * 4 <= int64_t(B.nodes[1]) * 5) {
+      // short fibres (nnz <= 1.25 x fibres) with the expansion built: the
+      // kernels that skip the pos -> crd chain
+      const bool expanded =
+          N == 3 && B.crd1_of_nnz && int64_t(B.nnz) * 4 <= int64_t(B.nodes[1]) * 5 && B.nnz > 0;
+      if constexpr (N == 3) {
+        if (expanded && vr.group > 0) {
+          const int64_t waves = (int64_t(B.nnz) + vr.group - 1) / vr.group;
+          slice_group_kernel<R><<<int((waves + 3) / 4), 256, 0, st>>>(B, F, A, Rr, vr.group);
+          TT_HIP_CHECK(hipGetLastError());
+          ktimer_end(st, "slice_group_kernel");
+          return TENTACO_OK;
+        }
+      }
+      if constexpr (N == 3 && (R > 0 || Row<R>::NV == 1)) {
+        if (expanded) {
           if constexpr (R == 16 || R == 32 || R == 64) {
             if (B.pair && vr.block >= 256) {
               slice_pair_kernel<R><<<B.npairs, 128, 0, st>>>(B.pair, B.pair_info, F, A, Rr);
@@ -1218,21 +1354,23 @@ int launch_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A,
               return TENTACO_OK;
             }
           }
-          if (B.pad && B.pad_width <= vr.block && B.pad_width % 64 == 0 && B.pad_width <= 512) {
-            const int id = dense_root ? 1 : 0;
-            switch (B.pad_width / 64) {
-              case 1: slice_pad_kernel<R, 1><<<B.nodes[0], 64, 0, st>>>(B, F, A, Rr, id); break;
-              case 2: slice_pad_kernel<R, 2><<<B.nodes[0], 128, 0, st>>>(B, F, A, Rr, id); break;
-              case 3: slice_pad_kernel<R, 3><<<B.nodes[0], 192, 0, st>>>(B, F, A, Rr, id); break;
-              case 4: slice_pad_kernel<R, 4><<<B.nodes[0], 256, 0, st>>>(B, F, A, Rr, id); break;
-              case 5: slice_pad_kernel<R, 5><<<B.nodes[0], 320, 0, st>>>(B, F, A, Rr, id); break;
-              case 6: slice_pad_kernel<R, 6><<<B.nodes[0], 384, 0, st>>>(B, F, A, Rr, id); break;
-              case 7: slice_pad_kernel<R, 7><<<B.nodes[0], 448, 0, st>>>(B, F, A, Rr, id); break;
-              default: slice_pad_kernel<R, 8><<<B.nodes[0], 512, 0, st>>>(B, F, A, Rr, id); break;
+          if constexpr (R > 0) {
+            if (B.pad && B.pad_width <= vr.block && B.pad_width % 64 == 0 && B.pad_width <= 512) {
+              const int id = dense_root ? 1 : 0;
+              switch (B.pad_width / 64) {
+                case 1: slice_pad_kernel<R, 1><<<B.nodes[0], 64, 0, st>>>(B, F, A, Rr, id); break;
+                case 2: slice_pad_kernel<R, 2><<<B.nodes[0], 128, 0, st>>>(B, F, A, Rr, id); break;
+                case 3: slice_pad_kernel<R, 3><<<B.nodes[0], 192, 0, st>>>(B, F, A, Rr, id); break;
+                case 4: slice_pad_kernel<R, 4><<<B.nodes[0], 256, 0, st>>>(B, F, A, Rr, id); break;
+                case 5: slice_pad_kernel<R, 5><<<B.nodes[0], 320, 0, st>>>(B, F, A, Rr, id); break;
+                case 6: slice_pad_kernel<R, 6><<<B.nodes[0], 384, 0, st>>>(B, F, A, Rr, id); break;
+                case 7: slice_pad_kernel<R, 7><<<B.nodes[0], 448, 0, st>>>(B, F, A, Rr, id); break;
+                default: slice_pad_kernel<R, 8><<<B.nodes[0], 512, 0, st>>>(B, F, A, Rr, id); break;
+              }
+              TT_HIP_CHECK(hipGetLastError());
+              ktimer_end(st, "slice_pad_kernel");
+              return TENTACO_OK;
             }
-            TT_HIP_CHECK(hipGetLastError());
-            ktimer_end(st, "slice_pad_kernel");
-            return TENTACO_OK;
           }
           slice_short_kernel<R><<<B.nodes[0], vr.block, 0, st>>>(B, F, A, Rr);
           TT_HIP_CHECK(hipGetLastError());

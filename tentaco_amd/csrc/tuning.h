@@ -53,8 +53,9 @@ struct CsfStats {
 // root slices are many and even, edge-parallel otherwise.
 int auto_variant(const CsfStats& s, int order, int R);
 
-// The tile that choice runs: an edge-parallel variant resized to the
-// tensor, any other unchanged.
-Variant auto_tile(const CsfStats& s, int order, int R);
+// The tile that choice runs: an edge-parallel variant or the slice-row kernel
+// of short fibres resized to the tensor, any other unchanged. paired: the
+// handle's paired slice layout applies.
+Variant auto_tile(const CsfStats& s, int order, int R, bool paired);
 
 }  // namespace tt
