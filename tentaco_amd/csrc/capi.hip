@@ -174,7 +174,8 @@ int ensure_ttv_plan(tentaco_csf* h, hipStream_t st) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   TT_HIP_CHECK(hipStreamIsCapturing(st, &cs));
   if (cs != hipStreamCaptureStatusNone) return TENTACO_OK;
-  return build_ttv_plan(h->view(), h->max_crd[h->order - 1] + 1, h->ttv_bands, &h->ttv, st);
+  return build_ttv_plan(h->view(), h->max_crd[h->order - 1] + 1, h->ttv_bands,
+                        int64_t(h->stats.child_max[h->order - 1]), &h->ttv, st);
 }
 
 // Grow a device buffer to at least `bytes` (contents are not kept).

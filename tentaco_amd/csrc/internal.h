@@ -168,6 +168,7 @@ constexpr int kMaxBands = 8;
 struct TtvPlan {
   bool built = false;
   bool ok = false;             // the unit kernel applies
+  bool whole = false;          // few units, no long or empty fibre: whole fibres by the wave
   void* mem = nullptr;         // one allocation holding the arrays below
   // with empty fibres, the bitmap and unit table index the non-empty fibres
   // only: ne_fid maps them to output positions and empty_ids lists the
@@ -222,7 +223,9 @@ struct TtvPlan {
 // coordinate + 1); beyond 2^30 - 8 the plan does not apply. bands: 0 picks
 // (the banded layout when the best window of c would serve under 3/4 of the
 // gathers), 1 keeps one window, 2..kMaxBands forces that many bands.
-int build_ttv_plan(const CsfDev& B, int32_t cdim, int bands, TtvPlan* plan, hipStream_t stream);
+// max_fibre: the most nonzeros of a level N-2 node.
+int build_ttv_plan(const CsfDev& B, int32_t cdim, int bands, int64_t max_fibre, TtvPlan* plan,
+                   hipStream_t stream);
 void free_ttv_plan(TtvPlan* plan);
 // Enqueue one TTV through the unit kernel (plan.ok must hold): every entry of
 // y is written exactly once, with no atomics on y, so results are bitwise

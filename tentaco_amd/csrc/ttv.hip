@@ -3,8 +3,9 @@
 // are the innermost fibers. Replaces ttv_kernel / ttv_csf_gpu_taco
 // (tensor_kernels/ttv_csf_gpu_taco.h:2-121).
 //
-// Two kernels. The unit kernel (below, ttv_unit_kernel) is the main path: it
-// reads a per-handle fibre-start bitmap instead of searching pos, keeps a
+// Three kernels. Up to a million nonzeros without long or empty fibres,
+// ttv_unit_fibres_kernel sums whole fibres by the wave. The unit kernel (below,
+// ttv_unit_kernel) is the main path otherwise: it reads a per-handle fibre-start bitmap instead of searching pos, keeps a
 // window of c in LDS and writes every y entry exactly once (no zero fill, no
 // atomics); with empty fibres its plan indexes the non-empty ones and maps
 // them to output positions. The bracket kernel (ttv_kernel) covers calls
@@ -521,6 +522,108 @@ __global__ __launch_bounds__(kUnitThreads) void ttv_unit_kernel(
                                     stage_window<LC>(s_c, crs, k0, lc);
                                     __syncthreads();
                                   });
+}
+
+// The unit kernel for tensors of few units and no long fibre: a wave sums
+// whole fibres, those that start in its unit, so there is no crossing table
+// and no second launch, and waves need neither each other nor a window of c
+// (which L2 serves at these sizes). The unit's products go to LDS in FP64
+// (exact) and a lane sums a fibre; one of more than kFibreLane nonzeros, and
+// what the last fibre has past the unit, is summed by the whole wave. y is
+// written once per entry, coalesced, without atomics (bitwise reproducible).
+// Two dependent rounds of loads bound it: 200k nonzeros, 27k fibres: 5.3 us
+// against 8.5 for ttv_unit_kernel (25 workgroups of 16 waves) and its fold;
+// the plan takes 0.1 ms, bands another 0.5 to 2 ms.
+// kFibreLane: 8 11.1 us, 16 6.9, 24 6.1, 48 5.3, 100 5.5 (a wave's sum is 12
+// cross-lane moves of latency, a lane's a serial chain).
+// Taken up to kFibreUnits units, us of this and of ttv_unit_kernel (banded
+// where c is past its window): 24k nonzeros 4.8 and 7.7, 445k 7.0 and 20.9, 1M
+// 6.2 and 8.9 (c of 4000) or 9.2 and 15.4 (c of 150000), 2M 10.1 and 9.7 or
+// 13.8 and 16.3, 4M 17.2 and 14.0 or 24.6 and 19.4. And up to fibres of
+// kFibreMax nonzeros, since a wave sums the rest of its last fibre alone.
+constexpr int kFibreWaves = 4;
+constexpr int32_t kFibreUnits = 2048;
+constexpr int64_t kFibreMax = 2048;
+constexpr int32_t kFibreLane = 48;
+__global__ __launch_bounds__(64 * kFibreWaves) void ttv_unit_fibres_kernel(
+    const int32_t* __restrict__ crd, const float* __restrict__ vals,
+    const uint32_t* __restrict__ flags, const int32_t* __restrict__ unit_fid,
+    const int32_t* __restrict__ pos, const float* __restrict__ cv, float* __restrict__ y,
+    int32_t nf, int32_t nnz, int32_t nunits) {
+  __shared__ double s_x[kFibreWaves][kUnit];
+  const int lane = int(threadIdx.x) & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int32_t u = int32_t(blockIdx.x) * kFibreWaves + wv;
+  if (u >= nunits) return;
+  double* x = s_x[wv];
+  const int32_t P = u * kUnit;
+  int32_t k[8];
+  float v[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int32_t p = min(P + j * 64 + lane, nnz - 1);
+    k[j] = crd[p];
+    v[j] = vals[p];
+  }
+  // fibres [f0, f1) start in this unit
+  const bool last = u + 1 == nunits;
+  const int32_t un = last ? u : u + 1;
+  const int32_t f0 = unit_fid[u] + ((flags[u * (kUnit / 32)] & 1u) ? 0 : 1);
+  const int32_t f1 = last ? nf : unit_fid[un] + ((flags[un * (kUnit / 32)] & 1u) ? 0 : 1);
+  if (f0 >= f1) return;  // one fibre that started earlier covers the unit
+  const int32_t end = pos[f1];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) x[j * 64 + lane] = double(v[j]) * cv[k[j]];
+  // the last fibre's nonzeros past the unit
+  double t = 0.0;
+  for (int32_t p0 = P + kUnit; p0 < end; p0 += 4 * 64) {
+    double a[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int32_t p = p0 + j * 64 + lane;
+      const int32_t q = min(p, end - 1);
+      a[j] = p < end ? double(vals[q]) * cv[crd[q]] : 0.0;
+    }
+    t += (a[0] + a[1]) + (a[2] + a[3]);
+  }
+  if (end > P + kUnit) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) t += __shfl_xor(t, o);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  for (int32_t fb = f0; fb < f1; fb += 64) {
+    const int32_t f = fb + lane;
+    const int32_t a = f < f1 ? pos[f] - P : 0;
+    const int32_t e = f < f1 ? min(pos[f + 1] - P, kUnit) : 0;
+    double s = 0.0;
+    if (e - a <= kFibreLane) {
+      double s1 = 0.0;
+      int32_t i = a;
+      for (; i + 4 <= e; i += 4) {
+        const double x0 = x[i], x1 = x[i + 1], x2 = x[i + 2], x3 = x[i + 3];
+        s += x0 + x1;
+        s1 += x2 + x3;
+      }
+      if (i + 2 <= e) {
+        s1 += x[i] + x[i + 1];
+        i += 2;
+      }
+      if (i < e) s += x[i];
+      s += s1;
+    }
+    for (uint64_t big = __ballot(e - a > kFibreLane); big; big &= big - 1) {
+      const int l = __builtin_ctzll(big);
+      const int32_t ba = __builtin_amdgcn_readlane(a, l);
+      const int32_t be = __builtin_amdgcn_readlane(e, l);
+      double b = 0.0;
+      for (int32_t i = ba + lane; i < be; i += 64) b += x[i];
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) b += __shfl_xor(b, o);
+      if (lane == l) s = b;
+    }
+    if (f < f1) y[f] = float(s + (f == f1 - 1 ? t : 0.0));
+  }
 }
 
 // First unit of wave i of the nwav waves that split a band's units
@@ -1353,7 +1456,8 @@ int build_ttv_bands(const CsfDev& B, int nb, int32_t band_w, int cus, TtvPlan* P
 
 }  // namespace
 
-int build_ttv_plan(const CsfDev& B, int32_t cdim, int bands, TtvPlan* P, hipStream_t st) {
+int build_ttv_plan(const CsfDev& B, int32_t cdim, int bands, int64_t max_fibre, TtvPlan* P,
+                   hipStream_t st) {
   free_ttv_plan(P);
   P->built = true;
   if (B.order < 2 || B.order > kMaxOrder || B.nnz <= 0 || cdim <= 0 || cdim > kUnitMaxC ||
@@ -1407,6 +1511,16 @@ int build_ttv_plan(const CsfDev& B, int32_t cdim, int bands, TtvPlan* P, hipStre
   }
   P->k0 = 0;
   P->lc = std::min(cdim, lds);
+  if (bands == 0 && max_fibre <= kFibreMax && nunits <= kFibreUnits) {
+    // whole fibres by the wave, unless there are empty ones to write too
+    uint32_t empty = 1;
+    TT_HIP_CHECK(hipMemcpyAsync(&empty, bad, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    TT_HIP_CHECK(hipStreamSynchronize(st));
+    if (!empty) {
+      P->whole = P->ok = true;
+      return TENTACO_OK;
+    }
+  }
   double window_share = 1.0;  // share of the sampled gathers the window serves
   if (cdim > lds) {
     // the window of `lds` consecutive entries of c that the most nonzeros
@@ -1523,6 +1637,15 @@ int launch_ttv_units(const CsfDev& B, const TtvPlan& P, const float* c, float* y
       case 16384: return launch_bands_typed<16384>(B, P, c, y, st);
       default: return launch_bands_typed<kTtvLdsMax>(B, P, c, y, st);
     }
+  }
+  if (P.whole) {
+    ktimer_begin(st);
+    ttv_unit_fibres_kernel<<<(P.nunits + kFibreWaves - 1) / kFibreWaves, 64 * kFibreWaves, 0, st>>>(
+        B.crd[B.order - 1], B.vals, P.flags, P.unit_fid, B.pos[B.order - 1], c, y,
+        B.nodes[B.order - 2], B.nnz, P.nunits);
+    TT_HIP_CHECK(hipGetLastError());
+    ktimer_end(st, "ttv_unit_kernel");
+    return TENTACO_OK;
   }
   switch (P.lds_floats) {
     case 4096: return launch_units_typed<4096>(B, P, c, y, st);
