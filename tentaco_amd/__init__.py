@@ -970,8 +970,8 @@ class Cpd:
         return np.array(fits[:])
 
     def factor(self, t: int, m: int):
-        a = np.zeros((self.dims[t][m], self.R), np.float32)
-        lam = np.zeros(self.R, np.float32)
+        a = np.empty((self.dims[t][m], self.R), np.float32)
+        lam = np.empty(self.R, np.float32)
         _check(lib().tentaco_cpd_factor(self.h, t, m, _fp(a), _fp(lam)))
         return a, lam
 

@@ -19,14 +19,15 @@
 using tt::fail;
 
 #include "handle.h"
+#include "host_copy.h"
 
 namespace tt {
 namespace {
 
 // Host-side structural validation (host_csf.cpp), copied into the handle.
-int validate_csf(const taco_tensor_t* B, int order, tentaco_csf* h) {
+int validate_csf(const taco_tensor_t* B, int order, tentaco_csf* h, const LevelFn& put = {}) {
   CsfCheck ck;
-  const int rc = validate_csf(B, order, &ck);
+  const int rc = validate_csf(B, order, &ck, put);
   if (rc) return rc;
   for (int m = 0; m < kMaxOrder; ++m) {
     h->dims[m] = ck.dims[m];
@@ -40,15 +41,14 @@ int validate_csf(const taco_tensor_t* B, int order, tentaco_csf* h) {
 }
 
 template <class T>
-int upload_array(T** dst, const T* src, int64_t n) {
+int upload_array(T** dst, const T* src, int64_t n, HostStage& stage) {
   *dst = nullptr;
   const size_t bytes = size_t(std::max<int64_t>(n, 1)) * sizeof(T);
   if (hipMalloc(reinterpret_cast<void**>(dst), bytes) != hipSuccess) {
     *dst = nullptr;
     return fail(TENTACO_ENOMEM, "hipMalloc of %zu bytes failed", bytes);
   }
-  if (n > 0) TT_HIP_CHECK(hipMemcpy(*dst, src, size_t(n) * sizeof(T), hipMemcpyHostToDevice));
-  return TENTACO_OK;
+  return stage.to_device(*dst, src, size_t(n) * sizeof(T));
 }
 
 void free_handle(tentaco_csf* h) {
@@ -297,6 +297,30 @@ int ensure_events() {
   return TENTACO_OK;
 }
 
+// A handle with B's arrays on the device once `stage` is drained; a level's
+// arrays are copied while its coordinates are still being checked.
+int upload_csf(const taco_tensor_t* B, int order, HostStage& stage, tentaco_csf** out) {
+  tentaco_csf* h = new tentaco_csf;
+  h->order = order;
+  bool warm = false;
+  int rc = validate_csf(B, order, h, [&](int m, int64_t parents, int64_t nodes) {
+    int r = warm ? TENTACO_OK : warm_device();
+    warm = true;
+    if (!r) r = upload_array(&h->d_pos[m], B->indices[m][0], parents + 1, stage);
+    if (!r) r = upload_array(&h->d_crd[m], B->indices[m][1], nodes, stage);
+    return r;
+  });
+  if (!rc) rc = upload_array(&h->d_crd0, B->indices[0][1], h->nodes[0], stage);
+  if (!rc) rc = upload_array(&h->d_vals, B->vals, h->nodes[order - 1], stage);
+  if (rc) {
+    (void)stage.drain();
+    free_handle(h);
+    return rc;
+  }
+  *out = h;
+  return TENTACO_OK;
+}
+
 // ---- per-call staging for the host-pointer entry points ------------------
 struct DevBuf {
   void* p = nullptr;
@@ -320,31 +344,36 @@ int host_mttkrp(int order, taco_tensor_t* A, taco_tensor_t* B,
   clear_error();
   if (!A || !A->dimensions || !A->vals) return fail(TENTACO_EINVAL, "A is NULL/incomplete");
   if (!factors) return fail(TENTACO_EINVAL, "factors is NULL");
+  DevBuf fb[kMaxOrder], abuf;
+  HostStage stage(kStageFirst);
   tentaco_csf* h = nullptr;
-  int rc = tentaco_csf_upload(B, order, &h);
+  int rc = upload_csf(B, order, stage, &h);
   if (rc) return rc;
   struct Guard {
     tentaco_csf* h;
-    ~Guard() { free_handle(h); }
-  } guard{h};
+    HostStage& stage;
+    ~Guard() {
+      (void)stage.drain();  // nothing is freed under a copy
+      free_handle(h);
+    }
+  } guard{h, stage};
   const int R = A->dimensions[1];
   const int32_t a_rows = A->dimensions[0];
   if (R <= 0) return fail(TENTACO_EINVAL, "A has %d columns", R);
   if (a_rows <= h->max_crd[0])
     return fail(TENTACO_EINVAL, "A has %d rows but root coordinates reach %d", a_rows,
                 h->max_crd[0]);
-  DevBuf fb[kMaxOrder];
   const float* fdev[kMaxOrder] = {};
   for (int m = 1; m < order; ++m) {
     rc = check_factor(factors[m - 1], m, h, R);
     if (rc) return rc;
     float* d = nullptr;
-    rc = upload_array(&d, factors[m - 1]->vals, int64_t(factors[m - 1]->dimensions[0]) * R);
+    rc = upload_array(&d, factors[m - 1]->vals, int64_t(factors[m - 1]->dimensions[0]) * R,
+                      stage);
     fb[m].p = d;
     if (rc) return rc;
     fdev[m - 1] = d;
   }
-  DevBuf abuf;
   const size_t abytes = size_t(a_rows) * size_t(R) * sizeof(float);
   if (hipMalloc(&abuf.p, std::max<size_t>(abytes, 4)) != hipSuccess)
     return fail(TENTACO_ENOMEM, "hipMalloc of A (%zu bytes) failed", abytes);
@@ -374,21 +403,26 @@ int host_mttkrp(int order, taco_tensor_t* A, taco_tensor_t* B,
     TT_HIP_CHECK(hipEventElapsedTime(&ms, g_ev0, g_ev1));
     g_last_ms.store(ms);
   }
-  TT_HIP_CHECK(hipMemcpy(A->vals, abuf.p, abytes, hipMemcpyDeviceToHost));
-  return TENTACO_OK;
+  return stage.to_host(A->vals, abuf.p, abytes);
 }
 
 int host_ttv(int order, taco_tensor_t* A, taco_tensor_t* B, taco_tensor_t* c) {
   clear_error();
   if (!A || !A->vals) return fail(TENTACO_EINVAL, "A is NULL/incomplete");
   if (!c || !c->dimensions || !c->vals) return fail(TENTACO_EINVAL, "c is NULL/incomplete");
+  DevBuf cbuf, ybuf;
+  HostStage stage(kStageFirst);
   tentaco_csf* h = nullptr;
-  int rc = tentaco_csf_upload(B, order, &h);
+  int rc = upload_csf(B, order, stage, &h);
   if (rc) return rc;
   struct Guard {
     tentaco_csf* h;
-    ~Guard() { free_handle(h); }
-  } guard{h};
+    HostStage& stage;
+    ~Guard() {
+      (void)stage.drain();  // nothing is freed under a copy
+      free_handle(h);
+    }
+  } guard{h, stage};
   // a handle for one call: the banded layout's build would cost more than
   // it saves
   h->ttv_bands = 1;
@@ -398,9 +432,8 @@ int host_ttv(int order, taco_tensor_t* A, taco_tensor_t* B, taco_tensor_t* c) {
   const int32_t nf = h->nodes[order - 2];
   if (A->dimensions && A->dimensions[0] < nf)
     return fail(TENTACO_EINVAL, "A has %d entries, B has %d fibers", A->dimensions[0], nf);
-  DevBuf cbuf, ybuf;
   float* cd = nullptr;
-  rc = upload_array(&cd, c->vals, c->dimensions[0]);
+  rc = upload_array(&cd, c->vals, c->dimensions[0], stage);
   cbuf.p = cd;
   if (rc) return rc;
   if (hipMalloc(&ybuf.p, std::max<size_t>(size_t(nf) * 4, 4)) != hipSuccess)
@@ -423,8 +456,7 @@ int host_ttv(int order, taco_tensor_t* A, taco_tensor_t* B, taco_tensor_t* c) {
     TT_HIP_CHECK(hipEventElapsedTime(&ms, g_ev0, g_ev1));
     g_last_ms.store(ms);
   }
-  if (nf > 0) TT_HIP_CHECK(hipMemcpy(A->vals, ybuf.p, size_t(nf) * 4, hipMemcpyDeviceToHost));
-  return TENTACO_OK;
+  return stage.to_host(A->vals, ybuf.p, size_t(nf) * 4);
 }
 
 // Legacy void entry points report failures on stderr (as gpuErrchk does,
@@ -553,20 +585,11 @@ int tentaco_csf_upload(const taco_tensor_t* B, int order, tentaco_csf** out) {
   clear_error();
   if (!out) return fail(TENTACO_EINVAL, "out is NULL");
   *out = nullptr;
-  tentaco_csf* h = new tentaco_csf;
-  h->order = order;
-  int rc = validate_csf(B, order, h);
-  if (rc) {
-    delete h;
-    return rc;
-  }
-  rc = warm_device();
-  if (!rc) rc = upload_array(&h->d_crd0, B->indices[0][1], h->nodes[0]);
-  for (int m = 1; m < order && !rc; ++m) {
-    rc = upload_array(&h->d_pos[m], B->indices[m][0], int64_t(h->nodes[m - 1]) + 1);
-    if (!rc) rc = upload_array(&h->d_crd[m], B->indices[m][1], h->nodes[m]);
-  }
-  if (!rc) rc = upload_array(&h->d_vals, B->vals, h->nodes[order - 1]);
+  HostStage stage(kStageFirst);
+  tentaco_csf* h = nullptr;
+  int rc = upload_csf(B, order, stage, &h);
+  if (rc) return rc;
+  rc = stage.drain();
   if (rc) {
     free_handle(h);
     return rc;

@@ -26,9 +26,11 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "handle.h"
+#include "host_copy.h"
 #include "internal.h"
 #include "rowops.h"
 
@@ -549,6 +551,9 @@ struct tentaco_cpd {
   // on this stream (default priority), forked from and joined to the sweep's
   hipStream_t side = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
+  // tentaco_cpd_factor copies through it, one caller at a time
+  mutable std::mutex stage_mu;
+  mutable HostStage stage{0};
 
   ~tentaco_cpd() {
     for (auto& s : step) {
@@ -941,12 +946,11 @@ int tentaco_cpd_factor(const tentaco_cpd* c, int t, int m, float* factor, float*
   clear_error();
   if (!c || t < 0 || t >= c->nt) return fail(TENTACO_EINVAL, "cpd: bad tensor index");
   if (m < 0 || m >= c->order[size_t(t)]) return fail(TENTACO_EINVAL, "cpd: bad mode");
-  if (factor)
-    TT_HIP_CHECK(hipMemcpy(factor, c->A[size_t(t)][size_t(m)],
-                           sizeof(float) * size_t(c->dims[size_t(t)][size_t(m)]) * c->R,
-                           hipMemcpyDeviceToHost));
-  if (lambda) TT_HIP_CHECK(hipMemcpy(lambda, c->lam[size_t(t)], sizeof(float) * c->R, hipMemcpyDeviceToHost));
-  return TENTACO_OK;
+  std::lock_guard<std::mutex> lk(c->stage_mu);
+  return c->stage.to_host(
+      factor, c->A[size_t(t)][size_t(m)],
+      factor ? sizeof(float) * size_t(c->dims[size_t(t)][size_t(m)]) * c->R : 0, lambda,
+      c->lam[size_t(t)], lambda ? sizeof(float) * c->R : 0);
 }
 
 int tentaco_cpd_set_factor(tentaco_cpd* c, int t, int m, const float* factor) {

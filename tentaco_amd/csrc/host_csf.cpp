@@ -13,6 +13,7 @@
 #include <memory>
 #include <mutex>
 #include <numeric>
+#include <system_error>
 #include <thread>
 #include <utility>
 #include <vector>
@@ -506,7 +507,57 @@ int check_threads(int64_t n) {
   return int(std::max<int64_t>(1, std::min<int64_t>({int64_t(8), int64_t(hw_threads()), n >> 19})));
 }
 
-int validate_csf(const taco_tensor_t* B, int order, CsfCheck* h) {
+// The smallest and largest of crd[0..n), 0 and -1 included, on T threads beside
+// the caller from start() to finish(); with T = 0 in finish() itself.
+class RangeScan {
+ public:
+  ~RangeScan() { join(); }
+  void start(const int32_t* crd, int64_t n, int T) {
+    crd_ = crd;
+    n_ = n;
+    parts_.assign(size_t(std::max(T, 1)), {0, -1});
+    started_ = 0;
+    for (int t = 0; t < T; ++t) {
+      try {
+        th_.emplace_back([this, t, T] { scan(t, T); });
+        ++started_;
+      } catch (const std::system_error&) {
+        break;  // no thread to be had: finish() scans the rest
+      }
+    }
+  }
+  void finish(int32_t* mn, int32_t* mx) {
+    const int T = int(parts_.size());
+    for (int t = started_; t < T; ++t) scan(t, T);
+    join();
+    for (const auto& p : parts_) {
+      *mn = std::min(*mn, p.first);
+      *mx = std::max(*mx, p.second);
+    }
+  }
+
+ private:
+  void scan(int t, int T) {
+    int32_t lo = 0, hi = -1;
+    for (int64_t x = n_ * t / T, e = n_ * (t + 1) / T; x < e; ++x) {
+      const int32_t v = crd_[x];
+      lo = v < lo ? v : lo;
+      hi = v > hi ? v : hi;
+    }
+    parts_[size_t(t)] = {lo, hi};
+  }
+  void join() {
+    for (auto& x : th_) x.join();
+    th_.clear();
+  }
+  const int32_t* crd_ = nullptr;
+  int64_t n_ = 0;
+  int started_ = 0;
+  std::vector<std::pair<int32_t, int32_t>> parts_;
+  std::vector<std::thread> th_;
+};
+
+int validate_csf(const taco_tensor_t* B, int order, CsfCheck* h, const LevelFn& put) {
   if (!B) return fail(TENTACO_EINVAL, "B is NULL");
   if (order < 2 || order > kMaxOrder)
     return fail(TENTACO_EUNSUPPORTED, "order %d outside 2..%d", order, kMaxOrder);
@@ -555,6 +606,7 @@ int validate_csf(const taco_tensor_t* B, int order, CsfCheck* h) {
   h->max_crd[0] = n0 > 0 ? crd0[n0 - 1] : -1;
   h->dense_root = dense;
   int64_t parents = n0;
+  int put_rc = TENTACO_OK;
   for (int m = 1; m < order; ++m) {
     const int32_t* pos = B->indices[m][0];
     const int32_t* crd = B->indices[m][1];
@@ -607,22 +659,13 @@ int validate_csf(const taco_tensor_t* B, int order, CsfCheck* h) {
     int32_t mn = 0, mx = -1;
     const int32_t dim = h->dims[m];
     {
+      // beside a put the caller's core is busy, so one and two threads pay
+      // from a quarter of a thread's usual share on
+      RangeScan scan;
       const int T = check_threads(nodes);
-      std::vector<int32_t> mn_t(size_t(T), 0), mx_t(size_t(T), -1);
-      run_chunks(T, nodes, [&](int t, int64_t a, int64_t e) {
-        int32_t lo = 0, hi = -1;
-        for (int64_t x = a; x < e; ++x) {
-          const int32_t v = crd[x];
-          lo = v < lo ? v : lo;
-          hi = v > hi ? v : hi;
-        }
-        mn_t[size_t(t)] = lo;
-        mx_t[size_t(t)] = hi;
-      });
-      for (int t = 0; t < T; ++t) {
-        mn = std::min(mn, mn_t[size_t(t)]);
-        mx = std::max(mx, mx_t[size_t(t)]);
-      }
+      scan.start(crd, nodes, put ? std::max(T > 1 ? T : 0, int(std::min<int64_t>(2, nodes >> 17))) : T > 1 ? T : 0);
+      if (put && !put_rc) put_rc = put(m, parents, nodes);
+      scan.finish(&mn, &mx);
     }
     if (mn < 0 || mx >= dim)
       for (int64_t x = 0; x < nodes; ++x) {
@@ -636,6 +679,7 @@ int validate_csf(const taco_tensor_t* B, int order, CsfCheck* h) {
     parents = nodes;
   }
   if (h->nodes[order - 1] > 0 && !B->vals) return fail(TENTACO_EINVAL, "B->vals is NULL");
+  if (put_rc) return put_rc;
   // per-slice nonzero counts (descend the pos arrays from each root node)
   CsfStats& st = h->stats;
   st.nnz = h->nodes[order - 1];

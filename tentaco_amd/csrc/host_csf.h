@@ -2,6 +2,7 @@
 #pragma once
 
 #include <cstdint>
+#include <functional>
 #include <vector>
 
 #include "../../include/taco_tensor_t.h"
@@ -27,8 +28,13 @@ constexpr int64_t kPairCap = 256;
 // The pairing above from the nonzero count of every root node.
 void pair_slices(const std::vector<int32_t>& counts, int64_t cap, std::vector<int32_t>* pairs);
 // Validate B as an order-`order` CSF (the device API's operand contract);
-// TENTACO_OK or an error code with tentaco_last_error() set.
-int validate_csf(const taco_tensor_t* B, int order, CsfCheck* out);
+// TENTACO_OK or an error code with tentaco_last_error() set. `put(m, parents,
+// nodes)`, if given, is called for each level m >= 1 once its arrays may be
+// read (pos checked, crd present) and may copy them while the check of a long
+// crd array still runs on other threads; an error of its own is returned only
+// for a B without faults.
+using LevelFn = std::function<int(int, int64_t, int64_t)>;
+int validate_csf(const taco_tensor_t* B, int order, CsfCheck* out, const LevelFn& put = {});
 
 struct HostCsf {
   int order = 0;
