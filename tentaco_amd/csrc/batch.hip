@@ -28,10 +28,7 @@ struct tentaco_batch {
   size_t brk_bytes = 0;
   tt::BatchLaunch L;
   std::vector<int64_t> h_fill, h_bnd;  // host prefix tables (ntasks + 1)
-  // side stream and events of the overlapped per-order preps
-  hipStream_t side = nullptr;
-  hipEvent_t ev[tt::kMaxOrder + 1] = {};
-  // streams and events of the concurrent order launches (retained outputs)
+  // streams and events of the concurrent order launches
   hipStream_t conc[tt::kMaxOrder + 1] = {};
   hipEvent_t cev[tt::kMaxOrder + 1] = {};
   // graph
@@ -155,6 +152,22 @@ int configure_tables(tentaco_batch* b) {
     L.grp_grid[N] = std::max(1, per_cu) * prop.multiProcessorCount;
     L.grid = std::max(L.grid, L.grp_grid[N]);
   }
+  int orders = 0, block = 0;
+  bool one_block = true;
+  for (int N = 2; N <= kMaxOrder; ++N) {
+    if (L.grp_task[N + 1] <= L.grp_task[N]) continue;
+    one_block = one_block && (orders == 0 || L.blk[N] == block);
+    block = L.blk[N];
+    ++orders;
+  }
+  L.all_grid = 0;
+  if (orders > 1 && one_block && L.total_items > 0) {
+    int per_cu = 1;
+    rc = batch_all_occupancy(block, b->R, &per_cu);
+    if (rc) return rc;
+    L.all_grid = std::max(1, per_cu) * prop.multiProcessorCount;
+    L.grid = L.all_grid;
+  }
   // the brackets depend on the CSFs and the tiles only: written once here,
   // read by every launch
   rc = launch_batch_brackets(L, nullptr);
@@ -220,16 +233,16 @@ int tentaco_batch_create(tentaco_csf* const* tasks, int ntasks, int R, tentaco_b
     delete b;
     return fail(TENTACO_ENOMEM, "counter allocation failed");
   }
-  // the side stream of the per-order preps (default priority); without it
-  // every launch runs in order on the caller's stream
-  bool side_ok = hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking) == hipSuccess;
-  for (int k = 0; k <= kMaxOrder && side_ok; ++k)
-    side_ok = hipEventCreateWithFlags(&b->ev[k], hipEventDisableTiming) == hipSuccess;
-  if (side_ok) {
-    b->L.side = b->side;
-    for (int k = 0; k <= kMaxOrder; ++k) b->L.ev[k] = b->ev[k];
+  // the streams of the concurrent order launches (default priority), where
+  // there are several; without them the orders run one after another
+  bool ok = b->tasks.front()->order != b->tasks.back()->order;
+  for (int k = 0; k <= kMaxOrder && ok; ++k)
+    ok = hipStreamCreateWithFlags(&b->conc[k], hipStreamNonBlocking) == hipSuccess &&
+         hipEventCreateWithFlags(&b->cev[k], hipEventDisableTiming) == hipSuccess;
+  for (int k = 0; k <= kMaxOrder && ok; ++k) {
+    b->L.conc[k] = b->conc[k];
+    b->L.cev[k] = b->cev[k];
   }
-
   *out = b;
   return TENTACO_OK;
 }
@@ -301,21 +314,6 @@ int tentaco_batch_set_output_mode(tentaco_batch* b, int mode) {
     return fail(TENTACO_EINVAL, "output mode %d", mode);
   drop_graph(b);
   b->L.retain = mode == TENTACO_BATCH_OUTPUTS_RETAINED ? 1 : 0;
-  if (b->L.retain && !b->L.conc[0]) {
-    // the streams of the concurrent order launches (default priority);
-    // without them the orders run one after another
-    bool ok = true;
-    for (int k = 0; k <= kMaxOrder && ok; ++k) {
-      if (!b->conc[k]) ok = hipStreamCreateWithFlags(&b->conc[k], hipStreamNonBlocking) == hipSuccess;
-      if (ok && !b->cev[k]) ok = hipEventCreateWithFlags(&b->cev[k], hipEventDisableTiming) == hipSuccess;
-    }
-    if (ok) {
-      for (int k = 0; k <= kMaxOrder; ++k) {
-        b->L.conc[k] = b->conc[k];
-        b->L.cev[k] = b->cev[k];
-      }
-    }
-  }
   return zero_retained_outputs(b);
 }
 
@@ -484,9 +482,8 @@ int tentaco_batch_autotune(tentaco_batch* b, int reps, void* stream, int* best_f
   if (!rc) rc = tentaco_batch_set_schedule(b, bs);
   if (rc) return rc;
   // 2. each order group's own tile, the others held at their best, timed as
-  // whole runs in the batch's output mode (written: the order launches run
-  // one after another; retained: together, so a group's best tile depends on
-  // the others' work beside it)
+  // whole runs in the batch's output mode (the orders run together, so a
+  // group's best tile depends on the others' work beside it)
   for (int N = 2; N <= kMaxOrder; ++N) {
     if (b->L.grp_task[N + 1] <= b->L.grp_task[N]) continue;
     int of = b->L.fam[N], ob = b->L.blk[N], og = b->L.grp[N], os = b->L.sch[N];
@@ -529,9 +526,6 @@ int tentaco_batch_free(tentaco_batch* b) {
   (void)hipFree(b->d_counter);
   (void)hipFree(b->d_fill_off);
   (void)hipFree(b->d_rowbits);
-  for (int k = 0; k <= kMaxOrder; ++k)
-    if (b->ev[k]) (void)hipEventDestroy(b->ev[k]);
-  if (b->side) (void)hipStreamDestroy(b->side);
   for (int k = 0; k <= kMaxOrder; ++k) {
     if (b->cev[k]) (void)hipEventDestroy(b->cev[k]);
     if (b->conc[k]) (void)hipStreamDestroy(b->conc[k]);

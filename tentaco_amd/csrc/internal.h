@@ -276,12 +276,9 @@ struct BatchLaunch {
   int32_t grp_task[kMaxOrder + 2] = {};
   int32_t grp_item[kMaxOrder + 2] = {};
   int grp_grid[kMaxOrder + 1] = {};
-  // prep of every order group after the first on `side` (default priority),
-  // overlapping the earlier groups' kernels: ev[0] forks side from the launch
-  // stream, ev[N] marks order N's prep done (the launch stream waits on it
-  // before order N's kernel). side == nullptr runs everything in order.
-  hipStream_t side = nullptr;
-  hipEvent_t ev[kMaxOrder + 1] = {};
+  // batches of several orders with one block size: the workgroups of the one
+  // launch that holds them all (0: launches per order)
+  int all_grid = 0;
   // host copies of fill_off and bnd_off with ntasks + 1 entries (the group
   // ranges of the per-order preps)
   const int64_t* h_fill_off = nullptr;
@@ -291,10 +288,10 @@ struct BatchLaunch {
   // a launch writes only the rows the walk stores and the rows of slices at
   // item boundaries, which it zeroes before their atomics)
   int retain = 0;
-  // with retained outputs the order groups' persistent launches run
-  // concurrently: each group after the largest on its own stream conc[N]
-  // (default priority), forked from and joined back to the launch stream
-  // through events cev[0] (fork) and cev[N] (group N done)
+  // launches per order run concurrently: each group after the largest on its
+  // own stream conc[N] (default priority), forked from and joined back to the
+  // launch stream through events cev[0] (fork) and cev[N] (group N done);
+  // conc[0] == nullptr runs them in order
   hipStream_t conc[kMaxOrder + 1] = {};
   hipEvent_t cev[kMaxOrder + 1] = {};
 };
@@ -312,6 +309,7 @@ int launch_batch_zero_outputs(const BatchLaunch& L, hipStream_t stream);
 // node of B that holds at least one nonzero.
 int launch_batch_rowbits(const CsfDev& B, uint32_t* bits, hipStream_t stream);
 int batch_occupancy(int family, int block, int R, int32_t NB, int order, int* per_cu);
+int batch_all_occupancy(int block, int R, int* per_cu);
 
 // Launch one empty kernel of the MTTKRP / TTV code objects on `stream`, so
 // that loading them falls outside any later timed region.

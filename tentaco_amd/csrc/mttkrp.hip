@@ -343,22 +343,40 @@ int launch_batch_prep_range(const BatchLaunch& L, int n_lo, int n_hi, hipStream_
   return TENTACO_OK;
 }
 
-// The prep of order group N (a group without tasks has none).
-int launch_batch_prep(const BatchLaunch& L, int N, hipStream_t st, int mode) {
-  return launch_batch_prep_range(L, N, N + 1, st, mode);
-}
-
 // Every order group's prep with the same mode, one launch.
 int launch_batch_preps(const BatchLaunch& L, hipStream_t st, int mode) {
   return launch_batch_prep_range(L, 2, kMaxOrder + 1, st, mode);
 }
 
 
+// One launch for all orders up to kAllItems items a workgroup of it, and one
+// per order beyond, on queues of their own: long batches keep every queue's
+// workgroups busy, and there the orders' own register footprints count. us of a
+// replay (retained outputs), 8 uneven tensors of 2 to 5 modes: R=32, 1 item a
+// workgroup 120 and 149, 2 80 and 86, 7 347 and 377, 12 571 and 533, 32 1384
+// and 1252; R=64: 10 473 and 490, 19 850 and 847, 48 2153 and 2050; R=16: 9 394
+// and 437, 24 933 and 953.
+constexpr int64_t kAllItems = 10;
+
 int launch_batch_orders(const BatchLaunch& L, hipStream_t st) {
   int first = -1;
-  for (int N = 2; N <= kMaxOrder && first < 0; ++N)
-    if (L.grp_task[N + 1] > L.grp_task[N]) first = N;
+  bool one_schedule = true;
+  for (int N = 2; N <= kMaxOrder; ++N) {
+    if (L.grp_task[N + 1] <= L.grp_task[N]) continue;
+    if (first < 0) first = N;
+    one_schedule = one_schedule && L.sch[N] == L.sch[first];
+  }
   if (first < 0) return TENTACO_OK;
+  // counters, boundary rows and (written outputs) the rows no launch stores
+  int rc = launch_batch_preps(L, st, L.retain ? kPrepBoundary : kPrepFill | kPrepBoundary);
+  if (rc) return rc;
+  if (L.all_grid > 0 && one_schedule && L.total_items <= kAllItems * L.all_grid) {
+    ktimer_begin(st);
+    rc = all_orders_batch(L, L.blk[first], L.sch[first], st);
+    if (rc) return rc;
+    ktimer_end(st, "batch_kernel");
+    return TENTACO_OK;
+  }
   auto launch_order = [&](int N, hipStream_t s) -> int {
     switch (N) {
       case 2: return order_batch<2>(L, s);
@@ -367,57 +385,27 @@ int launch_batch_orders(const BatchLaunch& L, hipStream_t st) {
       default: return order_batch<5>(L, s);
     }
   };
-  if (L.retain && L.conc[0]) {
-    // retained outputs: one prep for every group (counters, boundary rows)
-    // up front; then every order group's persistent launch at once, the
-    // group with the most items on the launch stream and each other on its
-    // own stream, so a group's tail overlaps the others' work
-    int rc = launch_batch_prep_range(L, 2, kMaxOrder + 1, st, kPrepBoundary);
-    if (rc) return rc;
-    int big = first;
-    for (int N = first; N <= kMaxOrder; ++N)
-      if (L.grp_item[N + 1] - L.grp_item[N] > L.grp_item[big + 1] - L.grp_item[big]) big = N;
-    TT_HIP_CHECK(hipEventRecord(L.cev[0], st));
-    ktimer_begin(st);
-    rc = launch_order(big, st);
-    if (rc) return rc;
-    for (int N = first; N <= kMaxOrder; ++N) {
-      if (N == big || L.grp_task[N + 1] <= L.grp_task[N]) continue;
-      TT_HIP_CHECK(hipStreamWaitEvent(L.conc[N], L.cev[0], 0));
-      rc = launch_order(N, L.conc[N]);
-      if (rc) return rc;
-      TT_HIP_CHECK(hipEventRecord(L.cev[N], L.conc[N]));
-    }
-    for (int N = first; N <= kMaxOrder; ++N) {
-      if (N == big || L.grp_task[N + 1] <= L.grp_task[N]) continue;
-      TT_HIP_CHECK(hipStreamWaitEvent(st, L.cev[N], 0));
-    }
-    ktimer_end(st, "batch_kernel");
-    return TENTACO_OK;
-  }
-  // every run zeroes the rows no launch stores: the later orders' fills run
-  // on the side stream beside the earlier orders' kernels
-  const int mode = L.retain ? kPrepBoundary : (kPrepFill | kPrepBoundary);
-  const bool split = L.side != nullptr && !L.retain;
-  int rc = launch_batch_prep(L, first, st, mode);
-  if (rc) return rc;
-  if (split) {
-    TT_HIP_CHECK(hipEventRecord(L.ev[0], st));
-    TT_HIP_CHECK(hipStreamWaitEvent(L.side, L.ev[0], 0));
-  }
-  for (int N = first + 1; N <= kMaxOrder; ++N) {
-    if (L.grp_task[N + 1] <= L.grp_task[N]) continue;
-    rc = launch_batch_prep(L, N, split ? L.side : st, mode);
-    if (rc) return rc;
-    if (split) TT_HIP_CHECK(hipEventRecord(L.ev[N], L.side));
-  }
+  // every order group's persistent launch at once, the group with the most
+  // items on the launch stream and each other on its own stream (one after
+  // another without those), so a group's tail overlaps the others' work
+  int big = first;
+  for (int N = first; N <= kMaxOrder; ++N)
+    if (L.grp_item[N + 1] - L.grp_item[N] > L.grp_item[big + 1] - L.grp_item[big]) big = N;
+  const bool conc = L.conc[0] != nullptr;
+  auto beside = [&](int N) { return N != big && L.grp_task[N + 1] > L.grp_task[N]; };
+  if (conc) TT_HIP_CHECK(hipEventRecord(L.cev[0], st));
   ktimer_begin(st);
+  rc = launch_order(big, st);
+  if (rc) return rc;
   for (int N = first; N <= kMaxOrder; ++N) {
-    if (L.grp_task[N + 1] <= L.grp_task[N]) continue;
-    if (split && N != first) TT_HIP_CHECK(hipStreamWaitEvent(st, L.ev[N], 0));
-    rc = launch_order(N, st);
+    if (!beside(N)) continue;
+    if (conc) TT_HIP_CHECK(hipStreamWaitEvent(L.conc[N], L.cev[0], 0));
+    rc = launch_order(N, conc ? L.conc[N] : st);
     if (rc) return rc;
+    if (conc) TT_HIP_CHECK(hipEventRecord(L.cev[N], L.conc[N]));
   }
+  for (int N = first; conc && N <= kMaxOrder; ++N)
+    if (beside(N)) TT_HIP_CHECK(hipStreamWaitEvent(st, L.cev[N], 0));
   ktimer_end(st, "batch_kernel");
   return TENTACO_OK;
 }
@@ -503,6 +491,8 @@ int launch_batch(const BatchLaunch& L, hipStream_t st) {
     return fail(TENTACO_EUNSUPPORTED, "batched launch supports R in {16,32,64}");
   return launch_batch_orders(L, st);
 }
+
+int batch_all_occupancy(int block, int R, int* per_cu) { return all_orders_batch_occupancy(block, R, per_cu); }
 
 int batch_occupancy(int family, int block, int R, int32_t NB, int order, int* per_cu) {
   if (R != 16 && R != 32 && R != 64)

@@ -44,6 +44,10 @@ template <int N>
 int order_batch(const BatchLaunch& L, hipStream_t st);
 template <int N>
 int order_batch_occupancy(int family, int block, int R, int32_t NB, int* per_cu);
+// Every order's items in one launch (mttkrp_batch.hip); all orders run blocks
+// of one size with one schedule.
+int all_orders_batch(const BatchLaunch& L, int block, int schedule, hipStream_t st);
+int all_orders_batch_occupancy(int block, int R, int* per_cu);
 
 // Defined in mttkrp.hip: zero z_elems floats of Z and write the brackets of
 // nblk blocks of NB nonzeros; A = FP32(W) over n elements.

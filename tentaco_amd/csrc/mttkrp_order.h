@@ -1236,25 +1236,19 @@ __global__ __launch_bounds__(128) void slice_pair_kernel(const uint2* __restrict
 }
 
 
-// Persistent workgroups over the items of one order's tasks (the device
-// task table is sorted by order: tasks [t_lo, t_hi) hold items [i_lo, i_hi)),
-// so each order runs with its own register and LDS footprint. Items go out
-// in chunks of `chunk` consecutive ones: a workgroup's first chunk is its own
-// index; later ones come from the order's device counter (schedule 0, reset
-// by the prep launch; not touched when the first chunks cover every item) or
-// by a static cyclic assignment (schedule 1). Either way a workgroup's items
-// increase, so its task cursor only moves forward.
-template <int N, int R, bool EP>
-__global__ __launch_bounds__(512, (edge_waves<N, R>())) void batch_kernel(const BatchTaskDev* __restrict__ tasks,
-                                                    int32_t t_lo, int32_t t_hi,
-                                                    const int64_t* __restrict__ item_off,
-                                                    int32_t i_lo, int32_t i_hi,
-                                                    int32_t* __restrict__ counter, int Rr,
-                                                    int32_t G, int32_t NB, int32_t chunk,
-                                                    int dynamic) {
-  // the batch has no FP64 row buffer, which the edge-serial walk needs
-  static_assert(EP, "the batch runs the edge-parallel walk only");
-  extern __shared__ __align__(16) unsigned char smem[];
+// Persistent workgroups over the items [i_lo, i_hi) of tasks [t_lo, t_hi):
+// item(T, b) runs item b of task T. Items go out in chunks of `chunk`
+// consecutive ones: a workgroup's first chunk is its own index; later ones
+// come from the device counter (schedule 0, reset by the prep launch; not
+// touched when the first chunks cover every item) or by a static cyclic
+// assignment (schedule 1). Either way a workgroup's items increase, so its
+// task cursor only moves forward.
+template <class F>
+__device__ __forceinline__ void batch_items(const BatchTaskDev* __restrict__ tasks, int32_t t_lo,
+                                            int32_t t_hi, const int64_t* __restrict__ item_off,
+                                            int32_t i_lo, int32_t i_hi,
+                                            int32_t* __restrict__ counter, int32_t chunk,
+                                            int dynamic, F&& run) {
   __shared__ int32_t s_chunk;
   const int32_t nchunks = (i_hi - i_lo + chunk - 1) / chunk;
   const int32_t grid = int32_t(gridDim.x);
@@ -1273,9 +1267,7 @@ __global__ __launch_bounds__(512, (edge_waves<N, R>())) void batch_kernel(const 
         ++t;
         t_end = item_off[t + 1];
       }
-      const BatchTaskDev& T = tasks[t];
-      const int32_t b = item - int32_t(item_off[t]);
-      edge_block<N, R, EP>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, G, NB, smem, nullptr);
+      run(tasks[t], item - int32_t(item_off[t]));
     }
     if (dynamic) {
       if (nchunks <= grid) break;
@@ -1289,6 +1281,31 @@ __global__ __launch_bounds__(512, (edge_waves<N, R>())) void batch_kernel(const 
   }
 }
 
+// An add to the one counter takes 10-12 ns whatever the workgroups do, so
+// items taken one at a time cost that each (8 tensors, 38k items of 512
+// nonzeros: 815 us a replay, 676 us in chunks and with the starts kept). About
+// eight chunks per workgroup keep the ends even.
+inline int32_t batch_chunk(int32_t items, int grid, int schedule) {
+  return schedule == 0 ? std::max(1, items / (8 * grid)) : 1;
+}
+
+// One order's tasks (the device task table is sorted by order: tasks [t_lo,
+// t_hi) hold items [i_lo, i_hi)), with the order's own register footprint:
+// batches of one order, and those whose orders differ in block or schedule.
+// The batch has no FP64 row buffer, which the edge-serial walk needs, so it
+// runs the edge-parallel walk only.
+template <int N, int R>
+__global__ __launch_bounds__(512, (edge_waves<N, R>())) void batch_kernel(
+    const BatchTaskDev* __restrict__ tasks, int32_t t_lo, int32_t t_hi,
+    const int64_t* __restrict__ item_off, int32_t i_lo, int32_t i_hi, int32_t* __restrict__ counter,
+    int Rr, int32_t G, int32_t NB, int32_t chunk, int dynamic) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  batch_items(tasks, t_lo, t_hi, item_off, i_lo, i_hi, counter, chunk, dynamic,
+              [&](const BatchTaskDev& T, int32_t b) {
+                edge_block<N, R, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, G, NB, smem, nullptr);
+              });
+}
+
 template <int N, int R>
 int launch_batch_order(const BatchLaunch& L, hipStream_t st) {
   const int32_t i_lo = L.grp_item[N], i_hi = L.grp_item[N + 1];
@@ -1296,12 +1313,8 @@ int launch_batch_order(const BatchLaunch& L, hipStream_t st) {
   const int blk = L.blk[N];
   const size_t lds = size_t(blk / 64) * edge_wave_lds<R>();
   const int grid = std::max(1, std::min<int>(L.grp_grid[N], i_hi - i_lo));
-  // An add to the one counter takes 10-12 ns whatever the workgroups do, so
-  // items taken one at a time cost that each (8 tensors, 38k items of 512
-  // nonzeros: 815 us a replay, 676 us in chunks and with the starts kept). About eight chunks per
-  // workgroup keep the ends even.
-  const int32_t chunk = L.sch[N] == 0 ? std::max(1, (i_hi - i_lo) / (8 * grid)) : 1;
-  batch_kernel<N, R, true><<<grid, blk, lds, st>>>(
+  const int32_t chunk = batch_chunk(i_hi - i_lo, grid, L.sch[N]);
+  batch_kernel<N, R><<<grid, blk, lds, st>>>(
       L.tasks, L.grp_task[N], L.grp_task[N + 1], L.item_off, i_lo, i_hi, L.counter + N, L.R,
       L.grp[N], L.nb[N], chunk, L.sch[N] == 0);
   TT_HIP_CHECK(hipGetLastError());
@@ -1314,7 +1327,7 @@ int batch_occupancy_order(int family, int block, int Rr, int32_t NB, int* per_cu
     return fail(TENTACO_EUNSUPPORTED, "the batch runs the edge-parallel walk only");
   const size_t lds = size_t(block / 64) * edge_wave_lds<R>();
   const hipError_t e =
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, batch_kernel<N, R, true>, block, lds);
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, batch_kernel<N, R>, block, lds);
   if (e != hipSuccess) return fail(TENTACO_EHIP, "occupancy query: %s", hipGetErrorString(e));
   return TENTACO_OK;
 }
