@@ -24,7 +24,9 @@ struct tentaco_batch {
   uint32_t* d_rowbits = nullptr;  // per task, one bit per output row
   int32_t* d_counter = nullptr;
   int32_t* d_starts = nullptr;
-  float4** d_bnd_rows = nullptr;  // the rows zeroed before every run
+  float4** d_bnd_rows = nullptr;  // the rows of slices that items share
+  double* d_bnd_w = nullptr;      // and their sums
+  int2* d_slots = nullptr;
   size_t brk_bytes = 0;
   tt::BatchLaunch L;
   std::vector<int64_t> h_fill, h_bnd;  // host prefix tables (ntasks + 1)
@@ -62,10 +64,14 @@ void free_tables(tentaco_batch* b) {
   (void)hipFree(b->d_item_off);
   (void)hipFree(b->d_starts);
   (void)hipFree(b->d_bnd_rows);
+  (void)hipFree(b->d_bnd_w);
+  (void)hipFree(b->d_slots);
   b->d_tasks = nullptr;
   b->d_bnd_off = b->d_item_off = nullptr;
   b->d_starts = nullptr;
   b->d_bnd_rows = nullptr;
+  b->d_bnd_w = nullptr;
+  b->d_slots = nullptr;
   b->brk_bytes = 0;
 }
 
@@ -111,8 +117,17 @@ int configure_tables(tentaco_batch* b) {
   if (!rc) rc = dev_alloc(&b->d_item_off, size_t(b->ntasks) + 1);  // + the total
   if (!rc) rc = dev_alloc(&b->d_starts, size_t(start_off[b->ntasks]));
   if (!rc) rc = dev_alloc(&b->d_bnd_rows, size_t(bnd[b->ntasks]) * 2);
+  const size_t wlen = size_t(bnd[b->ntasks]) * 2 * size_t(b->R);
+  if (!rc) rc = dev_alloc(&b->d_bnd_w, wlen);
+  if (!rc) rc = dev_alloc(&b->d_slots, size_t(item[b->ntasks]));
   if (rc) return rc;
-  for (int t = 0; t < b->ntasks; ++t) b->host_tasks[t].starts = b->d_starts + start_off[t];
+  TT_HIP_CHECK(hipMemset(b->d_bnd_w, 0, sizeof(double) * wlen));
+  for (int t = 0; t < b->ntasks; ++t) {
+    BatchTaskDev& T = b->host_tasks[t];
+    T.starts = b->d_starts + start_off[t];
+    T.W = b->d_bnd_w + bnd[t] * 2 * b->R;
+    T.slots = b->d_slots + item[t];
+  }
   TT_HIP_CHECK(hipMemcpy(b->d_tasks, b->host_tasks.data(), sizeof(BatchTaskDev) * b->ntasks,
                          hipMemcpyHostToDevice));
   TT_HIP_CHECK(hipMemcpy(b->d_bnd_off, bnd.data(), sizeof(int64_t) * b->ntasks,
@@ -127,6 +142,7 @@ int configure_tables(tentaco_batch* b) {
   L.bnd_off = b->d_bnd_off;
   L.total_bnd = bnd[b->ntasks];
   L.bnd_rows = b->d_bnd_rows;
+  L.bnd_w = b->d_bnd_w;
   L.item_off = b->d_item_off;
   L.total_items = int32_t(item[b->ntasks]);
   L.counter = b->d_counter;

@@ -240,6 +240,11 @@ struct BatchTaskDev {
   FactorsDev F;
   float* A = nullptr;
   int32_t* starts = nullptr;  // per item and wave, the nodes of its first nonzero
+  // FP64 rows that the items sharing a slice add to, and per item those of its
+  // first and last slice; row 2 i is of the slice that starts with item i, row
+  // 2 i + 1 of the one that starts inside item i and reaches its end
+  double* W = nullptr;
+  int2* slots = nullptr;
   // output rows, and one bit per row, set where a root node with at least
   // one nonzero writes the row
   int32_t rows = 0;
@@ -253,7 +258,8 @@ struct BatchLaunch {
   int64_t total_fill = 0;
   const int64_t* bnd_off = nullptr;     // device, prefix of (items+1) per task
   int64_t total_bnd = 0;
-  float4** bnd_rows = nullptr;          // device, two output rows (or null) per boundary
+  float4** bnd_rows = nullptr;          // device, output row (or null) of every FP64 row
+  double* bnd_w = nullptr;              // device, the tasks' FP64 rows (2 per boundary), zero between runs
   const int64_t* item_off = nullptr;    // device, prefix of items per task (ntasks + 1)
   int32_t total_items = 0;
   int32_t* counter = nullptr;           // device work counter

@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256) void fill_kernel(float* A, int64_t n, float va
 // ---------------------------------------------------------------------------
 // batched persistent launch: every (tensor, mode) task's nonzeros are cut into
 // the same NB-sized items; persistent workgroups pull items from a device
-// counter (reset by the batch prep launch) until the queue is empty, and run
+// counter (left at zero by batch_rows_kernel) until the queue is empty, and run
 // the edge walk of the item's task. Every workgroup leaves the loop when the
 // counter passes the item count.
 // Root node of CSF B that holds nonzero position p (the largest node at each
@@ -170,9 +170,10 @@ __device__ __forceinline__ int32_t root_of_position(const CsfDev& B, int32_t p) 
   return key;
 }
 
-// What a batch prep launch does (bits): zero the output rows no root node
-// stores, write the brackets, zero the rows of the slices at item boundaries.
-constexpr int kPrepFill = 1, kPrepBrackets = 2, kPrepBoundary = 4;
+// What a batch_rows_kernel launch does (bits): zero the output rows no root
+// node stores, write the waves' starts and the shared rows' list, write the
+// rows of the slices that items share.
+constexpr int kRowsFill = 1, kRowsList = 2, kRowsShared = 4;
 
 // Nonzeros per work item and waves per workgroup of each order group (kernel
 // argument, by value).
@@ -181,19 +182,20 @@ struct BatchNB {
   int32_t nw[kMaxOrder + 1];
 };
 
-// Prep of the order group holding sorted tasks [t_lo, t_hi): reset that
-// order's work counter; with kPrepFill zero the outputs (quads [q_lo,
-// q_hi)), skipping a row whose bit is set in the task's rowbits, because a
-// root node with nonzeros stores it; with kPrepBrackets write where the waves
-// of each item start (entries [b_lo, b_hi)) and, per boundary b, the output
-// rows of the slices holding positions b*NB and b*NB - 1: those are the
-// edge-parallel walk's only atomically updated rows (the slices holding an
-// item's first and last nonzero); with kPrepBoundary zero the listed rows.
-// The list (two row addresses per boundary, null where an earlier boundary
-// lists the row) depends on the CSFs, outputs and tiles only; finding the
-// rows on every run took 17 us a launch in a CP-ALS sweep over three tensors,
-// reading the list 4 us.
-__global__ __launch_bounds__(256) void batch_prep_kernel(const BatchTaskDev* __restrict__ tasks,
+// The rows of sorted tasks [t_lo, t_hi) that the walk does not store, after
+// it: with kRowsFill zero the outputs (quads [q_lo, q_hi)), skipping a row
+// whose bit is set in the task's rowbits, because a root node with nonzeros
+// stores it; with kRowsShared write the rows of the slices that hold an item's
+// first or last nonzero. Several items may share those, so the walk adds to FP64
+// rows for them, which are left zero for the next run, as the work counters are
+// (hundreds of FP32 additions to a long slice's row, in whichever order, were
+// most of a batch's error: a sweep's worst factor against FP64, 30 seeds, had
+// 7.5e-7 on average and 4.5e-6 at most, now 4.5e-7 and 8.1e-7). With kRowsList (once per configuration) write where the waves of
+// each item start, its slots of FP64 rows, and the list of their output rows
+// (entries [b_lo, b_hi), two per item, null where an earlier item has the
+// slice's). The list depends on the CSFs, outputs and tiles only; finding the
+// rows on every run took 17 us a launch in a CP-ALS sweep over three tensors.
+__global__ __launch_bounds__(256) void batch_rows_kernel(const BatchTaskDev* __restrict__ tasks,
                                                          int32_t t_lo, int32_t t_hi,
                                                          const int64_t* __restrict__ fill_off,
                                                          int64_t q_lo, int64_t q_hi,
@@ -202,13 +204,14 @@ __global__ __launch_bounds__(256) void batch_prep_kernel(const BatchTaskDev* __r
                                                          int32_t* __restrict__ counter,
                                                          int n_lo, int n_hi, BatchNB nbs, int R,
                                                          int qshift, int mode,
-                                                         float4** __restrict__ bnd_rows) {
+                                                         float4** __restrict__ bnd_rows,
+                                                         double* __restrict__ bnd_w) {
   const int64_t tid = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const int64_t nthr = int64_t(gridDim.x) * blockDim.x;
   // the work counters of order groups [n_lo, n_hi)
   if (tid < n_hi - n_lo) counter[n_lo + tid] = 0;
   const int32_t nt = t_hi - t_lo;
-  if (!(mode & kPrepFill)) q_hi = q_lo;
+  if (!(mode & kRowsFill)) q_hi = q_lo;
   // Zero the outputs as float4 quads (every output holds rows x R floats
   // with R a multiple of 4 and starts 16-byte aligned, which the host
   // checks). Each workgroup takes one contiguous range of quads, finds the
@@ -261,14 +264,18 @@ __global__ __launch_bounds__(256) void batch_prep_kernel(const BatchTaskDev* __r
         if (dst[u] && !((w[u] >> sh[u]) & 1u)) *dst[u] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
   }
-  if (mode & kPrepBoundary) {
+  if (mode & kRowsShared) {
     const int64_t n = (b_hi - b_lo) << (qshift + 1);
     for (int64_t i = tid; i < n; i += nthr) {
       float4* row = bnd_rows[2 * b_lo + (i >> qshift)];
-      if (row) row[i & ((1 << qshift) - 1)] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (!row) continue;
+      double2* w = reinterpret_cast<double2*>(bnd_w) + 2 * ((b_lo << (qshift + 1)) + i);
+      const double2 x = w[0], y = w[1];
+      w[0] = w[1] = make_double2(0.0, 0.0);
+      row[i & ((1 << qshift) - 1)] = make_float4(float(x.x), float(x.y), float(y.x), float(y.y));
     }
   }
-  if (!(mode & kPrepBrackets)) return;
+  if (!(mode & kRowsList)) return;
   for (int64_t i = b_lo + tid; i < b_hi; i += nthr) {
     const int32_t t = t_lo + upper_index(bnd_off + t_lo, nt, i);
     const BatchTaskDev& T = tasks[t];
@@ -287,20 +294,22 @@ __global__ __launch_bounds__(256) void batch_prep_kernel(const BatchTaskDev* __r
         key = x;
       }
     }
-    // the boundary's rows: the slice of position p, and that of p - 1 (the
-    // previous item's last nonzero), another one only when p is a slice's
-    // first position
-    const int64_t p = min(bi * int64_t(NB), int64_t(T.B.nnz) - 1);
+    // the item's first and last slice
+    const int64_t p = bi * int64_t(NB);
+    if (p >= T.B.nnz) continue;  // the boundary behind the last item
     const int32_t here = T.starts[bi * nw * (N - 1)];
-    const int32_t prev = bi > 0 ? root_of_position(T.B, int32_t((bi - 1) * NB)) : -1;
+    const int32_t back = root_of_position(T.B, int32_t(min(p + NB, int64_t(T.B.nnz)) - 1));
+    auto slot_of = [&](int32_t x) {
+      for (int m = 1; m < N; ++m) x = T.B.pos[m][x];
+      return 2 * (x / NB) + (x % NB ? 1 : 0);
+    };
     auto row_of = [&](int32_t x) {
       return reinterpret_cast<float4*>(T.A + int64_t(T.B.crd0[x]) * R);
     };
-    if (here != prev) bnd_rows[2 * i] = row_of(here);
-    if (bi > 0 && p == bi * int64_t(NB)) {
-      const int32_t before = root_of_position(T.B, int32_t(p - 1));
-      if (before != here && before != prev) bnd_rows[2 * i + 1] = row_of(before);
-    }
+    const int2 s = make_int2(slot_of(here), slot_of(back));
+    T.slots[bi] = s;
+    if (s.x == 2 * bi) bnd_rows[2 * i] = row_of(here);
+    if (s.y == 2 * bi + 1) bnd_rows[2 * i + 1] = row_of(back);
   }
 }
 
@@ -319,33 +328,33 @@ __global__ __launch_bounds__(256) void batch_rowbits_kernel(CsfDev B, uint32_t* 
   }
 }
 
-// The prep of order groups [n_lo, n_hi) in one launch (their tasks are
-// consecutive in the task table; groups without tasks add nothing).
-int launch_batch_prep_range(const BatchLaunch& L, int n_lo, int n_hi, hipStream_t st, int mode) {
+// batch_rows_kernel over order groups [n_lo, n_hi) (their tasks are consecutive
+// in the task table; groups without tasks add nothing).
+int launch_batch_rows_range(const BatchLaunch& L, int n_lo, int n_hi, hipStream_t st, int mode) {
   const int32_t t_lo = L.grp_task[n_lo], t_hi = L.grp_task[n_hi];
   if (t_hi <= t_lo) return TENTACO_OK;
   // the host prefix tables hold ntasks + 1 entries (the last is the total)
   const int64_t f0 = L.h_fill_off[t_lo], f1 = L.h_fill_off[t_hi];
   const int64_t b0 = L.h_bnd_off[t_lo], b1 = L.h_bnd_off[t_hi];
-  const int64_t fill_quads = (mode & kPrepFill) ? (f1 - f0) >> 2 : 0;
+  const int64_t fill_quads = (mode & kRowsFill) ? (f1 - f0) >> 2 : 0;
   const int qshift = L.R == 16 ? 2 : L.R == 32 ? 3 : 4;  // log2(R / 4), R in {16, 32, 64}
   const int64_t work = std::max<int64_t>(
-      fill_quads, (mode & kPrepBoundary) ? (b1 - b0) << (qshift + 1) : b1 - b0);
+      fill_quads, (mode & kRowsShared) ? (b1 - b0) << (qshift + 1) : b1 - b0);
   BatchNB nbs{};
   for (int N = 0; N <= kMaxOrder; ++N) {
     nbs.nb[N] = L.nb[N];
     nbs.nw[N] = std::max(1, L.blk[N] / 64);
   }
-  batch_prep_kernel<<<grid_for(work, 256, 16384), 256, 0, st>>>(
+  batch_rows_kernel<<<grid_for(work, 256, 16384), 256, 0, st>>>(
       L.tasks, t_lo, t_hi, L.fill_off, f0 >> 2, f1 >> 2, L.bnd_off, b0, b1, L.counter, n_lo, n_hi,
-      nbs, L.R, qshift, mode, L.bnd_rows);
+      nbs, L.R, qshift, mode, L.bnd_rows, L.bnd_w);
   TT_HIP_CHECK(hipGetLastError());
   return TENTACO_OK;
 }
 
-// Every order group's prep with the same mode, one launch.
-int launch_batch_preps(const BatchLaunch& L, hipStream_t st, int mode) {
-  return launch_batch_prep_range(L, 2, kMaxOrder + 1, st, mode);
+// Every order group's with the same mode, one launch.
+int launch_batch_rows(const BatchLaunch& L, hipStream_t st, int mode) {
+  return launch_batch_rows_range(L, 2, kMaxOrder + 1, st, mode);
 }
 
 
@@ -367,15 +376,17 @@ int launch_batch_orders(const BatchLaunch& L, hipStream_t st) {
     one_schedule = one_schedule && L.sch[N] == L.sch[first];
   }
   if (first < 0) return TENTACO_OK;
-  // counters, boundary rows and (written outputs) the rows no launch stores
-  int rc = launch_batch_preps(L, st, L.retain ? kPrepBoundary : kPrepFill | kPrepBoundary);
-  if (rc) return rc;
+  // the shared rows and (written outputs) the rows no launch stores
+  auto rows = [&]() {
+    return launch_batch_rows(L, st, L.retain ? kRowsShared : kRowsFill | kRowsShared);
+  };
+  int rc = TENTACO_OK;
   if (L.all_grid > 0 && one_schedule && L.total_items <= kAllItems * L.all_grid) {
     ktimer_begin(st);
     rc = all_orders_batch(L, L.blk[first], L.sch[first], st);
     if (rc) return rc;
     ktimer_end(st, "batch_kernel");
-    return TENTACO_OK;
+    return rows();
   }
   auto launch_order = [&](int N, hipStream_t s) -> int {
     switch (N) {
@@ -407,7 +418,7 @@ int launch_batch_orders(const BatchLaunch& L, hipStream_t st) {
   for (int N = first; conc && N <= kMaxOrder; ++N)
     if (beside(N)) TT_HIP_CHECK(hipStreamWaitEvent(st, L.cev[N], 0));
   ktimer_end(st, "batch_kernel");
-  return TENTACO_OK;
+  return rows();
 }
 
 }  // namespace
@@ -479,11 +490,11 @@ int launch_batch_rowbits(const CsfDev& B, uint32_t* bits, hipStream_t st) {
 }
 
 int launch_batch_brackets(const BatchLaunch& L, hipStream_t st) {
-  return launch_batch_preps(L, st, kPrepBrackets);
+  return launch_batch_rows(L, st, kRowsList);
 }
 
 int launch_batch_zero_outputs(const BatchLaunch& L, hipStream_t st) {
-  return launch_batch_preps(L, st, kPrepFill | kPrepBoundary);
+  return launch_batch_rows(L, st, kRowsFill | kRowsShared);
 }
 
 int launch_batch(const BatchLaunch& L, hipStream_t st) {

@@ -83,7 +83,7 @@ template <int N, int R, bool EP>
 __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F, float* out_a,
                                            int Rr, const int32_t* brk_p, const int32_t* starts_p,
                                            int32_t b, int32_t G, int32_t NB, unsigned char* smem,
-                                           double* out_w) {
+                                           double* out_w, const int2* slots = nullptr) {
   using RO = Row<R>;
   using V = typename RO::V;
   constexpr int NV = RO::NV;
@@ -474,8 +474,9 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
       const int64_t o = int64_t(global_ptr(B.crd0)[key]) * cols + col;
       const bool shared = key == first || key == last;
       if constexpr (EP) {
-        if (shared) unsafeAtomicAdd(A + o, float(s));
-        else A[o] = float(s);
+        if (!shared) A[o] = float(s);
+        else if (slots) unsafeAtomicAdd(W + int64_t(key == first ? slots->x : slots->y) * cols + col, s);
+        else unsafeAtomicAdd(A + o, float(s));
       } else {
         if (shared) unsafeAtomicAdd(W + o, s);
         else W[o] = s;
@@ -1239,7 +1240,7 @@ __global__ __launch_bounds__(128) void slice_pair_kernel(const uint2* __restrict
 // Persistent workgroups over the items [i_lo, i_hi) of tasks [t_lo, t_hi):
 // item(T, b) runs item b of task T. Items go out in chunks of `chunk`
 // consecutive ones: a workgroup's first chunk is its own index; later ones
-// come from the device counter (schedule 0, reset by the prep launch; not
+// come from the device counter (schedule 0, zero between runs; not
 // touched when the first chunks cover every item) or by a static cyclic
 // assignment (schedule 1). Either way a workgroup's items increase, so its
 // task cursor only moves forward.
@@ -1292,8 +1293,8 @@ inline int32_t batch_chunk(int32_t items, int grid, int schedule) {
 // One order's tasks (the device task table is sorted by order: tasks [t_lo,
 // t_hi) hold items [i_lo, i_hi)), with the order's own register footprint:
 // batches of one order, and those whose orders differ in block or schedule.
-// The batch has no FP64 row buffer, which the edge-serial walk needs, so it
-// runs the edge-parallel walk only.
+// The batch has FP64 rows for the slices that items share only, not for all
+// that the edge-serial walk adds to, so it runs the edge-parallel walk only.
 template <int N, int R>
 __global__ __launch_bounds__(512, (edge_waves<N, R>())) void batch_kernel(
     const BatchTaskDev* __restrict__ tasks, int32_t t_lo, int32_t t_hi,
@@ -1302,7 +1303,8 @@ __global__ __launch_bounds__(512, (edge_waves<N, R>())) void batch_kernel(
   extern __shared__ __align__(16) unsigned char smem[];
   batch_items(tasks, t_lo, t_hi, item_off, i_lo, i_hi, counter, chunk, dynamic,
               [&](const BatchTaskDev& T, int32_t b) {
-                edge_block<N, R, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, G, NB, smem, nullptr);
+                edge_block<N, R, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, G, NB, smem, T.W,
+                                       T.slots + b);
               });
 }
 
