@@ -62,6 +62,8 @@ void free_handle(tentaco_csf* h) {
   (void)hipFree(h->ws);
   for (void* w : h->ws_retired) (void)hipFree(w);
   for (int i = 0; i < h->starts.n; ++i) (void)hipFree(h->starts.p[i]);
+  for (int i = 0; i < h->starts.ns; ++i) (void)hipFree(h->starts.mem[i]);
+  (void)hipFree(h->starts.bits);
   for (int m = 0; m < kMaxOrder; ++m) (void)hipFree(h->stage_f[m]);
   (void)hipFree(h->stage_a);
   (void)hipFree(h->d_crd1_of_nnz);
@@ -216,36 +218,99 @@ int reserve_ws(tentaco_csf* h, size_t bytes, hipStream_t st) {
   return TENTACO_OK;
 }
 
-// The handle's wave starts for variant vr at rank R (edge families), or null.
+// Adds the shared rows of edge-parallel tiles of NB nonzeros at rank R to the
+// handle's tables, complete for every stream.
+int build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStream_t st) {
+  const CsfDev B = h->view();
+  WalkStarts& s = h->starts;
+  const int64_t nblk = (int64_t(B.nnz) + NB - 1) / NB;
+  const size_t o_rows = (size_t(nblk) * sizeof(int2) + 255) / 256 * 256;
+  const size_t o_w = o_rows + (size_t(nblk) * 2 * sizeof(int32_t) + 255) / 256 * 256;
+  const size_t wbytes = size_t(nblk) * 2 * size_t(R) * sizeof(double);
+  const int32_t nbits = h->max_crd[0] + 1;
+  const size_t bbytes = (size_t(nbits) + 31) / 32 * sizeof(uint32_t);
+  void* mem = nullptr;
+  uint32_t* bits = s.bits;
+  bool ok = hipMalloc(&mem, o_w + wbytes) == hipSuccess;
+  if (ok && !bits) {
+    ok = hipMalloc(reinterpret_cast<void**>(&bits), bbytes) == hipSuccess &&
+         hipMemsetAsync(bits, 0, bbytes, st) == hipSuccess && launch_batch_rowbits(B, bits, st) == TENTACO_OK;
+  }
+  char* base = static_cast<char*>(mem);
+  int2* slots = reinterpret_cast<int2*>(base);
+  int32_t* rows = reinterpret_cast<int32_t*>(base + o_rows);
+  double* W = reinterpret_cast<double*>(base + o_w);
+  ok = ok && hipMemsetAsync(W, 0, wbytes, st) == hipSuccess &&
+       launch_shared_rows(B, int32_t(NB), slots, rows, st) == TENTACO_OK;
+  ok = hipStreamSynchronize(st) == hipSuccess && ok;
+  if (!ok) {
+    (void)hipGetLastError();
+    clear_error();
+    (void)hipFree(mem);
+    if (!s.bits) (void)hipFree(bits);
+    return TENTACO_ENOMEM;
+  }
+  s.bits = bits;
+  s.nb[s.ns] = NB;
+  s.rank[s.ns] = R;
+  s.mem[s.ns] = mem;
+  WalkTables& t = s.sh[s.ns++];
+  t.slots = slots;
+  t.rows = rows;
+  t.bits = bits;
+  t.nbits = nbits;
+  t.W = W;
+  return TENTACO_OK;
+}
+
+// Workgroups from which they share rows in FP64. The FP32 error of a long slice's
+// row grows with the root of the number of workgroups that add to it: 100M
+// nonzeros in 48,828 workgroups 4.6e-7 against FP64, 1.2e-7 with FP64 rows, 30M
+// (5-mode) 5.8e-7 and 1.2e-7; in 700 workgroups 2.3e-7 and 1.5e-7. The rows'
+// kernel costs 3 us more than the fill it replaces (100M: 2027 and 2037 us, 5M
+// at rank 50 147 and 150; 20k 11.1 and 14.1, 1.5M 31.9 and 35.7).
+constexpr int64_t kSharedBlocks = 2048;
+
+// What the handle keeps for variant vr at rank R (edge families), or nulls.
 // With `build`, a missing table is built on st and waited for, so that it is
 // complete for every stream; not under capture. A failed build leaves the
-// calls on the brackets they write themselves.
-const int32_t* walk_starts(tentaco_csf* h, const Variant& vr, int R, bool build, hipStream_t st) {
+// calls on the brackets they write themselves and on FP32 atomics.
+WalkTables walk_tables(tentaco_csf* h, const Variant& vr, int R, bool build, hipStream_t st) {
   const CsfDev B = h->view();
-  if (vr.family == kSliceRow || vr.family < 0 || B.nnz <= 0) return nullptr;
-  const int64_t wn = nnz_per_wave(vr, R);
+  WalkTables t;
+  if (vr.family == kSliceRow || vr.family < 0 || B.nnz <= 0) return t;
+  const int64_t wn = nnz_per_wave(vr, R), NB = nnz_per_block(vr, R);
   WalkStarts& s = h->starts;
   std::lock_guard<std::mutex> lk(s.mu);
-  for (int i = 0; i < s.n; ++i)
-    if (s.wn[i] == wn) return s.p[i];
-  if (!build || s.n >= WalkStarts::kTables) return nullptr;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone)
-    return nullptr;
-  int32_t* p = nullptr;
-  if (hipMalloc(reinterpret_cast<void**>(&p), edge_brk_bytes(B, wn)) != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;
+  int i = 0;
+  while (i < s.n && s.wn[i] != wn) ++i;
+  int j = 0;
+  while (j < s.ns && (s.nb[j] != NB || s.rank[j] != R)) ++j;
+  const bool ep = vr.family == kEdgeParallel && B.nnz >= kSharedBlocks * NB;
+  if (build && (i == s.n || (ep && j == s.ns)) &&
+      (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone))
+    build = false;
+  if (i == s.n) {
+    if (!build || s.n >= WalkStarts::kTables) return t;
+    int32_t* p = nullptr;
+    if (hipMalloc(reinterpret_cast<void**>(&p), edge_brk_bytes(B, wn)) != hipSuccess) {
+      (void)hipGetLastError();
+      return t;
+    }
+    const int rc = launch_walk_starts(B, wn, p, st);
+    if (hipStreamSynchronize(st) != hipSuccess || rc) {
+      (void)hipFree(p);
+      clear_error();
+      return t;
+    }
+    s.wn[s.n] = wn;
+    s.p[s.n++] = p;
   }
-  const int rc = launch_walk_starts(B, wn, p, st);
-  if (hipStreamSynchronize(st) != hipSuccess || rc) {
-    (void)hipFree(p);
-    clear_error();
-    return nullptr;
-  }
-  s.wn[s.n] = wn;
-  s.p[s.n++] = p;
-  return p;
+  if (ep && j == s.ns && build && s.ns < WalkStarts::kTables) (void)build_shared_rows(h, NB, R, st);
+  if (ep && j < s.ns) t = s.sh[j];
+  t.starts = s.p[i];
+  return t;
 }
 
 int resolve_variant(const tentaco_csf* h, int R, int variant) {
@@ -749,7 +814,7 @@ int tentaco_csf_reserve_rows(tentaco_csf* h, int R, int variant, int32_t a_rows)
   rc = reserve_ws(h, need, nullptr);
   if (rc) return rc;
   // the wave starts of the variant that calls with this argument run
-  (void)walk_starts(h, tile_of(h, R, variant, resolve_variant(h, R, variant)), R, true, nullptr);
+  (void)walk_tables(h, tile_of(h, R, variant, resolve_variant(h, R, variant)), R, true, nullptr);
   h->reserved = true;
   return TENTACO_OK;
 }
@@ -846,10 +911,10 @@ int tentaco_mttkrp_dev(tentaco_csf* h, int R, const float* const* factors_dev, f
   const CsfDev B = h->view();
   rc = reserve_ws(h, mttkrp_workspace_bytes(B, R, vr, a_rows), static_cast<hipStream_t>(stream));
   if (rc) return rc;
-  const int32_t* starts =
-      walk_starts(h, vr, R, !h->reserved, static_cast<hipStream_t>(stream));
+  const WalkTables tables =
+      walk_tables(h, vr, R, !h->reserved, static_cast<hipStream_t>(stream));
   const bool dense = h->dense_root && a_rows == h->nodes[0];
-  return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws, starts,
+  return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws, tables,
                        static_cast<hipStream_t>(stream));
 }
 
@@ -886,7 +951,7 @@ int tentaco_mttkrp_dev_noalloc(tentaco_csf* h, int R, const float* const* factor
   // slice-row: the 3-mode expansion and padded layout are used when a
   // reserve call built them, never built here
   const bool dense = h->dense_root && a_rows == h->nodes[0];
-  return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, ws, nullptr,
+  return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, ws, WalkTables{},
                        static_cast<hipStream_t>(stream));
 }
 
@@ -906,7 +971,7 @@ static int sweep_impl(tentaco_csf* h, int R, const float* const* factors_dev, fl
     if (rc) return rc;
     for (int v = 0; v < kNumVariants; ++v)
       if ((!use || use[v]) && variant_fits(h->order, R, v))
-        (void)walk_starts(h, variant_of(v), R, true, st);
+        (void)walk_tables(h, variant_of(v), R, true, st);
   }
   hipEvent_t e0, e1;
   TT_HIP_CHECK(hipEventCreate(&e0));

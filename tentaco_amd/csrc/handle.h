@@ -21,6 +21,13 @@ struct WalkStarts {
   int n = 0;
   int64_t wn[kTables] = {};
   int32_t* p[kTables] = {};
+  // the shared rows of edge-parallel tiles, by nonzeros per workgroup and rank
+  int ns = 0;
+  int64_t nb[kTables] = {};
+  int rank[kTables] = {};
+  void* mem[kTables] = {};
+  WalkTables sh[kTables] = {};
+  uint32_t* bits = nullptr;
 };
 }  // namespace tt
 

@@ -91,11 +91,26 @@ size_t ttv_workspace_bytes(const CsfDev& B);
 // Enqueue one MTTKRP on `stream`. A (a_rows x R) is fully overwritten;
 // `dense_root` says crd0 == 0..n0-1 with n0 == a_rows (no zero fill needed
 // for the slice-row family). ws must hold mttkrp_workspace_bytes bytes.
-// starts: the walk's wave starts for nnz_per_wave(vr, R) (edge families; see
-// launch_walk_starts), or null: the call then writes the brackets into ws.
+// tables: what a handle keeps for the tile, or nulls.
+struct WalkTables {
+  // the walk's wave starts for nnz_per_wave(vr, R) (edge families; see
+  // launch_walk_starts); null: the call writes the brackets into ws
+  const int32_t* starts = nullptr;
+  // edge-parallel tiles (see launch_shared_rows): the FP64 rows that workgroups
+  // sharing a slice add to, zero between calls, two per workgroup; each
+  // workgroup's two; their output rows (-1: another's); and one bit per output
+  // row that a root node with nonzeros writes. slots null: FP32 atomics
+  const int2* slots = nullptr;
+  const int32_t* rows = nullptr;
+  const uint32_t* bits = nullptr;
+  int32_t nbits = 0;
+  double* W = nullptr;
+};
 int launch_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A,
                   int32_t a_rows, bool dense_root, const Variant& vr,
-                  void* ws, const int32_t* starts, hipStream_t stream);
+                  void* ws, const WalkTables& tables, hipStream_t stream);
+// Write the slots and rows of an edge-parallel tile of NB nonzeros.
+int launch_shared_rows(const CsfDev& B, int32_t NB, int2* slots, int32_t* rows, hipStream_t stream);
 // Nonzeros one wave of an edge-family variant walks at rank R.
 int64_t nnz_per_wave(const Variant& vr, int R);
 // Write the node at every level 0..N-2 that holds the first nonzero of each

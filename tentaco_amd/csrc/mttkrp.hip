@@ -170,6 +170,13 @@ __device__ __forceinline__ int32_t root_of_position(const CsfDev& B, int32_t p) 
   return key;
 }
 
+// Which FP64 row the slice of root node x adds to: 2 i if it starts with item
+// (or workgroup) i of NB nonzeros, 2 i + 1 if inside it.
+__device__ __forceinline__ int32_t slot_of_root(const CsfDev& B, int32_t x, int32_t NB) {
+  for (int m = 1; m < B.order; ++m) x = B.pos[m][x];
+  return 2 * (x / NB) + (x % NB ? 1 : 0);
+}
+
 // What a batch_rows_kernel launch does (bits): zero the output rows no root
 // node stores, write the waves' starts and the shared rows' list, write the
 // rows of the slices that items share.
@@ -299,14 +306,10 @@ __global__ __launch_bounds__(256) void batch_rows_kernel(const BatchTaskDev* __r
     if (p >= T.B.nnz) continue;  // the boundary behind the last item
     const int32_t here = T.starts[bi * nw * (N - 1)];
     const int32_t back = root_of_position(T.B, int32_t(min(p + NB, int64_t(T.B.nnz)) - 1));
-    auto slot_of = [&](int32_t x) {
-      for (int m = 1; m < N; ++m) x = T.B.pos[m][x];
-      return 2 * (x / NB) + (x % NB ? 1 : 0);
-    };
     auto row_of = [&](int32_t x) {
       return reinterpret_cast<float4*>(T.A + int64_t(T.B.crd0[x]) * R);
     };
-    const int2 s = make_int2(slot_of(here), slot_of(back));
+    const int2 s = make_int2(slot_of_root(T.B, here, NB), slot_of_root(T.B, back, NB));
     T.slots[bi] = s;
     if (s.x == 2 * bi) bnd_rows[2 * i] = row_of(here);
     if (s.y == 2 * bi + 1) bnd_rows[2 * i + 1] = row_of(back);
@@ -324,6 +327,73 @@ __global__ __launch_bounds__(256) void batch_rowbits_kernel(CsfDev B, uint32_t* 
     if (hi > lo) {
       const int32_t r = B.crd0[x];
       atomicOr(bits + (r >> 5), 1u << (r & 31));
+    }
+  }
+}
+
+// slots[b], rows[2 b], rows[2 b + 1] of the workgroups of one CSF, as
+// batch_rows_kernel lists an item's (rows: output row, or -1).
+__global__ __launch_bounds__(256) void shared_rows_kernel(CsfDev B, int32_t NB, int32_t nblk,
+                                                          int2* __restrict__ slots,
+                                                          int32_t* __restrict__ rows) {
+  const int32_t b = int32_t(blockIdx.x * 256 + threadIdx.x);
+  if (b >= nblk) return;
+  const int64_t p = int64_t(b) * NB;
+  const int32_t here = root_of_position(B, int32_t(p));
+  const int32_t back = root_of_position(B, int32_t(min(p + NB, int64_t(B.nnz)) - 1));
+  const int2 s = make_int2(slot_of_root(B, here, NB), slot_of_root(B, back, NB));
+  slots[b] = s;
+  rows[2 * b] = s.x == 2 * b ? B.crd0[here] : -1;
+  rows[2 * b + 1] = s.y == 2 * b + 1 ? B.crd0[back] : -1;
+}
+
+// After an edge-parallel walk: a wave per 32 output rows zeroes those whose bit
+// is clear (the walk stores the others), and waves write the shared rows, each
+// row's columns on the smallest power of two of lanes, and zero them for the
+// next call. In place of the fill of all of A before the walk.
+__global__ __launch_bounds__(256) void edge_rows_kernel(const int32_t* __restrict__ rows, int32_t nrows,
+                                                        double* __restrict__ W,
+                                                        const uint32_t* __restrict__ bits, int32_t nbits,
+                                                        float* __restrict__ A, int32_t a_rows, int R,
+                                                        int lshift) {
+  const int lane = int(threadIdx.x) & 63;
+  const int32_t wave = int32_t(blockIdx.x * 4 + (threadIdx.x >> 6)), nwave = int32_t(gridDim.x * 4);
+  const int32_t words = int32_t((int64_t(a_rows) + 31) / 32);
+  const int per = 64 >> lshift, sub = lane >> lshift, c0 = lane & ((1 << lshift) - 1);
+  // every load of a wave's first word, row number and column is in flight
+  // before the first of them is waited for
+  auto clear = [&](int32_t i) {  // the word's rows without a root node
+    const int32_t left = a_rows - 32 * i;
+    const uint32_t all = left >= 32 ? ~0u : (1u << left) - 1u;
+    const int32_t known = nbits - 32 * i;  // rows from nbits on have none
+    return known > 0 ? all & ~(known >= 32 ? bits[i] : bits[i] & ((1u << known) - 1u)) : all;
+  };
+  int64_t j = int64_t(wave) * per + sub;
+  uint32_t none = wave < words ? clear(wave) : 0u;
+  int32_t r = j < nrows ? rows[j] : -1;
+  double w = j < nrows && c0 < R ? W[j * R + c0] : 0.0;
+  for (int32_t i = wave; i < words;) {
+    for (; none; none &= none - 1u) {
+      float* row = A + (int64_t(32) * i + (__ffs(none) - 1)) * R;
+      for (int c = lane; c < R; c += 64) row[c] = 0.f;
+    }
+    i += nwave;
+    if (i < words) none = clear(i);
+  }
+  while (j < nrows) {
+    if (r >= 0 && c0 < R) {
+      for (int c = c0;;) {
+        A[int64_t(r) * R + c] = float(w);
+        W[j * R + c] = 0.0;
+        c += 1 << lshift;
+        if (c >= R) break;
+        w = W[j * R + c];
+      }
+    }
+    j += int64_t(nwave) * per;
+    if (j < nrows) {
+      r = rows[j];
+      w = c0 < R ? W[j * R + c0] : 0.0;
     }
   }
 }
@@ -427,6 +497,23 @@ int launch_edge_prep(const CsfDev& B, float* Z, int64_t z_elems, int32_t* brk, i
                      int32_t NB, hipStream_t st) {
   const int64_t work = std::max<int64_t>(z_elems / 4, int64_t(nblk) + 1);
   edge_prep_kernel<<<grid_for(work, 256, 16384), 256, 0, st>>>(B, Z, z_elems, brk, nblk, NB);
+  TT_HIP_CHECK(hipGetLastError());
+  return TENTACO_OK;
+}
+
+int launch_shared_rows(const CsfDev& B, int32_t NB, int2* slots, int32_t* rows, hipStream_t st) {
+  const int32_t nblk = int32_t((int64_t(B.nnz) + NB - 1) / NB);
+  shared_rows_kernel<<<(nblk + 255) / 256, 256, 0, st>>>(B, NB, nblk, slots, rows);
+  TT_HIP_CHECK(hipGetLastError());
+  return TENTACO_OK;
+}
+
+int launch_edge_rows(const WalkTables& wt, int32_t nblk, float* A, int32_t a_rows, int R, hipStream_t st) {
+  int lshift = 0;
+  while (lshift < 6 && (1 << lshift) < R) ++lshift;
+  const int64_t waves = std::max<int64_t>((int64_t(a_rows) + 31) / 32, (2 * int64_t(nblk)) >> (6 - lshift));
+  edge_rows_kernel<<<grid_for(waves, 4, 8192), 256, 0, st>>>(wt.rows, 2 * nblk, wt.W, wt.bits, wt.nbits, A,
+                                                             a_rows, R, lshift);
   TT_HIP_CHECK(hipGetLastError());
   return TENTACO_OK;
 }
@@ -657,15 +744,15 @@ int launch_mttkrp_level(const CsfDev& B, const FactorsDev& F, int level, int R, 
 
 int launch_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A,
                   int32_t a_rows, bool dense_root, const Variant& vr, void* ws,
-                  const int32_t* starts, hipStream_t st) {
+                  const WalkTables& tables, hipStream_t st) {
   if (R <= 0 || R > kMaxRankAny)
     return fail(TENTACO_EUNSUPPORTED, "rank R=%d outside 1..%d", R, kMaxRankAny);
   if (vr.family < 0) return fail(TENTACO_EINVAL, "invalid variant");
   switch (B.order) {
-    case 2: return order_mttkrp<2>(B, F, R, A, a_rows, dense_root, vr, ws, starts, st);
-    case 3: return order_mttkrp<3>(B, F, R, A, a_rows, dense_root, vr, ws, starts, st);
-    case 4: return order_mttkrp<4>(B, F, R, A, a_rows, dense_root, vr, ws, starts, st);
-    case 5: return order_mttkrp<5>(B, F, R, A, a_rows, dense_root, vr, ws, starts, st);
+    case 2: return order_mttkrp<2>(B, F, R, A, a_rows, dense_root, vr, ws, tables, st);
+    case 3: return order_mttkrp<3>(B, F, R, A, a_rows, dense_root, vr, ws, tables, st);
+    case 4: return order_mttkrp<4>(B, F, R, A, a_rows, dense_root, vr, ws, tables, st);
+    case 5: return order_mttkrp<5>(B, F, R, A, a_rows, dense_root, vr, ws, tables, st);
     default: return fail(TENTACO_EUNSUPPORTED, "order %d outside 2..5", B.order);
   }
 }

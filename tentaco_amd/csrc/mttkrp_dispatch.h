@@ -35,7 +35,7 @@ __device__ __forceinline__ int32_t upper_index(const int64_t* __restrict__ off, 
 // pick the order.
 template <int N>
 int order_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A, int32_t a_rows,
-                 bool dense_root, const Variant& vr, void* ws, const int32_t* starts,
+                 bool dense_root, const Variant& vr, void* ws, const WalkTables& wt,
                  hipStream_t st);
 template <int N>
 int order_level(const CsfDev& B, const FactorsDev& F, int level, int R, float* A, int32_t a_rows,
@@ -54,5 +54,8 @@ int all_orders_batch_occupancy(int block, int R, int* per_cu);
 int launch_edge_prep(const CsfDev& B, float* Z, int64_t z_elems, int32_t* brk, int32_t nblk,
                      int32_t NB, hipStream_t st);
 int launch_narrow(const double* W, float* A, int64_t n, hipStream_t st);
+// After an edge-parallel walk over nblk workgroups with shared rows: write them
+// (and zero them for the next call) and zero the rows that no root node writes.
+int launch_edge_rows(const WalkTables& wt, int32_t nblk, float* A, int32_t a_rows, int R, hipStream_t st);
 
 }  // namespace tt

@@ -104,6 +104,9 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
   const int32_t* __restrict__ brk = global_ptr(brk_p);
   const int32_t* __restrict__ starts = global_ptr(starts_p);
 
+  // read here: at the end its latency would stand alone
+  const int2 slot = slots ? *slots : make_int2(0, 0);
+
   const int lane = int(threadIdx.x) & 63;
   const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
   const int nwv = int(blockDim.x) >> 6;
@@ -475,7 +478,7 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
       const bool shared = key == first || key == last;
       if constexpr (EP) {
         if (!shared) A[o] = float(s);
-        else if (slots) unsafeAtomicAdd(W + int64_t(key == first ? slots->x : slots->y) * cols + col, s);
+        else if (slots) unsafeAtomicAdd(W + int64_t(key == first ? slot.x : slot.y) * cols + col, s);
         else unsafeAtomicAdd(A + o, float(s));
       } else {
         if (shared) unsafeAtomicAdd(W + o, s);
@@ -508,9 +511,11 @@ __global__ __launch_bounds__(512, (edge_waves<N, R>())) void edge_kernel(CsfDev 
                                                    const int32_t* __restrict__ brk,
                                                    const int32_t* __restrict__ starts,
                                                    int32_t G, int32_t NB,
-                                                   double* __restrict__ W) {
+                                                   double* __restrict__ W,
+                                                   const int2* __restrict__ slots) {
   extern __shared__ __align__(16) unsigned char smem[];
-  edge_block<N, R, EP>(B, F, A, Rr, brk, starts, blockIdx.x, G, NB, smem, W);
+  edge_block<N, R, EP>(B, F, A, Rr, brk, starts, blockIdx.x, G, NB, smem, W,
+                       EP && slots ? slots + blockIdx.x : nullptr);
 }
 
 
@@ -1337,7 +1342,7 @@ int batch_occupancy_order(int family, int block, int Rr, int32_t NB, int* per_cu
 template <int N, int R>
 int launch_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A,
                  int32_t a_rows, bool dense_root, const Variant& vr, void* ws,
-                 const int32_t* starts, hipStream_t st) {
+                 const WalkTables& wt, hipStream_t st) {
   const int64_t a_elems = int64_t(a_rows) * Rr;
   if (vr.family == kSliceRow) {
     if (!dense_root) {
@@ -1402,12 +1407,14 @@ int launch_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A,
   const int64_t NB = nnz_per_block(vr, Rr);
   const int64_t nblk = (int64_t(B.nnz) + NB - 1) / NB;
   int32_t* brk = static_cast<int32_t*>(ws);
+  const int32_t* starts = wt.starts;
+  const bool shared = vr.family == kEdgeParallel && starts && wt.slots && nblk > 0;
   // edge-serial: rows accumulate in FP64 (W, after the brackets), narrowed
   // to A at the end; the prep zeroes W instead of A
   double* W = (vr.family == kEdgeSerial && nblk > 0)
                   ? reinterpret_cast<double*>(static_cast<char*>(ws) + edge_brk_bytes(B, NB))
                   : nullptr;
-  {
+  if (!shared) {
     float* Z = W ? reinterpret_cast<float*>(W) : A;
     const int64_t z_elems = W ? 2 * a_elems : a_elems;
     const int rc = starts ? launch_fill(Z, z_elems, 0.f, st)
@@ -1424,13 +1431,16 @@ int launch_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A,
   ktimer_begin(st);
   if (vr.family == kEdgeSerial) {
     edge_kernel<N, R, false><<<int(nblk), vr.block, lds, st>>>(B, F, A, Rr, brk, starts,
-                                                               vr.group, int32_t(NB), W);
+                                                               vr.group, int32_t(NB), W, nullptr);
   } else {
     edge_kernel<N, R, true><<<int(nblk), vr.block, lds, st>>>(B, F, A, Rr, brk, starts,
-                                                              vr.group, int32_t(NB), nullptr);
+                                                              vr.group, int32_t(NB),
+                                                              shared ? wt.W : nullptr,
+                                                              shared ? wt.slots : nullptr);
   }
   TT_HIP_CHECK(hipGetLastError());
   ktimer_end(st, "edge_kernel");
+  if (shared) return launch_edge_rows(wt, int32_t(nblk), A, a_rows, Rr, st);
   return W ? launch_narrow(W, A, a_elems, st) : TENTACO_OK;
 }
 
@@ -1477,10 +1487,10 @@ int launch_level_order(const CsfDev& B, const FactorsDev& F, int level, int Rr, 
 // ---- one tensor order's entry points (mttkrp_dispatch.h) --------------------
 template <int N>
 int order_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A, int32_t a_rows,
-                 bool dense_root, const Variant& vr, void* ws, const int32_t* starts,
+                 bool dense_root, const Variant& vr, void* ws, const WalkTables& wt,
                  hipStream_t st) {
   return with_rank_layout(R, [&](auto r) {
-    return launch_typed<N, r()>(B, F, R, A, a_rows, dense_root, vr, ws, starts, st);
+    return launch_typed<N, r()>(B, F, R, A, a_rows, dense_root, vr, ws, wt, st);
   });
 }
 
@@ -1514,7 +1524,7 @@ int order_batch_occupancy(int family, int block, int R, int32_t NB, int* per_cu)
 // Instantiates order N's entry points (one source per order).
 #define TT_INSTANTIATE_ORDER(N)                                                                 \
   template int tt::order_mttkrp<N>(const CsfDev&, const FactorsDev&, int, float*, int32_t, bool, \
-                                   const Variant&, void*, const int32_t*, hipStream_t);         \
+                                   const Variant&, void*, const WalkTables&, hipStream_t);         \
   template int tt::order_level<N>(const CsfDev&, const FactorsDev&, int, int, float*, int32_t,  \
                                   hipStream_t);                                                 \
   template int tt::order_batch<N>(const BatchLaunch&, hipStream_t);                             \
