@@ -297,7 +297,11 @@ int tentaco_csf_tuned(const tentaco_csf* h, int R, int* variant, int* source);
 /* The variant a call with `variant` runs at rank R without consulting a
  * selector: AUTO gives the recorded choice, else the structural heuristic
  * (slice-row for many even slices; edge-parallel 256 x 16 below 300k
- * nonzeros and 512 x 64 from there, stepping down to tiles that fit). */
+ * nonzeros and 512 x 64 from there, stepping down to tiles that fit). These
+ * are names: a call that AUTO resolves by the heuristic runs the family at a
+ * size chosen from nnz and R (about 3000 runs of 32 to 512 nonzeros) or, for
+ * 3-mode short fibres, from the mean slice. A variant given by number runs as
+ * named. */
 int tentaco_csf_resolve_variant(const tentaco_csf* h, int R, int variant, int* out);
 
 /* ---- CP-ALS around the batched MTTKRP ---------------------------------- */

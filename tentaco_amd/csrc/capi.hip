@@ -62,7 +62,10 @@ void free_handle(tentaco_csf* h) {
   (void)hipFree(h->ws);
   for (void* w : h->ws_retired) (void)hipFree(w);
   for (int i = 0; i < h->starts.n; ++i) (void)hipFree(h->starts.p[i]);
-  for (int i = 0; i < h->starts.ns; ++i) (void)hipFree(h->starts.mem[i]);
+  for (int i = 0; i < h->starts.ns; ++i) {
+    (void)hipFree(h->starts.mem[i]);
+    (void)hipEventDestroy(h->starts.used[i]);
+  }
   (void)hipFree(h->starts.bits);
   for (int m = 0; m < kMaxOrder; ++m) (void)hipFree(h->stage_f[m]);
   (void)hipFree(h->stage_a);
@@ -231,7 +234,9 @@ int build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStream_t st) {
   const size_t bbytes = (size_t(nbits) + 31) / 32 * sizeof(uint32_t);
   void* mem = nullptr;
   uint32_t* bits = s.bits;
-  bool ok = hipMalloc(&mem, o_w + wbytes) == hipSuccess;
+  hipEvent_t used = nullptr;
+  bool ok = hipMalloc(&mem, o_w + wbytes) == hipSuccess &&
+            hipEventCreateWithFlags(&used, hipEventDisableTiming) == hipSuccess;
   if (ok && !bits) {
     ok = hipMalloc(reinterpret_cast<void**>(&bits), bbytes) == hipSuccess &&
          hipMemsetAsync(bits, 0, bbytes, st) == hipSuccess && launch_batch_rowbits(B, bits, st) == TENTACO_OK;
@@ -247,6 +252,7 @@ int build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStream_t st) {
     (void)hipGetLastError();
     clear_error();
     (void)hipFree(mem);
+    if (used) (void)hipEventDestroy(used);
     if (!s.bits) (void)hipFree(bits);
     return TENTACO_ENOMEM;
   }
@@ -254,6 +260,7 @@ int build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStream_t st) {
   s.nb[s.ns] = NB;
   s.rank[s.ns] = R;
   s.mem[s.ns] = mem;
+  s.used[s.ns] = used;
   WalkTables& t = s.sh[s.ns++];
   t.slots = slots;
   t.rows = rows;
@@ -288,9 +295,10 @@ WalkTables walk_tables(tentaco_csf* h, const Variant& vr, int R, bool build, hip
   int j = 0;
   while (j < s.ns && (s.nb[j] != NB || s.rank[j] != R)) ++j;
   const bool ep = vr.family == kEdgeParallel && B.nnz >= kSharedBlocks * NB;
-  if (build && (i == s.n || (ep && j == s.ns)) &&
-      (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone))
-    build = false;
+  const bool capturing =
+      (ep || i == s.n) &&
+      (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone);
+  if (capturing) build = false;
   if (i == s.n) {
     if (!build || s.n >= WalkStarts::kTables) return t;
     int32_t* p = nullptr;
@@ -308,7 +316,7 @@ WalkTables walk_tables(tentaco_csf* h, const Variant& vr, int R, bool build, hip
     s.p[s.n++] = p;
   }
   if (ep && j == s.ns && build && s.ns < WalkStarts::kTables) (void)build_shared_rows(h, NB, R, st);
-  if (ep && j < s.ns) t = s.sh[j];
+  if (ep && j < s.ns && !capturing) t = s.sh[j];
   t.starts = s.p[i];
   return t;
 }
@@ -914,8 +922,16 @@ int tentaco_mttkrp_dev(tentaco_csf* h, int R, const float* const* factors_dev, f
   const WalkTables tables =
       walk_tables(h, vr, R, !h->reserved, static_cast<hipStream_t>(stream));
   const bool dense = h->dense_root && a_rows == h->nodes[0];
-  return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws, tables,
-                       static_cast<hipStream_t>(stream));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (!tables.slots) return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws, tables, st);
+  WalkStarts& s = h->starts;
+  std::lock_guard<std::mutex> lk(s.mu);
+  int j = 0;
+  while (s.sh[j].slots != tables.slots) ++j;
+  TT_HIP_CHECK(hipStreamWaitEvent(st, s.used[j], 0));
+  rc = launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws, tables, st);
+  TT_HIP_CHECK(hipEventRecord(s.used[j], st));
+  return rc;
 }
 
 int tentaco_mttkrp_dev_noalloc(tentaco_csf* h, int R, const float* const* factors_dev,

@@ -21,11 +21,15 @@ struct WalkStarts {
   int n = 0;
   int64_t wn[kTables] = {};
   int32_t* p[kTables] = {};
-  // the shared rows of edge-parallel tiles, by nonzeros per workgroup and rank
+  // the shared rows of edge-parallel tiles, by nonzeros per workgroup and rank.
+  // A call adds to them, so each waits for the one before on whatever stream
+  // (`used`, recorded behind every call, both under mu); a call under capture,
+  // whose replays no one orders, does without them
   int ns = 0;
   int64_t nb[kTables] = {};
   int rank[kTables] = {};
   void* mem[kTables] = {};
+  hipEvent_t used[kTables] = {};
   WalkTables sh[kTables] = {};
   uint32_t* bits = nullptr;
 };

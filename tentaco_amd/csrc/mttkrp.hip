@@ -3,34 +3,32 @@
 //   A(i,:) = sum over the subtree of root node i of
 //            B(i,k,l,...) * C(k,:) (.) D(l,:) (.) ...
 //
-// computed in factorised form (the association of
-// tensor_kernels/mttkrp{3,4}_csf_cpu_taco_workspace.h and of
-// mttkrp5_csf_cpu_taco.h): the nonzeros of a level-(N-2) fiber are summed as
-// val * M_{N-1}(l,:), the fiber sum is multiplied by its own factor row once,
-// and so on up to the root. Factor rows are gathered as float4 fragments
-// over a row group of lanes (rowops.h).
+// computed in factorised form: the upper levels' row product of a fibre is
+// formed once, and multiplies the leaf rows of its nonzeros (the workspace
+// kernels of tensor_kernels/mttkrp{3,4}_csf_cpu_taco_workspace.h and
+// mttkrp5_csf_cpu_taco.h sum a fibre first). Factor rows are gathered as float4
+// fragments over a row group of lanes (rowops.h).
 //
 // Three kernel families form the variant table:
-//  * edge-serial (ES): the nonzeros are cut into equal runs of G consecutive
-//    positions, one run per row group (the reference's eb_sr work split,
-//    mttkrp3_csf_ebsr.h:4-77). A run walks its positions serially, closing
-//    fibers and slices as it crosses their ends. Slices that start and end
-//    inside one run are stored; a run's first and last slice may be shared
-//    with neighbouring runs and are added atomically into the pre-zeroed A.
-//  * edge-parallel (EP): the same runs, but the shared first/last slice
-//    partials of all runs of a workgroup are combined by a segmented
-//    parallel reduction in LDS (the role of segReduceGroup,
-//    gpu_library.h:295-321, redone for wave64 and R-wide rows); only the
-//    workgroup's first and last slice are added atomically.
+//  * edge-serial (ES) and edge-parallel (EP): the nonzeros are cut into equal
+//    runs, one per wave, of as many consecutive positions as the wave's row
+//    groups would walk at G each (the reference's eb_sr work split,
+//    mttkrp3_csf_ebsr.h:4-77, gives a run to a lane group). A slice that starts
+//    and ends inside one run is stored; the first and last slices of a
+//    workgroup's runs are summed in FP64 in LDS (the role of segReduceGroup,
+//    gpu_library.h:295-321), and only the workgroup's first and last slice can
+//    be another's too. ES adds them to FP64 rows of the whole output, EP to the
+//    pre-zeroed output with FP32 atomics or, from 2048 workgroups on, to FP64
+//    rows of the shared slices (edge_rows_kernel).
 //  * slice-row (SR): one workgroup per root node, its level-1 children
 //    spread over the workgroup's row groups, rows reduced with xor shuffles
 //    and LDS and stored once. No atomics, no zero fill for a dense root,
 //    deterministic; balanced only when slices are.
 //
-// Runs find their starting node at every level with an upper-bound binary
-// search inside the workgroup's bracket, which a prep kernel computes
-// together with the zero fill of A (the reference's two partition-search
-// launches plus cudaMemset, mttkrp3_csf_gpu_taco.h:88-94, in one launch).
+// Where a wave's run starts (its node at every level) is a table that the
+// handle or batch keeps for a run length, or comes from brackets that the call
+// itself writes, with the zero fill of A, in one prep launch (the reference's
+// two partition-search launches plus cudaMemset, mttkrp3_csf_gpu_taco.h:88-94).
 
 #include <algorithm>
 #include <climits>
