@@ -41,8 +41,10 @@ constexpr int kMaxR = 64;
 constexpr int kApplyRows = 64;    // rows per block of the apply / scale kernels
 constexpr int kStatRows = 2048;   // rows per block of the reduction kernels
 // Blocks of a mode step's fused update: the rows per block are chosen so that
-// about this many cover the chip without many partials to sum.
-constexpr int kUpdBlocks = 256;
+// about 256 cover the chip without many partials to sum, and for long modes up
+// to 1024, four a CU, to keep enough bytes in flight (64 tensors, 9.3M rows and
+// less per step, R = 32: 689 and 413 us a step, the finish 10 and 18).
+constexpr int kUpdBlocks = 256, kUpdBlocksMax = 1024;
 constexpr int kUpdUnit = 128;     // rows per block: a multiple of this
 
 struct CpdJob {
@@ -621,7 +623,8 @@ int build_jobs(tentaco_cpd* c, int m, const std::vector<int>& tensors, std::vect
   int32_t nu = 0;
   int64_t total = 0;
   for (int t : tensors) total += c->dims[size_t(t)][size_t(m)];
-  const int64_t per = (total + kUpdBlocks - 1) / kUpdBlocks;
+  const int64_t blocks = std::min<int64_t>(kUpdBlocksMax, std::max<int64_t>(kUpdBlocks, total / 4096));
+  const int64_t per = (total + blocks - 1) / blocks;
   const int32_t urows = int32_t((per + kUpdUnit - 1) / kUpdUnit * kUpdUnit);
   for (int t : tensors) {
     CpdJob J;
