@@ -225,7 +225,10 @@ int tentaco_csf_info(const tentaco_csf* h, int* order, int64_t* nnz,
  * the variant named here (AUTO: the one it resolves to) the call builds the
  * table of the waves' start nodes, which later calls read instead of writing
  * brackets (4(order-1) B per 16 to 1024 nonzeros; without a reserve call, the
- * first call of a run length builds it and synchronizes its stream); the
+ * first call of a run length builds it and synchronizes its stream), and for
+ * edge-parallel tiles of 2048 workgroups and more the FP64 rows of the slices
+ * that workgroups share (16 R B per workgroup; calls outside capture use them,
+ * each waiting for the one before on this handle); the
  * edge-serial family also accumulates its rows in FP64 (output rows x R
  * doubles), which keeps atomics on giant slices accurate. For 3-mode
  * handles it also builds the slice-row structures: the expansion (4 B per
@@ -472,7 +475,8 @@ int tentaco_csf_ttv_layout(const tentaco_csf* h, int* bands, int64_t* device_byt
  * CSF per mode ordering) in one persistent kernel: all tasks' nonzeros are cut
  * into equal work items that persistent workgroups pull from a device
  * counter, so uneven tensor sizes do not leave the GPU idle and the whole
- * batch costs two launches (prep + persistent), or one graph launch. No
+ * batch costs two launches (the walk and its shared rows; long batches of
+ * several orders one walk per order), or one graph launch. No
  * counterpart in the reference, which launches per tensor-mode
  * (mttkrp_csf_gpu.h:186-217). */
 typedef struct tentaco_batch tentaco_batch;
@@ -484,7 +488,7 @@ int tentaco_batch_create(tentaco_csf* const* tasks, int ntasks, int R,
  * the factor of level m (slots past order-1 ignored). outs_dev[t] holds
  * out_rows[t] x R floats and is fully overwritten by each run. Builds each
  * task's row bitmap (one bit per output row: rows that root nodes with
- * nonzeros store, which the edge-parallel prep does not zero) on the null
+ * nonzeros store, which are not zeroed) on the null
  * stream and synchronizes the device before returning. */
 int tentaco_batch_set_operands(tentaco_batch* b, const float* const* factors_dev,
                                float* const* outs_dev, const int32_t* out_rows);
@@ -495,14 +499,13 @@ int tentaco_batch_set_operands(tentaco_batch* b, const float* const* factors_dev
  * a captured graph. */
 int tentaco_batch_configure(tentaco_batch* b, int family, int block, int group);
 /* The tile and schedule (see tentaco_batch_set_schedule) of the tasks of one
- * tensor order (2..5) only; each order group runs its own persistent launch,
- * so the groups may differ. Drops a captured graph. */
+ * tensor order (2..5) only; the groups may differ. Drops a captured graph. */
 int tentaco_batch_configure_order(tentaco_batch* b, int order, int family, int block,
                                   int group, int schedule);
 /* The tile and schedule an order group runs with. */
 int tentaco_batch_get_config(const tentaco_batch* b, int order, int* family, int* block,
                              int* group, int* schedule);
-/* Enqueue prep + persistent kernel on `stream`. */
+/* Enqueue a run on `stream`. */
 int tentaco_batch_run(tentaco_batch* b, void* stream);
 /* Capture tentaco_batch_run into an instantiated hipGraph (kernels only). */
 int tentaco_batch_capture(tentaco_batch* b, void* stream);

@@ -19,7 +19,6 @@
 using tt::fail;
 
 #include "handle.h"
-#include "host_copy.h"
 
 namespace tt {
 namespace {
@@ -41,14 +40,15 @@ int validate_csf(const taco_tensor_t* B, int order, tentaco_csf* h, const LevelF
 }
 
 template <class T>
-int upload_array(T** dst, const T* src, int64_t n, HostStage& stage) {
+int upload_array(T** dst, const T* src, int64_t n) {
   *dst = nullptr;
   const size_t bytes = size_t(std::max<int64_t>(n, 1)) * sizeof(T);
   if (hipMalloc(reinterpret_cast<void**>(dst), bytes) != hipSuccess) {
     *dst = nullptr;
     return fail(TENTACO_ENOMEM, "hipMalloc of %zu bytes failed", bytes);
   }
-  return stage.to_device(*dst, src, size_t(n) * sizeof(T));
+  if (n > 0) TT_HIP_CHECK(hipMemcpy(*dst, src, size_t(n) * sizeof(T), hipMemcpyHostToDevice));
+  return TENTACO_OK;
 }
 
 void free_handle(tentaco_csf* h) {
@@ -370,23 +370,25 @@ int ensure_events() {
   return TENTACO_OK;
 }
 
-// A handle with B's arrays on the device once `stage` is drained; a level's
-// arrays are copied while its coordinates are still being checked.
-int upload_csf(const taco_tensor_t* B, int order, HostStage& stage, tentaco_csf** out) {
+// A handle with B's arrays on the device. A level's arrays are copied while its
+// coordinates are still being checked (2M nonzeros: of 0.4 ms of checks 0.15
+// are left in the way). Copying through pinned slabs of the call's own instead
+// gained as much as allocating them takes, and allocating them took several ms
+// now and then.
+int upload_csf(const taco_tensor_t* B, int order, tentaco_csf** out) {
   tentaco_csf* h = new tentaco_csf;
   h->order = order;
   bool warm = false;
   int rc = validate_csf(B, order, h, [&](int m, int64_t parents, int64_t nodes) {
     int r = warm ? TENTACO_OK : warm_device();
     warm = true;
-    if (!r) r = upload_array(&h->d_pos[m], B->indices[m][0], parents + 1, stage);
-    if (!r) r = upload_array(&h->d_crd[m], B->indices[m][1], nodes, stage);
+    if (!r) r = upload_array(&h->d_pos[m], B->indices[m][0], parents + 1);
+    if (!r) r = upload_array(&h->d_crd[m], B->indices[m][1], nodes);
     return r;
   });
-  if (!rc) rc = upload_array(&h->d_crd0, B->indices[0][1], h->nodes[0], stage);
-  if (!rc) rc = upload_array(&h->d_vals, B->vals, h->nodes[order - 1], stage);
+  if (!rc) rc = upload_array(&h->d_crd0, B->indices[0][1], h->nodes[0]);
+  if (!rc) rc = upload_array(&h->d_vals, B->vals, h->nodes[order - 1]);
   if (rc) {
-    (void)stage.drain();
     free_handle(h);
     return rc;
   }
@@ -418,18 +420,13 @@ int host_mttkrp(int order, taco_tensor_t* A, taco_tensor_t* B,
   if (!A || !A->dimensions || !A->vals) return fail(TENTACO_EINVAL, "A is NULL/incomplete");
   if (!factors) return fail(TENTACO_EINVAL, "factors is NULL");
   DevBuf fb[kMaxOrder], abuf;
-  HostStage stage(kStageFirst);
   tentaco_csf* h = nullptr;
-  int rc = upload_csf(B, order, stage, &h);
+  int rc = upload_csf(B, order, &h);
   if (rc) return rc;
   struct Guard {
     tentaco_csf* h;
-    HostStage& stage;
-    ~Guard() {
-      (void)stage.drain();  // nothing is freed under a copy
-      free_handle(h);
-    }
-  } guard{h, stage};
+    ~Guard() { free_handle(h); }
+  } guard{h};
   const int R = A->dimensions[1];
   const int32_t a_rows = A->dimensions[0];
   if (R <= 0) return fail(TENTACO_EINVAL, "A has %d columns", R);
@@ -441,8 +438,7 @@ int host_mttkrp(int order, taco_tensor_t* A, taco_tensor_t* B,
     rc = check_factor(factors[m - 1], m, h, R);
     if (rc) return rc;
     float* d = nullptr;
-    rc = upload_array(&d, factors[m - 1]->vals, int64_t(factors[m - 1]->dimensions[0]) * R,
-                      stage);
+    rc = upload_array(&d, factors[m - 1]->vals, int64_t(factors[m - 1]->dimensions[0]) * R);
     fb[m].p = d;
     if (rc) return rc;
     fdev[m - 1] = d;
@@ -476,7 +472,8 @@ int host_mttkrp(int order, taco_tensor_t* A, taco_tensor_t* B,
     TT_HIP_CHECK(hipEventElapsedTime(&ms, g_ev0, g_ev1));
     g_last_ms.store(ms);
   }
-  return stage.to_host(A->vals, abuf.p, abytes);
+  TT_HIP_CHECK(hipMemcpy(A->vals, abuf.p, abytes, hipMemcpyDeviceToHost));
+  return TENTACO_OK;
 }
 
 int host_ttv(int order, taco_tensor_t* A, taco_tensor_t* B, taco_tensor_t* c) {
@@ -484,18 +481,13 @@ int host_ttv(int order, taco_tensor_t* A, taco_tensor_t* B, taco_tensor_t* c) {
   if (!A || !A->vals) return fail(TENTACO_EINVAL, "A is NULL/incomplete");
   if (!c || !c->dimensions || !c->vals) return fail(TENTACO_EINVAL, "c is NULL/incomplete");
   DevBuf cbuf, ybuf;
-  HostStage stage(kStageFirst);
   tentaco_csf* h = nullptr;
-  int rc = upload_csf(B, order, stage, &h);
+  int rc = upload_csf(B, order, &h);
   if (rc) return rc;
   struct Guard {
     tentaco_csf* h;
-    HostStage& stage;
-    ~Guard() {
-      (void)stage.drain();  // nothing is freed under a copy
-      free_handle(h);
-    }
-  } guard{h, stage};
+    ~Guard() { free_handle(h); }
+  } guard{h};
   // a handle for one call: the banded layout's build would cost more than
   // it saves
   h->ttv_bands = 1;
@@ -506,7 +498,7 @@ int host_ttv(int order, taco_tensor_t* A, taco_tensor_t* B, taco_tensor_t* c) {
   if (A->dimensions && A->dimensions[0] < nf)
     return fail(TENTACO_EINVAL, "A has %d entries, B has %d fibers", A->dimensions[0], nf);
   float* cd = nullptr;
-  rc = upload_array(&cd, c->vals, c->dimensions[0], stage);
+  rc = upload_array(&cd, c->vals, c->dimensions[0]);
   cbuf.p = cd;
   if (rc) return rc;
   if (hipMalloc(&ybuf.p, std::max<size_t>(size_t(nf) * 4, 4)) != hipSuccess)
@@ -529,7 +521,8 @@ int host_ttv(int order, taco_tensor_t* A, taco_tensor_t* B, taco_tensor_t* c) {
     TT_HIP_CHECK(hipEventElapsedTime(&ms, g_ev0, g_ev1));
     g_last_ms.store(ms);
   }
-  return stage.to_host(A->vals, ybuf.p, size_t(nf) * 4);
+  if (nf > 0) TT_HIP_CHECK(hipMemcpy(A->vals, ybuf.p, size_t(nf) * 4, hipMemcpyDeviceToHost));
+  return TENTACO_OK;
 }
 
 // Legacy void entry points report failures on stderr (as gpuErrchk does,
@@ -658,17 +651,7 @@ int tentaco_csf_upload(const taco_tensor_t* B, int order, tentaco_csf** out) {
   clear_error();
   if (!out) return fail(TENTACO_EINVAL, "out is NULL");
   *out = nullptr;
-  HostStage stage(kStageFirst);
-  tentaco_csf* h = nullptr;
-  int rc = upload_csf(B, order, stage, &h);
-  if (rc) return rc;
-  rc = stage.drain();
-  if (rc) {
-    free_handle(h);
-    return rc;
-  }
-  *out = h;
-  return TENTACO_OK;
+  return upload_csf(B, order, out);
 }
 
 int tentaco_csf_upload_async(const taco_tensor_t* B, int order, void* stream, tentaco_csf** out) {

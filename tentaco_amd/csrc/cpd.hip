@@ -577,7 +577,7 @@ struct tentaco_cpd {
   hipEvent_t fork = nullptr, join = nullptr;
   // tentaco_cpd_factor copies through it, one caller at a time
   mutable std::mutex stage_mu;
-  mutable HostStage stage{0};
+  mutable HostStage stage;
 
   ~tentaco_cpd() {
     for (auto& s : step) {

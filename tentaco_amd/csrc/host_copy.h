@@ -1,4 +1,4 @@
-// Copies between pageable host memory and the device through pinned slabs.
+// Copies from the device to pageable host memory through pinned slabs.
 #pragma once
 
 #include <algorithm>
@@ -20,23 +20,21 @@ static __global__ __launch_bounds__(256) void stage_copy_kernel(const uint32_t* 
   for (int32_t i = 4 * n4 + tid; i < n; i += nt) dst[i] = src[i];
 }
 
-// A pageable hipMemcpy moves 17 to 35 GB/s here and takes 30 to 60 us however
+// A pageable hipMemcpy from the device moves 17 GB/s here and takes 70 us however
 // small it is; pinned memory moves at 50 GB/s. So a copy is cut into slabs of
-// pinned memory, and the core fills (or empties) one while the device moves
-// others. The device moves a slab with stage_copy_kernel: a hipMemcpyAsync of
-// 512 KB costs 24 us in a row of them (8 MB: 389 us from the device, 383 to
-// it), a kernel 12 (263 and 218). One core empties 512 KB in 16 us.
-// Twelve factors of 0.3 to 3.8 MB and their weights, 22 MB, from the device:
-// 1.86 -> 0.96 ms; a host MTTKRP's 22 MB to it and 1.3 MB back 0.93 -> 0.75 ms.
-// The slabs (kSlabs x kSlab bytes) belong to the object that stages through
-// them and are freed with it. Pinned or device operands, an object used from
-// another device than its own, and a failed allocation take hipMemcpy.
-// Sizes are in bytes, whole words.
-constexpr size_t kStageFirst = size_t(1) << 20;
+// pinned memory, and the core empties one while the device fills others. The
+// device fills a slab with stage_copy_kernel: a hipMemcpyAsync of 512 KB costs
+// 24 us in a row of them (8 MB: 389 us), a kernel 12 (263). One core empties
+// 512 KB in 16 us. Twelve factors of 0.3 to 3.8 MB and their weights, 22 MB:
+// 1.86 -> 0.96 ms.
+// The slabs (kSlabs x kSlab bytes) belong to the object that copies through
+// them, which has to live for several copies (allocating them takes 0.1 ms, and
+// several now and then), and are freed with it. Pinned or device operands, an
+// object used from another device than its own, and a failed allocation take
+// hipMemcpy. Sizes are in bytes, whole words.
 class HostStage {
  public:
-  // The slabs are allocated (0.1 ms) by the first copy of at least `first` bytes.
-  explicit HostStage(size_t first) : first_(first) {}
+  HostStage() = default;
   HostStage(const HostStage&) = delete;
   HostStage& operator=(const HostStage&) = delete;
   ~HostStage() {
@@ -47,28 +45,6 @@ class HostStage {
     (void)hipHostFree(mem_);
   }
 
-  // dst[0..n) = src[0..n), queued on the null stream: src may change when this
-  // returns, dst is whole after drain().
-  int to_device(void* dst, const void* src, size_t n) {
-    if (n == 0) return TENTACO_OK;
-    if (!usable(src, n)) {
-      TT_HIP_CHECK(hipMemcpy(dst, src, n, hipMemcpyHostToDevice));
-      return TENTACO_OK;
-    }
-    for (size_t o = 0; o < n; o += kSlab) {
-      const size_t k = std::min(kSlab, n - o);
-      const int i = next_;
-      if (busy_[i]) TT_HIP_CHECK(hipEventSynchronize(ev_[i]));
-      busy_[i] = false;
-      std::memcpy(slab(i), static_cast<const char*>(src) + o, k);
-      TT_HIP_CHECK(copy(static_cast<char*>(dst) + o, slab(i), k));
-      TT_HIP_CHECK(hipEventRecord(ev_[i], nullptr));
-      busy_[i] = true;
-      next_ = (i + 1) % kSlabs;
-    }
-    return TENTACO_OK;
-  }
-
   // dst[0..n) = src[0..n) and, if given, dst2[0..n2) = src2[0..n2) (at most a
   // slab) behind it; returns when both are whole. The core reads a slab that the
   // device has written from memory, which bounds this (two threads emptying
@@ -76,7 +52,7 @@ class HostStage {
   int to_host(void* dst, const void* src, size_t n, void* dst2 = nullptr, const void* src2 = nullptr,
               size_t n2 = 0) {
     if (n + n2 == 0) return TENTACO_OK;
-    if (n2 > kSlab || !usable(n ? dst : dst2, n + n2) || (n2 && !usable(dst2, n2))) {
+    if (n2 > kSlab || !usable(n ? dst : dst2) || (n2 && !usable(dst2))) {
       if (n) TT_HIP_CHECK(hipMemcpy(dst, src, n, hipMemcpyDeviceToHost));
       if (n2) TT_HIP_CHECK(hipMemcpy(dst2, src2, n2, hipMemcpyDeviceToHost));
       return TENTACO_OK;
@@ -105,7 +81,7 @@ class HostStage {
     return TENTACO_OK;
   }
 
-  // Waits for the copies queued by to_device.
+  // Waits for the slabs that a failed copy left in flight.
   int drain() {
     for (int i = 0; i < kSlabs; ++i) {
       if (busy_[i]) TT_HIP_CHECK(hipEventSynchronize(ev_[i]));
@@ -126,9 +102,8 @@ class HostStage {
 
   char* slab(int i) { return mem_ + size_t(i) * kSlab; }
 
-  // Whether a copy of n bytes from or to `host` goes through the slabs.
-  bool usable(const void* host, size_t n) {
-    if (!tried_ && n < first_) return false;
+  // Whether a copy to `host` goes through the slabs.
+  bool usable(const void* host) {
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess) return false;
     if (!tried_) {
@@ -156,11 +131,9 @@ class HostStage {
     return at.type == hipMemoryTypeUnregistered;
   }
 
-  size_t first_;
   char* mem_ = nullptr;
   hipEvent_t ev_[kSlabs] = {};
   bool busy_[kSlabs] = {};
-  int next_ = 0;
   int dev_ = -1;
   bool tried_ = false, failed_ = false;
 };

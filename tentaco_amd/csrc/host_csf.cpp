@@ -659,11 +659,11 @@ int validate_csf(const taco_tensor_t* B, int order, CsfCheck* h, const LevelFn& 
     int32_t mn = 0, mx = -1;
     const int32_t dim = h->dims[m];
     {
-      // beside a put the caller's core is busy, so one and two threads pay
-      // from a quarter of a thread's usual share on
+      // threads beside the caller only where the check alone would use them
+      // too: starting one stalls for a millisecond now and then
       RangeScan scan;
       const int T = check_threads(nodes);
-      scan.start(crd, nodes, put ? std::max(T > 1 ? T : 0, int(std::min<int64_t>(2, nodes >> 17))) : T > 1 ? T : 0);
+      scan.start(crd, nodes, T > 1 ? T : 0);
       if (put && !put_rc) put_rc = put(m, parents, nodes);
       scan.finish(&mn, &mx);
     }

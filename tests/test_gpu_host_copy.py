@@ -1,7 +1,6 @@
-"""Copies of the host-pointer calls through pinned slabs: sizes around a slab
-(512 KB), around all slabs (2 MB) and past them, sizes that are no whole
-float4, pinned operands, and a fault in an array that is copied while it is
-being checked."""
+"""Factors read back through pinned slabs: sizes around a slab (512 KB), around
+all slabs (2 MB) and past them; host-pointer calls with pageable and pinned
+operands; and a fault in an array that is copied while it is being checked."""
 
 import numpy as np
 import pytest
@@ -33,7 +32,7 @@ def test_cpd_factor_round_trip(gpu, R, dims):
 
 
 @pytest.mark.parametrize("pinned", [False, True])
-def test_host_mttkrp_larger_than_the_slabs(gpu, pinned):
+def test_host_mttkrp_operands(gpu, pinned):
     rng = np.random.default_rng(11)
     dims, n, R = (3001, 40_009, 9001), 1_300_003, 32
     B = tt.Csf.from_coo(dims, np.stack([rng.integers(0, d, n) for d in dims]).astype(np.int32),
