@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <climits>
 
+#include "index_range.h"
 #include "internal.h"
 #include "mttkrp_dispatch.h"
 #include "rowops.h"
@@ -168,11 +169,11 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
     // wc[k] lane j = coordinate of node cur[k]+j.
     int32_t wp[NL], wc[NL];
     auto window = [&](int k, int32_t x, int32_t& p, int32_t& cc) {
-      p = pos[k][min(x + 1 + lane, B.nodes[k])];
-      cc = crd[k][min(x + lane, B.nodes[k] - 1)];
+      p = pos[k][index_ahead(x, 1 + lane, B.nodes[k])];
+      cc = crd[k][index_ahead(x, lane, B.nodes[k] - 1)];
     };
     auto pairs = [&](int32_t q, int32_t& l, float& v) {
-      const int32_t t = min(q + lane, w1 - 1);
+      const int32_t t = index_ahead(q, lane, w1 - 1);
       l = lcrd[t];
       v = vals[t];
     };
@@ -238,7 +239,7 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
         const int32_t key = k == FL ? q : cur[k + 1];
         const int32_t m = k == FL ? n : cnt[k + 1];
         loc[k] = 0;
-        if (lane_of(wp[k], 0) < key + m) loc[k] = rank(wp[k], key);
+        if (lane_of(wp[k], 0) - key < m) loc[k] = rank(wp[k], key);
         cnt[k] = lane_of(loc[k], m - 1) + 1;
       }
       int32_t fc[NL];      // fc[k] lane f: coordinate at level k above fibre f
@@ -778,9 +779,10 @@ __device__ __forceinline__ void slice3_short(const CsfDev& B, const FactorsDev& 
   const float* __restrict__ vq = B.vals;
   const float* __restrict__ Cm = F.M[1];
   const float* __restrict__ Dm = F.M[2];
-  for (int32_t base = q0 + 64 * wv; base < q1; base += 64 * nwv) {
-    const int32_t q = base + lane;
-    const bool okq = q < q1;
+  // (unsigned: a base past the slice may pass 2^31 - 1)
+  for (uint32_t base = uint32_t(q0) + 64 * wv; base < uint32_t(q1); base += 64 * nwv) {
+    const uint32_t q = base + lane;
+    const bool okq = q < uint32_t(q1);
     const int32_t k = okq ? kq[q] : 0;
     const int32_t l = okq ? lq[q] : 0;
     const float v = okq ? vq[q] : 0.f;
@@ -964,10 +966,10 @@ __global__ __launch_bounds__(256) void slice_group_kernel(CsfDev B, FactorsDev F
   V carry[NV];
   RO::zero(carry);
   bool carried = false;
-  for (int32_t xb = x0; xb < x1; xb += 64) {
+  for (uint32_t xb = x0; xb < uint32_t(x1); xb += 64) {
     // a window of slices, one per lane
-    const int32_t nx = min(64, x1 - xb);
-    const int32_t x = min(xb + lane, x1 - 1);
+    const int32_t nx = min(64, x1 - int32_t(xb));
+    const int32_t x = index_ahead(int32_t(xb), lane, x1 - 1);
     const int32_t st = nzr[x];
     const int32_t en = nzr[x + 1];
     const int32_t row = B.crd0[x];
@@ -983,8 +985,8 @@ __global__ __launch_bounds__(256) void slice_group_kernel(CsfDev B, FactorsDev F
     }
     const int32_t q0 = __builtin_amdgcn_readlane(st, 0);
     const int32_t q1 = __builtin_amdgcn_readlane(en, nx - 1);
-    for (int32_t s0 = q0; s0 < q1; s0 += PB) {
-      const int32_t m = min(PB, q1 - s0);
+    for (int32_t s0 = q0, m = 0; s0 < q1; s0 += m) {
+      m = min(PB, q1 - s0);
       V cr[U][NV], dr[U][NV];
       float vt[U];
 #pragma unroll

@@ -32,6 +32,7 @@
 
 #include <rocprim/device/device_radix_sort.hpp>
 
+#include "index_range.h"
 #include "internal.h"
 #include "rowops.h"
 
@@ -144,7 +145,7 @@ __global__ __launch_bounds__(256) void tl_range_kernel(const int32_t* __restrict
   for (int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; t < n; t += nthr) {
     const int64_t p = order[t];
     range[t] = pos[p];
-    range[n + t] = pos[p + 1];
+    range[index_end(n, int32_t(t))] = pos[p + 1];
     for (int m = 0, i = 0; m < w; ++m)
       if (m != level) cor[int64_t(i++) * n + t] = anc[p * w + m];
   }
@@ -188,20 +189,21 @@ __global__ __launch_bounds__(512) void tleaf_kernel(const int32_t* __restrict__ 
   if (j < tdim) {
     const int32_t t0 = tpos[j];
     const int32_t t1 = tpos[j + 1];
-    const int32_t step = 64 * nwv;
+    const uint32_t step = 64 * nwv;
+    const uint32_t end = uint32_t(t1);  // (unsigned: the bases below may pass 2^31 - 1)
     // An entry's coordinates and value arrive one chunk ahead, a lane each;
     // where they are its level N-2 node's, the node two chunks ahead.
     uint2 raw = make_uint2(0u, 0u);
-    auto node_of = [&](int32_t base) {
+    auto node_of = [&](uint32_t base) {
       if constexpr (!kCoords) {
-        const int32_t t = min(base + lane, t1 - 1);
+        const int32_t t = index_ahead(int32_t(base), lane, t1 - 1);
         raw = static_cast<const uint2*>(entries)[t];
       }
     };
-    auto coords_of = [&](int32_t base) {
+    auto coords_of = [&](uint32_t base) {
       LeafEnt<N> e;
       if constexpr (kCoords) {
-        e = static_cast<const LeafEnt<N>*>(entries)[min(base + lane, t1 - 1)];
+        e = static_cast<const LeafEnt<N>*>(entries)[index_ahead(int32_t(base), lane, t1 - 1)];
       } else {
         const int32_t* a = anc + int64_t(raw.x) * (N - 1);
 #pragma unroll
@@ -210,22 +212,22 @@ __global__ __launch_bounds__(512) void tleaf_kernel(const int32_t* __restrict__ 
       }
       return e;
     };
-    const int32_t b0 = t0 + 64 * wv;
+    const uint32_t b0 = uint32_t(t0) + 64 * wv;
     LeafEnt<N> e{}, next{};
-    if (b0 < t1) {
+    if (b0 < end) {
       node_of(b0);
       next = coords_of(b0);
-      if (b0 + step < t1) node_of(b0 + step);
+      if (b0 + step < end) node_of(b0 + step);
     }
-    for (int32_t base = b0; base < t1; base += step) {
+    for (uint32_t base = b0; base < end; base += step) {
       e = next;
-      if (base + step < t1) {
+      if (base + step < end) {
         next = coords_of(base + step);
-        if (base + 2 * step < t1) node_of(base + 2 * step);
+        if (base + 2 * step < end) node_of(base + 2 * step);
       }
 #pragma unroll
       for (int u0 = 0; u0 < NT; u0 += TB) {
-        if (base + u0 * NG >= t1) break;
+        if (base + u0 * NG >= end) break;
         V rows[TB][N - 1][NV];
         float vt[TB];
 #pragma unroll
@@ -234,7 +236,7 @@ __global__ __launch_bounds__(512) void tleaf_kernel(const int32_t* __restrict__ 
           // read inactive source lanes as zero)
           const int src = (u0 + u) * NG + gi;
           const float v = __shfl(e.v, src);
-          const bool ok = base + src < t1;
+          const bool ok = base + src < end;
           vt[u] = ok ? v : 0.f;
 #pragma unroll
           for (int m = 0; m < N - 1; ++m) {
@@ -322,11 +324,12 @@ __global__ __launch_bounds__(512) void inner_leaf_kernel(const int32_t* __restri
   if (j < tdim) {
     const int32_t t1 = tpos[j + 1];
     const int32_t step = 64 * nwv;
-    for (int32_t base = tpos[j] + 64 * wv; base < t1; base += step) {
+    // (unsigned: a base past the last entry may pass 2^31 - 1)
+    for (uint32_t base = uint32_t(tpos[j]) + 64 * wv; base < uint32_t(t1); base += step) {
       // the window's nodes: lane i holds entry base + i
-      const int32_t t = min(base + lane, t1 - 1);
+      const int32_t t = index_ahead(int32_t(base), lane, t1 - 1);
       const int32_t first = range[t];
-      const int32_t len = base + lane < t1 ? range[nent + t] - first : 0;
+      const int32_t len = base + lane < uint32_t(t1) ? range[index_end(nent, t)] - first : 0;
       int32_t co[L];
 #pragma unroll
       for (int m = 0; m < L; ++m) co[m] = cor[int64_t(m) * nent + t];
@@ -334,34 +337,34 @@ __global__ __launch_bounds__(512) void inner_leaf_kernel(const int32_t* __restri
       const int32_t begin = end - len;
       const int32_t total = __builtin_amdgcn_readlane(end, 63);
       // list position p of the wave: its node, coordinate and value
-      auto fetch = [&](int32_t f0, int32_t& node, int32_t& l, float& v) {
-        const uint32_t s = uint32_t(end - f0);
+      auto fetch = [&](uint32_t f0, int32_t& node, int32_t& l, float& v) {
+        const uint32_t s = uint32_t(end) - f0;
         hist[lane] = 0;
         wave_lds_sync();
         if (s - 1u < 63u) atomicAdd(&hist[s], 1);
         wave_lds_sync();
         const int32_t h = hist[lane];
         wave_lds_sync();
-        node = min(__popcll(__ballot(end <= f0)) + wave_scan_add(h), 63);
-        const int32_t q = __shfl(first - begin, node) + min(f0 + lane, total - 1);
-        const bool ok = f0 + lane < total;
+        node = min(__popcll(__ballot(uint32_t(end) <= f0)) + wave_scan_add(h), 63);
+        const int32_t q = __shfl(first - begin, node) + index_ahead(int32_t(f0), lane, total - 1);
+        const bool ok = f0 + lane < uint32_t(total);
         l = ok ? crd[q] : 0;
         v = ok ? vals[q] : 0.f;
       };
       int32_t node, l, node_n = 0, l_n = 0;
       float v, v_n = 0.f;
       if (total > 0) fetch(0, node, l, v);
-      for (int32_t f0 = 0; f0 < total; f0 += 64) {
-        const int32_t n = min(64, total - f0);
+      for (uint32_t f0 = 0; f0 < uint32_t(total); f0 += 64) {
+        const int32_t n = min(64, total - int32_t(f0));
         rec[lane] = make_int4(l, __float_as_int(v), node, 0);
         wave_lds_sync();
         const int32_t a0 = __builtin_amdgcn_readlane(node, 0);
         const int32_t a1 = __builtin_amdgcn_readlane(node, n - 1);
-        if (f0 + 64 < total) fetch(f0 + 64, node_n, l_n, v_n);
+        if (f0 + 64 < uint32_t(total)) fetch(f0 + 64, node_n, l_n, v_n);
         // nodes [fa, fe) of the chunk hold its nonzeros [a, e)
         for (int32_t fa = a0, a = 0; a < n;) {
           const int32_t fe = min(fa + PF, a1 + 1);
-          const int32_t e = fe > a1 ? n : __builtin_amdgcn_readlane(begin, fe) - f0;
+          const int32_t e = fe > a1 ? n : __builtin_amdgcn_readlane(begin, fe) - int32_t(f0);
           for (int32_t g0 = fa; g0 < fe; g0 += 2 * NGW) {
             V p[2][NV];
 #pragma unroll
