@@ -797,6 +797,8 @@ __device__ __forceinline__ void slice3_short(const CsfDev& B, const FactorsDev& 
     }
 #pragma unroll
     for (int u = 0; u < NT; ++u) {
+      // (no zero weights: a row of the factors may hold infinities or NaN)
+      if (base + u * NG + gi >= uint32_t(q1)) continue;
       V w[NV];
       RO::zero(w);
       RO::axpy(w, vt[u], dr[u]);

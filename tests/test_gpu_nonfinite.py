@@ -1,0 +1,64 @@
+"""Infinities and NaN in factor rows stay where they belong. Row 0 of every
+factor is NaN and infinite and no nonzero uses it; the last row of every factor
+holds an infinity and is used by the last nonzero of some output rows only. So
+lanes without a nonzero of their own must add nothing at all (0 times such a
+row would be NaN): rows that use no such factor row are finite and right, and
+the others infinite in the columns that are."""
+
+import numpy as np
+import pytest
+
+import oracle
+import tentaco_amd as tt
+from helpers import REL_L2_TOL
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(rng, dims, R, mode, sizes):
+    """COO entries with sizes[j - 1] of them at coordinate j of `mode`, the
+    factors, and the 64-bit MTTKRP of that mode."""
+    rows = 1 + np.repeat(np.arange(sizes.size), sizes)
+    coords = np.stack([rows if m == mode else rng.integers(1, d - 1, rows.size) for m, d in enumerate(dims)])
+    some = 1 + np.arange(0, sizes.size, 5)
+    last = np.stack([some if m == mode else np.full(some.size, d - 1) for m, d in enumerate(dims)])
+    coords = np.concatenate([coords, last], axis=1).astype(np.int32)
+    vals = rng.uniform(0.5, 1.5, coords.shape[1]).astype(np.float32)
+    facs = [rng.uniform(0.5, 1.5, (d, R)).astype(np.float32) for d in dims]
+    for m, f in enumerate(facs):
+        f[0, 0::2] = np.nan
+        f[0, 1::2] = np.inf
+        f[-1, m % R] = np.inf
+    B = tt.Csf.from_coo(dims, coords, vals)
+    p = vals.astype(np.float64)[:, None]
+    for m, f in enumerate(facs):
+        if m != mode:
+            p = p * f[coords[m]].astype(np.float64)
+    ref = np.zeros((dims[mode], R))
+    np.add.at(ref, coords[mode], p)
+    assert np.isinf(ref).any() and not np.isnan(ref).any()
+    return B, facs, ref
+
+
+def _check(got, ref, what):
+    fin = np.isfinite(ref)
+    assert np.array_equal(got[~fin], ref[~fin].astype(np.float32)), what
+    assert np.all(np.isfinite(got[fin])), what
+    assert oracle.rel_l2(got[fin], ref[fin]) <= REL_L2_TOL, what
+
+
+@pytest.mark.parametrize("R", [2, 3, 7, 16, 20, 32, 50, 64, 100, 128])
+def test_short_fibre_slice_rows(gpu, R):
+    rng = np.random.default_rng(R)
+    # one slice too long for the padded and paired layouts
+    sizes = np.concatenate([rng.integers(1, 130, 300), [64, 128, 63, 65, 1, 2, 700]])
+    B, facs, ref = _case(rng, (sizes.size + 2, 4000, 3000), R, 0, sizes)
+    fd = [tt.DeviceArray.from_numpy(f) for f in facs[1:]]
+    names = tt.variants()
+    H = tt.DeviceCsf(B)
+    A = tt.DeviceArray.empty(ref.shape)
+    for v in ("sr_b128", "sr_b256", "sr_b512"):
+        A.upload(np.full(ref.shape, 7.0, np.float32))
+        H.mttkrp(fd, A, R, names.index(v))
+        _check(A.numpy(), ref, v)
+    H.close()
