@@ -558,7 +558,8 @@ __device__ __forceinline__ void children_sum(const CsfDev& B, const FactorsDev& 
 #pragma unroll
       for (int u = 0; u < U; ++u) RO::load(d[u], Ml, l[u], c, Rr);
 #pragma unroll
-      for (int u = 0; u < U; ++u) RO::axpy(out, v[u], d[u]);
+      for (int u = 0; u < U; ++u)
+        if (q0 + u < e) RO::axpy(out, v[u], d[u]);
     }
   } else {
     for (int32_t ch = a; ch < e; ++ch) {
@@ -847,7 +848,8 @@ __global__ __launch_bounds__(512) void slice_kernel(CsfDev B, FactorsDev F,
         RO::load(d[t], F.M[1], __shfl(lq, src), c, Rr);
       }
 #pragma unroll
-      for (int t = 0; t < NT; ++t) RO::axpy(acc, vt[t], d[t]);
+      for (int t = 0; t < NT; ++t)
+        if (base + t * NG + gi < e) RO::axpy(acc, vt[t], d[t]);
     }
   } else if constexpr (N == 3) {
     slice3_accumulate<R>(B, F, x, lane, gi, c, Rr, wv, nwv, acc);
@@ -1209,16 +1211,13 @@ __global__ __launch_bounds__(128) void slice_pair_kernel(const uint2* __restrict
     }
 #pragma unroll
     for (int u = 0; u < NT; ++u) {
-      const int slot = h * 128 + wv * 64 + u * NG + gi;
-      const float va = slot < inf.z ? vt[u] : 0.f;
-      const float vb = vt[u] - va;
+      // (the other slice adds nothing rather than 0 times the rows, which may
+      // hold infinities; an empty slot's are zeros)
       V w[NV];
       RO::zero(w);
-      RO::axpy(w, va, dr[u]);
-      RO::hfma(aa, w, cr[u]);
-      RO::zero(w);
-      RO::axpy(w, vb, dr[u]);
-      RO::hfma(ab, w, cr[u]);
+      RO::axpy(w, vt[u], dr[u]);
+      if (h * 128 + wv * 64 + u * NG + gi < inf.z) RO::hfma(aa, w, cr[u]);
+      else RO::hfma(ab, w, cr[u]);
     }
   }
   RO::wave_sum(aa);

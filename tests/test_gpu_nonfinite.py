@@ -62,3 +62,35 @@ def test_short_fibre_slice_rows(gpu, R):
         H.mttkrp(fd, A, R, names.index(v))
         _check(A.numpy(), ref, v)
     H.close()
+
+
+@pytest.mark.parametrize("order,R", [(2, 3), (2, 16), (2, 32), (2, 50), (2, 128), (4, 2), (4, 32), (4, 100), (5, 20), (5, 64)])
+def test_slice_rows(gpu, order, R):
+    rng = np.random.default_rng(order * 1000 + R)
+    sizes = np.concatenate([rng.integers(1, 130, 150), [64, 128, 63, 65, 1, 2, 700]])
+    dims = (sizes.size + 2,) + (12, 9, 8)[: order - 2] + (3000,)
+    B, facs, ref = _case(rng, dims, R, 0, sizes)
+    fd = [tt.DeviceArray.from_numpy(f) for f in facs[1:]]
+    names = tt.variants()
+    H = tt.DeviceCsf(B)
+    A = tt.DeviceArray.empty(ref.shape)
+    for v in ("sr_b128", "sr_b256", "sr_b512"):
+        A.upload(np.full(ref.shape, 7.0, np.float32))
+        H.mttkrp(fd, A, R, names.index(v))
+        _check(A.numpy(), ref, v)
+    H.close()
+
+
+@pytest.mark.parametrize("R", [16, 32, 64])
+def test_paired_slices(gpu, R):
+    rng = np.random.default_rng(R)
+    sizes = rng.integers(60, 190, 300)  # two slices to a workgroup
+    B, facs, ref = _case(rng, (sizes.size + 2, 4000, 3000), R, 0, sizes)
+    fd = [tt.DeviceArray.from_numpy(f) for f in facs[1:]]
+    H = tt.DeviceCsf(B)
+    A = tt.DeviceArray.from_numpy(np.full(ref.shape, 7.0, np.float32))
+    tt.ktimer_start()
+    H.mttkrp(fd, A, R, tt.variants().index("sr_b256"))
+    assert tt.ktimer_stop()[2] == "slice_pair_kernel"
+    _check(A.numpy(), ref, "sr_b256")
+    H.close()
