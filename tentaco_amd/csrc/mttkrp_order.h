@@ -403,15 +403,18 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
 #pragma unroll
           for (int u = 0; u < S(); ++u) {
             const int4 x = record(u);
-            const float w = t0 + u * NGW + gi < e ? __int_as_float(x.y) : 0.f;
+            const float w = __int_as_float(x.y);
+            // a step past the piece adds nothing (not its weight 0: the row it
+            // repeats may hold infinities)
+            const bool ok = t0 + u * NGW + gi < e;
             if constexpr (N > 2) {
               V p[NV], s[NV];
               RO::get(P + (x.z - fa) * KR, c, p);
               RO::zero(s);
               RO::axpy(s, w, p);
-              RO::hfma(acc, s, d[u]);
+              if (ok) RO::hfma(acc, s, d[u]);
             } else {
-              RO::axpy(acc, w, d[u]);
+              if (ok) RO::axpy(acc, w, d[u]);
             }
           }
         };

@@ -94,3 +94,42 @@ def test_paired_slices(gpu, R):
     assert tt.ktimer_stop()[2] == "slice_pair_kernel"
     _check(A.numpy(), ref, "sr_b256")
     H.close()
+
+
+@pytest.mark.parametrize("order,R", [(2, 32), (3, 3), (3, 16), (3, 32), (3, 50), (3, 128), (4, 64), (4, 20), (5, 200), (5, 32)])
+@pytest.mark.parametrize("case", ["long", "short"])
+def test_edge_walk(gpu, case, order, R):
+    rng = np.random.default_rng(order * 1000 + R)
+    # slices of several chunks of a wave, and many to a chunk
+    sizes = rng.integers(20, 900, 60) if case == "long" else rng.integers(0, 7, 3000)
+    dims = (sizes.size + 2,) + (40, 30, 50)[: order - 2] + (20_000,)
+    B, facs, ref = _case(rng, dims, R, 0, sizes)
+    fd = [tt.DeviceArray.from_numpy(f) for f in facs[1:]]
+    names = tt.variants()
+    H = tt.DeviceCsf(B)
+    A = tt.DeviceArray.empty(ref.shape)
+    for v in [names.index(n) for n in ("ep_b128_g4", "ep_b256_g16", "ep_b512_g64", "es_b256_g8")] + [tt.VARIANT_AUTO]:
+        if v >= 0 and not tt.variant_fits(order, R, v):
+            continue
+        A.upload(np.full(ref.shape, 7.0, np.float32))
+        H.mttkrp(fd, A, R, v)
+        _check(A.numpy(), ref, v)
+    H.close()
+
+
+@pytest.mark.parametrize("R", [16, 32, 64])
+def test_batch(gpu, R):
+    rng = np.random.default_rng(R)
+    cases = [_case(rng, (n + 2,) + (40, 30, 50)[: order - 2] + (9000,), R, 0, rng.integers(0, 400, n))
+             for order, n in ((2, 50), (3, 90), (4, 70), (5, 60))]
+    tasks = [tt.DeviceCsf(B) for B, _, _ in cases]
+    outs = [tt.DeviceArray.from_numpy(np.full(ref.shape, 7.0, np.float32)) for _, _, ref in cases]
+    bt = tt.Batch(tasks, R)
+    bt.set_operands([[tt.DeviceArray.from_numpy(f) for f in facs[1:]] for _, facs, _ in cases], outs,
+                    [ref.shape[0] for _, _, ref in cases])
+    for tile in (None, (1, 128, 4), (1, 512, 64)):
+        if tile:
+            bt.configure(*tile)
+        bt.run()
+        for t, (o, (_, _, ref)) in enumerate(zip(outs, cases)):
+            _check(o.numpy(), ref, (tile, t))
