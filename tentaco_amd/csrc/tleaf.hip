@@ -235,17 +235,15 @@ __global__ __launch_bounds__(512) void tleaf_kernel(const int32_t* __restrict__ 
           // every lane runs the shuffles (a shuffle inside a branch would
           // read inactive source lanes as zero)
           const int src = (u0 + u) * NG + gi;
-          const float v = __shfl(e.v, src);
-          const bool ok = base + src < end;
-          vt[u] = ok ? v : 0.f;
+          vt[u] = __shfl(e.v, src);
 #pragma unroll
-          for (int m = 0; m < N - 1; ++m) {
-            const int32_t x = __shfl(e.c[m], src);
-            RO::load(rows[u][m], F.M[m], ok ? x : 0, c, Rr);
-          }
+          for (int m = 0; m < N - 1; ++m)
+            RO::load(rows[u][m], F.M[m], __shfl(e.c[m], src), c, Rr);
         }
 #pragma unroll
         for (int u = 0; u < TB; ++u) {
+          // (a lane past the entries repeats the last one)
+          if (base + (u0 + u) * NG + gi >= end) continue;
 #pragma unroll
           for (int m = 1; m < N - 1; ++m) RO::hmul(rows[u][0], rows[u][m]);
           RO::axpy(acc, vt[u], rows[u][0]);
@@ -391,12 +389,13 @@ __global__ __launch_bounds__(512) void inner_leaf_kernel(const int32_t* __restri
 #pragma unroll
             for (int u = 0; u < S(); ++u) {
               const int4 x = record(u);
-              const float w = s0 + u * NGW + gi < e ? __int_as_float(x.y) : 0.f;
               V p[NV], s[NV];
               RO::get(P + (x.z - fa) * KR, c, p);
               RO::zero(s);
-              RO::axpy(s, w, p);
-              RO::hfma(acc, s, d[u]);
+              RO::axpy(s, __int_as_float(x.y), p);
+              // a step past the nonzeros adds nothing (not its weight 0: the
+              // row it repeats may hold infinities)
+              if (s0 + u * NGW + gi < e) RO::hfma(acc, s, d[u]);
             }
           };
           for (int32_t s0 = a; s0 < e;) {

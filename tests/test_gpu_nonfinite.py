@@ -133,3 +133,19 @@ def test_batch(gpu, R):
         bt.run()
         for t, (o, (_, _, ref)) in enumerate(zip(outs, cases)):
             _check(o.numpy(), ref, (tile, t))
+
+
+@pytest.mark.parametrize("order,R", [(2, 32), (3, 3), (3, 16), (3, 32), (3, 50), (3, 128), (4, 64), (4, 20), (5, 200), (5, 32)])
+@pytest.mark.parametrize("sizes", ["long", "short"])
+def test_level_modes(gpu, sizes, order, R):
+    rng = np.random.default_rng(order * 1000 + R)
+    n = rng.integers(20, 900, 60) if sizes == "long" else rng.integers(0, 7, 3000)
+    for level in range(1, order):
+        dims = [60, 40, 30, 50, 20_000][5 - order:]
+        dims[level] = n.size + 2
+        B, facs, ref = _case(rng, tuple(dims), R, level, n)
+        H = tt.DeviceCsf(B)
+        A = tt.DeviceArray.from_numpy(np.full(ref.shape, 7.0, np.float32))
+        H.mttkrp_level(level, [tt.DeviceArray.from_numpy(f) for f in facs], A, R)
+        _check(A.numpy(), ref, level)
+        H.close()
