@@ -5,6 +5,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cfloat>
 #include <climits>
 
 #include "index_range.h"
@@ -31,7 +32,11 @@ namespace {
 // a piece, the product of the upper levels' rows is formed once per fibre and
 // kept in LDS (P); the row groups take the piece's nonzeros in turn, each
 // step one leaf row by a global load and one P row from LDS:
-//   acc += (val * P(fibre, :)) (.) M_{N-1}(l, :).
+//   acc += (val * M_{N-1}(l, :)) (.) P(fibre, :).
+// (At orders 4 and 5 P is a product of rows itself. Where it leaves the normal
+// numbers, the piece multiplies the rows to the value's leaf row one by one, as
+// they would be without P: 1e30 * 1e-15 * 1e-15 * 1e-15 * 1e-15 is no 0. The
+// check is two instructions a column and fibre.)
 // Slice changes are uniform over the wave: the row groups' accumulators are
 // summed over the wave and the row is stored.
 //
@@ -287,28 +292,21 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
         for (int32_t s0 = 0; s0 < n; s0 += PB) {
           const int32_t m = min(PB, n - s0);
           V d[U][NV];
-          float w[U];
 #pragma unroll
           for (int u = 0; u < U; ++u) {
             const int4 x = rec[s0 + min(u * NGW + gi, m - 1)];
-            w[u] = __int_as_float(x.y);
             RO::load(d[u], Mleaf, x.x, c, Rr);
-            if constexpr (N > 2) {
+            RO::scale(d[u], __int_as_float(x.y));
 #pragma unroll
-              for (int k = FL; k >= 1; --k) {
-                V p[NV];
-                RO::load(p, M[k], __shfl(fc[k], x.z), c, Rr);
-                RO::hmul(d[u], p);
-              }
+            for (int k = FL; k >= 1; --k) {
+              V p[NV];
+              RO::load(p, M[k], __shfl(fc[k], x.z), c, Rr);
+              RO::hmul(d[u], p);
             }
           }
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
-            V p[NV];
-            RO::zero(p);
-            RO::axpy(p, w[u], d[u]);
-            if (u * NGW + gi < m) RO::put(P + (u * NGW + gi) * KR, c, p);
-          }
+          for (int u = 0; u < U; ++u)
+            if (u * NGW + gi < m) RO::put(P + (u * NGW + gi) * KR, c, d[u]);
           wave_lds_sync();
           const int32_t o0 = lane_of(ord, s0), o1 = lane_of(ord, s0 + m - 1);
           const int32_t r0 = lane_of(rq, s0);
@@ -366,9 +364,10 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
           open = cur[0] + r;
         }
         open_row = lane_of(wc[0], r);
-        bool staged = N == 2;
+        bool staged = N == 2, apart = false;
         auto stage = [&]() {
           constexpr int U = NV >= 4 ? 1 : 2;
+          float least = FLT_MAX, most = 0.f;
           for (int32_t f0 = fa; f0 < fe; f0 += U * NGW) {
             V p[U][NV];
 #pragma unroll
@@ -381,6 +380,7 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
                 RO::load(m, M[k], __shfl(fc[k], f), c, Rr);
                 RO::hmul(p[u], m);
               }
+              if constexpr (N > 3) RO::extent(p[u], c, Rr, least, most);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -388,7 +388,42 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
               if (f < fe) RO::put(P + (f - fa) * KR, c, p[u]);
             }
           }
+          if constexpr (N > 3) {
+            // a product below the normal numbers, or none: unless all of them
+            // come from a factor that is 0, the piece takes the rows apart
+            if (__ballot(!(least >= FLT_MIN && most <= FLT_MAX))) {
+              bool lost = false;
+              for (int32_t f0 = fa; f0 < fe; f0 += NGW) {
+                const int32_t f = min(f0 + gi, fe - 1);
+                V p[NV];
+                RO::load(p, M[FL], __shfl(fc[FL], f), c, Rr);
+#pragma unroll
+                for (int k = FL - 1; k >= 1; --k) {
+                  V m[NV];
+                  RO::load(m, M[k], __shfl(fc[k], f), c, Rr);
+                  lost = RO::hmul_lost(p, m) || lost;
+                }
+              }
+              apart = __ballot(lost) != 0;
+            }
+          }
           wave_lds_sync();
+        };
+        // the piece without P: the rows multiply each value's leaf row in turn
+        auto rows_apart = [&]() {
+          for (int32_t t0 = a; t0 < e; t0 += NGW) {
+            const int4 x = rec[min(t0 + gi, e - 1)];
+            V s[NV];
+            RO::load(s, Mleaf, x.x, c, Rr);
+            RO::scale(s, __int_as_float(x.y));
+#pragma unroll
+            for (int k = FL; k >= 1; --k) {
+              V m[NV];
+              RO::load(m, M[k], __shfl(fc[k], x.z), c, Rr);
+              RO::hmul(s, m);
+            }
+            if (t0 + gi < e) RO::add(acc, s);
+          }
         };
         auto steps = [&](auto S, int32_t t0) {
           V d[S()][NV];
@@ -398,6 +433,7 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
           if constexpr (N > 2) {
             if (!staged) stage();
             staged = true;
+            if (N > 3 && apart) return;
           }
           // (the records are read again rather than held: 16 registers less)
 #pragma unroll
@@ -408,11 +444,10 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
             // repeats may hold infinities)
             const bool ok = t0 + u * NGW + gi < e;
             if constexpr (N > 2) {
-              V p[NV], s[NV];
+              V p[NV];
               RO::get(P + (x.z - fa) * KR, c, p);
-              RO::zero(s);
-              RO::axpy(s, w, p);
-              if (ok) RO::hfma(acc, s, d[u]);
+              RO::scale(d[u], w);
+              if (ok) RO::hfma(acc, d[u], p);
             } else {
               if (ok) RO::axpy(acc, w, d[u]);
             }
@@ -428,6 +463,10 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
           } else {
             steps(std::integral_constant<int, 2>(), t0);
             t0 += 2 * NGW;
+          }
+          if (N > 3 && apart) {
+            rows_apart();
+            break;
           }
         }
         wave_lds_sync();

@@ -22,6 +22,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cfloat>
 #include <cstdint>
 #include <type_traits>
 
@@ -164,6 +165,62 @@ struct Row {
       for (int j = 0; j < NV; ++j)
         d[j] = *reinterpret_cast<const float4*>(p + col(j, c, Rr));
     }
+  }
+
+  // a *= s
+  __device__ __forceinline__ static void scale(V (&a)[NV], float s) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      if constexpr (R == 0) {
+        a[j] *= s;
+      } else {
+        a[j].x *= s;
+        a[j].y *= s;
+        a[j].z *= s;
+        a[j].w *= s;
+      }
+    }
+  }
+
+  // The smallest and largest magnitude of a's columns, with what least and most
+  // hold.
+  __device__ __forceinline__ static void extent(const V (&a)[NV], int c, int Rr, float& least,
+                                                float& most) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      if constexpr (R == 0) {
+        if (c < Rr) least = fminf(least, fabsf(a[j]));
+        most = fmaxf(most, fabsf(a[j]));
+      } else {
+        least = fminf(fminf(least, fabsf(a[j].x)), fabsf(a[j].y));
+        least = fminf(fminf(least, fabsf(a[j].z)), fabsf(a[j].w));
+        most = fmaxf(fmaxf(most, fabsf(a[j].x)), fabsf(a[j].y));
+        most = fmaxf(fmaxf(most, fabsf(a[j].z)), fabsf(a[j].w));
+      }
+    }
+  }
+
+  // a = a (.) y; whether a column left the normal numbers that neither a nor y
+  // has as 0.
+  __device__ __forceinline__ static bool hmul_lost(V (&a)[NV], const V (&y)[NV]) {
+    bool lost = false;
+    auto mul = [&](float& x, float z) {
+      const bool zero = x == 0.f || z == 0.f;
+      x *= z;
+      lost = lost || !(zero || (fabsf(x) >= FLT_MIN && fabsf(x) <= FLT_MAX));
+    };
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      if constexpr (R == 0) {
+        mul(a[j], y[j]);
+      } else {
+        mul(a[j].x, y[j].x);
+        mul(a[j].y, y[j].y);
+        mul(a[j].z, y[j].z);
+        mul(a[j].w, y[j].w);
+      }
+    }
+    return lost;
   }
 
   // a += s * d
