@@ -28,19 +28,19 @@ __global__ __launch_bounds__(512, (R == 32 ? 3 : 4)) void batch_all_kernel(
               [&](const BatchTaskDev& T, int32_t b) {
                 switch (T.B.order) {
                   case 2:
-                    edge_block<2, R, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[2], tl.NB[2],
+                    edge_block<2, R, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[2], tl.NB[2],
                                            smem, T.W, T.slots + b);
                     break;
                   case 3:
-                    edge_block<3, R, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[3], tl.NB[3],
+                    edge_block<3, R, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[3], tl.NB[3],
                                            smem, T.W, T.slots + b);
                     break;
                   case 4:
-                    edge_block<4, R, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[4], tl.NB[4],
+                    edge_block<4, R, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[4], tl.NB[4],
                                            smem, T.W, T.slots + b);
                     break;
                   default:
-                    edge_block<5, R, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[5], tl.NB[5],
+                    edge_block<5, R, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[5], tl.NB[5],
                                            smem, T.W, T.slots + b);
                     break;
                 }

@@ -85,7 +85,7 @@ __device__ __forceinline__ int32_t wave_search_le(const int32_t* __restrict__ a,
 // on the CSF and the run length only and that a handle or a batch keeps; or,
 // with starts null, from the block's brackets brk (the same per block) by a
 // search of its own.
-template <int N, int R, bool EP>
+template <int N, int R, bool EP, bool Batch = false>
 __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F, float* out_a,
                                            int Rr, const int32_t* brk_p, const int32_t* starts_p,
                                            int32_t b, int32_t G, int32_t NB, unsigned char* smem,
@@ -391,7 +391,7 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
           if constexpr (N > 3) {
             // a product below the normal numbers, or none: unless all of them
             // come from a factor that is 0, the piece takes the rows apart
-            if (__ballot(!(least >= FLT_MIN && most <= FLT_MAX))) {
+            if (__builtin_expect(__ballot(!(least >= FLT_MIN && most <= FLT_MAX)) != 0, 0)) {
               bool lost = false;
               for (int32_t f0 = fa; f0 < fe; f0 += NGW) {
                 const int32_t f = min(f0 + gi, fe - 1);
@@ -425,9 +425,15 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
             if (t0 + gi < e) RO::add(acc, s);
           }
         };
-        auto steps = [&](auto S, int32_t t0) {
+        // S steps of the row groups from nonzero t0. `whole`: none of them is past
+        // the piece, as most are; the batch, whose registers already spill, has
+        // no form for those (5-mode 1.5M nonzeros 30.6 us a call without the
+        // form and 28.2 with it, the batch of 8 tensors 546 and 580)
+        auto steps = [&](auto S, auto whole, int32_t t0) {
           V d[S()][NV];
-          auto record = [&](int u) { return rec[min(t0 + u * NGW + gi, e - 1)]; };
+          auto record = [&](int u) {
+            return rec[whole() ? t0 + u * NGW + gi : min(t0 + u * NGW + gi, e - 1)];
+          };
 #pragma unroll
           for (int u = 0; u < S(); ++u) RO::load(d[u], Mleaf, record(u).x, c, Rr);
           if constexpr (N > 2) {
@@ -442,7 +448,7 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
             const float w = __int_as_float(x.y);
             // a step past the piece adds nothing (not its weight 0: the row it
             // repeats may hold infinities)
-            const bool ok = t0 + u * NGW + gi < e;
+            const bool ok = whole() || t0 + u * NGW + gi < e;
             if constexpr (N > 2) {
               V p[NV];
               RO::get(P + (x.z - fa) * KR, c, p);
@@ -454,17 +460,20 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
           }
         };
         for (int32_t t0 = a; t0 < e;) {
-          if (SB == 8 && e - t0 > 4 * NGW) {
-            steps(std::integral_constant<int, SB>(), t0);
+          if (!Batch && SB >= 4 && e - t0 >= SB * NGW) {
+            steps(std::integral_constant<int, SB>(), std::true_type(), t0);
+            t0 += SB * NGW;
+          } else if (SB == 8 && e - t0 > 4 * NGW) {
+            steps(std::integral_constant<int, SB>(), std::false_type(), t0);
             t0 += SB * NGW;
           } else if (SB >= 4 && e - t0 > 2 * NGW) {
-            steps(std::integral_constant<int, SB < 4 ? SB : 4>(), t0);
+            steps(std::integral_constant<int, SB < 4 ? SB : 4>(), std::false_type(), t0);
             t0 += 4 * NGW;
           } else {
-            steps(std::integral_constant<int, 2>(), t0);
+            steps(std::integral_constant<int, 2>(), std::false_type(), t0);
             t0 += 2 * NGW;
           }
-          if (N > 3 && apart) {
+          if (N > 3 && __builtin_expect(apart, 0)) {
             rows_apart();
             break;
           }
@@ -1353,7 +1362,7 @@ __global__ __launch_bounds__(512, (edge_waves<N, R>())) void batch_kernel(
   extern __shared__ __align__(16) unsigned char smem[];
   batch_items(tasks, t_lo, t_hi, item_off, i_lo, i_hi, counter, chunk, dynamic,
               [&](const BatchTaskDev& T, int32_t b) {
-                edge_block<N, R, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, G, NB, smem, T.W,
+                edge_block<N, R, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, G, NB, smem, T.W,
                                        T.slots + b);
               });
 }
