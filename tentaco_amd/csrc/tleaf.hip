@@ -28,6 +28,7 @@
 // reproducible.
 
 #include <algorithm>
+#include <cfloat>
 #include <cstring>
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -363,6 +364,7 @@ __global__ __launch_bounds__(512) void inner_leaf_kernel(const int32_t* __restri
         for (int32_t fa = a0, a = 0; a < n;) {
           const int32_t fe = min(fa + PF, a1 + 1);
           const int32_t e = fe > a1 ? n : __builtin_amdgcn_readlane(begin, fe) - int32_t(f0);
+          float least = FLT_MAX, most = 0.f;
           for (int32_t g0 = fa; g0 < fe; g0 += 2 * NGW) {
             V p[2][NV];
 #pragma unroll
@@ -375,10 +377,49 @@ __global__ __launch_bounds__(512) void inner_leaf_kernel(const int32_t* __restri
                 RO::load(r, F.M[m], __shfl(co[m], f), c, Rr);
                 RO::hmul(p[u], r);
               }
+              if constexpr (L > 1) RO::extent(p[u], c, Rr, least, most);
             }
 #pragma unroll
             for (int u = 0; u < 2; ++u)
               if (g0 + u * NGW + gi < fe) RO::put(P + (g0 + u * NGW + gi - fa) * KR, c, p[u]);
+          }
+          if constexpr (L > 1) {
+            // as in the edge walk: products that are no normal numbers, other
+            // than by a factor that is 0, and the nonzeros take the rows apart
+            if (__builtin_expect(__ballot(!(least >= FLT_MIN && most <= FLT_MAX)) != 0, 0)) {
+              bool lost = false;
+              for (int32_t g0 = fa; g0 < fe; g0 += NGW) {
+                const int32_t f = min(g0 + gi, fe - 1);
+                V p[NV];
+                RO::load(p, F.M[0], __shfl(co[0], f), c, Rr);
+#pragma unroll
+                for (int m = 1; m < L; ++m) {
+                  V r[NV];
+                  RO::load(r, F.M[m], __shfl(co[m], f), c, Rr);
+                  lost = RO::hmul_lost(p, r) || lost;
+                }
+              }
+              if (__ballot(lost) != 0) {
+                wave_lds_sync();
+                for (int32_t s0 = a; s0 < e; s0 += NGW) {
+                  const int4 x = rec[min(s0 + gi, e - 1)];
+                  V s[NV];
+                  RO::load(s, Ml, x.x, c, Rr);
+                  RO::scale(s, __int_as_float(x.y));
+#pragma unroll
+                  for (int m = L - 1; m >= 0; --m) {
+                    V r[NV];
+                    RO::load(r, F.M[m], __shfl(co[m], x.z), c, Rr);
+                    RO::hmul(s, r);
+                  }
+                  if (s0 + gi < e) RO::add(acc, s);
+                }
+                wave_lds_sync();
+                a = e;
+                fa = fe;
+                continue;
+              }
+            }
           }
           auto steps = [&](auto S, int32_t s0) {
             V d[S()][NV];
@@ -389,13 +430,12 @@ __global__ __launch_bounds__(512) void inner_leaf_kernel(const int32_t* __restri
 #pragma unroll
             for (int u = 0; u < S(); ++u) {
               const int4 x = record(u);
-              V p[NV], s[NV];
+              V p[NV];
               RO::get(P + (x.z - fa) * KR, c, p);
-              RO::zero(s);
-              RO::axpy(s, __int_as_float(x.y), p);
+              RO::scale(d[u], __int_as_float(x.y));
               // a step past the nonzeros adds nothing (not its weight 0: the
               // row it repeats may hold infinities)
-              if (s0 + u * NGW + gi < e) RO::hfma(acc, s, d[u]);
+              if (s0 + u * NGW + gi < e) RO::hfma(acc, d[u], p);
             }
           };
           for (int32_t s0 = a; s0 < e;) {

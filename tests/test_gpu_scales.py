@@ -96,3 +96,20 @@ def test_batch(gpu, kind, R):
         bt.run()
         for t, (o, (_, _, ref)) in enumerate(zip(outs, cases)):
             _check(o.numpy(), ref, (tile, t))
+
+
+@pytest.mark.parametrize("order,R", [(4, 2), (4, 16), (4, 32), (4, 50), (4, 128), (5, 3), (5, 20), (5, 32), (5, 64), (5, 200)])
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("sizes", ["long", "short"])
+def test_inner_modes(gpu, sizes, kind, order, R):
+    rng = np.random.default_rng(order * 1000 + R)
+    n = rng.integers(20, 900, 60) if sizes == "long" else rng.integers(0, 7, 3000)
+    for level in range(1, order - 1):
+        dims = [10, 12, 14, 16, 5000][5 - order:]
+        dims[level] = n.size
+        B, facs, ref = _case(rng, tuple(dims), R, level, n, kind)
+        H = tt.DeviceCsf(B)
+        A = tt.DeviceArray.from_numpy(np.full(ref.shape, 7.0, np.float32))
+        H.mttkrp_level(level, [tt.DeviceArray.from_numpy(f) for f in facs], A, R)
+        _check(A.numpy(), ref, level)
+        H.close()
