@@ -1,0 +1,42 @@
+"""Sums of many nonzeros in FP32 take them in levels. One nonzero of 2^24 and
+many of 1, all factors 1: a sum that adds them to the large one one by one
+loses every 1 (2^24 + 1 rounds to 2^24), one that adds partial sums keeps them."""
+
+import numpy as np
+import pytest
+
+import tentaco_amd as tt
+
+pytestmark = pytest.mark.gpu
+
+BIG = 2.0 ** 24
+
+
+def _ones(dims, R):
+    return [tt.DeviceArray.from_numpy(np.ones((d, R), np.float32)) for d in dims]
+
+
+def _groups(R):
+    """Row groups of a wave (lanes that share a factor row)."""
+    p = next(p for p in (16, 32, 64, 128, 256) if p >= max(R, 16))
+    return 16 if R < 4 else 64 // min(16, p // 4)
+
+
+@pytest.mark.parametrize("order,R", [(3, 16), (3, 32), (3, 50), (4, 64), (4, 20), (5, 32), (5, 128)])
+def test_inner_mode_row(gpu, order, R):
+    # one output row of 8192 level N-2 nodes with 8 nonzeros each
+    n = np.arange(65536)
+    lead = [n // 8] if order == 3 else [n // 64, n // 8 % 8] if order == 4 else [n // 512, n // 64 % 8, n // 8 % 8]
+    coords = np.stack([lead[0], np.zeros_like(n), *lead[1:], n % 8]).astype(np.int32)
+    dims = tuple(int(c.max()) + 1 for c in coords)
+    vals = np.ones(n.size, np.float32)
+    vals[0] = BIG
+    H = tt.DeviceCsf(tt.Csf.from_coo(dims, coords, vals))
+    A = tt.DeviceArray.empty((1, R))
+    H.mttkrp_level(1, _ones(dims, R), A, R)
+    # what is added to the large one alone: its chunk's 64 / groups nonzeros of
+    # its row group; every other partial sum below 2^24 is exact, and adding an
+    # odd one to a total past 2^24 rounds by 1, at most once a wave of 8
+    got = A.numpy().astype(np.float64)
+    assert np.max(np.abs(got - (BIG + n.size - 1))) <= 64 // _groups(R) + 9
+    H.close()
