@@ -424,9 +424,12 @@ __global__ __launch_bounds__(512) void inner_leaf_kernel(const int32_t* __restri
               }
             }
           }
-          auto steps = [&](auto S, int32_t s0) {
+          // (`whole`: no step is past the nonzeros, as most are not)
+          auto steps = [&](auto S, auto whole, int32_t s0) {
             V d[S()][NV];
-            auto record = [&](int u) { return rec[min(s0 + u * NGW + gi, e - 1)]; };
+            auto record = [&](int u) {
+              return rec[whole() ? s0 + u * NGW + gi : min(s0 + u * NGW + gi, e - 1)];
+            };
 #pragma unroll
             for (int u = 0; u < S(); ++u) RO::load(d[u], Ml, record(u).x, c, Rr);
             wave_lds_sync();
@@ -438,15 +441,18 @@ __global__ __launch_bounds__(512) void inner_leaf_kernel(const int32_t* __restri
               RO::scale(d[u], __int_as_float(x.y));
               // a step past the nonzeros adds nothing (not its weight 0: the
               // row it repeats may hold infinities)
-              if (s0 + u * NGW + gi < e) RO::hfma(acc, d[u], p);
+              if (whole() || s0 + u * NGW + gi < e) RO::hfma(acc, d[u], p);
             }
           };
           for (int32_t s0 = a; s0 < e;) {
-            if (SB > 2 && e - s0 > 2 * NGW) {
-              steps(std::integral_constant<int, SB>(), s0);
+            if (SB > 2 && e - s0 >= SB * NGW) {
+              steps(std::integral_constant<int, SB>(), std::true_type(), s0);
+              s0 += SB * NGW;
+            } else if (SB > 2 && e - s0 > 2 * NGW) {
+              steps(std::integral_constant<int, SB>(), std::false_type(), s0);
               s0 += SB * NGW;
             } else {
-              steps(std::integral_constant<int, 2>(), s0);
+              steps(std::integral_constant<int, 2>(), std::false_type(), s0);
               s0 += 2 * NGW;
             }
           }
