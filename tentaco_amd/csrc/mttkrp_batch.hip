@@ -28,20 +28,20 @@ __global__ __launch_bounds__(512, (R == 32 ? 3 : 4)) void batch_all_kernel(
               [&](const BatchTaskDev& T, int32_t b) {
                 switch (T.B.order) {
                   case 2:
-                    edge_block<2, R, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[2], tl.NB[2],
-                                           smem, T.W, T.slots + b);
+                    edge_block<2, R, true, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[2],
+                                                       tl.NB[2], smem, T.W, T.slots + b);
                     break;
                   case 3:
-                    edge_block<3, R, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[3], tl.NB[3],
-                                           smem, T.W, T.slots + b);
+                    edge_block<3, R, true, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[3],
+                                                       tl.NB[3], smem, T.W, T.slots + b);
                     break;
                   case 4:
-                    edge_block<4, R, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[4], tl.NB[4],
-                                           smem, T.W, T.slots + b);
+                    edge_block<4, R, true, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[4],
+                                                       tl.NB[4], smem, T.W, T.slots + b);
                     break;
                   default:
-                    edge_block<5, R, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[5], tl.NB[5],
-                                           smem, T.W, T.slots + b);
+                    edge_block<5, R, true, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, tl.G[5],
+                                                       tl.NB[5], smem, T.W, T.slots + b);
                     break;
                 }
               });
@@ -54,7 +54,7 @@ int launch_all(const BatchLaunch& L, int block, int schedule, hipStream_t st) {
     tl.G[N] = L.grp[N];
     tl.NB[N] = L.nb[N];
   }
-  const size_t lds = size_t(block / 64) * edge_wave_lds<R>();
+  const size_t lds = size_t(block / 64) * edge_wave_lds<R, true>();
   const int grid = std::max(1, std::min<int>(L.all_grid, L.total_items));
   batch_all_kernel<R><<<grid, block, lds, st>>>(L.tasks, L.ntasks, L.item_off, L.total_items, L.counter + 2,
                                                 L.R, tl, batch_chunk(L.total_items, grid, schedule),
@@ -65,7 +65,7 @@ int launch_all(const BatchLaunch& L, int block, int schedule, hipStream_t st) {
 
 template <int R>
 int occupancy_all(int block, int* per_cu) {
-  const size_t lds = size_t(block / 64) * edge_wave_lds<R>();
+  const size_t lds = size_t(block / 64) * edge_wave_lds<R, true>();
   const hipError_t e =
       hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, batch_all_kernel<R>, block, lds);
   if (e != hipSuccess) return fail(TENTACO_EHIP, "occupancy query: %s", hipGetErrorString(e));

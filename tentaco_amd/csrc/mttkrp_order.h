@@ -51,16 +51,26 @@ namespace {
 // latency of a chunk's dependent steps and about 4 vector instructions a
 // nonzero.
 //
+// Rows: the workgroups' shared rows are FP64 ones. Without them a long slice's
+// row takes an FP32 addition per workgroup, and a run is summed in two levels
+// to leave that the room it had: a chunk's nonzeros, then (in LDS, a lane each)
+// the chunks. One chain over a run of 512 had 1.2 to 1.4 times the error at the
+// same tile: 1.85 and 1.43e-7 against FP64 for 400k nonzeros, 2.14 and 1.85 for
+// 12M at rank 128, in two levels 1.25 and 1.79. With FP64 rows the chain stays
+// (1.0 and 1.5e-7, 2044 us for 100M nonzeros; 2083 in two levels).
+//
 // LDS per wave (edge_wave_lds bytes): a record per nonzero of the chunk
-// (leaf row, value, fibre), the histogram, P, and the wave's first slice's
-// row; the block's combine reuses P and the histogram.
+// (leaf row, value, fibre), the histogram, P, the wave's first slice's row, and
+// without Rows the earlier chunks' sums; the block's combine reuses P and the
+// histogram.
 constexpr int kRecBytes = 64 * 16;
 constexpr int kHistBytes = 64 * 4;
 constexpr int kFibBytes = 4096;
 
-template <int R>
+template <int R, bool Rows>
 constexpr size_t edge_wave_lds() {
-  return kRecBytes + kHistBytes + kFibBytes + Lay<R>::kMaxRank * sizeof(float);
+  return kRecBytes + kHistBytes + kFibBytes + Lay<R>::kMaxRank * sizeof(float) +
+         (Rows ? 0 : 64 * Row<R>::NV * sizeof(typename Row<R>::V));
 }
 
 // Largest x in [lo, hi] with a[x] <= key (requires a[lo] <= key), 64 probes a
@@ -85,11 +95,11 @@ __device__ __forceinline__ int32_t wave_search_le(const int32_t* __restrict__ a,
 // on the CSF and the run length only and that a handle or a batch keeps; or,
 // with starts null, from the block's brackets brk (the same per block) by a
 // search of its own.
-template <int N, int R, bool EP, bool Batch = false>
+template <int N, int R, bool EP, bool Rows, bool Batch = false>
 __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F, float* out_a,
                                            int Rr, const int32_t* brk_p, const int32_t* starts_p,
                                            int32_t b, int32_t G, int32_t NB, unsigned char* smem,
-                                           double* out_w, const int2* slots = nullptr) {
+                                           double* out_w, const int2* slots) {
   using RO = Row<R>;
   using V = typename RO::V;
   constexpr int NV = RO::NV;
@@ -111,18 +121,19 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
   const int32_t* __restrict__ starts = global_ptr(starts_p);
 
   // read here: at the end its latency would stand alone
-  const int2 slot = slots ? *slots : make_int2(0, 0);
+  const int2 slot = Rows ? *slots : make_int2(0, 0);
 
   const int lane = int(threadIdx.x) & 63;
   const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
   const int nwv = int(blockDim.x) >> 6;
   const int gi = lane / LPR;
   const int c = lane % LPR;
-  auto wave_mem = [&](int w) { return smem + size_t(w) * edge_wave_lds<R>(); };
+  auto wave_mem = [&](int w) { return smem + size_t(w) * edge_wave_lds<R, Rows>(); };
   int4* rec = reinterpret_cast<int4*>(wave_mem(wv));
   int32_t* hist = reinterpret_cast<int32_t*>(wave_mem(wv) + kRecBytes);
   float* P = reinterpret_cast<float*>(wave_mem(wv) + kRecBytes + kHistBytes);
   float* head_row = P + kFibBytes / 4;
+  V* earlier = reinterpret_cast<V*>(head_row + KR) + lane * NV;  // this lane's
 
   // the wave's run [w0, w1)
   const int32_t blk0 = b * NB;
@@ -136,6 +147,15 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
   RO::zero(acc);
   int32_t head = INT_MAX, open = INT_MAX;
   bool head_closed = false;
+  bool has_earlier = false;  // of the open slice
+  auto take_earlier = [&]() {
+    if (!has_earlier) return;
+    has_earlier = false;
+    V t[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) t[j] = earlier[j];
+    RO::add(acc, t);
+  };
 
   if (active) {
     const int32_t* __restrict__ lcrd = global_ptr(B.crd[N - 1]);
@@ -197,6 +217,7 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
 
     int32_t open_row = 0;
     auto close_slice = [&]() {
+      take_earlier();
       RO::wave_sum(acc);
       if (open == head && !head_closed) {
         head_closed = true;
@@ -482,6 +503,13 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
         a = e;
         fa = fe;
       }
+      if (!Rows && !many && qn < w1) {
+        take_earlier();
+#pragma unroll
+        for (int j = 0; j < NV; ++j) earlier[j] = acc[j];
+        RO::zero(acc);
+        has_earlier = true;
+      }
       q = qn;
       l = lnext;
       v = vnext;
@@ -492,6 +520,7 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
         wc[k] = wcn[k];
       }
     }
+    take_earlier();
     RO::wave_sum(acc);
   }
 
@@ -530,7 +559,7 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
       const bool shared = key == first || key == last;
       if constexpr (EP) {
         if (!shared) A[o] = float(s);
-        else if (slots) unsafeAtomicAdd(W + int64_t(key == first ? slot.x : slot.y) * cols + col, s);
+        else if (Rows) unsafeAtomicAdd(W + int64_t(key == first ? slot.x : slot.y) * cols + col, s);
         else unsafeAtomicAdd(A + o, float(s));
       } else {
         if (shared) unsafeAtomicAdd(W + o, s);
@@ -557,7 +586,7 @@ constexpr int edge_waves() {
   return Row<R>::NV >= 4 ? 2 : Row<R>::NV == 2 ? 4 : N <= 3 ? 5 : 4;
 }
 
-template <int N, int R, bool EP>
+template <int N, int R, bool EP, bool Rows>
 __global__ __launch_bounds__(512, (edge_waves<N, R>())) void edge_kernel(CsfDev B, FactorsDev F,
                                                    float* __restrict__ A, int Rr,
                                                    const int32_t* __restrict__ brk,
@@ -566,8 +595,8 @@ __global__ __launch_bounds__(512, (edge_waves<N, R>())) void edge_kernel(CsfDev 
                                                    double* __restrict__ W,
                                                    const int2* __restrict__ slots) {
   extern __shared__ __align__(16) unsigned char smem[];
-  edge_block<N, R, EP>(B, F, A, Rr, brk, starts, blockIdx.x, G, NB, smem, W,
-                       EP && slots ? slots + blockIdx.x : nullptr);
+  edge_block<N, R, EP, Rows>(B, F, A, Rr, brk, starts, blockIdx.x, G, NB, smem, W,
+                             Rows ? slots + blockIdx.x : nullptr);
 }
 
 
@@ -1362,7 +1391,7 @@ __global__ __launch_bounds__(512, (edge_waves<N, R>())) void batch_kernel(
   extern __shared__ __align__(16) unsigned char smem[];
   batch_items(tasks, t_lo, t_hi, item_off, i_lo, i_hi, counter, chunk, dynamic,
               [&](const BatchTaskDev& T, int32_t b) {
-                edge_block<N, R, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, G, NB, smem, T.W,
+                edge_block<N, R, true, true, true>(T.B, T.F, T.A, Rr, nullptr, T.starts, b, G, NB, smem, T.W,
                                        T.slots + b);
               });
 }
@@ -1372,7 +1401,7 @@ int launch_batch_order(const BatchLaunch& L, hipStream_t st) {
   const int32_t i_lo = L.grp_item[N], i_hi = L.grp_item[N + 1];
   if (i_hi <= i_lo) return TENTACO_OK;
   const int blk = L.blk[N];
-  const size_t lds = size_t(blk / 64) * edge_wave_lds<R>();
+  const size_t lds = size_t(blk / 64) * edge_wave_lds<R, true>();
   const int grid = std::max(1, std::min<int>(L.grp_grid[N], i_hi - i_lo));
   const int32_t chunk = batch_chunk(i_hi - i_lo, grid, L.sch[N]);
   batch_kernel<N, R><<<grid, blk, lds, st>>>(
@@ -1386,7 +1415,7 @@ template <int N, int R>
 int batch_occupancy_order(int family, int block, int Rr, int32_t NB, int* per_cu) {
   if (family != kEdgeParallel)
     return fail(TENTACO_EUNSUPPORTED, "the batch runs the edge-parallel walk only");
-  const size_t lds = size_t(block / 64) * edge_wave_lds<R>();
+  const size_t lds = size_t(block / 64) * edge_wave_lds<R, true>();
   const hipError_t e =
       hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, batch_kernel<N, R>, block, lds);
   if (e != hipSuccess) return fail(TENTACO_EHIP, "occupancy query: %s", hipGetErrorString(e));
@@ -1481,17 +1510,19 @@ int launch_typed(const CsfDev& B, const FactorsDev& F, int Rr, float* A,
     return fail(TENTACO_EUNSUPPORTED, "edge tile of block %d and group %d at rank %d is over the "
                 "tile limit of order %d", vr.block, vr.group, Rr, N);
   }
-  const size_t lds = size_t(vr.block / 64) * edge_wave_lds<R>();
+  const size_t lds =
+      size_t(vr.block / 64) * (shared ? edge_wave_lds<R, true>() : edge_wave_lds<R, false>());
+  const int32_t nb = int32_t(NB), grid = int32_t(nblk);
   ktimer_begin(st);
-  if (vr.family == kEdgeSerial) {
-    edge_kernel<N, R, false><<<int(nblk), vr.block, lds, st>>>(B, F, A, Rr, brk, starts,
-                                                               vr.group, int32_t(NB), W, nullptr);
-  } else {
-    edge_kernel<N, R, true><<<int(nblk), vr.block, lds, st>>>(B, F, A, Rr, brk, starts,
-                                                              vr.group, int32_t(NB),
-                                                              shared ? wt.W : nullptr,
-                                                              shared ? wt.slots : nullptr);
-  }
+  if (shared)
+    edge_kernel<N, R, true, true><<<grid, vr.block, lds, st>>>(B, F, A, Rr, brk, starts, vr.group, nb,
+                                                               wt.W, wt.slots);
+  else if (vr.family == kEdgeParallel)
+    edge_kernel<N, R, true, false><<<grid, vr.block, lds, st>>>(B, F, A, Rr, brk, starts, vr.group, nb,
+                                                                nullptr, nullptr);
+  else
+    edge_kernel<N, R, false, false><<<grid, vr.block, lds, st>>>(B, F, A, Rr, brk, starts, vr.group, nb,
+                                                                 W, nullptr);
   TT_HIP_CHECK(hipGetLastError());
   ktimer_end(st, "edge_kernel");
   if (shared) return launch_edge_rows(wt, int32_t(nblk), A, a_rows, Rr, st);

@@ -40,3 +40,32 @@ def test_inner_mode_row(gpu, order, R):
     got = A.numpy().astype(np.float64)
     assert np.max(np.abs(got - (BIG + n.size - 1))) <= 64 // _groups(R) + 9
     H.close()
+
+
+@pytest.mark.parametrize("order,R", [(2, 32), (3, 2), (3, 16), (3, 32), (3, 50), (3, 128), (4, 64), (4, 20), (5, 32), (5, 256)])
+def test_edge_walk_run(gpu, order, R):
+    # two slices of 8192 nonzeros, 8 to a fibre
+    n = np.arange(16384)
+    lead = {2: [n // 8192], 3: [n // 8192, n // 8 % 1024], 4: [n // 8192, n // 64 % 128, n // 8 % 8],
+            5: [n // 8192, n // 512 % 16, n // 64 % 8, n // 8 % 8]}[order]
+    coords = np.stack([*lead, n % 8192 if order == 2 else n % 8]).astype(np.int32)
+    dims = tuple(int(c.max()) + 1 for c in coords)
+    vals = np.ones(n.size, np.float32)
+    vals[[0, 8192]] = BIG
+    names = tt.variants()
+    H = tt.DeviceCsf(tt.Csf.from_coo(dims, coords, vals))
+    A = tt.DeviceArray.empty((2, R))
+    fd = _ones(dims[1:], R)
+    ran = 0
+    for v in ("ep_b512_g64", "ep_b256_g64", "ep_b128_g32", "es_b512_g64", "es_b128_g64"):
+        if not tt.variant_fits(order, R, names.index(v)):
+            continue
+        ran += 1
+        H.mttkrp(fd, A, R, names.index(v))
+        # the large one's chunk of its row group, then a rounding by 1 for every
+        # odd total that a wave, a workgroup or (FP32 atomics, at most 32
+        # workgroups a slice) the output row adds to 2^24
+        got = A.numpy().astype(np.float64)
+        assert np.max(np.abs(got - (BIG + 8191))) <= 64 // _groups(R) + 6, v
+    assert ran >= 3
+    H.close()
