@@ -284,6 +284,30 @@ struct Row {
     }
   }
 
+  // Sums in FP64, a lane's 4 (layout 0: 1) columns per fragment.
+  static constexpr int NC = R == 0 ? 1 : 4;
+  using D = double[NV * NC];
+  __device__ __forceinline__ static void add(D& a, const V (&b)[NV]) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      if constexpr (R == 0) {
+        a[j] += double(b[j]);
+      } else {
+        a[4 * j] += double(b[j].x);
+        a[4 * j + 1] += double(b[j].y);
+        a[4 * j + 2] += double(b[j].z);
+        a[4 * j + 3] += double(b[j].w);
+      }
+    }
+  }
+  __device__ __forceinline__ static void narrow(V (&a)[NV], const D& b) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      if constexpr (R == 0) a[j] = float(b[j]);
+      else a[j] = make_float4(float(b[4 * j]), float(b[4 * j + 1]), float(b[4 * j + 2]), float(b[4 * j + 3]));
+    }
+  }
+
   __device__ __forceinline__ static void store(float* __restrict__ A,
                                                int64_t row, int c, int Rr,
                                                const V (&a)[NV]) {

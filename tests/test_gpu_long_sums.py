@@ -69,3 +69,25 @@ def test_edge_walk_run(gpu, order, R):
         assert np.max(np.abs(got - (BIG + 8191))) <= 64 // _groups(R) + 6, v
     assert ran >= 3
     H.close()
+
+
+@pytest.mark.parametrize("R", [2, 16, 20, 32, 50, 100, 128, 200])
+def test_short_slices(gpu, R):
+    # slices of 6 on average, 40 at most, one nonzero a fibre (the AUTO kernel of
+    # short slices); every slice starts with the large one
+    rng = np.random.default_rng(R)
+    sizes = np.where(rng.random(5000) < 0.02, 40, rng.integers(1, 12, 5000))
+    row = np.repeat(np.arange(sizes.size), sizes)
+    at = np.arange(row.size) - np.repeat(np.cumsum(sizes) - sizes, sizes)
+    coords = np.stack([row, at, rng.integers(0, 9, row.size)]).astype(np.int32)
+    vals = np.where(at == 0, BIG, 1.0).astype(np.float32)
+    dims = tuple(int(c.max()) + 1 for c in coords)
+    H = tt.DeviceCsf(tt.Csf.from_coo(dims, coords, vals))
+    A = tt.DeviceArray.empty((dims[0], R))
+    tt.ktimer_start()
+    H.mttkrp(_ones(dims[1:], R), A, R, tt.VARIANT_AUTO)
+    assert tt.ktimer_stop()[2] == "slice_group_kernel"
+    # FP64 sums: one rounding
+    ref = (BIG + sizes - 1).astype(np.float32)
+    assert np.array_equal(A.numpy(), np.repeat(ref[:, None], R, axis=1))
+    H.close()
