@@ -474,9 +474,11 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
               V p[NV];
               RO::get(P + (x.z - fa) * KR, c, p);
               RO::scale(d[u], w);
-              if (ok) RO::hfma(acc, d[u], p);
+              if constexpr (whole()) RO::hfma(acc, d[u], p);
+              else RO::hfma_if(ok, acc, d[u], p);
             } else {
-              if (ok) RO::axpy(acc, w, d[u]);
+              if constexpr (whole()) RO::axpy(acc, w, d[u]);
+              else RO::axpy_if(ok, acc, w, d[u]);
             }
           }
         };
@@ -639,7 +641,7 @@ __device__ __forceinline__ void children_sum(const CsfDev& B, const FactorsDev& 
       for (int u = 0; u < U; ++u) RO::load(d[u], Ml, l[u], c, Rr);
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        if (q0 + u < e) RO::axpy(out, v[u], d[u]);
+        RO::axpy_if(q0 + u < e, out, v[u], d[u]);
     }
   } else {
     for (int32_t ch = a; ch < e; ++ch) {
@@ -878,12 +880,10 @@ __device__ __forceinline__ void slice3_short(const CsfDev& B, const FactorsDev& 
     }
 #pragma unroll
     for (int u = 0; u < NT; ++u) {
-      // (no zero weights: a row of the factors may hold infinities or NaN)
-      if (base + u * NG + gi >= uint32_t(q1)) continue;
       V w[NV];
       RO::zero(w);
       RO::axpy(w, vt[u], dr[u]);
-      RO::hfma(acc, w, cr[u]);
+      RO::hfma_if(base + u * NG + gi < uint32_t(q1), acc, w, cr[u]);
     }
   }
 }
@@ -929,7 +929,7 @@ __global__ __launch_bounds__(512) void slice_kernel(CsfDev B, FactorsDev F,
       }
 #pragma unroll
       for (int t = 0; t < NT; ++t)
-        if (base + t * NG + gi < e) RO::axpy(acc, vt[t], d[t]);
+        RO::axpy_if(base + t * NG + gi < e, acc, vt[t], d[t]);
     }
   } else if constexpr (N == 3) {
     slice3_accumulate<R>(B, F, x, lane, gi, c, Rr, wv, nwv, acc);

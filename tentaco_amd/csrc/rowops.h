@@ -255,6 +255,40 @@ struct Row {
     }
   }
 
+  // axpy and hfma where ok, else a as it is, whatever the operands (weight 0
+  // would turn infinities and NaN of an idle lane's row into NaN). Selects, not a
+  // branch: behind one, the compiler moves the operands' loads to it, each waited
+  // for by itself (300k nonzeros in 40000 slices, 256 threads a slice: 84 us a
+  // call against 42).
+  __device__ __forceinline__ static void axpy_if(bool ok, V (&a)[NV], float s, const V (&d)[NV]) {
+    V t[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) t[j] = a[j];
+    axpy(t, s, d);
+    select(ok, a, t);
+  }
+  __device__ __forceinline__ static void hfma_if(bool ok, V (&a)[NV], const V (&x)[NV],
+                                                 const V (&y)[NV]) {
+    V t[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) t[j] = a[j];
+    hfma(t, x, y);
+    select(ok, a, t);
+  }
+  __device__ __forceinline__ static void select(bool ok, V (&a)[NV], const V (&t)[NV]) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      if constexpr (R == 0) {
+        a[j] = ok ? t[j] : a[j];
+      } else {
+        a[j].x = ok ? t[j].x : a[j].x;
+        a[j].y = ok ? t[j].y : a[j].y;
+        a[j].z = ok ? t[j].z : a[j].z;
+        a[j].w = ok ? t[j].w : a[j].w;
+      }
+    }
+  }
+
   // a = a (.) y
   __device__ __forceinline__ static void hmul(V (&a)[NV], const V (&y)[NV]) {
 #pragma unroll

@@ -243,11 +243,10 @@ __global__ __launch_bounds__(512) void tleaf_kernel(const int32_t* __restrict__ 
         }
 #pragma unroll
         for (int u = 0; u < TB; ++u) {
-          // (a lane past the entries repeats the last one)
-          if (base + (u0 + u) * NG + gi >= end) continue;
 #pragma unroll
           for (int m = 1; m < N - 1; ++m) RO::hmul(rows[u][0], rows[u][m]);
-          RO::axpy(acc, vt[u], rows[u][0]);
+          // (a lane past the entries repeats the last one)
+          RO::axpy_if(base + (u0 + u) * NG + gi < end, acc, vt[u], rows[u][0]);
         }
       }
     }
@@ -441,7 +440,8 @@ __global__ __launch_bounds__(512) void inner_leaf_kernel(const int32_t* __restri
               RO::scale(d[u], __int_as_float(x.y));
               // a step past the nonzeros adds nothing (not its weight 0: the
               // row it repeats may hold infinities)
-              if (whole() || s0 + u * NGW + gi < e) RO::hfma(acc, d[u], p);
+              if constexpr (whole()) RO::hfma(acc, d[u], p);
+              else RO::hfma_if(s0 + u * NGW + gi < e, acc, d[u], p);
             }
           };
           for (int32_t s0 = a; s0 < e;) {
