@@ -334,6 +334,10 @@ struct Row {
       }
     }
   }
+  __device__ __forceinline__ static void narrow(V (&a)[NV], const V (&b)[NV]) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) a[j] = b[j];
+  }
   __device__ __forceinline__ static void narrow(V (&a)[NV], const D& b) {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
