@@ -236,7 +236,7 @@ int build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStream_t st) {
   uint32_t* bits = s.bits;
   hipEvent_t used = nullptr;
   bool ok = hipMalloc(&mem, o_w + wbytes) == hipSuccess &&
-            hipEventCreateWithFlags(&used, hipEventDisableTiming) == hipSuccess;
+            hipEventCreateWithFlags(&used, hipEventDisableTiming | hipEventDisableSystemFence) == hipSuccess;
   if (ok && !bits) {
     ok = hipMalloc(reinterpret_cast<void**>(&bits), bbytes) == hipSuccess &&
          hipMemsetAsync(bits, 0, bbytes, st) == hipSuccess && launch_batch_rowbits(B, bits, st) == TENTACO_OK;
@@ -270,19 +270,20 @@ int build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStream_t st) {
   return TENTACO_OK;
 }
 
-// Workgroups from which they share rows in FP64. The FP32 error of a long slice's
-// row grows with the root of the number of workgroups that add to it: 100M
-// nonzeros in 48,828 workgroups 4.6e-7 against FP64, 1.2e-7 with FP64 rows, 30M
-// (5-mode) 5.8e-7 and 1.2e-7; in 700 workgroups 2.3e-7 and 1.5e-7. The rows'
-// kernel costs 3 us more than the fill it replaces (100M: 2027 and 2037 us, 5M
-// at rank 50 147 and 150; 20k 11.1 and 14.1, 1.5M 31.9 and 35.7).
+// Workgroups from which an edge-parallel variant's calls share rows in FP64 (AUTO's
+// sized tile: auto_needs_rows). A long slice's row takes an FP32 addition from every
+// workgroup, so its error grows with the root of their number: 100M nonzeros in
+// 48,828 workgroups 4.6e-7 against FP64, 1.2e-7 with FP64 rows, 30M (5-mode) 5.8e-7
+// and 1.2e-7. The rows' kernel and the event between calls cost 4 us more than the
+// fill (1.5M nonzeros 28.9 and 33.1), a few in 100 of a call of that many workgroups.
 constexpr int64_t kSharedBlocks = 2048;
 
 // What the handle keeps for variant vr at rank R (edge families), or nulls.
 // With `build`, a missing table is built on st and waited for, so that it is
 // complete for every stream; not under capture. A failed build leaves the
-// calls on the brackets they write themselves and on FP32 atomics.
-WalkTables walk_tables(tentaco_csf* h, const Variant& vr, int R, bool build, hipStream_t st) {
+// calls on the brackets they write themselves and on FP32 atomics. rows: shared
+// rows however few the workgroups.
+WalkTables walk_tables(tentaco_csf* h, const Variant& vr, int R, bool rows, bool build, hipStream_t st) {
   const CsfDev B = h->view();
   WalkTables t;
   if (vr.family == kSliceRow || vr.family < 0 || B.nnz <= 0) return t;
@@ -294,7 +295,7 @@ WalkTables walk_tables(tentaco_csf* h, const Variant& vr, int R, bool build, hip
   while (i < s.n && s.wn[i] != wn) ++i;
   int j = 0;
   while (j < s.ns && (s.nb[j] != NB || s.rank[j] != R)) ++j;
-  const bool ep = vr.family == kEdgeParallel && B.nnz >= kSharedBlocks * NB;
+  const bool ep = vr.family == kEdgeParallel && (rows || B.nnz >= kSharedBlocks * NB);
   const bool capturing =
       (ep || i == s.n) &&
       (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone);
@@ -337,6 +338,19 @@ Variant tile_of(const tentaco_csf* h, int R, int variant, int v) {
   if (variant == TENTACO_VARIANT_AUTO && h->tune.lookup(R) < 0)
     return auto_tile(h->stats, h->order, R, pairs_apply(h));
   return variant_of(v);
+}
+
+// Whether that tile is only run with FP64 rows (see auto_needs_rows).
+bool needs_rows(const tentaco_csf* h, int R, int variant, int v, const Variant& tile) {
+  return variant == TENTACO_VARIANT_AUTO && h->tune.lookup(R) < 0 &&
+         auto_needs_rows(h->stats, R, tile, variant_of(v));
+}
+
+// What such a call runs where FP64 rows are not to be had: for calls without
+// kept state.
+Variant plain_tile(const tentaco_csf* h, int R, int variant, int v) {
+  const Variant tile = tile_of(h, R, variant, v);
+  return needs_rows(h, R, variant, v, tile) ? variant_of(v) : tile;
 }
 
 // Load the MTTKRP and TTV code objects on the current device once, before
@@ -447,7 +461,7 @@ int host_mttkrp(int order, taco_tensor_t* A, taco_tensor_t* B,
   if (hipMalloc(&abuf.p, std::max<size_t>(abytes, 4)) != hipSuccess)
     return fail(TENTACO_ENOMEM, "hipMalloc of A (%zu bytes) failed", abytes);
   const int v = resolve_variant(h, R, variant);
-  const Variant vr = tile_of(h, R, variant, v);
+  const Variant vr = plain_tile(h, R, variant, v);
   if (vr.family < 0) return fail(TENTACO_EINVAL, "variant %d out of range", variant);
   rc = reserve_ws(h, mttkrp_workspace_bytes(h->view(), R, vr, a_rows), nullptr);
   if (rc) return rc;
@@ -804,8 +818,13 @@ int tentaco_csf_reserve_rows(tentaco_csf* h, int R, int variant, int32_t a_rows)
   if (rc) return rc;
   rc = reserve_ws(h, need, nullptr);
   if (rc) return rc;
-  // the wave starts of the variant that calls with this argument run
-  (void)walk_tables(h, tile_of(h, R, variant, resolve_variant(h, R, variant)), R, true, nullptr);
+  // the tables of the tile that calls with this argument run, and of the one
+  // that calls under capture run in its place
+  const int v = resolve_variant(h, R, variant);
+  const Variant tile = tile_of(h, R, variant, v);
+  const bool rows = needs_rows(h, R, variant, v, tile);
+  (void)walk_tables(h, tile, R, rows, true, nullptr);
+  if (rows) (void)walk_tables(h, variant_of(v), R, false, true, nullptr);
   h->reserved = true;
   return TENTACO_OK;
 }
@@ -893,19 +912,23 @@ int tentaco_mttkrp_dev(tentaco_csf* h, int R, const float* const* factors_dev, f
   } else {
     v = resolve_variant(h, R, variant);
   }
-  const Variant vr = tile_of(h, R, variant, v);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  Variant vr = tile_of(h, R, variant, v);
   if (vr.family < 0) return fail(TENTACO_EINVAL, "variant %d out of range", variant);
   if (vr.family == kSliceRow) {
-    rc = ensure_expand3(h, static_cast<hipStream_t>(stream));
+    rc = ensure_expand3(h, st);
     if (rc) return rc;
   }
   const CsfDev B = h->view();
-  rc = reserve_ws(h, mttkrp_workspace_bytes(B, R, vr, a_rows), static_cast<hipStream_t>(stream));
+  const bool rows = needs_rows(h, R, variant, v, vr);
+  WalkTables tables = walk_tables(h, vr, R, rows, !h->reserved, st);
+  if (rows && !tables.slots) {  // no FP64 rows here: the variant's own tile
+    vr = variant_of(v);
+    tables = walk_tables(h, vr, R, false, !h->reserved, st);
+  }
+  rc = reserve_ws(h, mttkrp_workspace_bytes(B, R, vr, a_rows), st);
   if (rc) return rc;
-  const WalkTables tables =
-      walk_tables(h, vr, R, !h->reserved, static_cast<hipStream_t>(stream));
   const bool dense = h->dense_root && a_rows == h->nodes[0];
-  hipStream_t st = static_cast<hipStream_t>(stream);
   if (!tables.slots) return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws, tables, st);
   WalkStarts& s = h->starts;
   std::lock_guard<std::mutex> lk(s.mu);
@@ -933,7 +956,7 @@ int tentaco_mttkrp_dev_noalloc(tentaco_csf* h, int R, const float* const* factor
   // AUTO: the recorded choice or the structural heuristic (the selector and
   // the sweep allocate and synchronise)
   const int v = resolve_variant(h, R, variant);
-  const Variant vr = tile_of(h, R, variant, v);
+  const Variant vr = plain_tile(h, R, variant, v);
   if (vr.family < 0) return fail(TENTACO_EINVAL, "variant %d out of range", variant);
   const CsfDev B = h->view();
   const size_t need = mttkrp_workspace_bytes(B, R, vr, a_rows);
@@ -970,7 +993,7 @@ static int sweep_impl(tentaco_csf* h, int R, const float* const* factors_dev, fl
     if (rc) return rc;
     for (int v = 0; v < kNumVariants; ++v)
       if ((!use || use[v]) && variant_fits(h->order, R, v))
-        (void)walk_tables(h, variant_of(v), R, true, st);
+        (void)walk_tables(h, variant_of(v), R, false, true, st);
   }
   hipEvent_t e0, e1;
   TT_HIP_CHECK(hipEventCreate(&e0));

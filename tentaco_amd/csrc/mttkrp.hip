@@ -674,6 +674,17 @@ Variant auto_tile(const CsfStats& s, int order, int R, bool paired) {
   return edge_tile_fits(order, R, t) ? t : vr;
 }
 
+bool auto_needs_rows(const CsfStats& s, int R, const Variant& tile, const Variant& v) {
+  // From 300k nonzeros on the sized tile has 2 to 8 times the variant's
+  // workgroups, whose FP32 additions to a long slice's row had 1.3 to 1.6 times
+  // the error of the variant's tile before the walk (400k nonzeros 2.0 and
+  // 1.4e-7 against FP64, 1.5M 5-mode 2.3 and 1.5, at rank 64 3.6 and 2.5; with
+  // FP64 rows 1.0, 1.2 and 1.5). Below, it has no more error than that tile
+  // had: 0.99 and 1.13e-7 at 10k, 1.9 and 2.7 at 250k.
+  return tile.family == kEdgeParallel && v.family == kEdgeParallel && s.nnz >= 300000 &&
+         nnz_per_block(tile, R) < nnz_per_block(v, R);
+}
+
 int batch_group(int64_t nnz, int R) {
   // runs of 512 nonzeros a wave from 4M nonzeros in all, 256 below: at 256
   // threads, 19.6M nonzeros, rank 32: group 64 547 us a replay, 16 669; 1.26M:

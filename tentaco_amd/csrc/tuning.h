@@ -58,4 +58,8 @@ int auto_variant(const CsfStats& s, int order, int R);
 // handle's paired slice layout applies.
 Variant auto_tile(const CsfStats& s, int order, int R, bool paired);
 
+// Whether that tile is to be run only with FP64 rows for the slices that its
+// workgroups share, and variant v's own tile without them.
+bool auto_needs_rows(const CsfStats& s, int R, const Variant& tile, const Variant& v);
+
 }  // namespace tt
