@@ -51,6 +51,14 @@ int upload_array(T** dst, const T* src, int64_t n) {
   return TENTACO_OK;
 }
 
+void free_shared(const WalkStarts::Shared& x) {
+  if (x.used) {
+    (void)hipEventSynchronize(x.used);  // the last call that adds to them
+    (void)hipEventDestroy(x.used);
+  }
+  (void)hipFree(x.mem);
+}
+
 void free_handle(tentaco_csf* h) {
   if (!h) return;
   (void)hipFree(h->d_crd0);
@@ -61,11 +69,8 @@ void free_handle(tentaco_csf* h) {
   (void)hipFree(h->d_vals);
   (void)hipFree(h->ws);
   for (void* w : h->ws_retired) (void)hipFree(w);
-  for (int i = 0; i < h->starts.n; ++i) (void)hipFree(h->starts.p[i]);
-  for (int i = 0; i < h->starts.ns; ++i) {
-    (void)hipFree(h->starts.mem[i]);
-    (void)hipEventDestroy(h->starts.used[i]);
-  }
+  for (const auto& x : h->starts.starts) (void)hipFree(x.p);
+  for (const auto& x : h->starts.shared) free_shared(x);
   (void)hipFree(h->starts.bits);
   for (int m = 0; m < kMaxOrder; ++m) (void)hipFree(h->stage_f[m]);
   (void)hipFree(h->stage_a);
@@ -221,27 +226,53 @@ int reserve_ws(tentaco_csf* h, size_t bytes, hipStream_t st) {
   return TENTACO_OK;
 }
 
-// Adds the shared rows of edge-parallel tiles of NB nonzeros at rank R to the
-// handle's tables, complete for every stream.
-int build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStream_t st) {
+// The wave starts of runs of wn nonzeros, complete for every stream; p null if
+// they cannot be built.
+WalkStarts::Starts build_starts(const CsfDev& B, int64_t wn, hipStream_t st) {
+  WalkStarts::Starts x;
+  x.wn = wn;
+  if (hipMalloc(reinterpret_cast<void**>(&x.p), edge_brk_bytes(B, wn)) != hipSuccess) {
+    (void)hipGetLastError();
+    x.p = nullptr;
+    return x;
+  }
+  const int rc = launch_walk_starts(B, wn, x.p, st);
+  if (hipStreamSynchronize(st) != hipSuccess || rc) {
+    (void)hipGetLastError();
+    clear_error();
+    (void)hipFree(x.p);
+    x.p = nullptr;
+  }
+  return x;
+}
+
+// The shared rows of edge-parallel tiles of NB nonzeros at rank R, complete for
+// every stream; mem null if they cannot be built. (under h->starts.mu, which
+// guards bits)
+WalkStarts::Shared build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStream_t st) {
   const CsfDev B = h->view();
   WalkStarts& s = h->starts;
+  WalkStarts::Shared x;
+  x.nb = NB;
+  x.rank = R;
   const int64_t nblk = (int64_t(B.nnz) + NB - 1) / NB;
   const size_t o_rows = (size_t(nblk) * sizeof(int2) + 255) / 256 * 256;
   const size_t o_w = o_rows + (size_t(nblk) * 2 * sizeof(int32_t) + 255) / 256 * 256;
   const size_t wbytes = size_t(nblk) * 2 * size_t(R) * sizeof(double);
   const int32_t nbits = h->max_crd[0] + 1;
   const size_t bbytes = (size_t(nbits) + 31) / 32 * sizeof(uint32_t);
-  void* mem = nullptr;
   uint32_t* bits = s.bits;
-  hipEvent_t used = nullptr;
-  bool ok = hipMalloc(&mem, o_w + wbytes) == hipSuccess &&
-            hipEventCreateWithFlags(&used, hipEventDisableTiming | hipEventDisableSystemFence) == hipSuccess;
+  bool ok = hipMalloc(&x.mem, o_w + wbytes) == hipSuccess;
+  if (!ok) x.mem = nullptr;
+  ok = ok && hipEventCreateWithFlags(&x.used, hipEventDisableTiming | hipEventDisableSystemFence) ==
+                 hipSuccess;
   if (ok && !bits) {
-    ok = hipMalloc(reinterpret_cast<void**>(&bits), bbytes) == hipSuccess &&
-         hipMemsetAsync(bits, 0, bbytes, st) == hipSuccess && launch_batch_rowbits(B, bits, st) == TENTACO_OK;
+    ok = hipMalloc(reinterpret_cast<void**>(&bits), bbytes) == hipSuccess;
+    if (!ok) bits = nullptr;
+    ok = ok && hipMemsetAsync(bits, 0, bbytes, st) == hipSuccess &&
+         launch_batch_rowbits(B, bits, st) == TENTACO_OK;
   }
-  char* base = static_cast<char*>(mem);
+  char* base = static_cast<char*>(x.mem);
   int2* slots = reinterpret_cast<int2*>(base);
   int32_t* rows = reinterpret_cast<int32_t*>(base + o_rows);
   double* W = reinterpret_cast<double*>(base + o_w);
@@ -251,23 +282,20 @@ int build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStream_t st) {
   if (!ok) {
     (void)hipGetLastError();
     clear_error();
-    (void)hipFree(mem);
-    if (used) (void)hipEventDestroy(used);
+    (void)hipFree(x.mem);
+    x.mem = nullptr;
+    if (x.used) (void)hipEventDestroy(x.used);
+    x.used = nullptr;
     if (!s.bits) (void)hipFree(bits);
-    return TENTACO_ENOMEM;
+    return x;
   }
   s.bits = bits;
-  s.nb[s.ns] = NB;
-  s.rank[s.ns] = R;
-  s.mem[s.ns] = mem;
-  s.used[s.ns] = used;
-  WalkTables& t = s.sh[s.ns++];
-  t.slots = slots;
-  t.rows = rows;
-  t.bits = bits;
-  t.nbits = nbits;
-  t.W = W;
-  return TENTACO_OK;
+  x.t.slots = slots;
+  x.t.rows = rows;
+  x.t.bits = bits;
+  x.t.nbits = nbits;
+  x.t.W = W;
+  return x;
 }
 
 // Workgroups from which an edge-parallel variant's calls share rows in FP64 (AUTO's
@@ -278,49 +306,101 @@ int build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStream_t st) {
 // fill (1.5M nonzeros 28.9 and 33.1), a few in 100 of a call of that many workgroups.
 constexpr int64_t kSharedBlocks = 2048;
 
+// The shared rows that the handle keeps for these, or null (under h->starts.mu).
+WalkStarts::Shared* find_shared(tentaco_csf* h, int64_t NB, int R) {
+  for (auto& x : h->starts.shared)
+    if (x.nb == NB && x.rank == R) return &x;
+  return nullptr;
+}
+
 // What the handle keeps for variant vr at rank R (edge families), or nulls.
 // With `build`, a missing table is built on st and waited for, so that it is
 // complete for every stream; not under capture. A failed build leaves the
 // calls on the brackets they write themselves and on FP32 atomics. rows: shared
-// rows however few the workgroups.
+// rows however few the workgroups. (under h->starts.mu, which the caller holds
+// until a call with shared rows is enqueued)
 WalkTables walk_tables(tentaco_csf* h, const Variant& vr, int R, bool rows, bool build, hipStream_t st) {
   const CsfDev B = h->view();
   WalkTables t;
   if (vr.family == kSliceRow || vr.family < 0 || B.nnz <= 0) return t;
   const int64_t wn = nnz_per_wave(vr, R), NB = nnz_per_block(vr, R);
   WalkStarts& s = h->starts;
-  std::lock_guard<std::mutex> lk(s.mu);
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  int i = 0;
-  while (i < s.n && s.wn[i] != wn) ++i;
-  int j = 0;
-  while (j < s.ns && (s.nb[j] != NB || s.rank[j] != R)) ++j;
+  const int32_t* starts = nullptr;
+  for (const auto& x : s.starts)
+    if (x.wn == wn) starts = x.p;
   const bool ep = vr.family == kEdgeParallel && (rows || B.nnz >= kSharedBlocks * NB);
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   const bool capturing =
-      (ep || i == s.n) &&
+      (ep || !starts) &&
       (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone);
   if (capturing) build = false;
-  if (i == s.n) {
-    if (!build || s.n >= WalkStarts::kTables) return t;
-    int32_t* p = nullptr;
-    if (hipMalloc(reinterpret_cast<void**>(&p), edge_brk_bytes(B, wn)) != hipSuccess) {
-      (void)hipGetLastError();
-      return t;
-    }
-    const int rc = launch_walk_starts(B, wn, p, st);
-    if (hipStreamSynchronize(st) != hipSuccess || rc) {
-      (void)hipFree(p);
-      clear_error();
-      return t;
-    }
-    s.wn[s.n] = wn;
-    s.p[s.n++] = p;
+  if (!starts) {
+    if (!build) return t;
+    const WalkStarts::Starts x = build_starts(B, wn, st);
+    if (!x.p) return t;
+    s.starts.push_back(x);
+    starts = x.p;
   }
-  if (ep && j == s.ns && build && s.ns < WalkStarts::kTables) (void)build_shared_rows(h, NB, R, st);
-  if (ep && j < s.ns && !capturing) t = s.sh[j];
-  t.starts = s.p[i];
+  WalkStarts::Shared* sh = ep && !capturing ? find_shared(h, NB, R) : nullptr;
+  if (ep && !sh && build) {
+    const WalkStarts::Shared x = build_shared_rows(h, NB, R, st);
+    if (x.mem) {
+      if (s.shared.size() >= WalkStarts::kShared + s.beyond) {
+        auto old = std::min_element(s.shared.begin(), s.shared.end(),
+                                    [](const auto& a, const auto& b) { return a.turn < b.turn; });
+        free_shared(*old);
+        s.shared.erase(old);
+      }
+      s.shared.push_back(x);
+      sh = &s.shared.back();
+    }
+  }
+  if (sh) {
+    sh->turn = ++s.turn;
+    t = sh->t;
+  }
+  t.starts = starts;
   return t;
 }
+
+// The tables that a sweep needs for one variant, held while it is timed: those
+// the handle did not keep before are dropped again. (Kept for all the variants of
+// a sweep, 100M nonzeros at rank 64 held 6 GB, and the rows of a later rank's
+// choice found no place.)
+class SweepTables {
+ public:
+  SweepTables(tentaco_csf* h, int v, int R, hipStream_t st) : h_(h) {
+    WalkStarts& s = h->starts;
+    std::lock_guard<std::mutex> lk(s.mu);
+    for (const auto& x : s.starts) starts_.push_back(x.p);
+    for (const auto& x : s.shared) shared_.push_back(x.mem);
+    ++s.beyond;
+    if (variant_fits(h->order, R, v)) (void)walk_tables(h, variant_of(v), R, false, true, st);
+  }
+  ~SweepTables() {
+    WalkStarts& s = h_->starts;
+    std::lock_guard<std::mutex> lk(s.mu);
+    --s.beyond;
+    auto kept = [](const auto& v, auto p) { return std::find(v.begin(), v.end(), p) != v.end(); };
+    for (size_t i = s.shared.size(); i-- > 0;)
+      if (!kept(shared_, s.shared[i].mem)) {
+        free_shared(s.shared[i]);
+        s.shared.erase(s.shared.begin() + ptrdiff_t(i));
+      }
+    for (size_t i = s.starts.size(); i-- > 0;)
+      if (!kept(starts_, s.starts[i].p)) {
+        (void)hipFree(s.starts[i].p);
+        s.starts.erase(s.starts.begin() + ptrdiff_t(i));
+      }
+  }
+  SweepTables(const SweepTables&) = delete;
+  SweepTables& operator=(const SweepTables&) = delete;
+
+ private:
+  tentaco_csf* h_;
+  std::vector<int32_t*> starts_;
+  std::vector<void*> shared_;
+};
 
 int resolve_variant(const tentaco_csf* h, int R, int variant) {
   if (variant == TENTACO_VARIANT_DEFAULT) return default_variant();
@@ -823,6 +903,7 @@ int tentaco_csf_reserve_rows(tentaco_csf* h, int R, int variant, int32_t a_rows)
   const int v = resolve_variant(h, R, variant);
   const Variant tile = tile_of(h, R, variant, v);
   const bool rows = needs_rows(h, R, variant, v, tile);
+  std::lock_guard<std::mutex> lk(h->starts.mu);
   (void)walk_tables(h, tile, R, rows, true, nullptr);
   if (rows) (void)walk_tables(h, variant_of(v), R, false, true, nullptr);
   h->reserved = true;
@@ -921,6 +1002,7 @@ int tentaco_mttkrp_dev(tentaco_csf* h, int R, const float* const* factors_dev, f
   }
   const CsfDev B = h->view();
   const bool rows = needs_rows(h, R, variant, v, vr);
+  std::unique_lock<std::mutex> lk(h->starts.mu);
   WalkTables tables = walk_tables(h, vr, R, rows, !h->reserved, st);
   if (rows && !tables.slots) {  // no FP64 rows here: the variant's own tile
     vr = variant_of(v);
@@ -929,14 +1011,14 @@ int tentaco_mttkrp_dev(tentaco_csf* h, int R, const float* const* factors_dev, f
   rc = reserve_ws(h, mttkrp_workspace_bytes(B, R, vr, a_rows), st);
   if (rc) return rc;
   const bool dense = h->dense_root && a_rows == h->nodes[0];
-  if (!tables.slots) return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws, tables, st);
-  WalkStarts& s = h->starts;
-  std::lock_guard<std::mutex> lk(s.mu);
-  int j = 0;
-  while (s.sh[j].slots != tables.slots) ++j;
-  TT_HIP_CHECK(hipStreamWaitEvent(st, s.used[j], 0));
+  if (!tables.slots) {
+    lk.unlock();
+    return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws, tables, st);
+  }
+  const hipEvent_t used = find_shared(h, nnz_per_block(vr, R), R)->used;
+  TT_HIP_CHECK(hipStreamWaitEvent(st, used, 0));
   rc = launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws, tables, st);
-  TT_HIP_CHECK(hipEventRecord(s.used[j], st));
+  TT_HIP_CHECK(hipEventRecord(used, st));
   return rc;
 }
 
@@ -991,9 +1073,6 @@ static int sweep_impl(tentaco_csf* h, int R, const float* const* factors_dev, fl
       need = std::max(need, mttkrp_workspace_bytes(h->view(), R, variant_of(v), a_rows));
     int rc = reserve_ws(h, need, st);
     if (rc) return rc;
-    for (int v = 0; v < kNumVariants; ++v)
-      if ((!use || use[v]) && variant_fits(h->order, R, v))
-        (void)walk_tables(h, variant_of(v), R, false, true, st);
   }
   hipEvent_t e0, e1;
   TT_HIP_CHECK(hipEventCreate(&e0));
@@ -1026,6 +1105,7 @@ static int sweep_impl(tentaco_csf* h, int R, const float* const* factors_dev, fl
     times_ms[v] = -1.f;
     if (use && !use[v]) continue;
     float p = 0.f;
+    SweepTables tables(h, v, R, st);
     int rc = timed(v, 1, &p);
     if (rc == TENTACO_EUNSUPPORTED) {
       clear_error();
@@ -1048,6 +1128,7 @@ static int sweep_impl(tentaco_csf* h, int R, const float* const* factors_dev, fl
     const float p = times_ms[v];
     if (p < 0.f) continue;
     if (cut > 0.f && p > cut * best_probe) continue;
+    SweepTables tables(h, v, R, st);
     int calls = int(std::ceil(0.1f / std::max(p, 1e-4f)));
     calls = std::min(32, std::max(1, calls));
     for (int r = 0; r < reps; ++r) {

@@ -16,21 +16,29 @@ namespace tt {
 // a search of its own (1.5M nonzeros, 5-mode, rank 16: 67 us a call, 47 us
 // with the table).
 struct WalkStarts {
-  static constexpr int kTables = 8;
+  struct Starts {
+    int64_t wn = 0;
+    int32_t* p = nullptr;
+  };
+  // The shared rows of edge-parallel tiles of nb nonzeros per workgroup at one
+  // rank. A call adds to them, so each waits for the one before on whatever
+  // stream (`used`, recorded behind every call, both under mu); a call under
+  // capture, whose replays no one orders, does without them. At most kShared
+  // are kept, the least recently used goes first (no graph holds them).
+  struct Shared {
+    int64_t nb = 0;
+    int rank = 0;
+    uint64_t turn = 0;
+    void* mem = nullptr;
+    hipEvent_t used = nullptr;
+    WalkTables t;
+  };
+  static constexpr size_t kShared = 8;
   std::mutex mu;
-  int n = 0;
-  int64_t wn[kTables] = {};
-  int32_t* p[kTables] = {};
-  // the shared rows of edge-parallel tiles, by nonzeros per workgroup and rank.
-  // A call adds to them, so each waits for the one before on whatever stream
-  // (`used`, recorded behind every call, both under mu); a call under capture,
-  // whose replays no one orders, does without them
-  int ns = 0;
-  int64_t nb[kTables] = {};
-  int rank[kTables] = {};
-  void* mem[kTables] = {};
-  hipEvent_t used[kTables] = {};
-  WalkTables sh[kTables] = {};
+  size_t beyond = 0;  // entries past kShared that a running sweep may add
+  uint64_t turn = 0;
+  std::vector<Starts> starts;
+  std::vector<Shared> shared;
   uint32_t* bits = nullptr;
 };
 }  // namespace tt

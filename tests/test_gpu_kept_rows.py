@@ -1,0 +1,72 @@
+"""The FP64 rows that a handle keeps for tiles of many workgroups: a sweep, which
+runs every such tile, leaves none behind but the handle's own, and the tiles
+that calls name have them whatever was swept or called before (at most 8 are
+kept, the least recently used goes)."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+import tentaco_amd as tt
+from test_gpu_graph import _hip
+
+pytestmark = pytest.mark.gpu
+
+
+def _free_bytes(hip):
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def _ones(dims, R):
+    return [tt.DeviceArray.from_numpy(np.ones((d, R), np.float32)) for d in dims]
+
+
+def test_sweep_keeps_no_rows(gpu):
+    hip = _hip()
+    n = np.arange(1 << 22)
+    coords = np.stack([n >> 12, n >> 3 & 511, n & 7]).astype(np.int32)
+    dims = (1024, 512, 8)
+    R = 64
+    H = tt.DeviceCsf(tt.Csf.from_coo(dims, coords, np.ones(n.size, np.float32)))
+    fd = _ones(dims[1:], R)
+    A = tt.DeviceArray.empty((dims[0], R))
+    H.reserve(R)
+    H.mttkrp(fd, A, R)
+    tt.synchronize()
+    before = _free_bytes(hip)
+    H.sweep(fd, A, R, reps=1)
+    # the smallest tile's rows alone take 16 R B for each of 131072 workgroups
+    assert before - _free_bytes(hip) < 16 * R * (1 << 22) // 32 // 4
+    H.autotune(fd, A, R, reps=1)
+    assert before - _free_bytes(hip) <= 16 * R * (1 << 22) // 32 + (32 << 20)
+    H.close()
+
+
+def test_later_ranks_have_rows(gpu):
+    # one slice, 2^24 in its first workgroup, then parts that FP32 additions to
+    # 2^24 would lose (see test_gpu_auto_rows)
+    n = np.arange(1 << 20)
+    coords = np.stack([np.zeros_like(n), n // 8, n % 8]).astype(np.int32)
+    vals = np.full(n.size, 2.0 ** -11, np.float32)
+    vals[:4096] = 0
+    vals[0] = 2.0 ** 24
+    dims = (1, n.size // 8, 8)
+    total = np.float32(2.0 ** 24 + (n.size - 4096) / 2048)
+    H = tt.DeviceCsf(tt.Csf.from_coo(dims, coords, vals))
+    names = tt.variants()
+    fd = _ones(dims[1:], 32)
+    A = tt.DeviceArray.empty((1, 32))
+    H.sweep(fd, A, 32, reps=1)
+    ranks = [16, 64, 128, 20, 48, 8, 100, 12, 24, 16, 32]
+    ops = {R: (_ones(dims[1:], R), tt.DeviceArray.empty((1, R))) for R in ranks}
+    for v in ("ep_b128_g4", "ep_b128_g8"):
+        for R in ranks:
+            f, out = ops[R]
+            for _ in range(2):
+                out.upload(np.full((1, R), 7.0, np.float32))
+                H.mttkrp(f, out, R, names.index(v))
+                assert np.all(out.numpy() == total), (v, R)
+    H.close()
