@@ -51,6 +51,8 @@ int upload_array(T** dst, const T* src, int64_t n) {
   return TENTACO_OK;
 }
 
+void free_starts(int32_t* p) { (void)hipFree(p); }
+
 void free_shared(const WalkStarts::Shared& x) {
   if (x.used) {
     (void)hipEventSynchronize(x.used);  // the last call that adds to them
@@ -69,8 +71,8 @@ void free_handle(tentaco_csf* h) {
   (void)hipFree(h->d_vals);
   (void)hipFree(h->ws);
   for (void* w : h->ws_retired) (void)hipFree(w);
-  for (const auto& x : h->starts.starts) (void)hipFree(x.p);
-  for (const auto& x : h->starts.shared) free_shared(x);
+  h->starts.starts.clear(free_starts);
+  h->starts.shared.clear(free_shared);
   (void)hipFree(h->starts.bits);
   for (int m = 0; m < kMaxOrder; ++m) (void)hipFree(h->stage_f[m]);
   (void)hipFree(h->stage_a);
@@ -226,35 +228,32 @@ int reserve_ws(tentaco_csf* h, size_t bytes, hipStream_t st) {
   return TENTACO_OK;
 }
 
-// The wave starts of runs of wn nonzeros, complete for every stream; p null if
-// they cannot be built.
-WalkStarts::Starts build_starts(const CsfDev& B, int64_t wn, hipStream_t st) {
-  WalkStarts::Starts x;
-  x.wn = wn;
-  if (hipMalloc(reinterpret_cast<void**>(&x.p), edge_brk_bytes(B, wn)) != hipSuccess) {
+// The wave starts of runs of wn nonzeros, complete for every stream; whether they
+// could be built.
+bool build_starts(const CsfDev& B, int64_t wn, hipStream_t st, int32_t** out) {
+  int32_t* p = nullptr;
+  if (hipMalloc(reinterpret_cast<void**>(&p), edge_brk_bytes(B, wn)) != hipSuccess) {
     (void)hipGetLastError();
-    x.p = nullptr;
-    return x;
+    return false;
   }
-  const int rc = launch_walk_starts(B, wn, x.p, st);
+  const int rc = launch_walk_starts(B, wn, p, st);
   if (hipStreamSynchronize(st) != hipSuccess || rc) {
     (void)hipGetLastError();
     clear_error();
-    (void)hipFree(x.p);
-    x.p = nullptr;
+    (void)hipFree(p);
+    return false;
   }
-  return x;
+  *out = p;
+  return true;
 }
 
 // The shared rows of edge-parallel tiles of NB nonzeros at rank R, complete for
-// every stream; mem null if they cannot be built. (under h->starts.mu, which
-// guards bits)
-WalkStarts::Shared build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStream_t st) {
+// every stream; whether they could be built. (under h->starts.mu, which guards
+// bits)
+bool build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStream_t st, WalkStarts::Shared* out) {
   const CsfDev B = h->view();
   WalkStarts& s = h->starts;
   WalkStarts::Shared x;
-  x.nb = NB;
-  x.rank = R;
   const int64_t nblk = (int64_t(B.nnz) + NB - 1) / NB;
   const size_t o_rows = (size_t(nblk) * sizeof(int2) + 255) / 256 * 256;
   const size_t o_w = o_rows + (size_t(nblk) * 2 * sizeof(int32_t) + 255) / 256 * 256;
@@ -283,11 +282,9 @@ WalkStarts::Shared build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStrea
     (void)hipGetLastError();
     clear_error();
     (void)hipFree(x.mem);
-    x.mem = nullptr;
     if (x.used) (void)hipEventDestroy(x.used);
-    x.used = nullptr;
     if (!s.bits) (void)hipFree(bits);
-    return x;
+    return false;
   }
   s.bits = bits;
   x.t.slots = slots;
@@ -295,7 +292,8 @@ WalkStarts::Shared build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStrea
   x.t.bits = bits;
   x.t.nbits = nbits;
   x.t.W = W;
-  return x;
+  *out = x;
+  return true;
 }
 
 // Workgroups from which an edge-parallel variant's calls share rows in FP64 (AUTO's
@@ -306,60 +304,42 @@ WalkStarts::Shared build_shared_rows(tentaco_csf* h, int64_t NB, int R, hipStrea
 // fill (1.5M nonzeros 28.9 and 33.1), a few in 100 of a call of that many workgroups.
 constexpr int64_t kSharedBlocks = 2048;
 
-// The shared rows that the handle keeps for these, or null (under h->starts.mu).
-WalkStarts::Shared* find_shared(tentaco_csf* h, int64_t NB, int R) {
-  for (auto& x : h->starts.shared)
-    if (x.nb == NB && x.rank == R) return &x;
-  return nullptr;
-}
+// What walk_tables may build: nothing, what was not tried yet, or anything.
+enum class Build { kNo, kYes, kAgain };
 
 // What the handle keeps for variant vr at rank R (edge families), or nulls.
 // With `build`, a missing table is built on st and waited for, so that it is
-// complete for every stream; not under capture. A failed build leaves the
-// calls on the brackets they write themselves and on FP32 atomics. rows: shared
-// rows however few the workgroups. (under h->starts.mu, which the caller holds
-// until a call with shared rows is enqueued)
-WalkTables walk_tables(tentaco_csf* h, const Variant& vr, int R, bool rows, bool build, hipStream_t st) {
+// complete for every stream; not under capture. One that cannot be built leaves
+// the calls on the brackets they write themselves and on FP32 atomics, and only
+// reserve tries again. rows: shared rows however few the workgroups. used: the
+// event of the shared rows. (under h->starts.mu, which the caller holds until a
+// call with shared rows is enqueued)
+WalkTables walk_tables(tentaco_csf* h, const Variant& vr, int R, bool rows, Build build, hipStream_t st,
+                       hipEvent_t* used = nullptr) {
   const CsfDev B = h->view();
   WalkTables t;
   if (vr.family == kSliceRow || vr.family < 0 || B.nnz <= 0) return t;
   const int64_t wn = nnz_per_wave(vr, R), NB = nnz_per_block(vr, R);
   WalkStarts& s = h->starts;
-  const int32_t* starts = nullptr;
-  for (const auto& x : s.starts)
-    if (x.wn == wn) starts = x.p;
   const bool ep = vr.family == kEdgeParallel && (rows || B.nnz >= kSharedBlocks * NB);
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   const bool capturing =
-      (ep || !starts) &&
+      (ep || build != Build::kNo) &&
       (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone);
-  if (capturing) build = false;
-  if (!starts) {
-    if (!build) return t;
-    const WalkStarts::Starts x = build_starts(B, wn, st);
-    if (!x.p) return t;
-    s.starts.push_back(x);
-    starts = x.p;
-  }
-  WalkStarts::Shared* sh = ep && !capturing ? find_shared(h, NB, R) : nullptr;
-  if (ep && !sh && build) {
-    const WalkStarts::Shared x = build_shared_rows(h, NB, R, st);
-    if (x.mem) {
-      if (s.shared.size() >= WalkStarts::kShared + s.beyond) {
-        auto old = std::min_element(s.shared.begin(), s.shared.end(),
-                                    [](const auto& a, const auto& b) { return a.turn < b.turn; });
-        free_shared(*old);
-        s.shared.erase(old);
-      }
-      s.shared.push_back(x);
-      sh = &s.shared.back();
+  const bool make = build != Build::kNo && !capturing, again = build == Build::kAgain;
+  int32_t** starts = s.starts.get(
+      wn, make, again, [&](int32_t** p) { return build_starts(B, wn, st, p); }, free_starts);
+  if (!starts) return t;
+  if (ep && !capturing) {
+    const WalkStarts::Shared* x = s.shared.get(
+        {NB, R}, make, again, [&](WalkStarts::Shared* y) { return build_shared_rows(h, NB, R, st, y); },
+        free_shared);
+    if (x) {
+      t = x->t;
+      if (used) *used = x->used;
     }
   }
-  if (sh) {
-    sh->turn = ++s.turn;
-    t = sh->t;
-  }
-  t.starts = starts;
+  t.starts = *starts;
   return t;
 }
 
@@ -370,36 +350,23 @@ WalkTables walk_tables(tentaco_csf* h, const Variant& vr, int R, bool rows, bool
 class SweepTables {
  public:
   SweepTables(tentaco_csf* h, int v, int R, hipStream_t st) : h_(h) {
-    WalkStarts& s = h->starts;
-    std::lock_guard<std::mutex> lk(s.mu);
-    for (const auto& x : s.starts) starts_.push_back(x.p);
-    for (const auto& x : s.shared) shared_.push_back(x.mem);
-    ++s.beyond;
-    if (variant_fits(h->order, R, v)) (void)walk_tables(h, variant_of(v), R, false, true, st);
+    std::lock_guard<std::mutex> lk(h->starts.mu);
+    starts_ = h->starts.starts.mark();
+    shared_ = h->starts.shared.mark();
+    if (variant_fits(h->order, R, v)) (void)walk_tables(h, variant_of(v), R, false, Build::kYes, st);
   }
   ~SweepTables() {
-    WalkStarts& s = h_->starts;
-    std::lock_guard<std::mutex> lk(s.mu);
-    --s.beyond;
-    auto kept = [](const auto& v, auto p) { return std::find(v.begin(), v.end(), p) != v.end(); };
-    for (size_t i = s.shared.size(); i-- > 0;)
-      if (!kept(shared_, s.shared[i].mem)) {
-        free_shared(s.shared[i]);
-        s.shared.erase(s.shared.begin() + ptrdiff_t(i));
-      }
-    for (size_t i = s.starts.size(); i-- > 0;)
-      if (!kept(starts_, s.starts[i].p)) {
-        (void)hipFree(s.starts[i].p);
-        s.starts.erase(s.starts.begin() + ptrdiff_t(i));
-      }
+    std::lock_guard<std::mutex> lk(h_->starts.mu);
+    h_->starts.shared.back_to(shared_, free_shared);
+    h_->starts.starts.back_to(starts_, free_starts);
   }
   SweepTables(const SweepTables&) = delete;
   SweepTables& operator=(const SweepTables&) = delete;
 
  private:
   tentaco_csf* h_;
-  std::vector<int32_t*> starts_;
-  std::vector<void*> shared_;
+  decltype(WalkStarts::starts)::Mark starts_;
+  decltype(WalkStarts::shared)::Mark shared_;
 };
 
 int resolve_variant(const tentaco_csf* h, int R, int variant) {
@@ -904,8 +871,8 @@ int tentaco_csf_reserve_rows(tentaco_csf* h, int R, int variant, int32_t a_rows)
   const Variant tile = tile_of(h, R, variant, v);
   const bool rows = needs_rows(h, R, variant, v, tile);
   std::lock_guard<std::mutex> lk(h->starts.mu);
-  (void)walk_tables(h, tile, R, rows, true, nullptr);
-  if (rows) (void)walk_tables(h, variant_of(v), R, false, true, nullptr);
+  (void)walk_tables(h, tile, R, rows, Build::kAgain, nullptr);
+  if (rows) (void)walk_tables(h, variant_of(v), R, false, Build::kAgain, nullptr);
   h->reserved = true;
   return TENTACO_OK;
 }
@@ -1003,10 +970,12 @@ int tentaco_mttkrp_dev(tentaco_csf* h, int R, const float* const* factors_dev, f
   const CsfDev B = h->view();
   const bool rows = needs_rows(h, R, variant, v, vr);
   std::unique_lock<std::mutex> lk(h->starts.mu);
-  WalkTables tables = walk_tables(h, vr, R, rows, !h->reserved, st);
+  const Build build = h->reserved ? Build::kNo : Build::kYes;
+  hipEvent_t used = nullptr;
+  WalkTables tables = walk_tables(h, vr, R, rows, build, st, &used);
   if (rows && !tables.slots) {  // no FP64 rows here: the variant's own tile
     vr = variant_of(v);
-    tables = walk_tables(h, vr, R, false, !h->reserved, st);
+    tables = walk_tables(h, vr, R, false, build, st, &used);
   }
   rc = reserve_ws(h, mttkrp_workspace_bytes(B, R, vr, a_rows), st);
   if (rc) return rc;
@@ -1015,7 +984,6 @@ int tentaco_mttkrp_dev(tentaco_csf* h, int R, const float* const* factors_dev, f
     lk.unlock();
     return launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws, tables, st);
   }
-  const hipEvent_t used = find_shared(h, nnz_per_block(vr, R), R)->used;
   TT_HIP_CHECK(hipStreamWaitEvent(st, used, 0));
   rc = launch_mttkrp(B, F, R, A_dev, a_rows, dense, vr, h->ws, tables, st);
   TT_HIP_CHECK(hipEventRecord(used, st));

@@ -5,6 +5,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "kept.h"
 #include "tuning.h"
 
 namespace tt {
@@ -16,29 +17,23 @@ namespace tt {
 // a search of its own (1.5M nonzeros, 5-mode, rank 16: 67 us a call, 47 us
 // with the table).
 struct WalkStarts {
-  struct Starts {
-    int64_t wn = 0;
-    int32_t* p = nullptr;
-  };
   // The shared rows of edge-parallel tiles of nb nonzeros per workgroup at one
   // rank. A call adds to them, so each waits for the one before on whatever
   // stream (`used`, recorded behind every call, both under mu); a call under
-  // capture, whose replays no one orders, does without them. At most kShared
-  // are kept, the least recently used goes first (no graph holds them).
-  struct Shared {
+  // capture, whose replays no one orders, does without them.
+  struct Tile {
     int64_t nb = 0;
     int rank = 0;
-    uint64_t turn = 0;
+    bool operator==(const Tile& o) const { return nb == o.nb && rank == o.rank; }
+  };
+  struct Shared {
     void* mem = nullptr;
     hipEvent_t used = nullptr;
     WalkTables t;
   };
-  static constexpr size_t kShared = 8;
   std::mutex mu;
-  size_t beyond = 0;  // entries past kShared that a running sweep may add
-  uint64_t turn = 0;
-  std::vector<Starts> starts;
-  std::vector<Shared> shared;
+  Kept<int64_t, int32_t*> starts{8};  // (there are 7 run lengths: none goes while in use)
+  Kept<Tile, Shared> shared{8};       // (no graph holds them)
   uint32_t* bits = nullptr;
 };
 }  // namespace tt
