@@ -891,6 +891,15 @@ static int sweep_impl(tentaco_csf* h, int R, const float* const* factors_dev, fl
                       int32_t a_rows, int reps, float cut, void* stream, const bool* use,
                       float* times_ms);
 
+// Records v for AUTO at rank R, with its tables: calls on a reserved handle build
+// none, and this one may (it was chosen by measuring or by the selector, which
+// allocate too). Not under capture.
+static void choose(tentaco_csf* h, int R, int v, int source, hipStream_t st) {
+  h->tune.set(R, v, source);
+  std::lock_guard<std::mutex> lk(h->starts.mu);
+  (void)walk_tables(h, variant_of(v), R, false, Build::kYes, st);
+}
+
 static int auto_with_selector(tentaco_csf* h, int R, const float* const* factors_dev,
                               float* A_dev, int32_t a_rows, hipStream_t st, int* out) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -908,7 +917,7 @@ static int auto_with_selector(tentaco_csf* h, int R, const float* const* factors
   rc = mlp_select(h->selector, h->order, R, f, &pick, &margin, pred);
   if (rc) return rc;
   if (margin >= h->min_margin) {
-    h->tune.set(R, pick, TENTACO_TUNED_SELECTOR);
+    choose(h, R, pick, TENTACO_TUNED_SELECTOR, st);
     *out = pick;
     return TENTACO_OK;
   }
@@ -928,7 +937,7 @@ static int auto_with_selector(tentaco_csf* h, int R, const float* const* factors
     for (int v = 0; v < kNumVariants; ++v)
       if (t[v] >= 0.f && (best < 0 || t[v] < t[best])) best = v;
     if (best < 0) best = pick;
-    h->tune.set(R, best, TENTACO_TUNED_SELECTOR_TIMED);
+    choose(h, R, best, TENTACO_TUNED_SELECTOR_TIMED, st);
     *out = best;
     return TENTACO_OK;
   }
@@ -1182,7 +1191,7 @@ int tentaco_csf_autotune(tentaco_csf* h, int R, const float* const* factors_dev,
   for (int v = 0; v < kNumVariants; ++v)
     if (t[size_t(v)] >= 0.f && (best_v < 0 || t[size_t(v)] < t[size_t(best_v)])) best_v = v;
   if (best_v < 0) return fail(TENTACO_EUNSUPPORTED, "no variant ran");
-  h->tune.set(R, best_v, TENTACO_TUNED_SWEEP);
+  choose(h, R, best_v, TENTACO_TUNED_SWEEP, static_cast<hipStream_t>(stream));
   if (best) *best = best_v;
   if (times_ms) std::copy(t.begin(), t.end(), times_ms);
   return TENTACO_OK;

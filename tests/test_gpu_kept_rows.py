@@ -70,3 +70,39 @@ def test_later_ranks_have_rows(gpu):
                 H.mttkrp(f, out, R, names.index(v))
                 assert np.all(out.numpy() == total), (v, R)
     H.close()
+
+
+def _lossy_slice():
+    n = np.arange(1 << 20)
+    coords = np.stack([np.zeros_like(n), n // 8, n % 8]).astype(np.int32)
+    vals = np.full(n.size, 2.0 ** -11, np.float32)
+    vals[:4096] = 0
+    vals[0] = 2.0 ** 24
+    dims = (1, n.size // 8, 8)
+    return tt.Csf.from_coo(dims, coords, vals), dims, np.float32(2.0 ** 24 + (n.size - 4096) / 2048)
+
+
+def test_a_choice_after_reserve_has_rows(gpu):
+    """A handle reserved for AUTO, then given a selector: its pick's tables are
+    built with the pick, as later calls build none."""
+    B, dims, total = _lossy_slice()
+    R = 32
+    H = tt.DeviceCsf(B)
+    fd = _ones(dims[1:], R)
+    A = tt.DeviceArray.empty((1, R))
+    pick = tt.variants().index("ep_b128_g4")
+    sel = tt.Selector()
+    p = np.zeros_like(sel.params())
+    p[-len(tt.variants()):] = 1.0  # the output layer's biases
+    p[-len(tt.variants()) + pick] = -1.0
+    sel.set_params(p)
+    assert sel.select(3, R, H.features(R))[0] == pick
+    H.reserve(R)
+    H.set_selector(sel, 0.0)
+    for _ in range(3):
+        A.upload(np.full((1, R), 7.0, np.float32))
+        H.mttkrp(fd, A, R)
+        assert H.tuned(R)[0] == pick
+        assert np.all(A.numpy() == total)
+    H.close()
+    sel.close()
