@@ -3,12 +3,13 @@
 // are the innermost fibers. Replaces ttv_kernel / ttv_csf_gpu_taco
 // (tensor_kernels/ttv_csf_gpu_taco.h:2-121).
 //
-// Three kernels. Up to a million nonzeros without long or empty fibres,
-// ttv_unit_fibres_kernel sums whole fibres by the wave. The unit kernel (below,
-// ttv_unit_kernel) is the main path otherwise: it reads a per-handle fibre-start bitmap instead of searching pos, keeps a
-// window of c in LDS and writes every y entry exactly once (no zero fill, no
-// atomics); with empty fibres its plan indexes the non-empty ones and maps
-// them to output positions. The bracket kernel (ttv_kernel) covers calls
+// Two kernels. The unit kernel (below, ttv_unit_kernel) is the main path: it
+// reads a per-handle fibre-start bitmap instead of searching pos and writes
+// every y entry exactly once (no zero fill, no atomics). It has two forms: up to
+// a million nonzeros without long or empty fibres a wave sums whole fibres;
+// otherwise a wave walks a range of units, with a window of c in LDS, and with
+// empty fibres the plan indexes the non-empty ones and maps them to output
+// positions. The bracket kernel (ttv_kernel) covers calls
 // captured before a handle's plan exists and c beyond 2^30 entries:
 //
 // Work split: each workgroup owns 8*BS consecutive nonzeros, each lane 8
@@ -524,7 +525,7 @@ __global__ __launch_bounds__(kUnitThreads) void ttv_unit_kernel(
                                   });
 }
 
-// The unit kernel for tensors of few units and no long fibre: a wave sums
+// The unit kernel's form for tensors of few units and no long fibre: a wave sums
 // whole fibres, those that start in its unit, so there is no crossing table
 // and no second launch, and waves need neither each other nor a window of c
 // (which L2 serves at these sizes). The unit's products go to LDS in FP64
@@ -532,11 +533,11 @@ __global__ __launch_bounds__(kUnitThreads) void ttv_unit_kernel(
 // what the last fibre has past the unit, is summed by the whole wave. y is
 // written once per entry, coalesced, without atomics (bitwise reproducible).
 // Two dependent rounds of loads bound it: 200k nonzeros, 27k fibres: 5.3 us
-// against 8.5 for ttv_unit_kernel (25 workgroups of 16 waves) and its fold;
+// against 8.5 for the form with the window (25 workgroups of 16 waves) and its fold;
 // the plan takes 0.1 ms, bands another 0.5 to 2 ms.
 // kFibreLane: 8 11.1 us, 16 6.9, 24 6.1, 48 5.3, 100 5.5 (a wave's sum is 12
 // cross-lane moves of latency, a lane's a serial chain).
-// Taken up to kFibreUnits units, us of this and of ttv_unit_kernel (banded
+// Taken up to kFibreUnits units, us of this and of the other form (banded
 // where c is past its window): 24k nonzeros 4.8 and 7.7, 445k 7.0 and 20.9, 1M
 // 6.2 and 8.9 (c of 4000) or 9.2 and 15.4 (c of 150000), 2M 10.1 and 9.7 or
 // 13.8 and 16.3, 4M 17.2 and 14.0 or 24.6 and 19.4. And up to fibres of
@@ -545,7 +546,7 @@ constexpr int kFibreWaves = 4;
 constexpr int32_t kFibreUnits = 2048;
 constexpr int64_t kFibreMax = 2048;
 constexpr int32_t kFibreLane = 48;
-__global__ __launch_bounds__(64 * kFibreWaves) void ttv_unit_fibres_kernel(
+__global__ __launch_bounds__(64 * kFibreWaves) void ttv_unit_kernel(
     const int32_t* __restrict__ crd, const float* __restrict__ vals,
     const uint32_t* __restrict__ flags, const int32_t* __restrict__ unit_fid,
     const int32_t* __restrict__ pos, const float* __restrict__ cv, float* __restrict__ y,
@@ -1640,7 +1641,7 @@ int launch_ttv_units(const CsfDev& B, const TtvPlan& P, const float* c, float* y
   }
   if (P.whole) {
     ktimer_begin(st);
-    ttv_unit_fibres_kernel<<<(P.nunits + kFibreWaves - 1) / kFibreWaves, 64 * kFibreWaves, 0, st>>>(
+    ttv_unit_kernel<<<(P.nunits + kFibreWaves - 1) / kFibreWaves, 64 * kFibreWaves, 0, st>>>(
         B.crd[B.order - 1], B.vals, P.flags, P.unit_fid, B.pos[B.order - 1], c, y,
         B.nodes[B.order - 2], B.nnz, P.nunits);
     TT_HIP_CHECK(hipGetLastError());
