@@ -106,3 +106,66 @@ def test_a_choice_after_reserve_has_rows(gpu):
         assert np.all(A.numpy() == total)
     H.close()
     sel.close()
+
+
+def test_streams_and_a_graph_on_one_handle(gpu):
+    """Calls that add to one handle's rows on two streams wait for each other, and
+    a captured call's replays, which use none, run between them."""
+    from test_gpu_graph import _capture
+
+    hip = _hip()
+    n = np.arange(1 << 18)
+    rng = np.random.default_rng(5)
+    coords = np.stack([n >> 15, n >> 3 & 4095, n & 7]).astype(np.int32)
+    vals = rng.integers(-8, 9, n.size).astype(np.float32)  # whole numbers: every sum is exact
+    dims = (8, 4096, 8)
+    R = 32
+    B = tt.Csf.from_coo(dims, coords, vals)
+    H = tt.DeviceCsf(B)
+    v = tt.variants().index("ep_b128_g4")  # 4096 workgroups
+    facs = [rng.integers(-2, 3, (d, R)).astype(np.float32) for d in dims[1:]]
+    other = [rng.integers(-2, 3, (d, R)).astype(np.float32) for d in dims[1:]]
+
+    def exact(f):
+        ref = np.zeros((8, R))
+        np.add.at(ref, coords[0], vals[:, None].astype(np.float64) * f[0][coords[1]] * f[1][coords[2]])
+        assert np.abs(ref).max() < 2 ** 24
+        return ref
+
+    refs = [exact(facs), exact(other)]
+    ops = [[tt.DeviceArray.from_numpy(x) for x in f] for f in (facs, other)]
+    outs = [[tt.DeviceArray.empty((8, R)) for _ in range(6)] for _ in range(2)]
+    streams = [tt.Stream(), tt.Stream()]
+    H.reserve(R, v)
+    G = tt.DeviceArray.empty((8, R))
+    g, ex = _capture(hip, streams[0], lambda: H.mttkrp(ops[1], G, R, v, stream=streams[0].h))
+    try:
+        for rep in range(3):
+            for o in outs[0] + outs[1] + [G]:
+                o.upload(np.full((8, R), 7.0 + rep, np.float32))
+            for i in range(6):
+                for k in (0, 1):
+                    H.mttkrp(ops[k], outs[k][i], R, v, stream=streams[k].h)
+                # (a replay writes the handle's workspace: it waits for the calls)
+                for s in streams:
+                    s.synchronize()
+                assert hip.hipGraphLaunch(ex, streams[0].h) == 0
+                streams[0].synchronize()
+                assert np.array_equal(G.numpy(), refs[1]), (rep, i)
+            for k in (0, 1):
+                for o in outs[k]:
+                    assert np.array_equal(o.numpy(), refs[k]), (rep, k)
+        for i in range(6):  # without a wait between them
+            for k in (0, 1):
+                H.mttkrp(ops[k], outs[k][i], R, v, stream=streams[k].h)
+        for s in streams:
+            s.synchronize()
+        for k in (0, 1):
+            for o in outs[k]:
+                assert np.array_equal(o.numpy(), refs[k]), k
+    finally:
+        hip.hipGraphExecDestroy(ex)
+        hip.hipGraphDestroy(g)
+    H.close()
+    for s in streams:
+        s.close()
