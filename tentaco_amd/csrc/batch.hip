@@ -27,7 +27,6 @@ struct tentaco_batch {
   float4** d_bnd_rows = nullptr;  // the rows of slices that items share
   double* d_bnd_w = nullptr;      // and their sums
   int2* d_slots = nullptr;
-  size_t brk_bytes = 0;
   tt::BatchLaunch L;
   std::vector<int64_t> h_fill, h_bnd;  // host prefix tables (ntasks + 1)
   // streams and events of the concurrent order launches
@@ -72,7 +71,6 @@ void free_tables(tentaco_batch* b) {
   b->d_bnd_rows = nullptr;
   b->d_bnd_w = nullptr;
   b->d_slots = nullptr;
-  b->brk_bytes = 0;
 }
 
 // The batch runs the edge-parallel walk only: its block-level combine keeps

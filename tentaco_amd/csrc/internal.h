@@ -72,8 +72,8 @@ constexpr int kNumVariants = 2 * kNumGridBlocks * kNumGridGroups + kNumGridBlock
 Variant variant_of(int v);
 int default_variant();
 
-// Lanes that share one factor row for rank R (float4 per lane); 16 for the
-// generic (non-specialised) rank path.
+// Lanes that share one factor row for rank R: 4, 8 or 16, a float4 each and from
+// rank 65 on several (ranks 1 to 3: 4, a column each).
 int lanes_per_row(int R);
 // Nonzeros per lane group of a batch tile of 256 threads that nobody chose,
 // for tasks of nnz nonzeros in all.
@@ -88,10 +88,7 @@ size_t mttkrp_workspace_bytes(const CsfDev& B, int R, const Variant& vr, int32_t
 size_t edge_brk_bytes(const CsfDev& B, int64_t NB);
 size_t ttv_workspace_bytes(const CsfDev& B);
 
-// Enqueue one MTTKRP on `stream`. A (a_rows x R) is fully overwritten;
-// `dense_root` says crd0 == 0..n0-1 with n0 == a_rows (no zero fill needed
-// for the slice-row family). ws must hold mttkrp_workspace_bytes bytes.
-// tables: what a handle keeps for the tile, or nulls.
+// What a handle keeps for a tile, or nulls.
 struct WalkTables {
   // the walk's wave starts for nnz_per_wave(vr, R) (edge families; see
   // launch_walk_starts); null: the call writes the brackets into ws
@@ -106,6 +103,10 @@ struct WalkTables {
   int32_t nbits = 0;
   double* W = nullptr;
 };
+// Enqueue one MTTKRP on `stream`. A (a_rows x R) is fully overwritten;
+// `dense_root` says crd0 == 0..n0-1 with n0 == a_rows (no zero fill needed
+// for the slice-row family). ws must hold mttkrp_workspace_bytes bytes.
+// tables: what the handle keeps for the tile.
 int launch_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A,
                   int32_t a_rows, bool dense_root, const Variant& vr,
                   void* ws, const WalkTables& tables, hipStream_t stream);
@@ -306,8 +307,8 @@ struct BatchLaunch {
   const int64_t* h_bnd_off = nullptr;
   // output rows no root node stores: 0 = zeroed by every launch; 1 =
   // retained (zeroed once by launch_batch_zero_outputs, then left alone, so
-  // a launch writes only the rows the walk stores and the rows of slices at
-  // item boundaries, which it zeroes before their atomics)
+  // a launch writes only the rows the walk stores and, behind it from their FP64
+  // sums, the rows of slices that items share)
   int retain = 0;
   // launches per order run concurrently: each group after the largest on its
   // own stream conc[N] (default priority), forked from and joined back to the

@@ -22,7 +22,9 @@
 //    rows of the shared slices (edge_rows_kernel).
 //  * slice-row (SR): one workgroup per root node, its level-1 children
 //    spread over the workgroup's row groups, rows reduced with xor shuffles
-//    and LDS and stored once. No atomics, no zero fill for a dense root,
+//    and LDS and stored once; for 3-mode short fibres two slices to a workgroup
+//    (slice_pair_kernel) or, for short slices under AUTO, whole slices by the wave
+//    (slice_group_kernel). No atomics, no zero fill for a dense root,
 //    deterministic; balanced only when slices are.
 //
 // Where a wave's run starts (its node at every level) is a table that the
@@ -187,8 +189,8 @@ struct BatchNB {
   int32_t nw[kMaxOrder + 1];
 };
 
-// The rows of sorted tasks [t_lo, t_hi) that the walk does not store, after
-// it: with kRowsFill zero the outputs (quads [q_lo, q_hi)), skipping a row
+// The tasks' rows that the walk does not store, after it: with kRowsFill zero the
+// outputs (quads [0, q_hi)), skipping a row
 // whose bit is set in the task's rowbits, because a root node with nonzeros
 // stores it; with kRowsShared write the rows of the slices that hold an item's
 // first or last nonzero. Several items may share those, so the walk adds to FP64
@@ -197,40 +199,38 @@ struct BatchNB {
 // most of a batch's error: a sweep's worst factor against FP64, 30 seeds, had
 // 7.5e-7 on average and 4.5e-6 at most, now 4.5e-7 and 8.1e-7). With kRowsList (once per configuration) write where the waves of
 // each item start, its slots of FP64 rows, and the list of their output rows
-// (entries [b_lo, b_hi), two per item, null where an earlier item has the
+// (entries [0, b_hi), two per item, null where an earlier item has the
 // slice's). The list depends on the CSFs, outputs and tiles only; finding the
 // rows on every run took 17 us a launch in a CP-ALS sweep over three tensors.
 __global__ __launch_bounds__(256) void batch_rows_kernel(const BatchTaskDev* __restrict__ tasks,
-                                                         int32_t t_lo, int32_t t_hi,
+                                                         int32_t nt,
                                                          const int64_t* __restrict__ fill_off,
-                                                         int64_t q_lo, int64_t q_hi,
+                                                         int64_t q_hi,
                                                          const int64_t* __restrict__ bnd_off,
-                                                         int64_t b_lo, int64_t b_hi,
+                                                         int64_t b_hi,
                                                          int32_t* __restrict__ counter,
-                                                         int n_lo, int n_hi, BatchNB nbs, int R,
+                                                         BatchNB nbs, int R,
                                                          int qshift, int mode,
                                                          float4** __restrict__ bnd_rows,
                                                          double* __restrict__ bnd_w) {
   const int64_t tid = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const int64_t nthr = int64_t(gridDim.x) * blockDim.x;
-  // the work counters of order groups [n_lo, n_hi)
-  if (tid < n_hi - n_lo) counter[n_lo + tid] = 0;
-  const int32_t nt = t_hi - t_lo;
-  if (!(mode & kRowsFill)) q_hi = q_lo;
+  // the work counters of the orders
+  if (tid >= 2 && tid <= kMaxOrder) counter[tid] = 0;
+  if (!(mode & kRowsFill)) q_hi = 0;
   // Zero the outputs as float4 quads (every output holds rows x R floats
   // with R a multiple of 4 and starts 16-byte aligned, which the host
   // checks). Each workgroup takes one contiguous range of quads, finds the
   // task of its first quad with one search and walks forward across task
   // boundaries (empty tasks included).
   // (quad e of a task is in row e >> qshift, with R / 4 == 1 << qshift)
-  const int64_t total_q = q_hi - q_lo;
-  const int64_t per = (total_q + gridDim.x - 1) / gridDim.x;
-  const int64_t q0 = q_lo + int64_t(blockIdx.x) * per;
+  const int64_t per = (q_hi + gridDim.x - 1) / gridDim.x;
+  const int64_t q0 = int64_t(blockIdx.x) * per;
   const int64_t q1 = q0 + per < q_hi ? q0 + per : q_hi;
   if (q0 < q1) {
-    int32_t t = t_lo + upper_index(fill_off + t_lo, nt, q0 << 2);
+    int32_t t = upper_index(fill_off, nt, q0 << 2);
     int64_t base = fill_off[t] >> 2;
-    int64_t next = t + 1 < t_hi ? fill_off[t + 1] >> 2 : q_hi;
+    int64_t next = t + 1 < nt ? fill_off[t + 1] >> 2 : q_hi;
     float4* A4 = reinterpret_cast<float4*>(tasks[t].A);
     const uint32_t* bits = tasks[t].rowbits;
     // four quads per thread and pass, their bitmap words loaded before any
@@ -249,7 +249,7 @@ __global__ __launch_bounds__(256) void batch_rows_kernel(const BatchTaskDev* __r
         if (qq >= next) {
           do {
             ++t;
-            next = t + 1 < t_hi ? fill_off[t + 1] >> 2 : q_hi;
+            next = t + 1 < nt ? fill_off[t + 1] >> 2 : q_hi;
           } while (qq >= next);
           base = fill_off[t] >> 2;
           A4 = reinterpret_cast<float4*>(tasks[t].A);
@@ -270,19 +270,19 @@ __global__ __launch_bounds__(256) void batch_rows_kernel(const BatchTaskDev* __r
     }
   }
   if (mode & kRowsShared) {
-    const int64_t n = (b_hi - b_lo) << (qshift + 1);
+    const int64_t n = b_hi << (qshift + 1);
     for (int64_t i = tid; i < n; i += nthr) {
-      float4* row = bnd_rows[2 * b_lo + (i >> qshift)];
+      float4* row = bnd_rows[i >> qshift];
       if (!row) continue;
-      double2* w = reinterpret_cast<double2*>(bnd_w) + 2 * ((b_lo << (qshift + 1)) + i);
+      double2* w = reinterpret_cast<double2*>(bnd_w) + 2 * i;
       const double2 x = w[0], y = w[1];
       w[0] = w[1] = make_double2(0.0, 0.0);
       row[i & ((1 << qshift) - 1)] = make_float4(float(x.x), float(x.y), float(y.x), float(y.y));
     }
   }
   if (!(mode & kRowsList)) return;
-  for (int64_t i = b_lo + tid; i < b_hi; i += nthr) {
-    const int32_t t = t_lo + upper_index(bnd_off + t_lo, nt, i);
+  for (int64_t i = tid; i < b_hi; i += nthr) {
+    const int32_t t = upper_index(bnd_off, nt, i);
     const BatchTaskDev& T = tasks[t];
     bnd_rows[2 * i] = bnd_rows[2 * i + 1] = nullptr;
     if (T.B.nnz <= 0) continue;
@@ -396,35 +396,25 @@ __global__ __launch_bounds__(256) void edge_rows_kernel(const int32_t* __restric
   }
 }
 
-// batch_rows_kernel over order groups [n_lo, n_hi) (their tasks are consecutive
-// in the task table; groups without tasks add nothing).
-int launch_batch_rows_range(const BatchLaunch& L, int n_lo, int n_hi, hipStream_t st, int mode) {
-  const int32_t t_lo = L.grp_task[n_lo], t_hi = L.grp_task[n_hi];
-  if (t_hi <= t_lo) return TENTACO_OK;
+// batch_rows_kernel over every task with one mode (bits), one launch.
+int launch_batch_rows(const BatchLaunch& L, hipStream_t st, int mode) {
+  if (L.ntasks <= 0) return TENTACO_OK;
   // the host prefix tables hold ntasks + 1 entries (the last is the total)
-  const int64_t f0 = L.h_fill_off[t_lo], f1 = L.h_fill_off[t_hi];
-  const int64_t b0 = L.h_bnd_off[t_lo], b1 = L.h_bnd_off[t_hi];
-  const int64_t fill_quads = (mode & kRowsFill) ? (f1 - f0) >> 2 : 0;
+  const int64_t fill = L.h_fill_off[L.ntasks], bnd = L.h_bnd_off[L.ntasks];
+  const int64_t fill_quads = (mode & kRowsFill) ? fill >> 2 : 0;
   const int qshift = L.R == 16 ? 2 : L.R == 32 ? 3 : 4;  // log2(R / 4), R in {16, 32, 64}
-  const int64_t work = std::max<int64_t>(
-      fill_quads, (mode & kRowsShared) ? (b1 - b0) << (qshift + 1) : b1 - b0);
+  const int64_t work = std::max<int64_t>(fill_quads, (mode & kRowsShared) ? bnd << (qshift + 1) : bnd);
   BatchNB nbs{};
   for (int N = 0; N <= kMaxOrder; ++N) {
     nbs.nb[N] = L.nb[N];
     nbs.nw[N] = std::max(1, L.blk[N] / 64);
   }
-  batch_rows_kernel<<<grid_for(work, 256, 16384), 256, 0, st>>>(
-      L.tasks, t_lo, t_hi, L.fill_off, f0 >> 2, f1 >> 2, L.bnd_off, b0, b1, L.counter, n_lo, n_hi,
-      nbs, L.R, qshift, mode, L.bnd_rows, L.bnd_w);
+  batch_rows_kernel<<<grid_for(work, 256, 16384), 256, 0, st>>>(L.tasks, L.ntasks, L.fill_off, fill >> 2,
+                                                                L.bnd_off, bnd, L.counter, nbs, L.R, qshift,
+                                                                mode, L.bnd_rows, L.bnd_w);
   TT_HIP_CHECK(hipGetLastError());
   return TENTACO_OK;
 }
-
-// Every order group's with the same mode, one launch.
-int launch_batch_rows(const BatchLaunch& L, hipStream_t st, int mode) {
-  return launch_batch_rows_range(L, 2, kMaxOrder + 1, st, mode);
-}
-
 
 // One launch for all orders up to kAllItems items a workgroup of it, and one
 // per order beyond, on queues of their own: long batches keep every queue's

@@ -395,8 +395,7 @@ struct Row {
     }
   }
 
-  // FP64 row output (the edge-serial family's accumulation buffer): store,
-  // and device-scope FP64 atomic add (global_atomic_add_f64).
+  // FP64 row output (the edge-serial family's accumulation buffer).
   __device__ __forceinline__ static void store_f64(double* __restrict__ W, int64_t row, int c,
                                                    int Rr, const V (&a)[NV]) {
     if constexpr (R == 0) {
@@ -419,34 +418,6 @@ struct Row {
         double2* q = reinterpret_cast<double2*>(p + col(j, c, Rr));
         q[0] = make_double2(double(a[j].x), double(a[j].y));
         q[1] = make_double2(double(a[j].z), double(a[j].w));
-      }
-    }
-  }
-
-  __device__ __forceinline__ static void atomic_add_f64(double* __restrict__ W, int64_t row, int c,
-                                                        int Rr, const V (&a)[NV]) {
-    if constexpr (R == 0) {
-      if (c < Rr) unsafeAtomicAdd(W + row * Rr + c, double(a[0]));
-    } else if constexpr (R < 0) {
-      double* p = W + row * Rr;
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        const int own = slot(j, c);
-        const int k = col(j, c, Rr);
-        if (k >= own) unsafeAtomicAdd(p + k, double(a[j].x));
-        if (k + 1 >= own) unsafeAtomicAdd(p + k + 1, double(a[j].y));
-        if (k + 2 >= own) unsafeAtomicAdd(p + k + 2, double(a[j].z));
-        if (k + 3 >= own) unsafeAtomicAdd(p + k + 3, double(a[j].w));
-      }
-    } else {
-      double* p = W + row * R;
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        double* q = p + col(j, c, Rr);
-        unsafeAtomicAdd(q + 0, double(a[j].x));
-        unsafeAtomicAdd(q + 1, double(a[j].y));
-        unsafeAtomicAdd(q + 2, double(a[j].z));
-        unsafeAtomicAdd(q + 3, double(a[j].w));
       }
     }
   }
