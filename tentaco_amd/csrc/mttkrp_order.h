@@ -33,10 +33,14 @@ namespace {
 // kept in LDS (P); the row groups take the piece's nonzeros in turn, each
 // step one leaf row by a global load and one P row from LDS:
 //   acc += (val * M_{N-1}(l, :)) (.) P(fibre, :).
-// (At orders 4 and 5 P is a product of rows itself. Where it leaves the normal
-// numbers, the piece multiplies the rows to the value's leaf row one by one, as
-// they would be without P: 1e30 * 1e-15 * 1e-15 * 1e-15 * 1e-15 is no 0. The
-// check is two instructions a column and fibre.)
+// (At orders 4 and 5 P is a product of rows itself. Where it passes FP32's range,
+// or falls below the normal numbers under a value times leaf row above kSafe, the
+// rows multiply the value's leaf row one by one: 1e30 * 1e-15 * 1e-15 * 1e-15 *
+// 1e-15 is no 0. The check is an instruction a column and product. Products that
+// underflow under ordinary values are common, in CP-ALS on skewed tensors columns
+// concentrate within a few sweeps, and what is lost there is below 2^-139: a sweep
+// of three tensors 560 us without the check, 690 with the rows one by one whenever
+// a product underflows.)
 // Slice changes are uniform over the wave: the row groups' accumulators are
 // summed over the wave and the row is stored.
 //
@@ -388,7 +392,8 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
           open = cur[0] + r;
         }
         open_row = lane_of(wc[0], r);
-        bool staged = N == 2, apart = false;
+        bool staged = N == 2;
+        bool odd = false, over = false;  // P has products that are no normal numbers, or past them
         auto stage = [&]() {
           constexpr int U = NV >= 4 ? 1 : 2;
           float least = FLT_MAX, most = 0.f;
@@ -403,8 +408,8 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
                 V m[NV];
                 RO::load(m, M[k], __shfl(fc[k], f), c, Rr);
                 RO::hmul(p[u], m);
+                RO::extent(p[u], c, Rr, least, most);
               }
-              if constexpr (N > 3) RO::extent(p[u], c, Rr, least, most);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -413,30 +418,73 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
             }
           }
           if constexpr (N > 3) {
-            // a product below the normal numbers, or none: unless all of them
-            // come from a factor that is 0, the piece takes the rows apart
-            if (__builtin_expect(__ballot(!(least >= FLT_MIN && most <= FLT_MAX)) != 0, 0)) {
-              bool lost = false;
-              for (int32_t f0 = fa; f0 < fe; f0 += NGW) {
-                const int32_t f = min(f0 + gi, fe - 1);
-                V p[NV];
-                RO::load(p, M[FL], __shfl(fc[FL], f), c, Rr);
-#pragma unroll
-                for (int k = FL - 1; k >= 1; --k) {
-                  V m[NV];
-                  RO::load(m, M[k], __shfl(fc[k], f), c, Rr);
-                  lost = RO::hmul_lost(p, m) || lost;
-                }
-              }
-              apart = __ballot(lost) != 0;
-            }
+            odd = __ballot(!(least >= FLT_MIN && most <= FLT_MAX)) != 0;
+            over = odd && __ballot(!(most <= FLT_MAX)) != 0;
           }
           wave_lds_sync();
         };
-        // the piece without P: the rows multiply each value's leaf row in turn
-        auto rows_apart = [&]() {
-          for (int32_t t0 = a; t0 < e; t0 += NGW) {
-            const int4 x = rec[min(t0 + gi, e - 1)];
+        // (cold) whether a product of the piece's rows left the normal numbers
+        // where no row has a 0
+        auto product_lost = [&]() {
+          bool l = false;
+          for (int32_t f0 = fa; f0 < fe; f0 += NGW) {
+            const int32_t f = min(f0 + gi, fe - 1);
+            V p[NV];
+            RO::load(p, M[FL], __shfl(fc[FL], f), c, Rr);
+#pragma unroll
+            for (int k = FL - 1; k >= 1; --k) {
+              V m[NV];
+              RO::load(m, M[k], __shfl(fc[k], f), c, Rr);
+              l = RO::hmul_lost(p, m) || l;
+            }
+          }
+          return __ballot(l) != 0;
+        };
+        // (cold) whether a row that multiplies a product of others is above 1
+        auto raised = [&]() {
+          float peak = 0.f;
+          for (int32_t f0 = fa; N > 4 && f0 < fe; f0 += NGW) {
+            V m[NV];
+            RO::load(m, M[1], __shfl(fc[1], min(f0 + gi, fe - 1)), c, Rr);
+            peak = RO::peak(m, peak);
+          }
+          return __ballot(!(peak <= 1.f)) != 0;
+        };
+        // (cold) nonzeros [t, e) with P, unless a value times leaf row is above
+        // kSafe: whether they are added
+        auto with_p = [&](int32_t t) {
+          constexpr int S = SB < 4 ? 2 : 4;
+          V sum[NV];
+#pragma unroll
+          for (int j = 0; j < NV; ++j) sum[j] = acc[j];
+          float peak = 0.f;
+          for (; t < e; t += S * NGW) {
+            V d[S][NV];
+            int4 x[S];
+#pragma unroll
+            for (int u = 0; u < S; ++u) {
+              x[u] = rec[min(t + u * NGW + gi, e - 1)];
+              RO::load(d[u], Mleaf, x[u].x, c, Rr);
+            }
+#pragma unroll
+            for (int u = 0; u < S; ++u) {
+              V p[NV];
+              RO::get(P + (x[u].z - fa) * KR, c, p);
+              RO::scale(d[u], __int_as_float(x[u].y));
+              peak = RO::peak(d[u], peak);
+              RO::hfma_if(t + u * NGW + gi < e, sum, d[u], p);
+            }
+          }
+          if (__ballot(!(peak <= kSafe))) return false;
+#pragma unroll
+          for (int j = 0; j < NV; ++j) acc[j] = sum[j];
+          return true;
+        };
+        // (cold) nonzeros [t, te) without P: the rows multiply each value's leaf
+        // row in turn
+        auto rows_apart = [&](int32_t t, int32_t te) {
+          for (; t < te; t += NGW) {
+            const int4 x = rec[min(t + gi, te - 1)];
             V s[NV];
             RO::load(s, Mleaf, x.x, c, Rr);
             RO::scale(s, __int_as_float(x.y));
@@ -446,14 +494,15 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
               RO::load(m, M[k], __shfl(fc[k], x.z), c, Rr);
               RO::hmul(s, m);
             }
-            if (t0 + gi < e) RO::add(acc, s);
+            if (t + gi < te) RO::add(acc, s);
           }
         };
         // S steps of the row groups from nonzero t0. `whole`: none of them is past
         // the piece, as most are; the batch, whose registers already spill, has
         // no form for those (5-mode 1.5M nonzeros 30.6 us a call without the
         // form and 28.2 with it, the batch of 8 tensors 546 and 580)
-        auto steps = [&](auto S, auto whole, int32_t t0) {
+        // False, with nothing done, where P may not do.
+        auto steps = [&](auto S, auto whole, int32_t t0) -> bool {
           V d[S()][NV];
           auto record = [&](int u) {
             return rec[whole() ? t0 + u * NGW + gi : min(t0 + u * NGW + gi, e - 1)];
@@ -463,7 +512,7 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
           if constexpr (N > 2) {
             if (!staged) stage();
             staged = true;
-            if (N > 3 && apart) return;
+            if (N > 3 && __builtin_expect(odd, 0)) return false;
           }
           // (the records are read again rather than held: 16 registers less)
 #pragma unroll
@@ -484,25 +533,35 @@ __device__ __forceinline__ void edge_block(const CsfDev& B, const FactorsDev& F,
               else RO::axpy_if(ok, acc, w, d[u]);
             }
           }
+          return true;
         };
         for (int32_t t0 = a; t0 < e;) {
+          bool done;
+          int32_t t1;
           if (!Batch && SB >= 4 && e - t0 >= SB * NGW) {
-            steps(std::integral_constant<int, SB>(), std::true_type(), t0);
-            t0 += SB * NGW;
+            done = steps(std::integral_constant<int, SB>(), std::true_type(), t0);
+            t1 = t0 + SB * NGW;
           } else if (SB == 8 && e - t0 > 4 * NGW) {
-            steps(std::integral_constant<int, SB>(), std::false_type(), t0);
-            t0 += SB * NGW;
+            done = steps(std::integral_constant<int, SB>(), std::false_type(), t0);
+            t1 = t0 + SB * NGW;
           } else if (SB >= 4 && e - t0 > 2 * NGW) {
-            steps(std::integral_constant<int, SB < 4 ? SB : 4>(), std::false_type(), t0);
-            t0 += 4 * NGW;
+            done = steps(std::integral_constant<int, SB < 4 ? SB : 4>(), std::false_type(), t0);
+            t1 = t0 + 4 * NGW;
           } else {
-            steps(std::integral_constant<int, 2>(), std::false_type(), t0);
-            t0 += 2 * NGW;
+            done = steps(std::integral_constant<int, 2>(), std::false_type(), t0);
+            t1 = t0 + 2 * NGW;
           }
-          if (N > 3 && __builtin_expect(apart, 0)) {
-            rows_apart();
-            break;
+          if (N > 3 && __builtin_expect(!done, 0)) {
+            t1 = e;
+            if (over || raised() || !with_p(t0)) {
+              if (!product_lost()) {
+                odd = false;
+                continue;
+              }
+              rows_apart(t0, e);
+            }
           }
+          t0 = t1;
         }
         wave_lds_sync();
         a = e;

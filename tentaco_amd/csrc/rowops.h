@@ -57,6 +57,10 @@ __device__ __forceinline__ int32_t wave_scan_add(int32_t x) {
 
 constexpr int kMaxRankAny = 256;
 
+// Where a product of factor rows underflows, a value times leaf row up to this
+// makes of what is lost (2^-150) no more than 2^-140.
+constexpr float kSafe = 1024.f;
+
 template <int R>
 struct Lay {
   static constexpr int K = R < 0 ? -R : R;
@@ -198,6 +202,20 @@ struct Row {
         most = fmaxf(fmaxf(most, fabsf(a[j].z)), fabsf(a[j].w));
       }
     }
+  }
+
+  // The largest magnitude of a's columns and m.
+  __device__ __forceinline__ static float peak(const V (&a)[NV], float m) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      if constexpr (R == 0) {
+        m = fmaxf(m, fabsf(a[j]));
+      } else {
+        m = fmaxf(fmaxf(m, fabsf(a[j].x)), fabsf(a[j].y));
+        m = fmaxf(fmaxf(m, fabsf(a[j].z)), fabsf(a[j].w));
+      }
+    }
+    return m;
   }
 
   // a = a (.) y; whether a column left the normal numbers that neither a nor y

@@ -362,6 +362,82 @@ __global__ __launch_bounds__(512) void inner_leaf_kernel(const int32_t* __restri
         const int32_t a0 = __builtin_amdgcn_readlane(node, 0);
         const int32_t a1 = __builtin_amdgcn_readlane(node, n - 1);
         if (f0 + 64 < uint32_t(total)) fetch(f0 + 64, node_n, l_n, v_n);
+        // (cold) whether a row that multiplies a product of others is above 1
+        auto raised = [&](int32_t f, int32_t fe) {
+          float peak = 0.f;
+          for (; L > 2 && f < fe; f += NGW) {
+            V r[NV];
+            RO::load(r, F.M[L - 1], __shfl(co[L - 1], min(f + gi, fe - 1)), c, Rr);
+            peak = RO::peak(r, peak);
+          }
+          return __ballot(!(peak <= 1.f)) != 0;
+        };
+        // (cold) whether a product of the nodes' rows left the normal numbers where
+        // no row has a 0
+        auto product_lost = [&](int32_t f, int32_t fe) {
+          bool lost = false;
+          for (; f < fe; f += NGW) {
+            const int32_t x = min(f + gi, fe - 1);
+            V p[NV];
+            RO::load(p, F.M[0], __shfl(co[0], x), c, Rr);
+#pragma unroll
+            for (int m = 1; m < L; ++m) {
+              V r[NV];
+              RO::load(r, F.M[m], __shfl(co[m], x), c, Rr);
+              lost = RO::hmul_lost(p, r) || lost;
+            }
+          }
+          return __ballot(lost) != 0;
+        };
+        // (cold) nonzeros [t, e) with P, whose first node is fa; the largest value
+        // times leaf row
+        auto add_p = [&](int32_t fa, int32_t t, int32_t e) {
+          float peak = 0.f;
+          for (; t < e; t += 2 * NGW) {
+            V d[2][NV];
+            int4 x[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              x[u] = rec[min(t + u * NGW + gi, e - 1)];
+              RO::load(d[u], Ml, x[u].x, c, Rr);
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+              V p[NV];
+              RO::get(P + (x[u].z - fa) * KR, c, p);
+              RO::scale(d[u], __int_as_float(x[u].y));
+              peak = RO::peak(d[u], peak);
+              RO::hfma_if(t + u * NGW + gi < e, acc, d[u], p);
+            }
+          }
+          return peak;
+        };
+        // (cold) the same unless that is above kSafe: whether they are added
+        auto with_p = [&](int32_t fa, int32_t t, int32_t e) {
+          V before[NV];
+#pragma unroll
+          for (int i = 0; i < NV; ++i) before[i] = acc[i];
+          if (!__ballot(!(add_p(fa, t, e) <= kSafe))) return true;
+#pragma unroll
+          for (int i = 0; i < NV; ++i) acc[i] = before[i];
+          return false;
+        };
+        // (cold) nonzeros [t, e) without P
+        auto rows_apart = [&](int32_t t, int32_t e) {
+          for (; t < e; t += NGW) {
+            const int4 x = rec[min(t + gi, e - 1)];
+            V s[NV];
+            RO::load(s, Ml, x.x, c, Rr);
+            RO::scale(s, __int_as_float(x.y));
+#pragma unroll
+            for (int m = L - 1; m >= 0; --m) {
+              V r[NV];
+              RO::load(r, F.M[m], __shfl(co[m], x.z), c, Rr);
+              RO::hmul(s, r);
+            }
+            if (t + gi < e) RO::add(acc, s);
+          }
+        };
         // nodes [fa, fe) of the chunk hold its nonzeros [a, e)
         for (int32_t fa = a0, a = 0; a < n;) {
           const int32_t fe = min(fa + PF, a1 + 1);
@@ -378,49 +454,26 @@ __global__ __launch_bounds__(512) void inner_leaf_kernel(const int32_t* __restri
                 V r[NV];
                 RO::load(r, F.M[m], __shfl(co[m], f), c, Rr);
                 RO::hmul(p[u], r);
+                RO::extent(p[u], c, Rr, least, most);
               }
-              if constexpr (L > 1) RO::extent(p[u], c, Rr, least, most);
             }
 #pragma unroll
             for (int u = 0; u < 2; ++u)
               if (g0 + u * NGW + gi < fe) RO::put(P + (g0 + u * NGW + gi - fa) * KR, c, p[u]);
           }
           if constexpr (L > 1) {
-            // as in the edge walk: products that are no normal numbers, other
-            // than by a factor that is 0, and the nonzeros take the rows apart
+            // as in the edge walk: products that are no normal numbers, and the
+            // nonzeros take the rows apart where that matters
             if (__builtin_expect(__ballot(!(least >= FLT_MIN && most <= FLT_MAX)) != 0, 0)) {
-              bool lost = false;
-              for (int32_t g0 = fa; g0 < fe; g0 += NGW) {
-                const int32_t f = min(g0 + gi, fe - 1);
-                V p[NV];
-                RO::load(p, F.M[0], __shfl(co[0], f), c, Rr);
-#pragma unroll
-                for (int m = 1; m < L; ++m) {
-                  V r[NV];
-                  RO::load(r, F.M[m], __shfl(co[m], f), c, Rr);
-                  lost = RO::hmul_lost(p, r) || lost;
-                }
+              wave_lds_sync();
+              if (__ballot(!(most <= FLT_MAX)) != 0 || raised(fa, fe) || !with_p(fa, a, e)) {
+                if (product_lost(fa, fe)) rows_apart(a, e);
+                else add_p(fa, a, e);
               }
-              if (__ballot(lost) != 0) {
-                wave_lds_sync();
-                for (int32_t s0 = a; s0 < e; s0 += NGW) {
-                  const int4 x = rec[min(s0 + gi, e - 1)];
-                  V s[NV];
-                  RO::load(s, Ml, x.x, c, Rr);
-                  RO::scale(s, __int_as_float(x.y));
-#pragma unroll
-                  for (int m = L - 1; m >= 0; --m) {
-                    V r[NV];
-                    RO::load(r, F.M[m], __shfl(co[m], x.z), c, Rr);
-                    RO::hmul(s, r);
-                  }
-                  if (s0 + gi < e) RO::add(acc, s);
-                }
-                wave_lds_sync();
-                a = e;
-                fa = fe;
-                continue;
-              }
+              wave_lds_sync();
+              a = e;
+              fa = fe;
+              continue;
             }
           }
           // (`whole`: no step is past the nonzeros, as most are not)

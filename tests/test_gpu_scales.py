@@ -113,3 +113,62 @@ def test_inner_modes(gpu, sizes, kind, order, R):
         H.mttkrp_level(level, [tt.DeviceArray.from_numpy(f) for f in facs], A, R)
         _check(A.numpy(), ref, level)
         H.close()
+
+
+def _raised(rng, dims, R, mode, sizes):
+    """Order 5: two of the other rows underflow together (1e-23 each) and a third
+    brings their product back (1e22), whichever is multiplied first; or two
+    overflow together and a third holds zeros."""
+    B, facs, _ = _case(rng, dims, R, mode, sizes, "zeros")
+    others = [m for m in range(5) if m != mode]
+    out = []
+    for big in others[:-1]:
+        f = [x.copy() for x in facs]
+        for m in others[:-1]:
+            f[m][f[m] == 0] = 1
+            f[m] *= np.float32(1e22 if m == big else 1e-23)
+        out.append(f)
+        g = [x.copy() for x in facs]
+        for m in others[:-1]:
+            if m != big:
+                g[m][g[m] == 0] = 1
+                g[m] *= np.float32(1e20)
+        g[others[-1]] *= np.float32(1e-38)
+        out.append(g)
+    B.vals = B.vals * np.float32(1e10)  # (the rows one by one, in either order, stay in range)
+    return B, out
+
+
+@pytest.mark.parametrize("R", [3, 16, 32, 50, 64])
+@pytest.mark.parametrize("mode", [0, 1, 2, 3])
+def test_products_lost_on_the_way(gpu, mode, R):
+    rng = np.random.default_rng(R)
+    n = rng.integers(20, 400, 40)
+    dims = [10, 12, 14, 16, 3000]
+    dims[mode] = n.size
+    B, cases = _raised(rng, tuple(dims), R, mode, n)
+    # (the tensor's coordinates and values, from its CSF)
+    node = np.arange(B.nnz)
+    coords = [None] * 4 + [B.crd[4]]
+    for m in range(4, 0, -1):
+        node = np.searchsorted(B.pos[m], node, side="right") - 1
+        coords[m - 1] = B.crd[m - 1][node]
+    H = tt.DeviceCsf(B)
+    A = tt.DeviceArray.empty((dims[mode], R))
+    for facs in cases:
+        p = B.vals.astype(np.float64)[:, None]
+        for m in range(5):
+            if m != mode:
+                p = p * facs[m][coords[m]].astype(np.float64)
+        ref = np.zeros((dims[mode], R))
+        np.add.at(ref, coords[mode], p)
+        used = ref[ref > 0]
+        assert used.max() < 1e37 and used.min() > 1e-30
+        fd = [tt.DeviceArray.from_numpy(f) for f in facs]
+        A.upload(np.full(ref.shape, 7.0, np.float32))
+        if mode == 0:
+            H.mttkrp(fd[1:], A, R, tt.variants().index("ep_b256_g16"))
+        else:
+            H.mttkrp_level(mode, fd, A, R)
+        _check(A.numpy(), ref, mode)
+    H.close()
