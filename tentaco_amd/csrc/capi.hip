@@ -400,23 +400,24 @@ Variant plain_tile(const tentaco_csf* h, int R, int variant, int v) {
   return needs_rows(h, R, variant, v, tile) ? variant_of(v) : tile;
 }
 
-// Load the MTTKRP and TTV code objects on the current device once, before
-// the first timed region (the first launch from a code object loads it,
-// which would otherwise land inside get_gpu_timer_result's region).
-int warm_device() {
+// Load the code objects of MTTKRPs of this order and of TTV on the current device
+// once, before the first timed region (the first launch from a code object loads
+// it, which would otherwise land inside get_gpu_timer_result's region: 3.8 ms for
+// an order's kernels).
+int warm_device(int order) {
   constexpr int kMaxDevices = 64;
   static std::mutex mu;
-  static bool done[kMaxDevices] = {};
+  static bool done[kMaxDevices][kMaxOrder + 1] = {};
   int dev = 0;
   TT_HIP_CHECK(hipGetDevice(&dev));
   if (dev < 0 || dev >= kMaxDevices) return TENTACO_OK;
   std::lock_guard<std::mutex> lk(mu);
-  if (done[dev]) return TENTACO_OK;
-  int rc = warm_mttkrp_module(nullptr);
+  if (done[dev][order]) return TENTACO_OK;
+  int rc = warm_mttkrp_module(order, nullptr);
   if (!rc) rc = warm_ttv_module(nullptr);
   if (rc) return rc;
   TT_HIP_CHECK(hipStreamSynchronize(nullptr));
-  done[dev] = true;
+  done[dev][order] = true;
   return TENTACO_OK;
 }
 
@@ -441,7 +442,7 @@ int upload_csf(const taco_tensor_t* B, int order, tentaco_csf** out) {
   h->order = order;
   bool warm = false;
   int rc = validate_csf(B, order, h, [&](int m, int64_t parents, int64_t nodes) {
-    int r = warm ? TENTACO_OK : warm_device();
+    int r = warm ? TENTACO_OK : warm_device(order);
     warm = true;
     if (!r) r = upload_array(&h->d_pos[m], B->indices[m][0], parents + 1);
     if (!r) r = upload_array(&h->d_crd[m], B->indices[m][1], nodes);
@@ -517,7 +518,7 @@ int host_mttkrp(int order, taco_tensor_t* A, taco_tensor_t* B,
     rc = ensure_expand3(h, nullptr);  // per-handle structure, outside the timed region
     if (rc) return rc;
   }
-  rc = warm_device();
+  rc = warm_device(order);
   if (rc) return rc;
   TT_HIP_CHECK(hipDeviceSynchronize());
   {
@@ -566,7 +567,7 @@ int host_ttv(int order, taco_tensor_t* A, taco_tensor_t* B, taco_tensor_t* c) {
     return fail(TENTACO_ENOMEM, "hipMalloc of y failed");
   rc = ensure_ttv_plan(h, nullptr);  // outside the timed region
   if (rc) return rc;
-  rc = warm_device();
+  rc = warm_device(order);
   if (rc) return rc;
   TT_HIP_CHECK(hipDeviceSynchronize());
   {

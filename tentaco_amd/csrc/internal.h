@@ -333,9 +333,9 @@ int launch_batch_rowbits(const CsfDev& B, uint32_t* bits, hipStream_t stream);
 int batch_occupancy(int family, int block, int R, int32_t NB, int order, int* per_cu);
 int batch_all_occupancy(int block, int R, int* per_cu);
 
-// Launch one empty kernel of the MTTKRP / TTV code objects on `stream`, so
-// that loading them falls outside any later timed region.
-int warm_mttkrp_module(hipStream_t stream);
+// Launch one empty kernel of each code object that an MTTKRP of this order / a
+// TTV uses on `stream`, so that loading them falls outside any later timed region.
+int warm_mttkrp_module(int order, hipStream_t stream);
 int warm_ttv_module(hipStream_t stream);
 
 // Read n floats of buf (16-byte aligned) through the caches on `stream`;

@@ -543,11 +543,16 @@ int launch_pair3(const CsfDev& B, const int32_t* nzr, const int2* pairs, int32_t
   return TENTACO_OK;
 }
 
-int warm_mttkrp_module(hipStream_t st) {
-  // no elements: the launch writes nothing, it only loads the code object
+int warm_mttkrp_module(int order, hipStream_t st) {
+  // no elements: the launches write nothing, they only load the code objects
   fill_kernel<<<1, 256, 0, st>>>(nullptr, 0, 0.f);
   TT_HIP_CHECK(hipGetLastError());
-  return TENTACO_OK;
+  switch (order) {
+    case 2: return order_warm<2>(st);
+    case 3: return order_warm<3>(st);
+    case 4: return order_warm<4>(st);
+    default: return order_warm<5>(st);
+  }
 }
 
 int launch_fill(float* p, int64_t n, float value, hipStream_t st) {

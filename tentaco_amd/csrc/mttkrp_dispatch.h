@@ -32,7 +32,9 @@ __device__ __forceinline__ int32_t upper_index(const int64_t* __restrict__ off, 
 }
 
 // Defined per order N in mttkrp_o<N>.hip; the public launches of internal.h
-// pick the order.
+// pick the order. (order_warm: an empty launch, which loads the code object.)
+template <int N>
+int order_warm(hipStream_t st);
 template <int N>
 int order_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A, int32_t a_rows,
                  bool dense_root, const Variant& vr, void* ws, const WalkTables& wt,

@@ -1636,9 +1636,23 @@ int launch_level_order(const CsfDev& B, const FactorsDev& F, int level, int Rr, 
   return fail(TENTACO_EINVAL, "level %d outside 1..%d", level, N - 1);
 }
 
+// Writes nothing; holds as much scratch as the walk's kernels spill at most, which
+// the runtime allocates for a queue on its first use (1.8 ms).
+__global__ __launch_bounds__(512) void order_warm_kernel(int n) {
+  volatile int32_t spill[40];
+  for (int i = 0; i < n; ++i) spill[(i * 7 + int(threadIdx.x)) % 40] = i;
+}
+
 }  // namespace
 
 // ---- one tensor order's entry points (mttkrp_dispatch.h) --------------------
+template <int N>
+int order_warm(hipStream_t st) {
+  order_warm_kernel<<<2048, 512, 0, st>>>(0);
+  TT_HIP_CHECK(hipGetLastError());
+  return TENTACO_OK;
+}
+
 template <int N>
 int order_mttkrp(const CsfDev& B, const FactorsDev& F, int R, float* A, int32_t a_rows,
                  bool dense_root, const Variant& vr, void* ws, const WalkTables& wt,
@@ -1677,6 +1691,7 @@ int order_batch_occupancy(int family, int block, int R, int32_t NB, int* per_cu)
 
 // Instantiates order N's entry points (one source per order).
 #define TT_INSTANTIATE_ORDER(N)                                                                 \
+  template int tt::order_warm<N>(hipStream_t);                                                  \
   template int tt::order_mttkrp<N>(const CsfDev&, const FactorsDev&, int, float*, int32_t, bool, \
                                    const Variant&, void*, const WalkTables&, hipStream_t);         \
   template int tt::order_level<N>(const CsfDev&, const FactorsDev&, int, int, float*, int32_t,  \
