@@ -1365,8 +1365,9 @@ __global__ __launch_bounds__(128) void slice_pair_kernel(const uint2* __restrict
       V w[NV];
       RO::zero(w);
       RO::axpy(w, vt[u], dr[u]);
-      if (h * 128 + wv * 64 + u * NG + gi < inf.z) RO::hfma(aa, w, cr[u]);
-      else RO::hfma(ab, w, cr[u]);
+      const bool first = h * 128 + wv * 64 + u * NG + gi < inf.z;
+      RO::hfma_if(first, aa, w, cr[u]);
+      RO::hfma_if(!first, ab, w, cr[u]);
     }
   }
   RO::wave_sum(aa);
