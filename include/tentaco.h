@@ -226,9 +226,12 @@ int tentaco_csf_info(const tentaco_csf* h, int* order, int64_t* nnz,
  * table of the waves' start nodes, which later calls read instead of writing
  * brackets (4(order-1) B per 16 to 1024 nonzeros; without a reserve call, the
  * first call of a run length builds it and synchronizes its stream), and for
- * edge-parallel tiles of 2048 workgroups and more the FP64 rows of the slices
- * that workgroups share (16 R B per workgroup; calls outside capture use them,
- * each waiting for the one before on this handle); the
+ * edge-parallel tiles of 2048 workgroups and more, and AUTO's from 300k nonzeros,
+ * the FP64 rows of the slices that workgroups share (16 R B per workgroup, the 8
+ * last used kept; calls outside capture use them, each waiting for the one before
+ * on this handle; AUTO runs its variant's own tile where it has none). Memory
+ * that does not suffice for these leaves calls without them, and only a reserve
+ * call tries again; the
  * edge-serial family also accumulates its rows in FP64 (output rows x R
  * doubles), which keeps atomics on giant slices accurate. For 3-mode
  * handles it also builds the slice-row structures: the expansion (4 B per

@@ -656,11 +656,13 @@ Variant auto_tile(const CsfStats& s, int order, int R, bool paired) {
   // all (12 waves per CU) shorter runs are faster; beyond that more runs only
   // add each one's start and end. Runs hold 32 to 512 nonzeros, in 512-thread
   // workgroups below 300k nonzeros (fewer workgroups to combine) and 256 from
-  // there. From 30M nonzeros on 512 threads and runs of 256 are 2-4% faster
-  // again (100M, 3-mode, rank 32: 2023 us against 2101). Over 60 tensors drawn
-  // from 10k to 12.6M nonzeros, orders 3-5, ranks 7-128, this is 1.08x the
-  // sweep's best edge-parallel tile (geometric mean); the variants' own sizes
-  // (256 x 16 and 512 x 64) are 1.33x.
+  // there. From 30M nonzeros on 512 threads and runs of 256 are 3-6% faster than
+  // 256 and 512 (3-mode, rank 32, us of both: 30M 584 and 601, 45M 899 and 946, 60M
+  // 1246 and 1327; 4-mode 30M, rank 64 1216 and 1250; 40M, rank 16 672 and 705), at
+  // 20M 1 to 3% (403 and 415; rank 64 831 and 843), at 13M the same (244). Over
+  // 60 tensors drawn from 10k to 12.6M nonzeros, orders 3-5, ranks 7-128, the
+  // sizes are 1.08x the sweep's best edge-parallel tile (geometric mean); the
+  // variants' own (256 x 16 and 512 x 64) are 1.33x.
   const int groups = 64 / lanes_per_row(R);
   const bool large = s.nnz >= 30000000;
   const int64_t want = std::max<int64_t>(32, std::min<int64_t>(large ? 256 : 512, s.nnz / 3000));
@@ -675,7 +677,9 @@ bool auto_needs_rows(const CsfStats& s, int R, const Variant& tile, const Varian
   // the error of the variant's tile before the walk (400k nonzeros 2.0 and
   // 1.4e-7 against FP64, 1.5M 5-mode 2.3 and 1.5, at rank 64 3.6 and 2.5; with
   // FP64 rows 1.0, 1.2 and 1.5). Below, it has no more error than that tile
-  // had: 0.99 and 1.13e-7 at 10k, 1.9 and 2.7 at 250k.
+  // had but for a tenth in one of seven (12 seeds each: 1.12 and 1.17e-7 at 10k,
+  // 1.25 and 1.15 at 120k, 4-mode, 1.97 and 2.03 at 200k, 5-mode, 1.02 and 1.20 at
+  // 290k), and the rows' kernel would be 4 of 11 us.
   return tile.family == kEdgeParallel && v.family == kEdgeParallel && s.nnz >= 300000 &&
          nnz_per_block(tile, R) < nnz_per_block(v, R);
 }
