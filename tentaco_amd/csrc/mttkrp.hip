@@ -18,8 +18,9 @@
 //    workgroup's runs are summed in FP64 in LDS (the role of segReduceGroup,
 //    gpu_library.h:295-321), and only the workgroup's first and last slice can
 //    be another's too. ES adds them to FP64 rows of the whole output, EP to the
-//    pre-zeroed output with FP32 atomics or, from 2048 workgroups on, to FP64
-//    rows of the shared slices (edge_rows_kernel).
+//    pre-zeroed output with FP32 atomics or, from 2048 workgroups on and under
+//    AUTO from 300k nonzeros on, to FP64 rows of the shared slices
+//    (edge_rows_kernel).
 //  * slice-row (SR): one workgroup per root node, its level-1 children
 //    spread over the workgroup's row groups, rows reduced with xor shuffles
 //    and LDS and stored once; for 3-mode short fibres two slices to a workgroup
